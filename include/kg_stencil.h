@@ -55,8 +55,11 @@ int kg_h2d(kg_ctx* ctx, void* dst, const void* src, size_t bytes);
 int kg_d2h(kg_ctx* ctx, void* dst, const void* src, size_t bytes);
 int kg_d2d(kg_ctx* ctx, void* dst, const void* src, size_t bytes);
 int kg_sync(kg_ctx* ctx);
-/* Per-launch device timing with HIP events (on by default).  Each launch is
- * bracketed by an event pair from a ring of KG_TIMING_RING pairs. */
+/* Per-launch device timing with HIP events (on by default): the newest
+ * KG_TIMING_RING launches are kept.  A launch that queues behind the previous
+ * one, still running, is timed from that one's end to its own (so it holds the
+ * microsecond or so between them); a launch on an idle stream, or after work
+ * that is not timed, from a start marker of its own. */
 #define KG_TIMING_RING 8192
 int kg_timing_enable(kg_ctx* ctx, int on);
 /* Duration in seconds of the most recent launch (waits for it). */

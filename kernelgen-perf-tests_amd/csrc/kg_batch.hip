@@ -927,14 +927,14 @@ int build_work(kg_batch* b, int only_class = -1, int li_force = 0, int kc_force 
     if (!descs.empty()) {
         std::memcpy(b->h_desc, descs.data(), descs.size() * sizeof(GridDesc));
         KG_HIP(hipMemcpyAsync(b->d_desc, b->h_desc, descs.size() * sizeof(GridDesc),
-                              hipMemcpyHostToDevice, b->ctx->stream));
+                              hipMemcpyHostToDevice, kg_stream(b->ctx)));
     }
     if (!items.empty()) {
         std::memcpy(b->h_items, items.data(), items.size() * sizeof(Item));
         KG_HIP(hipMemcpyAsync(b->d_items, b->h_items, items.size() * sizeof(Item),
-                              hipMemcpyHostToDevice, b->ctx->stream));
+                              hipMemcpyHostToDevice, kg_stream(b->ctx)));
     }
-    KG_HIP(hipEventRecord(b->staged, b->ctx->stream));
+    KG_HIP(hipEventRecord(b->staged, kg_stream(b->ctx)));
     b->nitems = (int)items.size();
     if (only_class < 0) {
         b->pts_per_step = pts;
@@ -950,10 +950,10 @@ int launch_steps(kg_batch* b, int n, bool trial = false)
 {
     for (int s = 0; s < n; s++) {
         if (trial)
-            hipLaunchKernelGGL(batch_k<true>, dim3(b->nwg), dim3(64 * BW), 0, b->ctx->stream,
+            hipLaunchKernelGGL(batch_k<true>, dim3(b->nwg), dim3(64 * BW), 0, kg_stream(b->ctx),
                                b->d_desc, b->d_items, b->nitems, b->d_state);
         else
-            hipLaunchKernelGGL(batch_k<false>, dim3(b->nwg), dim3(64 * BW), 0, b->ctx->stream,
+            hipLaunchKernelGGL(batch_k<false>, dim3(b->nwg), dim3(64 * BW), 0, kg_stream(b->ctx),
                                b->d_desc, b->d_items, b->nitems, b->d_state);
     }
     KG_HIP(hipGetLastError());
@@ -996,12 +996,12 @@ extern "C" int kg_batch_create(kg_ctx* ctx, kg_batch** out)
         delete b;
         return kg_set_error(KG_ERR_NOMEM, "kg_batch_create: %s", hipGetErrorString(e));
     }
-    hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, ctx->stream, b->d_state, 0ull);
+    hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, kg_stream(ctx), b->d_state, 0ull);
     int per_cu = 0, cus = 0;
     KG_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, batch_k<false>, 64 * BW, 0));
     KG_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
     b->nwg = std::max(1, per_cu) * std::max(1, cus);
-    KG_HIP(hipStreamSynchronize(ctx->stream));
+    KG_HIP(hipStreamSynchronize(kg_stream(ctx)));
     *out = b;
     return KG_OK;
 }
@@ -1039,7 +1039,7 @@ extern "C" int kg_batch_remove(kg_batch* b, int id)
     if (id < 0 || id >= (int)b->grids.size() || !b->grids[id].alive)
         return kg_set_error(KG_ERR_INVALID, "kg_batch_remove: no grid %d", id);
     // Work already queued on the stream may still read the levels.
-    KG_HIP(hipStreamSynchronize(b->ctx->stream));
+    KG_HIP(hipStreamSynchronize(kg_stream(b->ctx)));
     HostGrid& g = b->grids[id];
     for (int l = 0; l < nlev_of(g.spec.kind); l++) b->arena.release(g.lev[l], g.level_bytes);
     g.alive = false;
@@ -1062,11 +1062,11 @@ static int level_copy(kg_batch* b, int id, int level, void* host, bool up)
     const size_t h = (size_t)g.spec.ny * g.spec.ns;
     if (up)
         KG_HIP(hipMemcpy2DAsync(g.lev[level], dp, host, w, w, h, hipMemcpyHostToDevice,
-                                b->ctx->stream));
+                                kg_stream(b->ctx)));
     else
         KG_HIP(hipMemcpy2DAsync(host, w, g.lev[level], dp, w, h, hipMemcpyDeviceToHost,
-                                b->ctx->stream));
-    KG_HIP(hipStreamSynchronize(b->ctx->stream));
+                                kg_stream(b->ctx)));
+    KG_HIP(hipStreamSynchronize(kg_stream(b->ctx)));
     return KG_OK;
 }
 
@@ -1117,9 +1117,9 @@ extern "C" int kg_batch_step(kg_batch* b, int nsteps, int use_graph)
             auto it = b->graphs.find(nsteps);
             if (it == b->graphs.end()) {
                 hipGraph_t graph;
-                KG_HIP(hipStreamBeginCapture(b->ctx->stream, hipStreamCaptureModeThreadLocal));
+                KG_HIP(hipStreamBeginCapture(kg_stream(b->ctx), hipStreamCaptureModeThreadLocal));
                 int rc = launch_steps(b, nsteps);
-                hipError_t e = hipStreamEndCapture(b->ctx->stream, &graph);
+                hipError_t e = hipStreamEndCapture(kg_stream(b->ctx), &graph);
                 if (rc) return rc;
                 KG_HIP(e);
                 hipGraphExec_t exec;
@@ -1128,13 +1128,15 @@ extern "C" int kg_batch_step(kg_batch* b, int nsteps, int use_graph)
                 KG_HIP(e);
                 it = b->graphs.emplace(nsteps, exec).first;
             }
-            KG_HIP(hipGraphLaunch(it->second, b->ctx->stream));
-        } else if (int rc = launch_steps(b, nsteps)) {
-            return rc;
+            KG_HIP(hipGraphLaunch(it->second, kg_stream(b->ctx)));
+        } else {   // the last step's kernel carries the stop event
+            if (int rc = launch_steps(b, nsteps - 1)) return rc;
+            kg_launch(b->ctx, batch_k<false>, dim3(b->nwg), dim3(64 * BW), 0, b->d_desc, b->d_items,
+                      b->nitems, b->d_state);
         }
     } else {
         // nothing to compute: the step counter still advances
-        hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, b->ctx->stream, b->d_state,
+        hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, kg_stream(b->ctx), b->d_state,
                            (unsigned long long)(b->steps + nsteps));
     }
     b->steps += nsteps;
@@ -1158,7 +1160,7 @@ extern "C" int kg_batch_tune(kg_batch* b, int reps, int* classes_tuned)
 {
     if (int rc = check_batch(b)) return rc;
     if (reps < 1) reps = 1;
-    KG_HIP(hipStreamSynchronize(b->ctx->stream));
+    KG_HIP(hipStreamSynchronize(kg_stream(b->ctx)));
     std::map<int, int> classes;
     for (const auto& g : b->grids)
         if (g.alive) classes[size_class(g.spec)]++;
@@ -1180,20 +1182,20 @@ extern "C" int kg_batch_tune(kg_batch* b, int reps, int* classes_tuned)
             for (int ki = 0; ki < NKC && !rc; ki++) {
                 if ((rc = build_work(b, c, li, KCS[ki]))) break;
                 b->d_state = scratch;
-                hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, b->ctx->stream, scratch,
+                hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, kg_stream(b->ctx), scratch,
                                    (unsigned long long)b->steps);
                 float ms = 0;
                 rc = launch_steps(b, 1, true);   // warm-up
                 if (!rc) {
-                    hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, b->ctx->stream, scratch,
+                    hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, kg_stream(b->ctx), scratch,
                                        (unsigned long long)b->steps);
-                    (void)hipEventRecord(e0, b->ctx->stream);
+                    (void)hipEventRecord(e0, kg_stream(b->ctx));
                     for (int r = 0; r < reps && !rc; r++) {
-                        hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, b->ctx->stream,
+                        hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, kg_stream(b->ctx),
                                            scratch, (unsigned long long)b->steps);
                         rc = launch_steps(b, 1, true);
                     }
-                    (void)hipEventRecord(e1, b->ctx->stream);
+                    (void)hipEventRecord(e1, kg_stream(b->ctx));
                     if (hipEventSynchronize(e1) != hipSuccess ||
                         hipEventElapsedTime(&ms, e0, e1) != hipSuccess)
                         rc = kg_set_error(KG_ERR_HIP, "kg_batch_tune: event timing failed");
@@ -1273,10 +1275,10 @@ static void fill_grid(kg_batch* b, const HostGrid& g, unsigned long long seed)
         const unsigned long long s =
             bs + (g.spec.kind == KG_KIND_JACOBI2 ? 0ull : (unsigned long long)l);
         if (g.spec.dtype == KG_F64)
-            launch_fill<double>(b->ctx->stream, g.lev[l], g.spec.nx, g.spec.ny, g.spec.ns, g.sy,
+            launch_fill<double>(kg_stream(b->ctx), g.lev[l], g.spec.nx, g.spec.ny, g.spec.ns, g.sy,
                                 g.sz, s, bs, box);
         else
-            launch_fill<float>(b->ctx->stream, g.lev[l], g.spec.nx, g.spec.ny, g.spec.ns, g.sy,
+            launch_fill<float>(kg_stream(b->ctx), g.lev[l], g.spec.nx, g.spec.ny, g.spec.ns, g.sy,
                                g.sz, s, bs, box);
     }
 }
@@ -1297,7 +1299,7 @@ extern "C" int kg_batch_fill(kg_batch* b, unsigned long long seed)
     for (size_t gi = 0; gi < b->grids.size(); gi++)
         if (b->grids[gi].alive) fill_grid(b, b->grids[gi], seed * 7919ull + gi);
     KG_HIP(hipGetLastError());
-    KG_HIP(hipStreamSynchronize(b->ctx->stream));
+    KG_HIP(hipStreamSynchronize(kg_stream(b->ctx)));
     return KG_OK;
 }
 
@@ -1326,7 +1328,7 @@ extern "C" int kg_batch_step_sequential(kg_batch* b, int nsteps)
                 switch (g.spec.kind * NTYPE + g.spec.dtype) {
 #define KG_SEQ_FLAT(K, DT)                                                                      \
     case K * NTYPE + DT:                                                                        \
-        hipLaunchKernelGGL((seq_flat_k<K, DT>), dim3(nkc), dim3(64 * BW), 0, b->ctx->stream, gp, \
+        hipLaunchKernelGGL((seq_flat_k<K, DT>), dim3(nkc), dim3(64 * BW), 0, kg_stream(b->ctx), gp, \
                            step);                                                               \
         break;
                     KG_FLAT_LIST(KG_SEQ_FLAT)
@@ -1342,7 +1344,7 @@ extern "C" int kg_batch_step_sequential(kg_batch* b, int nsteps)
 #define KG_SEQ_ROW2(K, DT)                                                                      \
     case K * NTYPE + DT:                                                                        \
         hipLaunchKernelGGL((seq_rows2_k<K, DT>), dim3((unsigned)(ntx * nty * nzi)), dim3(64 * BW), \
-                           0, b->ctx->stream, gp, ntx, nty, step);                              \
+                           0, kg_stream(b->ctx), gp, ntx, nty, step);                              \
         break;
                     KG_ROW2_LIST(KG_SEQ_ROW2)
 #undef KG_SEQ_ROW2
@@ -1359,7 +1361,7 @@ extern "C" int kg_batch_step_sequential(kg_batch* b, int nsteps)
 #define KG_SEQ_COL(K, DT)                                                                       \
     case K * NTYPE + DT:                                                                        \
         hipLaunchKernelGGL((seq_col_k<K, DT>), dim3((unsigned)(ntx * nty * nkb)), dim3(64 * BW), \
-                           0, b->ctx->stream, gp, ntx, nty, step);                              \
+                           0, kg_stream(b->ctx), gp, ntx, nty, step);                              \
         break;
                     KG_ROW2_LIST(KG_SEQ_COL)
 #undef KG_SEQ_COL
@@ -1375,7 +1377,7 @@ extern "C" int kg_batch_step_sequential(kg_batch* b, int nsteps)
 #define KG_SEQ_PACK(K, DT)                                                                      \
     case K * NTYPE + DT:                                                                        \
         hipLaunchKernelGGL((seq_pack_k<K, DT>), dim3((unsigned)(nty * nkc)), dim3(64 * BW), 0,  \
-                           b->ctx->stream, gp, nty, step);                                      \
+                           kg_stream(b->ctx), gp, nty, step);                                      \
         break;
                     KG_FLAT_LIST(KG_SEQ_PACK)
 #undef KG_SEQ_PACK
@@ -1390,7 +1392,7 @@ extern "C" int kg_batch_step_sequential(kg_batch* b, int nsteps)
 #define KG_SEQ_CASE(K, DT, LI)                                                                  \
     case var_id(K, DT, LI):                                                                     \
         hipLaunchKernelGGL((seq_k<K, DT, LPRS[LI]>), dim3((unsigned)(ntx * nty * nkc)),         \
-                           dim3(64 * BW), 0, b->ctx->stream, gp, ntx, nty, step);               \
+                           dim3(64 * BW), 0, kg_stream(b->ctx), gp, ntx, nty, step);               \
         break;
                 KG_VAR_LIST(KG_SEQ_CASE)
 #undef KG_SEQ_CASE
@@ -1401,7 +1403,7 @@ extern "C" int kg_batch_step_sequential(kg_batch* b, int nsteps)
     KG_HIP(hipGetLastError());
     // keep the device step counter in line with the host's
     b->steps += nsteps;
-    hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, b->ctx->stream, b->d_state,
+    hipLaunchKernelGGL(state_set_k, dim3(1), dim3(64), 0, kg_stream(b->ctx), b->d_state,
                        (unsigned long long)b->steps);
     return kg_launch_end(b->ctx);
 }
@@ -1416,8 +1418,8 @@ extern "C" int kg_fill_uniform(kg_ctx* ctx, int dtype, size_t n, void* p, unsign
     const int nx = (n % 64 == 0) ? 64 : (int)n, ny = (n % 64 == 0) ? (int)(n / 64) : 1;
     if (n && n % 64 && n > (size_t)INT32_MAX)
         return kg_set_error(KG_ERR_INVALID, "kg_fill_uniform: field too large");
-    if (dtype == KG_F64) launch_fill<double>(ctx->stream, p, nx, ny, 1, nx, (long long)nx * ny, seed);
-    else if (dtype == KG_F32) launch_fill<float>(ctx->stream, p, nx, ny, 1, nx, (long long)nx * ny, seed);
+    if (dtype == KG_F64) launch_fill<double>(kg_stream(ctx), p, nx, ny, 1, nx, (long long)nx * ny, seed);
+    else if (dtype == KG_F32) launch_fill<float>(kg_stream(ctx), p, nx, ny, 1, nx, (long long)nx * ny, seed);
     else return kg_set_error(KG_ERR_INVALID, "kg_fill_uniform: dtype %d (F64 or F32)", dtype);
     KG_HIP(hipGetLastError());
     return KG_OK;
@@ -1426,7 +1428,7 @@ extern "C" int kg_fill_uniform(kg_ctx* ctx, int dtype, size_t n, void* p, unsign
 extern "C" int kg_batch_destroy(kg_batch* b)
 {
     if (!b) return KG_OK;
-    if (b->ctx) (void)hipStreamSynchronize(b->ctx->stream);
+    if (b->ctx) (void)hipStreamSynchronize(kg_stream(b->ctx));
     drop_graphs(b);
     b->arena.destroy();
     if (b->d_desc) (void)hipFree(b->d_desc);
@@ -1647,11 +1649,11 @@ extern "C" int kg_serve_run(kg_ctx* ctx, const kg_job* jobs, int njobs, size_t h
                 const HostGrid& g = b->grids[x.id];
                 int lev = 0;
                 if ((rc = kg_batch_newest_level(b, x.id, &lev))) break;
-                if ((rc = kg_field_stats_launch(ctx->stream, j.dtype, (size_t)g.sz * j.ns, g.lev[lev],
+                if ((rc = kg_field_stats_launch(kg_stream(ctx), j.dtype, (size_t)g.sz * j.ns, g.lev[lev],
                                                 j.dtype, g.lev[lev ^ 1], ctx->stats)))
                     break;
                 if (hipMemcpyAsync(check_res + 5 * x.job, stats_res, 5 * sizeof(double),
-                                   hipMemcpyDeviceToHost, ctx->stream) != hipSuccess) {
+                                   hipMemcpyDeviceToHost, kg_stream(ctx)) != hipSuccess) {
                     rc = kg_set_error(KG_ERR_HIP, "kg_serve_run: convergence check copy failed");
                     break;
                 }
@@ -1661,7 +1663,7 @@ extern "C" int kg_serve_run(kg_ctx* ctx, const kg_job* jobs, int njobs, size_t h
             a++;
         }
         if (!rc && issued) {
-            if (hipEventRecord(checked, ctx->stream) != hipSuccess)
+            if (hipEventRecord(checked, kg_stream(ctx)) != hipSuccess)
                 rc = kg_set_error(KG_ERR_HIP, "kg_serve_run: event record failed");
             else
                 checks_live = true;

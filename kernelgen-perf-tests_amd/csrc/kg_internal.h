@@ -2,20 +2,30 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 
 #include <cstddef>
 #include <cstdint>
+#include <tuple>
 #include <type_traits>
 #include <utility>
 
 #include "../../include/kg_stencil.h"
 
+// Slots of the timing ring: one more than the launches it reports, because a
+// launch's start may be the stop event of the launch before it.
+constexpr int KG_RING_SLOTS = KG_TIMING_RING + 1;
+
 struct kg_ctx {
     int device;
-    hipStream_t stream;
-    int timing;                       // per-launch event pairs on/off
-    hipEvent_t* ev_start;             // ring of KG_TIMING_RING pairs
-    hipEvent_t* ev_stop;
+    hipStream_t queue;                // the context's stream; see kg_stream()
+    int timing;                       // per-launch timing on/off
+    hipEvent_t* ev_start;             // ring of KG_RING_SLOTS start markers
+    hipEvent_t* ev_stop;              // and of stop events
+    unsigned char* chained;           // slot's start is the previous slot's stop
+    bool last_is_stop;                // the stream's last operation is the newest stop event
+    bool stopped;                     // the open launch has its stop event on a kernel
+    hipError_t launch_err;            // first error of the open launch's kernels
     long long launches;               // launches recorded so far
     long long drained;                // launches already returned by kg_timing_drain
     const char* last_kernel;          // name of the most recent launch
@@ -46,11 +56,46 @@ int kg_set_error(int code, const char* fmt, ...);
                                 hipGetErrorString(kg_e_), __FILE__, __LINE__);             \
     } while (0)
 
-// Launch bookkeeping used by every entry point: kg_launch_begin() records the
-// start event of the next ring slot, kg_launch_end() checks the launch and
-// records the stop event.
+// The context's stream, for work outside kg_launch(): whatever is put on it
+// must not count as part of the next launch's duration.
+inline hipStream_t kg_stream(kg_ctx* ctx)
+{
+    ctx->last_is_stop = false;
+    return ctx->queue;
+}
+
+// Launch bookkeeping used by every entry point: kg_launch_begin() opens the
+// next ring slot and settles where its duration starts, kg_launch() starts a
+// kernel with the slot's stop event attached (a second kernel of the same
+// entry point takes the event over), kg_launch_end() checks the launch and
+// records the stop event where no kernel carries it (graphs, plain launches).
+//
+// Two event records around every kernel cost the stream two barrier packets:
+// 11.2 us per launch of an empty kernel back to back against 2.7 without
+// timing, 35.6 against 28.1 for a 27.7 us one.  An event attached to the
+// kernel's own packet costs 0-1.3 us (4.0 and 28.1 us per launch); attaching
+// a start event too makes the runtime add a marker and more host work (14 and
+// 32.8 us).  So a launch that queues behind the previous one, still running,
+// starts where that one stops (27.56 us reported for the 27.7 us kernel, 3.60
+// for the empty one's 3.5), and only a launch on an idle stream, where nothing
+// waits for it, records a start marker.
 int kg_launch_begin(kg_ctx* ctx, const char* name);
 int kg_launch_end(kg_ctx* ctx);
+
+template <class... P, class... A>
+inline void kg_launch(kg_ctx* ctx, void (*kern)(P...), dim3 grid, dim3 block, size_t smem, A... a)
+{
+    static_assert(sizeof...(P) == sizeof...(A), "one argument per kernel parameter");
+    std::tuple<P...> args(static_cast<P>(a)...);
+    hipEvent_t stop = ctx->timing ? ctx->ev_stop[ctx->launches % KG_RING_SLOTS] : nullptr;
+    std::apply([&](P&... p) {
+        void* ptr[] = {(void*)&p...};
+        const hipError_t e = hipExtLaunchKernel((const void*)kern, grid, block, ptr, smem, ctx->queue,
+                                                nullptr, stop, 0);
+        if (e != hipSuccess && ctx->launch_err == hipSuccess) ctx->launch_err = e;
+    }, args);
+    ctx->stopped = stop != nullptr;
+}
 
 // Registry of entry-point name -> kernel symbol, for kg_kernel_regcount.
 struct kg_kernel_entry {

@@ -224,13 +224,12 @@ extern "C" int kg_life_u8(kg_ctx* ctx, int nx, int ny, const uint8_t* c0, uint8_
         if (vec) {
             const unsigned nsx = (unsigned)((nx + LIFE_TX - 1) / LIFE_TX);
             const unsigned nb = (unsigned)((ny - 2 + LIFE_YC - 1) / LIFE_YC);
-            hipLaunchKernelGGL(life_u8_k, dim3(nsx * nb), dim3(64 * LIFE_WAVES), 0, ctx->stream, nx,
-                               ny, (int)nsx, c0, c1);
+            kg_launch(ctx, life_u8_k, dim3(nsx * nb), dim3(64 * LIFE_WAVES), 0, nx, ny, (int)nsx,
+                      c0, c1);
         } else {
             const unsigned ntx = (unsigned)((nx - 2 + 255) / 256);
             const unsigned nb = (unsigned)((ny - 2 + LIFE_SLOW_YC - 1) / LIFE_SLOW_YC);
-            hipLaunchKernelGGL(life_u8_cells_k, dim3(ntx * nb), dim3(256), 0, ctx->stream, nx, ny,
-                               (int)ntx, c0, c1);
+            kg_launch(ctx, life_u8_cells_k, dim3(ntx * nb), dim3(256), 0, nx, ny, (int)ntx, c0, c1);
         }
     }
     return kg_launch_end(ctx);

@@ -126,8 +126,8 @@ extern "C" int kg_matmul(kg_ctx* ctx, int nx, int ny, int ns, const double* A, c
     kg_register_kernel("matmul_", (const void*)matmul_k);
     if (int rc = kg_launch_begin(ctx, "matmul_")) return rc;
     if (tiles > 0)
-        hipLaunchKernelGGL(matmul_k, dim3((unsigned)tiles), dim3(64 * KS), 0, ctx->stream,
-                           nx, ny, ns, ti, kq, A, B, C);
+        kg_launch(ctx, matmul_k, dim3((unsigned)tiles), dim3(64 * KS), 0, nx, ny, ns, ti, kq, A, B,
+                  C);
     return kg_launch_end(ctx);
 }
 

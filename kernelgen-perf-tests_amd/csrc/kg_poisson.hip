@@ -549,7 +549,7 @@ int solve(kg_ctx* ctx, int n, const double* f, double* u, double tol, int max_ou
           Workspace& ws, kg_poisson_report* rep, int* outer_out, int* cycles_out, double* rel_out,
           Start&& t_start)
 {
-    hipStream_t st = ctx->stream;
+    hipStream_t st = kg_stream(ctx);
     const int N = n + 1;
     const long long np = (long long)N * N;
     const double h = 1.0 / n;
@@ -646,7 +646,7 @@ extern "C" int kg_poisson_solve(kg_ctx* ctx, int n, const double* f, double* u, 
 {
     if (int rc = check_args(ctx, "kg_poisson_solve", n, MAX_N, f, u)) return rc;
     KG_HIP(hipSetDevice(ctx->device));
-    hipStream_t st = ctx->stream;
+    hipStream_t st = kg_stream(ctx);
     Workspace ws;
     workspace_shape(ws, n);
     const size_t bytes = workspace_bytes(n, kg_stats_scratch_bytes());
@@ -694,7 +694,7 @@ extern "C" int kg_poisson_solve_noalloc(kg_ctx* ctx, int n, const double* f, dou
         return kg_set_error(KG_ERR_STATE, "kg_poisson_solve_noalloc: workspace of device %d not set up",
                             ctx->device);
     KG_HIP(hipSetDevice(ctx->device));
-    hipStream_t st = ctx->stream;
+    hipStream_t st = kg_stream(ctx);
     Workspace ws;
     workspace_shape(ws, n);
     if (workspace_bytes(n, STATS_BYTES) > NOALLOC_BYTES)

@@ -135,16 +135,17 @@ extern "C" int kg_init(kg_ctx** out, int device)
         free(c);
         return kg_set_error(KG_ERR_HIP, "kg_init: cannot read the compute unit count or LDS size");
     }
-    c->ev_start = (hipEvent_t*)calloc(KG_TIMING_RING, sizeof(hipEvent_t));
-    c->ev_stop = (hipEvent_t*)calloc(KG_TIMING_RING, sizeof(hipEvent_t));
-    if (!c->ev_start || !c->ev_stop) {
-        free(c->ev_start); free(c->ev_stop); free(c);
+    c->ev_start = (hipEvent_t*)calloc(KG_RING_SLOTS, sizeof(hipEvent_t));
+    c->ev_stop = (hipEvent_t*)calloc(KG_RING_SLOTS, sizeof(hipEvent_t));
+    c->chained = (unsigned char*)calloc(KG_RING_SLOTS, 1);
+    if (!c->ev_start || !c->ev_stop || !c->chained) {
+        free(c->ev_start); free(c->ev_stop); free(c->chained); free(c);
         return kg_set_error(KG_ERR_INVALID, "kg_init: host allocation failed");
     }
     // Default-priority, non-blocking stream: no implicit sync with the null stream.
-    hipError_t se = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
+    hipError_t se = hipStreamCreateWithFlags(&c->queue, hipStreamNonBlocking);
     if (se != hipSuccess) {
-        free(c->ev_start); free(c->ev_stop); free(c);
+        free(c->ev_start); free(c->ev_stop); free(c->chained); free(c);
         return kg_set_error(KG_ERR_HIP, "hipStreamCreateWithFlags: %s", hipGetErrorString(se));
     }
     c->last_kernel = "";
@@ -184,15 +185,16 @@ extern "C" int kg_destroy(kg_ctx* ctx)
 {
     if (!ctx) return KG_OK;
     (void)hipSetDevice(ctx->device);
-    (void)hipStreamSynchronize(ctx->stream);
-    for (int i = 0; i < KG_TIMING_RING; i++) {
+    (void)hipStreamSynchronize(ctx->queue);
+    for (int i = 0; i < KG_RING_SLOTS; i++) {
         if (ctx->ev_start[i]) (void)hipEventDestroy(ctx->ev_start[i]);
         if (ctx->ev_stop[i]) (void)hipEventDestroy(ctx->ev_stop[i]);
     }
     if (ctx->stats) (void)hipFree(ctx->stats);
-    (void)hipStreamDestroy(ctx->stream);
+    (void)hipStreamDestroy(ctx->queue);
     free(ctx->ev_start);
     free(ctx->ev_stop);
+    free(ctx->chained);
     free(ctx);
     return KG_OK;
 }
@@ -220,7 +222,7 @@ extern "C" int kg_free(kg_ctx* ctx, void* dptr)
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (!dptr) return KG_OK;
     KG_HIP(hipSetDevice(ctx->device));
-    KG_HIP(hipStreamSynchronize(ctx->stream));
+    KG_HIP(hipStreamSynchronize(ctx->queue));
     KG_HIP(hipFree(dptr));
     return KG_OK;
 }
@@ -231,8 +233,9 @@ static int kg_copy(kg_ctx* ctx, void* dst, const void* src, size_t bytes, hipMem
     if (bytes == 0) return KG_OK;
     if (!dst || !src) return kg_set_error(KG_ERR_INVALID, "copy: null pointer");
     KG_HIP(hipSetDevice(ctx->device));
-    KG_HIP(hipMemcpyAsync(dst, src, bytes, kind, ctx->stream));
-    KG_HIP(hipStreamSynchronize(ctx->stream));
+    hipStream_t st = kg_stream(ctx);
+    KG_HIP(hipMemcpyAsync(dst, src, bytes, kind, st));
+    KG_HIP(hipStreamSynchronize(st));
     return KG_OK;
 }
 
@@ -254,7 +257,7 @@ extern "C" int kg_d2d(kg_ctx* ctx, void* dst, const void* src, size_t bytes)
 extern "C" int kg_sync(kg_ctx* ctx)
 {
     if (int rc = kg_check_ctx(ctx)) return rc;
-    KG_HIP(hipStreamSynchronize(ctx->stream));
+    KG_HIP(hipStreamSynchronize(ctx->queue));
     return KG_OK;
 }
 
@@ -263,25 +266,55 @@ int kg_launch_begin(kg_ctx* ctx, const char* name)
 {
     KG_HIP(hipSetDevice(ctx->device));
     ctx->last_kernel = name;
+    ctx->stopped = false;
+    ctx->launch_err = hipSuccess;
     if (!ctx->timing) return KG_OK;
     if (ctx->launches - ctx->drained >= KG_TIMING_RING)
-        ctx->drained = ctx->launches - KG_TIMING_RING + 1;   // oldest pair is reused
-    int slot = (int)(ctx->launches % KG_TIMING_RING);
-    if (!ctx->ev_start[slot]) {
-        KG_HIP(hipEventCreate(&ctx->ev_start[slot]));
-        KG_HIP(hipEventCreate(&ctx->ev_stop[slot]));
+        ctx->drained = ctx->launches - KG_TIMING_RING + 1;   // the oldest slot is reused
+    const int slot = (int)(ctx->launches % KG_RING_SLOTS);
+    if (!ctx->ev_stop[slot]) KG_HIP(hipEventCreate(&ctx->ev_stop[slot]));
+    ctx->chained[slot] = 0;
+    if (ctx->last_is_stop) {
+        const int prev = (int)((ctx->launches - 1) % KG_RING_SLOTS);
+        const hipError_t q = hipEventQuery(ctx->ev_stop[prev]);
+        if (q == hipErrorNotReady) {
+            (void)hipGetLastError();
+            ctx->chained[slot] = 1;
+            return KG_OK;
+        }
+        KG_HIP(q);
     }
-    KG_HIP(hipEventRecord(ctx->ev_start[slot], ctx->stream));
+    // a marker for timing only: no cache write-back at system scope
+    if (!ctx->ev_start[slot])
+        KG_HIP(hipEventCreateWithFlags(&ctx->ev_start[slot], hipEventDisableSystemFence));
+    KG_HIP(hipEventRecord(ctx->ev_start[slot], ctx->queue));
     return KG_OK;
 }
 
 int kg_launch_end(kg_ctx* ctx)
 {
+    KG_HIP(ctx->launch_err);
     KG_HIP(hipGetLastError());
-    if (!ctx->timing) return KG_OK;
-    int slot = (int)(ctx->launches % KG_TIMING_RING);
-    KG_HIP(hipEventRecord(ctx->ev_stop[slot], ctx->stream));
+    if (!ctx->timing) {
+        ctx->last_is_stop = false;
+        return KG_OK;
+    }
+    if (!ctx->stopped)
+        KG_HIP(hipEventRecord(ctx->ev_stop[ctx->launches % KG_RING_SLOTS], ctx->queue));
     ctx->launches++;
+    ctx->last_is_stop = true;
+    return KG_OK;
+}
+
+// Duration of recorded launch l, whose stop event has completed.
+static int kg_launch_time(kg_ctx* ctx, long long l, double* seconds)
+{
+    const int slot = (int)(l % KG_RING_SLOTS);
+    const hipEvent_t from = ctx->chained[slot] ? ctx->ev_stop[(l - 1) % KG_RING_SLOTS]
+                                               : ctx->ev_start[slot];
+    float ms = 0.f;
+    KG_HIP(hipEventElapsedTime(&ms, from, ctx->ev_stop[slot]));
+    *seconds = ms * 1e-3;
     return KG_OK;
 }
 
@@ -298,12 +331,8 @@ extern "C" int kg_last_kernel_time(kg_ctx* ctx, double* seconds)
     if (!seconds) return kg_set_error(KG_ERR_INVALID, "kg_last_kernel_time: null argument");
     if (!ctx->timing || ctx->launches == 0)
         return kg_set_error(KG_ERR_STATE, "kg_last_kernel_time: no timed launch");
-    int slot = (int)((ctx->launches - 1) % KG_TIMING_RING);
-    KG_HIP(hipEventSynchronize(ctx->ev_stop[slot]));
-    float ms = 0.f;
-    KG_HIP(hipEventElapsedTime(&ms, ctx->ev_start[slot], ctx->ev_stop[slot]));
-    *seconds = ms * 1e-3;
-    return KG_OK;
+    KG_HIP(hipEventSynchronize(ctx->ev_stop[(ctx->launches - 1) % KG_RING_SLOTS]));
+    return kg_launch_time(ctx, ctx->launches - 1, seconds);
 }
 
 extern "C" int kg_timing_drain(kg_ctx* ctx, double* seconds, int cap, int* count)
@@ -311,13 +340,10 @@ extern "C" int kg_timing_drain(kg_ctx* ctx, double* seconds, int cap, int* count
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (!count || (cap > 0 && !seconds)) return kg_set_error(KG_ERR_INVALID, "kg_timing_drain: null argument");
     *count = 0;
-    KG_HIP(hipStreamSynchronize(ctx->stream));
+    KG_HIP(hipStreamSynchronize(ctx->queue));
     int n = 0;
     for (long long l = ctx->drained; l < ctx->launches && n < cap; l++, n++) {
-        int slot = (int)(l % KG_TIMING_RING);
-        float ms = 0.f;
-        KG_HIP(hipEventElapsedTime(&ms, ctx->ev_start[slot], ctx->ev_stop[slot]));
-        seconds[n] = ms * 1e-3;
+        if (int rc = kg_launch_time(ctx, l, &seconds[n])) return rc;
     }
     ctx->drained = ctx->launches;
     *count = n;

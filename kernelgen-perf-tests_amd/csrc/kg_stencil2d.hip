@@ -171,8 +171,7 @@ static int launch_row(kg_ctx* ctx, const char* name, int nx, int ny, bool al, Fi
         kg_register_kernel(name, (const void*)kern);
         if (int rc = kg_launch_begin(ctx, name)) return rc;
         if (!g.empty)
-            hipLaunchKernelGGL(kern, dim3(g.blocks), dim3(64 * C::W), 0, ctx->stream, nx, ny,
-                               g.ntx, op);
+            kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * C::W), 0, nx, ny, g.ntx, op);
         return kg_launch_end(ctx);
     };
     if (VEC_EVEN == 2 && nx % 2 == 0 && al) return go(std::integral_constant<int, VEC_EVEN>{});
@@ -238,8 +237,7 @@ static int launch_direct(kg_ctx* ctx, const char* name, int nx, int ny, const vo
     kg_register_kernel(name, (const void*)kern);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
     if (!g.empty)
-        hipLaunchKernelGGL(kern, dim3(g.blocks), dim3(64 * DC::ROWS), 0, ctx->stream, nx, ny,
-                           g.ntx, op);
+        kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * DC::ROWS), 0, nx, ny, g.ntx, op);
     return kg_launch_end(ctx);
 }
 

@@ -477,8 +477,8 @@ static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
         const unsigned blocks = ORD == kgp::KG_ORD_REGION
             ? kgp::region_blocks((unsigned)g.ntx * (unsigned)g.nty, (unsigned)g.nkc) : g.blocks;
         if (!g.empty)
-            hipLaunchKernelGGL(kern, dim3(blocks), dim3(64 * C::W), smem, ctx->stream,
-                               nx, ny, ns, g.ntx, g.nty, kc, op);
+            kg_launch(ctx, kern, dim3(blocks), dim3(64 * C::W), smem, nx, ny, ns, g.ntx, g.nty, kc,
+                      op);
         return kg_launch_end(ctx);
     };
     if (nx % 2 == 0 && al) return go(std::integral_constant<int, 2>{});
@@ -497,8 +497,8 @@ static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
         kg_register_kernel(NAME, (const void*)KERNEL);                                     \
         if (int rc_ = kg_launch_begin(ctx, NAME)) return rc_;                              \
         if (!g.empty)                                                                      \
-            hipLaunchKernelGGL(KERNEL, dim3(g.blocks), dim3(TX, TY), 0, ctx->stream,       \
-                               nx, ny, ns, g.ntx, g.nty, __VA_ARGS__);                     \
+            kg_launch(ctx, KERNEL, dim3(g.blocks), dim3(TX, TY), 0, nx, ny, ns, g.ntx,     \
+                      g.nty, __VA_ARGS__);                                                 \
         return kg_launch_end(ctx);                                                         \
     } while (0)
 
@@ -529,8 +529,8 @@ extern "C" int kg_divergence(kg_ctx* ctx, int nx, int ny, int ns, double alpha, 
         kg_register_kernel("divergence", (const void*)divergence2_k);
         if (int rc = kg_launch_begin(ctx, "divergence")) return rc;
         if (!g.empty)
-            hipLaunchKernelGGL(divergence2_k, dim3(g.blocks), dim3(64 * DIV_ROWS), kg_occupancy_lds(ctx, DIV_OCC, 0), ctx->stream,
-                               nx, ny, ns, g.ntx, g.nty, alpha, beta, gamma, u, ux, uy, uz);
+            kg_launch(ctx, divergence2_k, dim3(g.blocks), dim3(64 * DIV_ROWS), kg_occupancy_lds(ctx,
+                      DIV_OCC, 0), nx, ny, ns, g.ntx, g.nty, alpha, beta, gamma, u, ux, uy, uz);
         return kg_launch_end(ctx);
     }
     KG_LAUNCH3("divergence", divergence_k, 1, 1, alpha, beta, gamma, u, ux, uy, uz);
@@ -587,8 +587,8 @@ extern "C" int kg_uxx1(kg_ctx* ctx, int nx, int ny, int ns, double c1, double c2
         kg_register_kernel("uxx1", (const void*)uxx1_2_k);
         if (int rc = kg_launch_begin(ctx, "uxx1")) return rc;
         if (!g.empty)
-            hipLaunchKernelGGL(uxx1_2_k, dim3(g.blocks), dim3(64 * UXX_ROWS), 0, ctx->stream,
-                               nx, ny, ns, g.ntx, g.nty, c1, c2, dth, u0, u1, d1, xx, xy, xz);
+            kg_launch(ctx, uxx1_2_k, dim3(g.blocks), dim3(64 * UXX_ROWS), 0, nx, ny, ns, g.ntx,
+                      g.nty, c1, c2, dth, u0, u1, d1, xx, xy, xz);
         return kg_launch_end(ctx);
     }
     KG_LAUNCH3("uxx1", uxx1_k, 2, 1, c1, c2, dth, u0, u1, d1, xx, xy, xz);

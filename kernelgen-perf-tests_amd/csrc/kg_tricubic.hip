@@ -153,8 +153,8 @@ static int launch_tricubic(const char* name, kg_ctx* ctx, int nx, int ny, int ns
     kg_register_kernel(name, (const void*)kern);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
     if (!g.empty)
-        hipLaunchKernelGGL(kern, dim3(g.blocks), dim3(TX, TY), 0, ctx->stream,
-                           nx, ny, ns, g.ntx, g.nty, u0, u1, a, b, c);
+        kg_launch(ctx, kern, dim3(g.blocks), dim3(TX, TY), 0, nx, ny, ns, g.ntx, g.nty, u0, u1, a,
+                  b, c);
     return kg_launch_end(ctx);
 }
 

@@ -96,8 +96,8 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
         kg_register_kernel(name, (const void*)kern);
         if (int rc = kg_launch_begin(ctx, name)) return rc;
         if (!g.empty)
-            hipLaunchKernelGGL(kern, dim3(g.blocks), dim3(64 * C::W), 0, ctx->stream,
-                               nx, ny, ns, g.ntx, g.nty, KC, op);
+            kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * C::W), 0, nx, ny, ns, g.ntx, g.nty, KC,
+                      op);
         return kg_launch_end(ctx);
     };
     if (nx % VMAX == 0 && al) return go(std::integral_constant<int, VMAX>{});
@@ -128,8 +128,8 @@ static int launch_rows2(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
     kg_register_kernel(name, (const void*)kern);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
     if (nxi > 0 && nyi > 0 && ns > 0)
-        hipLaunchKernelGGL(kern, dim3((unsigned)ntx * (unsigned)nty * (unsigned)ns), dim3(64 * C::W),
-                           0, ctx->stream, nx, ny, ntx, nty, op);
+        kg_launch(ctx, kern, dim3((unsigned)ntx * (unsigned)nty * (unsigned)ns), dim3(64 * C::W), 0,
+                  nx, ny, ntx, nty, op);
     return kg_launch_end(ctx);
 }
 
@@ -186,8 +186,8 @@ static int launch_colmarch(kg_ctx* ctx, const char* name, int nx, int ny, int ns
     kg_register_kernel(name, (const void*)kern);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
     if (nxi > 0 && nyi > 0 && ns > 0)
-        hipLaunchKernelGGL(kern, dim3((unsigned)ntx * (unsigned)nty * (unsigned)ns), dim3(64 * W),
-                           0, ctx->stream, nx, ny, ns, ntx, nty, YC, op);
+        kg_launch(ctx, kern, dim3((unsigned)ntx * (unsigned)nty * (unsigned)ns), dim3(64 * W), 0,
+                  nx, ny, ns, ntx, nty, YC, op);
     return kg_launch_end(ctx);
 }
 
@@ -331,9 +331,9 @@ extern "C" int kg_convert(kg_ctx* ctx, int dst_dtype, void* dst, int src_dtype, 
 {
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (n && (!dst || !src)) return kg_set_error(KG_ERR_INVALID, "kg_convert: null buffer");
-    if (src_dtype == KG_F64) return convert_to<KG_F64>(ctx->stream, dst_dtype, n, src, dst);
-    if (src_dtype == KG_F32) return convert_to<KG_F32>(ctx->stream, dst_dtype, n, src, dst);
-    if (src_dtype == KG_BF16) return convert_to<KG_BF16>(ctx->stream, dst_dtype, n, src, dst);
+    if (src_dtype == KG_F64) return convert_to<KG_F64>(kg_stream(ctx), dst_dtype, n, src, dst);
+    if (src_dtype == KG_F32) return convert_to<KG_F32>(kg_stream(ctx), dst_dtype, n, src, dst);
+    if (src_dtype == KG_BF16) return convert_to<KG_BF16>(kg_stream(ctx), dst_dtype, n, src, dst);
     return kg_set_error(KG_ERR_INVALID, "kg_convert: unknown dtype %d", src_dtype);
 }
 
@@ -519,11 +519,11 @@ extern "C" int kg_field_stats(kg_ctx* ctx, int dtype, size_t n, const void* x, i
     double* dev = ctx->stats;   // KG_STATS_BLOCKS*5 partials followed by 5 results
     kg_register_kernel("field_stats", (const void*)stats_final_k);
     if ((rc = kg_launch_begin(ctx, "field_stats"))) return rc;
-    if ((rc = kg_field_stats_launch(ctx->stream, dtype, n, x, ref_dtype, ref, dev))) return rc;
+    if ((rc = kg_field_stats_launch(kg_stream(ctx), dtype, n, x, ref_dtype, ref, dev))) return rc;
     if ((rc = kg_launch_end(ctx))) return rc;
     KG_HIP(hipMemcpyAsync(out, dev + KG_STATS_BLOCKS * 5, 5 * sizeof(double), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    KG_HIP(hipStreamSynchronize(ctx->stream));
+                          kg_stream(ctx)));
+    KG_HIP(hipStreamSynchronize(kg_stream(ctx)));
     return KG_OK;
 }
 

@@ -34,12 +34,11 @@ extern "C" int kg_stream_copy(kg_ctx* ctx, double* dst, const double* src, size_
     if (n2 > 0) {
         long long blocks = (n2 + 255) / 256;
         if (blocks > 256 * 64) blocks = 256 * 64;   // 64 workgroups per CU, grid-stride
-        hipLaunchKernelGGL(stream_copy_k, dim3((unsigned)blocks), dim3(256), 0, ctx->stream,
-                           (double2*)dst, (const double2*)src, n2);
+        kg_launch(ctx, stream_copy_k, dim3((unsigned)blocks), dim3(256), 0, (double2*)dst, (const
+                  double2*)src, n2);
     }
     if (n & 1)
-        hipLaunchKernelGGL(stream_copy_tail_k, dim3(1), dim3(64), 0, ctx->stream, dst, src,
-                           (long long)n);
+        kg_launch(ctx, stream_copy_tail_k, dim3(1), dim3(64), 0, dst, src, (long long)n);
     return kg_launch_end(ctx);
 }
 

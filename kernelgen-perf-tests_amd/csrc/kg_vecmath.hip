@@ -222,11 +222,10 @@ int vecadd(kg_ctx* ctx, const char* who, const char* name, int nx, int ny, int n
     if (n > 0) {
         if (al) {
             const long long npc = n / per16<T>();
-            hipLaunchKernelGGL(vecadd_k<T>, dim3(blocks_for(std::max(npc, 1LL))), dim3(256), 0,
-                               ctx->stream, npc, n, w0, w1, w2);
+            kg_launch(ctx, vecadd_k<T>, dim3(blocks_for(std::max(npc, 1LL))), dim3(256), 0, npc, n,
+                      w0, w1, w2);
         } else {
-            hipLaunchKernelGGL(vecadd1_k<T>, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, n, w0,
-                               w1, w2);
+            kg_launch(ctx, vecadd1_k<T>, dim3(blocks_for(n)), dim3(256), 0, n, w0, w1, w2);
         }
     }
     return kg_launch_end(ctx);
@@ -245,11 +244,11 @@ int matvec(kg_ctx* ctx, const char* who, const char* name, int nx, int ny, const
     kg_register_kernel(name, rows16 ? (const void*)matvec_rows_k<T> : (const void*)matvec_k<T>);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
     if (ny > 0 && rows16 && nx > 0)
-        hipLaunchKernelGGL(matvec_rows_k<T>, dim3((ny + 63) / 64), dim3(64), 0, ctx->stream, nx, ny,
-                           A, x, y, (unsigned)a_bytes);
+        kg_launch(ctx, matvec_rows_k<T>, dim3((ny + 63) / 64), dim3(64), 0, nx, ny, A, x, y,
+                  (unsigned)a_bytes);
     else if (ny > 0)
-        hipLaunchKernelGGL(matvec_k<T>, dim3((ny + MV_ROWS - 1) / MV_ROWS), dim3(MV_ROWS), 0,
-                           ctx->stream, nx, ny, A, x, y);
+        kg_launch(ctx, matvec_k<T>, dim3((ny + MV_ROWS - 1) / MV_ROWS), dim3(MV_ROWS), 0, nx, ny, A,
+                  x, y);
     return kg_launch_end(ctx);
 }
 
@@ -270,11 +269,10 @@ int sincos_(kg_ctx* ctx, const char* who, const char* name, int nx, int ny, int 
     if (n > 0) {
         if (al) {
             const long long npc = n / per16<T>();
-            hipLaunchKernelGGL(sincos_k<T>, dim3(blocks_for(std::max(npc, 1LL))), dim3(256), 0,
-                               ctx->stream, npc, n, x, y, xy);
+            kg_launch(ctx, sincos_k<T>, dim3(blocks_for(std::max(npc, 1LL))), dim3(256), 0, npc, n,
+                      x, y, xy);
         } else {
-            hipLaunchKernelGGL(sincos1_k<T>, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, n, x,
-                               y, xy);
+            kg_launch(ctx, sincos1_k<T>, dim3(blocks_for(n)), dim3(256), 0, n, x, y, xy);
         }
     }
     return kg_launch_end(ctx);
