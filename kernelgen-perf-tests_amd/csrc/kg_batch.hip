@@ -613,6 +613,25 @@ void launch_fill(hipStream_t st, void* p, int nx, int ny, int ns, long long sy, 
                            sy, sz, seed, bseed, box);
 }
 
+// Rows of nx values between a padded level (row pitch sy) and a dense block,
+// one value per lane and turn; n = rows * nx values.  Moved by a strided host
+// copy instead, every row is a transfer of its own: 7 us a row (840 ms for the
+// 117,000 rows of 40 grids up to 128 points wide, 6 M values, that the packed
+// blocks bring to the host in 9 ms).  The rows are only touched once and the
+// link to the host is a hundred times slower than HBM, so the simplest mapping
+// does.
+template <class S, bool PACK_ROWS>
+__global__ __launch_bounds__(256)
+void pitch_rows_k(unsigned n, unsigned nx, long long sy, S* __restrict__ level, S* __restrict__ dense)
+{
+    for (unsigned e = blockIdx.x * 256u + threadIdx.x; e < n; e += gridDim.x * 256u) {
+        const unsigned r = e / nx;
+        S* p = level + (long long)r * sy + (e - r * nx);
+        if (PACK_ROWS) dense[e] = *p;
+        else *p = dense[e];
+    }
+}
+
 __global__ void state_set_k(BatchState* st, unsigned long long step)
 {
     if (threadIdx.x == 0) {
@@ -752,6 +771,9 @@ struct kg_batch {
     Item* h_items = nullptr;
     size_t h_item_cap = 0;
     hipEvent_t staged = nullptr;
+    // dense rows on their way to or from the host (level_copy)
+    char* rows = nullptr;
+    size_t rows_cap = 0;
 };
 
 namespace {
@@ -1048,6 +1070,41 @@ extern "C" int kg_batch_remove(kg_batch* b, int id)
     return KG_OK;
 }
 
+// The dense block of level_copy: at least `bytes`, or KG_ROWS_MAX where a level
+// is larger (it then moves block by block).  Kept with the batch; without
+// memory for it the old one stays, or none.
+constexpr size_t KG_ROWS_MAX = (size_t)64 << 20;
+
+static int rows_reserve(kg_batch* b, size_t bytes)
+{
+    bytes = std::min(bytes, KG_ROWS_MAX);
+    if (b->rows_cap >= bytes) return KG_OK;
+    KG_HIP(hipSetDevice(b->ctx->device));
+    char* p = nullptr;
+    if (hipMalloc((void**)&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return KG_OK;
+    }
+    if (b->rows) KG_HIP(hipFree(b->rows));
+    b->rows = p;
+    b->rows_cap = bytes;
+    return KG_OK;
+}
+
+template <class S>
+static void launch_pitch(hipStream_t st, bool up, size_t rows, int nx, long long sy, char* level,
+                         char* dense)
+{
+    const unsigned n = (unsigned)(rows * (size_t)nx);   // at most KG_ROWS_MAX / sizeof(S)
+    const unsigned blocks = std::min((n + 255u) / 256u, 256u * 8u);
+    if (up)
+        hipLaunchKernelGGL((pitch_rows_k<S, false>), dim3(blocks), dim3(256), 0, st, n, (unsigned)nx,
+                           sy, (S*)level, (S*)dense);
+    else
+        hipLaunchKernelGGL((pitch_rows_k<S, true>), dim3(blocks), dim3(256), 0, st, n, (unsigned)nx,
+                           sy, (S*)level, (S*)dense);
+}
+
 static int level_copy(kg_batch* b, int id, int level, void* host, bool up)
 {
     if (int rc = check_batch(b)) return rc;
@@ -1060,13 +1117,33 @@ static int level_copy(kg_batch* b, int id, int level, void* host, bool up)
     const size_t es = g.spec.dtype == KG_F64 ? 8 : 4;
     const size_t w = (size_t)g.spec.nx * es, dp = (size_t)g.sy * es;
     const size_t h = (size_t)g.spec.ny * g.spec.ns;
-    if (up)
-        KG_HIP(hipMemcpy2DAsync(g.lev[level], dp, host, w, w, h, hipMemcpyHostToDevice,
-                                kg_stream(b->ctx)));
-    else
-        KG_HIP(hipMemcpy2DAsync(host, w, g.lev[level], dp, w, h, hipMemcpyDeviceToHost,
-                                kg_stream(b->ctx)));
-    KG_HIP(hipStreamSynchronize(kg_stream(b->ctx)));
+    hipStream_t st = kg_stream(b->ctx);
+    const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
+    if (w == dp) {   // rows without padding: the level is dense
+        void* lev = g.lev[level];
+        KG_HIP(hipMemcpyAsync(up ? lev : host, up ? host : lev, w * h, kind, st));
+        KG_HIP(hipStreamSynchronize(st));
+        return KG_OK;
+    }
+    if (int rc = rows_reserve(b, w * h)) return rc;
+    if (b->rows_cap < w) {   // no memory for even one row: row by row
+        KG_HIP(up ? hipMemcpy2DAsync(g.lev[level], dp, host, w, w, h, kind, st)
+                  : hipMemcpy2DAsync(host, w, g.lev[level], dp, w, h, kind, st));
+        KG_HIP(hipStreamSynchronize(st));
+        return KG_OK;
+    }
+    const size_t per = b->rows_cap / w;   // rows per block
+    for (size_t r = 0; r < h; r += per) {
+        const size_t nr = std::min(per, h - r);
+        char* lev = (char*)g.lev[level] + r * dp;
+        char* dense = (char*)host + r * w;
+        if (up) KG_HIP(hipMemcpyAsync(b->rows, dense, nr * w, kind, st));
+        if (g.spec.dtype == KG_F64) launch_pitch<double>(st, up, nr, g.spec.nx, g.sy, lev, b->rows);
+        else launch_pitch<float>(st, up, nr, g.spec.nx, g.sy, lev, b->rows);
+        KG_HIP(hipGetLastError());
+        if (!up) KG_HIP(hipMemcpyAsync(dense, b->rows, nr * w, kind, st));
+    }
+    KG_HIP(hipStreamSynchronize(st));
     return KG_OK;
 }
 
@@ -1437,6 +1514,7 @@ extern "C" int kg_batch_destroy(kg_batch* b)
     if (b->h_desc) (void)hipHostFree(b->h_desc);
     if (b->h_items) (void)hipHostFree(b->h_items);
     if (b->staged) (void)hipEventDestroy(b->staged);
+    if (b->rows) (void)hipFree(b->rows);
     delete b;
     return KG_OK;
 }

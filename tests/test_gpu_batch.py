@@ -280,3 +280,21 @@ def test_batch_column_march_2d_kinds(gpu_ctx, kgmod, dtype):
         b.close()
     for o in outs[1:]:
         assert o == outs[0]
+
+
+@pytest.mark.parametrize("dtype,dims", [(F64, (1, 1, 1)), (F64, (17, 3, 2)), (F32, (19, 5, 3)),
+                                        (F32, (64, 9, 4)), (F64, (1001, 1000, 9)),
+                                        (F32, (4099, 4097, 1))])
+def test_batch_levels_round_trip(batch, dtype, dims):
+    """Rows with and without padding, one value, and levels larger than the
+    block they move through; the other level stays as it was."""
+    t = np.float64 if dtype == F64 else np.float32
+    nx, ny, ns = dims
+    rng = np.random.default_rng(5)
+    gid = batch.add("laplacian", dtype, dims, COEFS["laplacian"])
+    lv = [rng.uniform(-1, 1, (ns, ny, nx)).astype(t) for _ in range(2)]
+    for level, a in enumerate(lv):
+        batch.upload(gid, level, a)
+    for level in (1, 0, 1):
+        got = batch.download(gid, level)
+        assert np.array_equal(got, lv[level])
