@@ -324,8 +324,9 @@ int kg_batch_info(kg_batch* b, double* points_per_step, double* bytes_per_step,
  * the flat body (lanes_per_row 0: points swept from cache, for small grids)
  * -- with 8/16/32/64 planes per tile, over reps launches on the batch's own
  * grids, and keeps the fastest.  Untuned classes take the direct row body
- * (jacobi2, life2), packed rows (rows up to 64 lanes) or 64 lanes per row.  Grid
- * contents are preserved. */
+ * (jacobi2, life2), packed rows (rows up to 64 lanes) or 64 lanes per row, with
+ * fewer planes per tile while the batch has too few tiles to fill the device.
+ * Grid contents are preserved. */
 int kg_batch_tune(kg_batch* b, int reps, int* classes_tuned);
 int kg_batch_grid_shape(kg_batch* b, int id, int* lanes_per_row, int* planes_per_tile);
 /* Forces the tile shape of the size class of grid id. */

@@ -458,6 +458,12 @@ void batch_k(const GridDesc* __restrict__ grids, const Item* __restrict__ items,
     // and takes items from part b % 8 first: neighbouring tiles, which share
     // halo rows and planes, then run on one XCD and share its L2.  A
     // workgroup whose part is empty moves on to the next part.
+    // The first item of a workgroup follows from its number; only further ones
+    // cost an atomic, and a workgroup that finds a part empty reads all eight
+    // counters at once to see what is left, so that a step of few tiles is not
+    // spent asking eight counters in turn (63 tiles of 8 grids up to 64^3: 10.4
+    // us a step against 33.4 with every item taken by atomics; 2426 tiles of
+    // 200 grids of 64..128 points a side: 307 against 316).
     // Taking runs of several items per atomic (fewer atomics, neighbouring
     // tiles in sequence on one workgroup) measured slower: 2, 4, 8 and 32
     // items per take cost 4 %, 7 %, 10 % and 17 % (FP32).  So did taking the
@@ -467,24 +473,22 @@ void batch_k(const GridDesc* __restrict__ grids, const Item* __restrict__ items,
     // (3 %), which saves the callee-saved registers once per run of items
     // instead of once per item.
     const int home = (int)(blockIdx.x % KG_NUM_XCD);
-    int part = home, lo = 0, hi = 0, parts_left = KG_NUM_XCD;
-    lo = (int)((long long)part * nitems / KG_NUM_XCD);
-    hi = (int)((long long)(part + 1) * nitems / KG_NUM_XCD);
+    auto part_lo = [&](int p) { return (int)((long long)p * nitems / KG_NUM_XCD); };
+    // items of part p that are nobody's first
+    auto queued = [&](int p) {
+        return part_lo(p + 1) - part_lo(p) - (int)((gridDim.x + KG_NUM_XCD - 1 - p) / KG_NUM_XCD);
+    };
+    const int rank = (int)(blockIdx.x / KG_NUM_XCD);
+    int i = part_lo(home) + rank < part_lo(home + 1) ? part_lo(home) + rank : -1;
+    // parts that may still hold queued items, home first (wave 0 keeps it)
+    unsigned left = 0;
+    for (int q = 0; q < KG_NUM_XCD; q++)
+        if (queued((home + q) % KG_NUM_XCD) > 0) left |= 1u << q;
     for (;;) {
-        if (threadIdx.x == 0) next = lo + (int)atomicAdd(&st->counter[part], 1u);
-        __syncthreads();
-        const int i = next;
-        __syncthreads();
-        if (i >= hi) {
-            if (--parts_left == 0) break;
-            part = (part + 1) % KG_NUM_XCD;
-            lo = (int)((long long)part * nitems / KG_NUM_XCD);
-            hi = (int)((long long)(part + 1) * nitems / KG_NUM_XCD);
-            continue;
-        }
-        const Item it = items[i];
-        const GridDesc* g = grids + it.grid;
-        switch (it.var) {
+        if (i >= 0) {
+            const Item it = items[i];
+            const GridDesc* g = grids + it.grid;
+            switch (it.var) {
 #define KG_VAR_CASE(K, DT, LI) \
     case var_id(K, DT, LI): run_tile<K, DT, LPRS[LI]>(g, it.bx, it.by, it.bz, step); break;
             KG_VAR_LIST(KG_VAR_CASE)
@@ -499,18 +503,43 @@ void batch_k(const GridDesc* __restrict__ grids, const Item* __restrict__ items,
     case var_id(K, DT, COL): run_col<K, DT>(g, it.bx, it.by, it.bz, step); break;
             KG_ROW2_LIST(KG_ROW2_CASE)
 #undef KG_ROW2_CASE
-        default: break;
+            default: break;
+            }
+        }
+        if (threadIdx.x < 64) {
+            int got = -1;
+            while (left) {
+                const int p = (home + __builtin_ctz(left)) % KG_NUM_XCD;
+                int n = 0;
+                if (threadIdx.x == 0) n = (int)atomicAdd(&st->counter[p], 1u);
+                n = __builtin_amdgcn_readfirstlane(n);
+                if (n < queued(p)) {
+                    got = part_lo(p + 1) - queued(p) + n;
+                    break;
+                }
+                // lane q looks at the q-th part from home
+                const int o = (home + (int)threadIdx.x) % KG_NUM_XCD;
+                bool some = false;
+                if (threadIdx.x < KG_NUM_XCD)
+                    some = (int)__hip_atomic_load(&st->counter[o], __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT) < queued(o);
+                left &= (unsigned)__ballot(some);
+            }
+            if (threadIdx.x == 0) next = got;
         }
         __syncthreads();   // the next tile restages LDS
+        i = next;
+        if (i < 0) break;
+        __syncthreads();
     }
+    // No fence: the state is only touched by atomics, each of them waited for,
+    // and the levels are read by later launches.
     if (threadIdx.x == 0) {
-        __threadfence();
         if (atomicAdd(&st->done, 1u) == gridDim.x - 1) {
             // every workgroup has taken its last item and read `step`
             for (int x = 0; x < KG_NUM_XCD; x++) atomicExch(&st->counter[x], 0u);
             atomicExch(&st->done, 0u);
             atomicExch(&st->step, step + 1);
-            __threadfence();
         }
     }
 }
@@ -784,46 +813,42 @@ void drop_graphs(kg_batch* b)
     b->graphs.clear();
 }
 
-// Tiles of grid g with shape (li, kc), appended to out.
-void cut_tiles(const HostGrid& g, int gi, int li, int kc, std::vector<Item>& out)
+// How grid g is cut with shape (li, kc): ntx x nty tiles of the plane and nz
+// pieces along z, of planes of work in all.
+struct Cut {
+    int ntx, nty, nz, planes;
+    long long items() const { return (long long)ntx * nty * nz; }
+};
+
+Cut cut_of(const HostGrid& g, int li, int kc)
 {
-    const int var = var_id(g.spec.kind, g.spec.dtype, li);
-    const VarInfo& v = VARS[var];
+    const VarInfo& v = VARS[var_id(g.spec.kind, g.spec.dtype, li)];
     const int nx = g.spec.nx, ny = g.spec.ny, ns = g.spec.ns;
     const int nxi = nx - v.lo - v.hi, nyi = ny - v.lo - v.hi, nzi = ns - v.zlo - v.zhi;
-    if (nxi <= 0 || nyi <= 0 || nzi <= 0) return;
-    if (li == FLAT) {
-        for (int bz = 0; bz < (nzi + kc - 1) / kc; bz++) out.push_back(Item{gi, 0, 0, bz, var});
-        return;
-    }
-    if (li == ROW2) {   // one plane per item
-        const int ntx = (int)((g.sy + v.txw - 1) / v.txw), nty = (nyi + v.ty - 1) / v.ty;
-        for (int bz = 0; bz < nzi; bz++)
-            for (int by = 0; by < nty; by++)
-                for (int bx = 0; bx < ntx; bx++) out.push_back(Item{gi, bx, by, bz, var});
-        return;
-    }
+    if (nxi <= 0 || nyi <= 0 || nzi <= 0) return Cut{0, 0, 0, 0};
+    const int nkc = (nzi + kc - 1) / kc;
+    if (li == FLAT) return Cut{1, 1, nkc, nzi};
+    if (li == ROW2)   // one plane per item
+        return Cut{(int)((g.sy + v.txw - 1) / v.txw), (nyi + v.ty - 1) / v.ty, nzi, nzi};
     if (li == COL) {   // COLZ planes by 16/COLZ row chunks of kc rows per item
-        const int ntx = (int)((g.sy + v.txw - 1) / v.txw);
         const int rows = (BW / COLZ) * kc;
-        const int nty = (nyi + rows - 1) / rows, nkb = (ns + COLZ - 1) / COLZ;
-        for (int bk = 0; bk < nkb; bk++)
-            for (int by = 0; by < nty; by++)
-                for (int bx = 0; bx < ntx; bx++) out.push_back(Item{gi, bx, by, bk, var});
-        return;
+        return Cut{(int)((g.sy + v.txw - 1) / v.txw), (nyi + rows - 1) / rows, (ns + COLZ - 1) / COLZ, ns};
     }
     if (li == PACK) {
         const int ty = pack_rows_of(v, g.sy) - 2 * v.h;   // > 0: checked by build_work
-        for (int bz = 0; bz < (nzi + kc - 1) / kc; bz++)
-            for (int by = 0; by < (nyi + ty - 1) / ty; by++) out.push_back(Item{gi, 0, by, bz, var});
-        return;
+        return Cut{1, (nyi + ty - 1) / ty, nkc, nzi};
     }
-    const int ntx = (nx + v.txw - 1) / v.txw;
-    const int nty = (nyi + v.ty - 1) / v.ty;
-    const int nkc = (nzi + kc - 1) / kc;
-    for (int bz = 0; bz < nkc; bz++)
-        for (int by = 0; by < nty; by++)
-            for (int bx = 0; bx < ntx; bx++) out.push_back(Item{gi, bx, by, bz, var});
+    return Cut{(nx + v.txw - 1) / v.txw, (nyi + v.ty - 1) / v.ty, nkc, nzi};
+}
+
+// Tiles of grid g with shape (li, kc), appended to out.
+void cut_tiles(const HostGrid& g, int gi, int li, int kc, std::vector<Item>& out)
+{
+    const Cut c = cut_of(g, li, kc);
+    const int var = var_id(g.spec.kind, g.spec.dtype, li);
+    for (int bz = 0; bz < c.nz; bz++)
+        for (int by = 0; by < c.nty; by++)
+            for (int bx = 0; bx < c.ntx; bx++) out.push_back(Item{gi, bx, by, bz, var});
 }
 
 GridDesc make_desc(const HostGrid& g, int li, int kc)
@@ -887,6 +912,46 @@ void shape_of(const kg_batch* b, const HostGrid& g, int& li, int& kc)
     }
 }
 
+// Most planes per tile for the untuned grids of a batch (shape_of's kc is cut
+// down to it).  A batch of few or small grids has fewer tiles than there are
+// workgroups, and a step then takes as long as its thickest tile.  A tile costs
+// about as much as KG_ITEM_PLANES planes to start, and the workgroups take the
+// tiles in rounds: the cap with the least of the longest tile and of the rounds
+// at the mean cost.  A step, against the default's 8 to 32 planes: 8 grids up to
+// 64^3 8.7 us (33.9), 40 FP32 grids up to 128^3 28.5 us (49.7), 40 FP64 ones
+// 45.8 us (53.8); 200 grids keep the default (306 us).  2 to 12 planes a tile's
+// start all choose alike; halving every tile until there are 1, 2 or 4 per
+// workgroup gave 35-43 us for the 40 FP32 grids and 47-59 for the FP64 ones.
+constexpr int KG_ITEM_PLANES = 5;
+
+int planes_cap(const kg_batch* b, const std::vector<int>& order)
+{
+    double best = 0;
+    int pick = KCS[NKC - 1];
+    for (int cap = KCS[NKC - 1]; cap >= 2; cap /= 2) {
+        long long items = 0, longest = 0;
+        double cost = 0;
+        for (int gi : order) {
+            const HostGrid& g = b->grids[gi];
+            const int kc = b->tuned.count(size_class(g.spec)) ? g.kc : std::min(g.kc, cap);
+            const Cut c = cut_of(g, g.li, kc);
+            if (!c.items()) continue;
+            const int thick = g.li == ROW2 ? 1 : kc;
+            items += c.items();
+            cost += (double)c.items() * KG_ITEM_PLANES + (double)c.ntx * c.nty * c.planes;
+            longest = std::max<long long>(longest, KG_ITEM_PLANES + std::min(thick, c.planes));
+        }
+        if (!items) break;
+        const double est = std::max((double)longest,
+                                    (double)((items + b->nwg - 1) / b->nwg) * cost / items);
+        if (best == 0 || est < best) {
+            best = est;
+            pick = cap;
+        }
+    }
+    return pick;
+}
+
 // Upload descriptors and the work list (largest grids' tiles first).  With
 // only_class >= 0, only that size class is listed, with shape (li, kc).
 int build_work(kg_batch* b, int only_class = -1, int li_force = 0, int kc_force = 0)
@@ -921,6 +986,13 @@ int build_work(kg_batch* b, int only_class = -1, int li_force = 0, int kc_force 
         const kg_grid_spec &x = b->grids[a].spec, &y = b->grids[c].spec;
         return (double)x.nx * x.ny * x.ns > (double)y.nx * y.ny * y.ns;
     });
+    if (only_class < 0) {
+        const int cap = planes_cap(b, order);
+        for (int gi : order) {
+            HostGrid& g = b->grids[gi];
+            if (!b->tuned.count(size_class(g.spec))) g.kc = descs[gi].kc = std::min(g.kc, cap);
+        }
+    }
     std::vector<Item> items;
     for (int gi : order) cut_tiles(b->grids[gi], gi, b->grids[gi].li, b->grids[gi].kc, items);
     if (int rc = ensure_device_arrays(b, (int)std::max<size_t>(descs.size(), 1),

@@ -298,3 +298,18 @@ def test_batch_levels_round_trip(batch, dtype, dims):
     for level in (1, 0, 1):
         got = batch.download(gid, level)
         assert np.array_equal(got, lv[level])
+
+
+@pytest.mark.parametrize("ns,kc", [(6, 1), (260, 1), (1202, 1), (600, 0)])
+def test_batch_work_queue_lengths(gpu_ctx, batch, ns, kc):
+    """Fewer tiles than workgroups, a few more, several rounds, and the
+    default cut (kc 0): every tile is stepped exactly once a step."""
+    dims = (20, 9, ns)
+    specs = [("laplacian", F32, dims), ("wave13pt", F32, dims)]
+    ids, init = _fill(batch, specs, np.random.default_rng(16))
+    if kc:
+        for gid in ids:
+            batch.set_shape(gid, -1, kc)
+    batch.step(3, graph=False)
+    batch.step(4, graph=True)
+    _check_all(gpu_ctx, batch, specs, ids, init, 7, f"{ns} planes by {kc}")
