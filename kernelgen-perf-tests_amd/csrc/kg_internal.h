@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
 #include <tuple>
@@ -160,6 +161,32 @@ inline size_t kg_occupancy_lds(const kg_ctx* ctx, int occ, size_t static_lds)
     if (occ <= 0) return 0;
     const size_t per = (size_t)ctx->lds_cu / (size_t)occ;
     return per > static_lds + 256 ? per - static_lds - 256 : 0;
+}
+
+// Planes each workgroup marches when its launch covers nz of them with
+// `tiles` tiles side by side: kc on large grids; on small ones, where the kc of a
+// full chip would leave compute units idle or a last round nearly empty, the
+// number below kc that takes the least time.  A workgroup takes about kc + fill
+// planes' time (fill: the planes it loads before the first result) and the
+// device runs per_cu workgroups per compute unit at once.
+// Whole chunks against these: 64x32x32 lapgsrb 30 -> 5.7 us, wave13pt 20 -> 5.6,
+// tricubic 20 -> 6.2; 128^3 lapgsrb 35 -> 12.7, wave13pt 22 -> 11.2, its FP32 form
+// 55 -> 10.6 and BF16 72 -> 13.1; 200^3 wave13pt 54 -> 43.5, FP32 55 -> 19.9, BF16
+// 72 -> 26.  From four rounds of workgroups on the chunk of the large grids is
+// kept: there the last round is a small part and longer chunks read less.
+inline int kg_fit_chunk(const kg_ctx* ctx, long long tiles, int nz, int kc, int per_cu, int fill)
+{
+    const long long room = (long long)per_cu * ctx->cus;
+    if (tiles <= 0 || nz <= 0 || tiles * ((nz + kc - 1) / kc) >= 4 * room) return kc;
+    auto time = [&](int k) {
+        const long long wgs = tiles * ((nz + k - 1) / k);
+        return (wgs + room - 1) / room * (std::min(k, nz) + fill);
+    };
+    int best = kc;
+    for (int k = std::min(kc, nz); k >= 1; k--)
+        if (time(k) < time(best)) best = k;
+    // the planes two chunks share are read twice: a small gain is none
+    return time(best) * 100 < time(kc) * 85 ? best : kc;
 }
 
 // kg_xcd_chunk deals runs of `chunk` consecutive logical tiles to the XCDs in

@@ -63,7 +63,7 @@ void divergence_k(int nx, int ny, int ns, int ntx, int nty, double alpha, double
                   const double* __restrict__ uy, const double* __restrict__ uz)
 {
     kg_ztile t;
-    if (!kg_ztile_get<TX, TY, KC, 1, 1, false>(nx, ny, ns, ntx, nty, t)) return;
+    if (!kg_ztile_get<TX, TY, 1, 1, false>(nx, ny, ns, ntx, nty, KC, t)) return;
     const long long sz = (long long)nx * ny;
     const int sy = nx;
     long long o = kg_off3(t.i, t.j, t.k0, nx, sz);
@@ -166,7 +166,7 @@ void uxx1_k(int nx, int ny, int ns, int ntx, int nty, double c1, double c2, doub
             const double* __restrict__ xy, const double* __restrict__ xz)
 {
     kg_ztile t;
-    if (!kg_ztile_get<TX, TY, KC, 2, 1>(nx, ny, ns, ntx, nty, t)) return;
+    if (!kg_ztile_get<TX, TY, 2, 1>(nx, ny, ns, ntx, nty, KC, t)) return;
     const long long sz = (long long)nx * ny;
     const int sy = nx;
     long long o = kg_off3(t.i, t.j, t.k0, nx, sz);
@@ -459,10 +459,11 @@ static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
         using Op = OpT<C>;
         Op op{};
         fill(op);
-        int kc = C::KC;
+        const kgp::Grid g0 = kgp::make_grid<C>(nx, ny, ns, LO, HI);
+        const long long xy = (long long)g0.ntx * g0.nty;
+        int kc = kg_fit_chunk(ctx, xy, ns - LO - HI, C::KC, 1, C::RS);
         if (WGPC > 0) {
-            const kgp::Grid g0 = kgp::make_grid<C>(nx, ny, ns, LO, HI);
-            const long long xy = (long long)g0.ntx * g0.nty, want = (long long)WGPC * ctx->cus;
+            const long long want = (long long)WGPC * ctx->cus;
             if (!g0.empty && xy * g0.nkc > want) {
                 const long long chunks = want > xy ? want / xy : 1;
                 const long long nzi = ns - LO - HI;

@@ -73,14 +73,14 @@ __device__ __forceinline__ double point(const double (&win)[4][4][4], double av,
 
 template <int LO, int HI, bool FROM_ZERO>
 __global__ __launch_bounds__(TX * TY)
-void tricubic_k(int nx, int ny, int ns, int ntx, int nty,
+void tricubic_k(int nx, int ny, int ns, int ntx, int nty, int kc,
                 const double* __restrict__ u0, double* __restrict__ u1,
                 const double* __restrict__ a, const double* __restrict__ b,
                 const double* __restrict__ c)
 {
     static_assert(HI >= PFA, "a/b/c look-ahead must stay inside the grid");
     kg_ztile t;
-    if (!kg_ztile_get<TX, TY, KC, LO, HI, false>(nx, ny, ns, ntx, nty, t)) return;
+    if (!kg_ztile_get<TX, TY, LO, HI, false>(nx, ny, ns, ntx, nty, kc, t)) return;
     const long long sz = (long long)nx * ny;
     const int sy = nx;
     long long o = kg_off3(t.i, t.j, t.k0, nx, sz);
@@ -148,12 +148,14 @@ static int launch_tricubic(const char* name, kg_ctx* ctx, int nx, int ny, int ns
     if (!u0 || !u1 || !a || !b || !c) return kg_set_error(KG_ERR_INVALID, "kg_%s: null buffer", name);
     if (u1 == u0 || u1 == a || u1 == b || u1 == c)
         return kg_set_error(KG_ERR_INVALID, "kg_%s: u1 aliases an input", name);
-    const kg_zgrid g = kg_zgrid_make(nx, ny, ns, LO, HI, TX, TY, KC);
+    const kg_zgrid g0 = kg_zgrid_make(nx, ny, ns, LO, HI, TX, TY, KC);
+    const int kc = kg_fit_chunk(ctx, (long long)g0.ntx * g0.nty, ns - LO - HI, KC, 2, 3);
+    const kg_zgrid g = kg_zgrid_make(nx, ny, ns, LO, HI, TX, TY, kc);
     auto kern = tricubic_k<LO, HI, FROM_ZERO>;
     kg_register_kernel(name, (const void*)kern);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
     if (!g.empty)
-        kg_launch(ctx, kern, dim3(g.blocks), dim3(TX, TY), 0, nx, ny, ns, g.ntx, g.nty, u0, u1, a,
+        kg_launch(ctx, kern, dim3(g.blocks), dim3(TX, TY), 0, nx, ny, ns, g.ntx, g.nty, kc, u0, u1, a,
                   b, c);
     return kg_launch_end(ctx);
 }

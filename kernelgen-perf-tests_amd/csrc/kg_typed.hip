@@ -91,12 +91,14 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
         using Op = OpT<C>;
         Op op{};
         fill(op);
-        const kgp::Grid g = kgp::make_grid<C>(nx, ny, ns, LO, HI, ZLO, ZHI, KC);
+        const kgp::Grid g0 = kgp::make_grid<C>(nx, ny, ns, LO, HI, ZLO, ZHI, KC);
+        const int kc = kg_fit_chunk(ctx, (long long)g0.ntx * g0.nty, ns - ZLO - ZHI, KC, 1, C::RS);
+        const kgp::Grid g = kgp::make_grid<C>(nx, ny, ns, LO, HI, ZLO, ZHI, kc);
         auto kern = kgp::plane_kernel<C, LO, HI, Op, ZLO, ZHI, ORD>;
         kg_register_kernel(name, (const void*)kern);
         if (int rc = kg_launch_begin(ctx, name)) return rc;
         if (!g.empty)
-            kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * C::W), 0, nx, ny, ns, g.ntx, g.nty, KC,
+            kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * C::W), 0, nx, ny, ns, g.ntx, g.nty, kc,
                       op);
         return kg_launch_end(ctx);
     };

@@ -1,7 +1,7 @@
 // kg_zmarch.h -- tiling shared by the 3D stencil kernels.
 //
 // A workgroup of TX x TY threads owns a TX x TY column tile of the xy-plane
-// and marches it through a chunk of KC interior z-planes.  x is the fastest
+// and marches it through a chunk of kc interior z-planes.  x is the fastest
 // (coalesced) axis: one wave64 covers 64 consecutive x points of one row.
 // Tiles are aligned to x = 0 / y = 0 and cover the whole plane; threads whose
 // (i, j) lies outside the interior return at once (no barriers are used).
@@ -20,8 +20,9 @@ struct kg_ztile {
 };
 
 // lo / hi: interior is [lo, n - hi) along every axis.
-template <int TX, int TY, int KC, int LO, int HI, bool SWZ = true>
-__device__ __forceinline__ bool kg_ztile_get(int nx, int ny, int ns, int ntx, int nty, kg_ztile& t)
+template <int TX, int TY, int LO, int HI, bool SWZ = true>
+__device__ __forceinline__ bool kg_ztile_get(int nx, int ny, int ns, int ntx, int nty, int kc,
+                                             kg_ztile& t)
 {
     unsigned b = SWZ ? kg_xcd_swizzle(blockIdx.x, gridDim.x) : blockIdx.x;
     const int bx = (int)(b % (unsigned)ntx);
@@ -30,8 +31,8 @@ __device__ __forceinline__ bool kg_ztile_get(int nx, int ny, int ns, int ntx, in
     const int bz = (int)(b / (unsigned)nty);
     t.i = bx * TX + (int)threadIdx.x;
     t.j = by * TY + (int)threadIdx.y;
-    t.k0 = LO + bz * KC;
-    t.k1 = min(t.k0 + KC, ns - HI);
+    t.k0 = LO + bz * kc;
+    t.k1 = min(t.k0 + kc, ns - HI);
     return t.i >= LO && t.i < nx - HI && t.j >= LO && t.j < ny - HI && t.k0 < t.k1;
 }
 

@@ -158,6 +158,21 @@ def test_gpu_lapgsrb_long_z_chunks(gpu_ctx, oracle, dims):
         assert_bit_equal(got[role], want[role], f"lapgsrb {dims} {role}")
 
 
+@pytest.mark.parametrize("name", ["laplacian", "gradient", "wave13pt", "lapgsrb", "tricubic",
+                                  "tricubic2", "whispering"])
+def test_gpu_matches_oracle_thin_chunks(gpu_ctx, oracle, name):
+    """Grids with too few tiles for the device, whose z- or y-chunks are cut
+    down to one or a few planes, a last chunk of its own among them."""
+    spec = K.SPECS[name]
+    for si, dims in enumerate([(64, 32, 32), (100, 60, 80), (33, 57, 41), (130, 11, 257)]
+                              if spec.dim == 3 else [(64, 1000), (97, 2003), (512, 700)]):
+        coefs, arrays = K.random_case(spec, dims, 1200 + si)
+        want = oracle.run(spec, dims, coefs, arrays, 2)
+        got = K.GpuBackend(gpu_ctx).run(spec, dims, coefs, arrays, 2)
+        for role in want:
+            assert_bit_equal(got[role], want[role], f"{name} {dims} {role}")
+
+
 @pytest.mark.parametrize("name", ["laplacian", "wave13pt", "whispering", "gameoflife", "uxx1"])
 def test_gpu_matches_oracle_ten_steps(gpu_ctx, oracle, name):
     """Ten ping-pong steps (the suite's nt) at a mid size."""
