@@ -21,6 +21,7 @@
 namespace kgr {
 
 typedef double d2 __attribute__((ext_vector_type(2)));
+typedef d2 d2u __attribute__((aligned(8)));   // at any double
 
 template <int VEC_, int W_, int H_, int NF_, int LL_, int LR_, int ZL_, int ZR_, int D_, int NAUX_,
           int YC_>
@@ -208,7 +209,7 @@ __device__ __forceinline__ void store(double* dst, long long o, int x, const dou
         d2 t;
         t.x = r[0];
         t.y = r[VEC - 1];
-        kg_st((d2*)(dst + o + x), t);
+        __builtin_nontemporal_store(t, (d2u*)(dst + o + x));
     } else {
 #pragma unroll
         for (int v = 0; v < VEC; v++)
@@ -230,6 +231,13 @@ __device__ __forceinline__ void store(double* dst, long long o, int x, const dou
 // own piece and taking the pieces at x-2 and x+2 from the neighbouring lanes
 // by DPP shifts (one load per row instead of three) was bit-identical but
 // slower: jacobi 100 -> 110 us, gameoflife 100 -> 103, gaussblur 94 -> 122.
+//
+// Rows of an odd number of points, and fields that are only 8-byte aligned, take
+// the same form (ODD): the hardware loads and stores 16 bytes at any multiple of
+// 4, and the pair at the last point of an odd row is read one point further left
+// and shifted, so no load leaves its row.  301 x 30653: jacobi 30 us against 54 in
+// the row engine with 8-byte lanes, gaussblur 31 against 58, gameoflife 32
+// against 55; 511 x 65536: 78, 78 and 83 against 86, 111 and 86.
 template <int PY_, int ROWS_, int H_>
 struct DCfg {
     static constexpr int VEC = 2;
@@ -271,9 +279,23 @@ static inline DGrid<C> make_dgrid(int nx, int ny, int lo, int hi)
     return g;
 }
 
-// Requires an even nx and 16-byte aligned fields (checked by the host).
-// ORD: tile order (kg_tile_order).
-template <class C, int LO, int HI, class Op, int ORD = 0>
+// Points x, x+1 of a row of nx points (x even, x < nx).  ODD: x may be the last
+// point; with `last` the pair is then (last point, undefined).
+template <bool ODD>
+__device__ __forceinline__ d2 row_pair(const kgp::gmem<double>* row, int x, bool last = false)
+{
+    if constexpr (!ODD) {
+        return *(const kgp::gmem<d2>*)(row + x);
+    } else {
+        d2 p = *(const kgp::gmem<d2u>*)(row + (last ? x - 1 : x));
+        if (last) p.x = p.y;
+        return p;
+    }
+}
+
+// ODD: any nx and 8-byte aligned fields; otherwise an even nx and 16-byte
+// aligned fields (chosen by the host).  ORD: tile order (kg_tile_order).
+template <class C, int LO, int HI, class Op, int ORD = 0, bool ODD = false>
 __global__ __launch_bounds__(64 * C::ROWS)
 void direct_kernel(int nx, int ny, int ntx, Op op)
 {
@@ -283,7 +305,7 @@ void direct_kernel(int nx, int ny, int ntx, Op op)
     const int by = (int)(b / (unsigned)ntx);
     const int x = bx * C::TXW + 2 * lane;
     const int j0 = LO + (by * C::ROWS + r) * C::PY;
-    if (x >= nx || j0 >= ny - HI) return;   // no barriers in this kernel
+    if (x >= nx - HI || j0 >= ny - HI) return;   // no barriers in this kernel
     // The pairs at x-2 and x+2 are clamped into the row at the grid's
     // x-edges; there they only feed points outside the interior.  Rows past
     // ny-1 are clamped likewise (they feed rows >= ny-HI, never stored).
@@ -294,9 +316,9 @@ void direct_kernel(int nx, int ny, int ntx, Op op)
 #pragma unroll
     for (int q = 0; q < C::NR; q++) {
         const kgp::gmem<double>* row = src + (long long)min(j0 - C::H + q, ny - 1) * nx;
-        const d2 a = *(const kgp::gmem<d2>*)(row + xl);
-        const d2 c = *(const kgp::gmem<d2>*)(row + x);
-        const d2 e = *(const kgp::gmem<d2>*)(row + xr);
+        const d2 a = row_pair<ODD>(row, xl);
+        const d2 c = row_pair<ODD>(row, x);
+        const d2 e = row_pair<ODD>(row, xr, xr + 1 >= nx);
         win[q][0] = a.x;
         win[q][1] = a.y;
         win[q][2] = c.x;

@@ -148,8 +148,6 @@ struct WhisperingOp {
 // per SIMD, 3 values spilled) it ran slower: 614-618 us against 572-573
 // (YC=6 615-628, 12 631-634, 16 660; D=1 605-622).
 //                     VEC W      H  NF LL LR ZL ZR D  NAUX YC
-template <int V> using J9Cfg = kgr::Cfg<V, 4, 1, 1, 1, 1, 0, 0, 2, 0, 64>;
-template <int V> using G25Cfg = kgr::Cfg<V, 4, 2, 1, 2, 2, 0, 0, 2, 0, 32>;
 template <int V> using WhCfg = kgr::Cfg<V, 8 / V, 1, 5, 0, 0, 1, 1, 2, 3, 8>;
 
 // Launch Op on the row engine; 16-byte lanes (VEC=2) need an even nx and
@@ -218,22 +216,21 @@ using J9D = kgr::DCfg<KG_J9_PY, KG_J9_ROWS, 1>;
 using JacD = kgr::DCfg<KG_JAC_PY, KG_J9_ROWS, 1>;
 using G25D = kgr::DCfg<KG_G25_PY, KG_G25_ROWS, 2>;
 
-// Single-field stencils: the direct march when nx is even and both fields
-// are 16-byte aligned, else the row engine.
-template <class DC, template <int> class CfgT, template <class> class OpT, int LO, int HI,
-          int ORD, class Fill>
+// Single-field stencils on the direct march: its aligned form when nx is even and
+// both fields are 16-byte aligned, else the form for any row length.
+template <class DC, template <class> class OpT, int LO, int HI, int ORD, class Fill>
 static int launch_direct(kg_ctx* ctx, const char* name, int nx, int ny, const void* in,
                          const void* out, Fill fill)
 {
-    const bool al = kg_aligned16(in, out);
-    if (nx % 2 != 0 || !al) return launch_row<CfgT, OpT, LO, HI, 2>(ctx, name, nx, ny, al, fill);
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims2(nx, ny)) return rc;
     using Op = OpT<DC>;
     Op op{};
     fill(op);
     const kgr::DGrid<DC> g = kgr::make_dgrid<DC>(nx, ny, LO, HI);
-    auto kern = kgr::direct_kernel<DC, LO, HI, Op, ORD>;
+    const bool even = nx % 2 == 0 && kg_aligned16(in, out);
+    auto kern = even ? kgr::direct_kernel<DC, LO, HI, Op, ORD, false>
+                     : kgr::direct_kernel<DC, LO, HI, Op, ORD, true>;
     kg_register_kernel(name, (const void*)kern);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
     if (!g.empty)
@@ -251,7 +248,7 @@ extern "C" int kg_jacobi(kg_ctx* ctx, int nx, int ny, double c0, double c1, doub
 {
     KG_REQUIRE(w0 && w1, "kg_jacobi: null buffer");
     KG_REQUIRE(w0 != w1, "kg_jacobi: w0 and w1 must be distinct");
-    return launch_direct<JacD, J9Cfg, JacobiOp, 1, 1, KG_ORD_JAC>(ctx, "jacobi_", nx, ny, w0, w1, [&](auto& op) {
+    return launch_direct<JacD, JacobiOp, 1, 1, KG_ORD_JAC>(ctx, "jacobi_", nx, ny, w0, w1, [&](auto& op) {
         op.src[0] = w0;
         op.dst = w1;
         op.c0 = c0;
@@ -266,7 +263,7 @@ extern "C" int kg_gaussblur(kg_ctx* ctx, int nx, int ny, double s0, double s1, d
     KG_REQUIRE(w0 && w1, "kg_gaussblur: null buffer");
     KG_REQUIRE(w0 != w1, "kg_gaussblur: w0 and w1 must be distinct");
     const double f = 1. / (s0 + 4 * (s1 + s2 + s4 + s8) + 8 * s5);   // gaussblur/gaussblur.c:65
-    return launch_direct<G25D, G25Cfg, GaussblurOp, 2, 2, KG_ORD_GAUSS>(ctx, "gaussblur", nx, ny, w0, w1, [&](auto& op) {
+    return launch_direct<G25D, GaussblurOp, 2, 2, KG_ORD_GAUSS>(ctx, "gaussblur", nx, ny, w0, w1, [&](auto& op) {
         op.src[0] = w0;
         op.dst = w1;
         op.f = f;
@@ -283,7 +280,7 @@ extern "C" int kg_gameoflife(kg_ctx* ctx, int nx, int ny, const double* u0, doub
 {
     KG_REQUIRE(u0 && u1, "kg_gameoflife: null buffer");
     KG_REQUIRE(u0 != u1, "kg_gameoflife: u0 and u1 must be distinct");
-    return launch_direct<J9D, J9Cfg, GameoflifeOp, 1, 1, KG_ORD_LIFE>(ctx, "gameoflife", nx, ny, u0, u1, [&](auto& op) {
+    return launch_direct<J9D, GameoflifeOp, 1, 1, KG_ORD_LIFE>(ctx, "gameoflife", nx, ny, u0, u1, [&](auto& op) {
         op.src[0] = u0;
         op.dst = u1;
     });
@@ -322,5 +319,5 @@ extern "C" int kg_whispering(kg_ctx* ctx, int nx, int ny, double mu, double epsi
 
 int kg_preload_stencil2d()
 {
-    return kg_preload_kernel((const void*)kgr::row_kernel<J9Cfg<2>, 1, 1, JacobiOp<J9Cfg<2>>>);
+    return kg_preload_kernel((const void*)kgr::direct_kernel<JacD, 1, 1, JacobiOp<JacD>>);
 }

@@ -4,11 +4,9 @@
 // laplacian, gradient, wave13pt and lapgsrb run on the plane-staged engine
 // (kg_plane.h): xy-neighbours from LDS, z-neighbours from a register column,
 // every global load prefetched a few planes ahead.  divergence and uxx1 read
-// each of their inputs at only a few offsets along one axis: with an even nx
-// and 16-byte aligned fields they run the direct form (two points and a few
-// planes per lane, every operand a 16-byte load through the caches, all
-// issued up front), otherwise the plain z-march (kg_zmarch.h): a TX x TY
-// column tile marched through KC planes, one point per thread.
+// each of their inputs at only a few offsets along one axis and run the direct
+// form: two points and a few planes per lane, every operand a 16-byte load
+// through the caches, all issued up front.
 // Arithmetic is written in the reference's source order and the library is
 // built with -ffp-contract=off: results are bit-identical to an IEEE build of
 // the reference kernels.
@@ -48,49 +46,23 @@ namespace {
 using kgops::LaplacianOp;
 using kgops::Wave13ptOp;
 
-constexpr int TX = 64;   // one wave64 per x-row segment
-constexpr int TY = 4;    // 4 rows -> 256 threads per workgroup
-constexpr int KC = 16;   // z-planes per workgroup
-
 #define KG_REQUIRE(cond, msg) \
     do { if (!(cond)) return kg_set_error(KG_ERR_INVALID, "%s", msg); } while (0)
 
 // --------------------------------------------------------------- divergence
 // divergence/divergence.c:93-96
-__global__ __launch_bounds__(TX * TY)
-void divergence_k(int nx, int ny, int ns, int ntx, int nty, double alpha, double beta, double gamma,
-                  double* __restrict__ u, const double* __restrict__ ux,
-                  const double* __restrict__ uy, const double* __restrict__ uz)
-{
-    kg_ztile t;
-    if (!kg_ztile_get<TX, TY, 1, 1, false>(nx, ny, ns, ntx, nty, KC, t)) return;
-    const long long sz = (long long)nx * ny;
-    const int sy = nx;
-    long long o = kg_off3(t.i, t.j, t.k0, nx, sz);
-    double zm = uz[o - sz];
-    double zc = uz[o];
-#pragma unroll 4
-    for (int k = t.k0; k < t.k1; k++) {
-        const double zp = uz[o + sz];
-        kg_st(&u[o], alpha * (ux[o + 1] - ux[o - 1]) +
-                     beta * (uy[o + sy] - uy[o - sy]) +
-                     gamma * (zp - zm));
-        zm = zc;
-        zc = zp;
-        o += sz;
-    }
-}
-
-// Direct form (even nx, 16-byte aligned fields): a lane owns points x, x+1
-// (x even) of row j and PZ consecutive planes; every operand is a 16-byte
-// load through the caches (ux as the aligned pairs at x-2, x, x+2; uy at rows
+//
+// A lane owns points x, x+1 (x even) of row j and PZ consecutive planes; every
+// operand is a 16-byte load through the caches (ux as the aligned pairs at x-2, x, x+2; uy at rows
 // j-1, j+1; uz at planes k0-1 .. k0+PZ), all issued before the first use.
 // Workgroups stay in hardware order, at most DIV_OCC (16 waves) per compute
 // unit: 183 us at 512x256x256 (unlimited 187, 3 per CU 196; uxx1 gains
 // nothing from such a cap).  Other tile orders (kg_tile_order) measured no
 // better: chunks of 2, 4 or 8 tile rows per XCD 183-186 us (uxx1 286-295
 // against 284-286 in hardware order), XCD-contiguous eighths 188 us (uxx1
-// 310).  Same expression as divergence_k.
+// 310).  ODD: rows of an odd length and fields at any double, with loads and
+// stores of 16 bytes all the same: 58 us at 301x203x151 against 75 with a point
+// per lane marching through z, 198 against 223 at 511x256x256 (181 at 512).
 #ifndef KG_DIV_PZ
 #define KG_DIV_PZ 4
 #endif
@@ -101,11 +73,26 @@ constexpr int DIV_PZ = KG_DIV_PZ, DIV_ROWS = KG_DIV_ROWS, DIV_OCC = 4;
 
 typedef double d2v __attribute__((ext_vector_type(2)));
 
+typedef d2v d2vu __attribute__((aligned(8)));   // at any double
+
+// The pair at p.  ODD: any alignment.
+template <bool ODD>
 __device__ __forceinline__ d2v ld2(const double* p)
 {
-    return *(const kgp::gmem<d2v>*)kgp::as_global(p);
+    if constexpr (ODD) return *(const kgp::gmem<d2vu>*)kgp::as_global(p);
+    else return *(const kgp::gmem<d2v>*)kgp::as_global(p);
+}
+// The pair at p, or with `last` (ODD: p is the last point of an odd row) the pair
+// (last point, undefined), read from one point further left.
+template <bool ODD>
+__device__ __forceinline__ d2v ld2(const double* p, bool last)
+{
+    d2v v = ld2<ODD>(p - (ODD && last ? 1 : 0));
+    if (ODD && last) v.x = v.y;
+    return v;
 }
 
+template <bool ODD>
 __global__ __launch_bounds__(64 * DIV_ROWS)
 void divergence2_k(int nx, int ny, int ns, int ntx, int nty, double alpha, double beta,
                    double gamma, double* __restrict__ u, const double* __restrict__ ux,
@@ -120,25 +107,26 @@ void divergence2_k(int nx, int ny, int ns, int ntx, int nty, double alpha, doubl
     const int x = bx * 128 + 2 * lane;
     const int j = 1 + by * DIV_ROWS + r;
     const int k0 = 1 + bz * DIV_PZ;
-    if (x >= nx || j >= ny - 1 || k0 >= ns - 1) return;
+    if (x >= nx - 1 || j >= ny - 1 || k0 >= ns - 1) return;
     // pairs at x-2 / x+2 clamped into the row at the x-edges (they then feed
     // boundary points only); planes past ns-2 clamped (never stored)
     const int xl = x >= 2 ? x - 2 : x;
     const int xr = x + 2 < nx ? x + 2 : x;
+    const bool er = xr + 1 >= nx;   // the last point of an odd row
     const long long sz = (long long)nx * ny;
     const long long oj = (long long)j * nx;
     d2v xm[DIV_PZ], xc[DIV_PZ], xp[DIV_PZ], ym[DIV_PZ], yp[DIV_PZ], z[DIV_PZ + 2];
 #pragma unroll
     for (int p = 0; p < DIV_PZ; p++) {
         const long long o = (long long)min(k0 + p, ns - 2) * sz + oj;
-        xm[p] = ld2(ux + o + xl);
-        xc[p] = ld2(ux + o + x);
-        xp[p] = ld2(ux + o + xr);
-        ym[p] = ld2(uy + o - nx + x);
-        yp[p] = ld2(uy + o + nx + x);
+        xm[p] = ld2<ODD>(ux + o + xl);
+        xc[p] = ld2<ODD>(ux + o + x);
+        xp[p] = ld2<ODD>(ux + o + xr, er);
+        ym[p] = ld2<ODD>(uy + o - nx + x);
+        yp[p] = ld2<ODD>(uy + o + nx + x);
     }
 #pragma unroll
-    for (int p = 0; p < DIV_PZ + 2; p++) z[p] = ld2(uz + (long long)min(k0 - 1 + p, ns - 1) * sz + oj + x);
+    for (int p = 0; p < DIV_PZ + 2; p++) z[p] = ld2<ODD>(uz + (long long)min(k0 - 1 + p, ns - 1) * sz + oj + x);
     const bool m0 = x >= 1 && x < nx - 1, m1 = x + 1 < nx - 1;
 #pragma unroll
     for (int p = 0; p < DIV_PZ; p++) {
@@ -149,7 +137,7 @@ void divergence2_k(int nx, int ny, int ns, int ntx, int nty, double alpha, doubl
         double* o = u + (long long)(k0 + p) * sz + oj + x;
         if (m0 && m1) {
             d2v t = {res[0], res[1]};
-            kg_st((d2v*)o, t);
+            __builtin_nontemporal_store(t, (d2vu*)o);
         } else {
             if (m0) kg_st(o, res[0]);
             if (m1) kg_st(o + 1, res[1]);
@@ -159,46 +147,11 @@ void divergence2_k(int nx, int ny, int ns, int ntx, int nty, double alpha, doubl
 
 // --------------------------------------------------------------------- uxx1
 // uxx1/uxx1.c:95-105, interior [2,n-1)^3, dth = 1/nx (:70)
-__global__ __launch_bounds__(TX * TY)
-void uxx1_k(int nx, int ny, int ns, int ntx, int nty, double c1, double c2, double dth,
-            const double* __restrict__ u0, double* __restrict__ u1,
-            const double* __restrict__ d1, const double* __restrict__ xx,
-            const double* __restrict__ xy, const double* __restrict__ xz)
-{
-    kg_ztile t;
-    if (!kg_ztile_get<TX, TY, 2, 1>(nx, ny, ns, ntx, nty, KC, t)) return;
-    const long long sz = (long long)nx * ny;
-    const int sy = nx;
-    long long o = kg_off3(t.i, t.j, t.k0, nx, sz);
-    // z-columns kept in registers: d1 at (i,j) and (i,j-1), planes k-1..k;
-    // xz at (i,j), planes k-2..k+1.
-    double d_c_m = d1[o - sz], d_y_m = d1[o - sy - sz];
-    double xz_m2 = xz[o - 2 * sz], xz_m1 = xz[o - sz], xz_c = xz[o];
-#pragma unroll 2
-    for (int k = t.k0; k < t.k1; k++) {
-        const double d_c = d1[o], d_y = d1[o - sy];
-        const double xz_p1 = xz[o + sz];
-        const double d = 0.25 * (d_c + d_y + d_c_m + d_y_m);
-        kg_st(&u1[o], u0[o] + (dth / d) * (
-            c1 * (xx[o] - xx[o - 1]) +
-            c2 * (xx[o + 1] - xx[o - 2]) +
-            c1 * (xy[o] - xy[o - sy]) +
-            c2 * (xy[o + sy] - xy[o - 2 * sy]) +
-            c1 * (xz_c - xz_m1) +
-            c2 * (xz_p1 - xz_m2)));
-        d_c_m = d_c;
-        d_y_m = d_y;
-        xz_m2 = xz_m1;
-        xz_m1 = xz_c;
-        xz_c = xz_p1;
-        o += sz;
-    }
-}
-
-// Direct uxx1 (even nx, 16-byte aligned fields): a lane owns points x, x+1
-// of row j and PZ planes; xx as the aligned pairs at x-2, x, x+2; xy at rows
+//
+// A lane owns points x, x+1 of row j and PZ planes; xx as the aligned pairs at x-2, x, x+2; xy at rows
 // j-2 .. j+1; d1 at rows j-1, j of planes k0-1 .. k0+PZ-1; xz at planes
-// k0-2 .. k0+PZ; u0 at the point.  Same expression as uxx1_k.
+// k0-2 .. k0+PZ; u0 at the point.  ODD as for divergence: 95 us at 301x203x151
+// against 131 marching through z, 303 against 360 at 511x256x256 (283 at 512).
 #ifndef KG_UXX_PZ
 #define KG_UXX_PZ 4
 #endif
@@ -207,6 +160,7 @@ void uxx1_k(int nx, int ny, int ns, int ntx, int nty, double c1, double c2, doub
 #endif
 constexpr int UXX_PZ = KG_UXX_PZ, UXX_ROWS = KG_UXX_ROWS;
 
+template <bool ODD>
 __global__ __launch_bounds__(64 * UXX_ROWS)
 void uxx1_2_k(int nx, int ny, int ns, int ntx, int nty, double c1, double c2, double dth,
               const double* __restrict__ u0, double* __restrict__ u1,
@@ -222,9 +176,10 @@ void uxx1_2_k(int nx, int ny, int ns, int ntx, int nty, double c1, double c2, do
     const int x = bx * 128 + 2 * lane;
     const int j = 2 + by * UXX_ROWS + r;
     const int k0 = 2 + bz * UXX_PZ;
-    if (x >= nx || j >= ny - 1 || k0 >= ns - 1) return;
+    if (x >= nx - 1 || j >= ny - 1 || k0 >= ns - 1) return;
     const int xl = x >= 2 ? x - 2 : x;
     const int xr = x + 2 < nx ? x + 2 : x;
+    const bool er = xr + 1 >= nx;   // the last point of an odd row
     const long long sz = (long long)nx * ny;
     const long long oj = (long long)j * nx;
     d2v uc[UXX_PZ], xa[UXX_PZ], xc[UXX_PZ], xb[UXX_PZ], y2[UXX_PZ], y1[UXX_PZ], y0[UXX_PZ],
@@ -232,23 +187,23 @@ void uxx1_2_k(int nx, int ny, int ns, int ntx, int nty, double c1, double c2, do
 #pragma unroll
     for (int p = 0; p < UXX_PZ; p++) {
         const long long o = (long long)min(k0 + p, ns - 2) * sz + oj;
-        uc[p] = ld2(u0 + o + x);
-        xa[p] = ld2(xx + o + xl);
-        xc[p] = ld2(xx + o + x);
-        xb[p] = ld2(xx + o + xr);
-        y2[p] = ld2(xy + o - 2 * nx + x);
-        y1[p] = ld2(xy + o - nx + x);
-        y0[p] = ld2(xy + o + x);
-        y3[p] = ld2(xy + o + nx + x);
+        uc[p] = ld2<ODD>(u0 + o + x);
+        xa[p] = ld2<ODD>(xx + o + xl);
+        xc[p] = ld2<ODD>(xx + o + x);
+        xb[p] = ld2<ODD>(xx + o + xr, er);
+        y2[p] = ld2<ODD>(xy + o - 2 * nx + x);
+        y1[p] = ld2<ODD>(xy + o - nx + x);
+        y0[p] = ld2<ODD>(xy + o + x);
+        y3[p] = ld2<ODD>(xy + o + nx + x);
     }
 #pragma unroll
     for (int p = 0; p < UXX_PZ + 1; p++) {
         const long long o = (long long)min(k0 - 1 + p, ns - 2) * sz + oj + x;
-        dc[p] = ld2(d1 + o);
-        dy[p] = ld2(d1 + o - nx);
+        dc[p] = ld2<ODD>(d1 + o);
+        dy[p] = ld2<ODD>(d1 + o - nx);
     }
 #pragma unroll
-    for (int p = 0; p < UXX_PZ + 3; p++) z[p] = ld2(xz + (long long)min(k0 - 2 + p, ns - 1) * sz + oj + x);
+    for (int p = 0; p < UXX_PZ + 3; p++) z[p] = ld2<ODD>(xz + (long long)min(k0 - 2 + p, ns - 1) * sz + oj + x);
     const bool m0 = x >= 2 && x < nx - 1, m1 = x + 1 >= 2 && x + 1 < nx - 1;
 #pragma unroll
     for (int p = 0; p < UXX_PZ; p++) {
@@ -274,7 +229,7 @@ void uxx1_2_k(int nx, int ny, int ns, int ntx, int nty, double c1, double c2, do
         double* o = u1 + (long long)(k0 + p) * sz + oj + x;
         if (m0 && m1) {
             d2v t = {res[0], res[1]};
-            kg_st((d2v*)o, t);
+            __builtin_nontemporal_store(t, (d2vu*)o);
         } else {
             if (m0) kg_st(o, res[0]);
             if (m1) kg_st(o + 1, res[1]);
@@ -490,19 +445,6 @@ static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
 
 // ============================================================ entry points
 
-#define KG_LAUNCH3(NAME, KERNEL, LO, HI, ...)                                              \
-    do {                                                                                   \
-        if (int rc_ = kg_check_ctx(ctx)) return rc_;                                       \
-        if (int rc_ = kg_check_dims3(nx, ny, ns)) return rc_;                              \
-        const kg_zgrid g = kg_zgrid_make(nx, ny, ns, LO, HI, TX, TY, KC);                  \
-        kg_register_kernel(NAME, (const void*)KERNEL);                                     \
-        if (int rc_ = kg_launch_begin(ctx, NAME)) return rc_;                              \
-        if (!g.empty)                                                                      \
-            kg_launch(ctx, KERNEL, dim3(g.blocks), dim3(TX, TY), 0, nx, ny, ns, g.ntx,     \
-                      g.nty, __VA_ARGS__);                                                 \
-        return kg_launch_end(ctx);                                                         \
-    } while (0)
-
 extern "C" int kg_laplacian(kg_ctx* ctx, int nx, int ny, int ns, double alpha, double beta,
                             const double* w0, double* w1)
 {
@@ -523,18 +465,17 @@ extern "C" int kg_divergence(kg_ctx* ctx, int nx, int ny, int ns, double alpha, 
 {
     KG_REQUIRE(u && ux && uy && uz, "kg_divergence: null buffer");
     KG_REQUIRE(u != ux && u != uy && u != uz, "kg_divergence: output aliases an input");
-    if (nx % 2 == 0 && !(((uintptr_t)u | (uintptr_t)ux | (uintptr_t)uy | (uintptr_t)uz) & 15)) {
-        if (int rc = kg_check_ctx(ctx)) return rc;
-        if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
-        const kg_zgrid g = kg_zgrid_make(nx, ny, ns, 1, 1, 128, DIV_ROWS, DIV_PZ);
-        kg_register_kernel("divergence", (const void*)divergence2_k);
-        if (int rc = kg_launch_begin(ctx, "divergence")) return rc;
-        if (!g.empty)
-            kg_launch(ctx, divergence2_k, dim3(g.blocks), dim3(64 * DIV_ROWS), kg_occupancy_lds(ctx,
-                      DIV_OCC, 0), nx, ny, ns, g.ntx, g.nty, alpha, beta, gamma, u, ux, uy, uz);
-        return kg_launch_end(ctx);
-    }
-    KG_LAUNCH3("divergence", divergence_k, 1, 1, alpha, beta, gamma, u, ux, uy, uz);
+    if (int rc = kg_check_ctx(ctx)) return rc;
+    if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
+    const kg_zgrid g = kg_zgrid_make(nx, ny, ns, 1, 1, 128, DIV_ROWS, DIV_PZ);
+    const bool even = nx % 2 == 0 && kg_aligned16(u, ux, uy, uz);
+    auto kern = even ? divergence2_k<false> : divergence2_k<true>;
+    kg_register_kernel("divergence", (const void*)kern);
+    if (int rc = kg_launch_begin(ctx, "divergence")) return rc;
+    if (!g.empty)
+        kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * DIV_ROWS), kg_occupancy_lds(ctx, DIV_OCC, 0),
+                  nx, ny, ns, g.ntx, g.nty, alpha, beta, gamma, u, ux, uy, uz);
+    return kg_launch_end(ctx);
 }
 
 extern "C" int kg_gradient(kg_ctx* ctx, int nx, int ny, int ns, double alpha, double beta,
@@ -579,20 +520,18 @@ extern "C" int kg_uxx1(kg_ctx* ctx, int nx, int ny, int ns, double c1, double c2
     KG_REQUIRE(u1 != u0 && u1 != d1 && u1 != xx && u1 != xy && u1 != xz,
                "kg_uxx1: u1 aliases an input");
     const double dth = 1. / nx;   // uxx1/uxx1.c:70
-    if (nx % 2 == 0 && !(((uintptr_t)u0 | (uintptr_t)u1 | (uintptr_t)d1 | (uintptr_t)xx |
-                          (uintptr_t)xy | (uintptr_t)xz) & 15)) {
-        if (int rc = kg_check_ctx(ctx)) return rc;
-        if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
-        // rows/planes from 2: the grid helper counts tiles from 0, one spare
-        const kg_zgrid g = kg_zgrid_make(nx, ny, ns, 2, 1, 128, UXX_ROWS, UXX_PZ);
-        kg_register_kernel("uxx1", (const void*)uxx1_2_k);
-        if (int rc = kg_launch_begin(ctx, "uxx1")) return rc;
-        if (!g.empty)
-            kg_launch(ctx, uxx1_2_k, dim3(g.blocks), dim3(64 * UXX_ROWS), 0, nx, ny, ns, g.ntx,
-                      g.nty, c1, c2, dth, u0, u1, d1, xx, xy, xz);
-        return kg_launch_end(ctx);
-    }
-    KG_LAUNCH3("uxx1", uxx1_k, 2, 1, c1, c2, dth, u0, u1, d1, xx, xy, xz);
+    if (int rc = kg_check_ctx(ctx)) return rc;
+    if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
+    // rows/planes from 2: the grid helper counts tiles from 0, one spare
+    const kg_zgrid g = kg_zgrid_make(nx, ny, ns, 2, 1, 128, UXX_ROWS, UXX_PZ);
+    const bool even = nx % 2 == 0 && kg_aligned16(u0, u1, d1, xx, xy, xz);
+    auto kern = even ? uxx1_2_k<false> : uxx1_2_k<true>;
+    kg_register_kernel("uxx1", (const void*)kern);
+    if (int rc = kg_launch_begin(ctx, "uxx1")) return rc;
+    if (!g.empty)
+        kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * UXX_ROWS), 0, nx, ny, ns, g.ntx, g.nty, c1,
+                  c2, dth, u0, u1, d1, xx, xy, xz);
+    return kg_launch_end(ctx);
 }
 
 extern "C" int kg_lapgsrb(kg_ctx* ctx, int nx, int ny, int ns, double c0, double c1, double c2,
@@ -611,4 +550,4 @@ extern "C" int kg_lapgsrb(kg_ctx* ctx, int nx, int ny, int ns, double c0, double
     });
 }
 
-int kg_preload_stencil3d() { return kg_preload_kernel((const void*)divergence_k); }
+int kg_preload_stencil3d() { return kg_preload_kernel((const void*)divergence2_k<false>); }

@@ -65,6 +65,22 @@ def test_gpu_matches_oracle_unaligned(gpu_ctx, oracle, name):
             assert_bit_equal(got[role], want[role], f"{name} {dims} unaligned {role}")
 
 
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("name", K.STENCILS)
+def test_gpu_matches_oracle_odd_rows(gpu_ctx, oracle, name, offset):
+    """Rows of an odd length, whose 16-byte lanes start at any double: the last
+    lane holds one point, at the end of a tile, beside it and across tiles."""
+    spec = K.SPECS[name]
+    sizes = ([(5, 6, 7), (127, 9, 12), (129, 5, 6), (255, 6, 11), (301, 13, 9)] if spec.dim == 3
+             else [(5, 6), (127, 37), (129, 40), (255, 70), (511, 33), (513, 20)])
+    for si, dims in enumerate(sizes):
+        coefs, arrays = K.random_case(spec, dims, 1300 + si)
+        want = oracle.run(spec, dims, coefs, arrays, 2)
+        got = K.GpuBackend(gpu_ctx).run(spec, dims, coefs, arrays, 2, offset=offset)
+        for role in want:
+            assert_bit_equal(got[role], want[role], f"{name} {dims} offset {offset} {role}")
+
+
 FULL3 = (512, 256, 256)
 FULL2 = (512, 65536)
 
