@@ -199,10 +199,10 @@ template <> struct Shape<Life2Op> { static constexpr int H = 1, LL = 0, LR = 0, 
 
 // Engine configuration of op Op with storage type T, VEC points per lane, W
 // waves, prefetch depth D, KC planes per single-grid tile, LPR lanes per row,
-// XS the x-shift mode (LPR = 64 only).
+// XS the x-shift mode (LPR = 64 only), RAG rows of any length.
 template <template <class> class Op, class T, int VEC, int W, int D, int KC, int LPR = 64,
-          bool XS = false>
+          bool XS = false, bool RAG = false>
 using OpCfg = kgp::Cfg<VEC, W, Shape<Op>::H, Shape<Op>::LL, Shape<Op>::LR, Shape<Op>::ZL,
-                       Shape<Op>::ZR, D, Shape<Op>::NAUX, KC, T, LPR, false, XS>;
+                       Shape<Op>::ZR, D, Shape<Op>::NAUX, KC, T, LPR, false, XS, RAG>;
 
 }  // namespace kgops

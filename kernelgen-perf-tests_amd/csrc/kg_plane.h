@@ -156,7 +156,7 @@ __device__ __forceinline__ void bload(__amdgpu_buffer_rsrc_t r, unsigned off,
 template <class C, class V>
 __device__ __forceinline__ typename C::F xrow(const V& p, int v, int dx);
 template <int VEC_, int W_, int H_, int LL_, int LR_, int ZL_, int ZR_, int D_, int NAUX_, int KC_,
-          class T_ = F64, int LPR_ = 64, bool FULL_ = false, bool XS_ = false>
+          class T_ = F64, int LPR_ = 64, bool FULL_ = false, bool XS_ = false, bool RAG_ = false>
 struct Cfg {
     using T = T_;
     using S = typename T::S;           // storage type
@@ -182,6 +182,18 @@ struct Cfg {
     // the H halo values left of the tile and the last lane the H values right
     // of it.  One row per wave (LPR = 64).
     static constexpr bool XS = XS_;
+    // RAG: rows of any length nx >= VEC and fields at any element.  The hardware
+    // loads and stores VEC values from wherever they start; the last lane of a
+    // row that is no multiple of VEC reads the row's last VEC values and shifts
+    // them down when they are first used (shift_down), so no load leaves its
+    // row.  One value per lane, which such rows took before, against this: FP32
+    // at 333x257x131 laplacian 34 -> 22 us, wave13pt 58 -> 36, gaussblur3 39 -> 24;
+    // BF16 33 -> 21 and 47 -> 26; FP64 laplacian 42 -> 36, wave13pt 65 -> 55, lapgsrb
+    // (with LDS for every neighbour then) 72 -> 49, gaussblur3 57 -> 39.  FP64
+    // gradient, bound by its three stores, gains 3 % there and loses 14 % at
+    // 201x199x203, where its 128-point tiles make five rounds instead of nine of
+    // half the size.
+    static constexpr bool RAG = RAG_;
     static constexpr int NH = XS ? H : 1;             // halo values per ring slot
     static constexpr int RPW = 64 / LPR;             // rows per wave
     static constexpr int ROWS = W * RPW;             // tile rows, halo rows included
@@ -208,6 +220,26 @@ struct Slot {
     // row, or (x-shift mode) H values on the first and on the last lane
     F h[NH];
 };
+
+// v[i] becomes v[i + n] (the last n are then undefined), n = past % VEC; for
+// lanes whose `past` is a multiple of VEC nothing changes.
+template <class F, int VEC>
+__device__ __forceinline__ void shift_down(F (&v)[VEC], int past)
+{
+    static_assert(VEC == 1 || VEC == 2 || VEC == 4 || VEC == 8, "VEC values");
+    auto by = [&](auto width) {
+        constexpr int n = decltype(width)::value;
+        const bool on = past & n;
+        kg_static_for<VEC - n>([&](auto i) {
+            constexpr int q = decltype(i)::value;
+            const F below = v[q], above = v[q + n];   // values: a choice of lvalues would go to memory
+            v[q] = on ? above : below;
+        });
+    };
+    if constexpr (VEC > 4) by(std::integral_constant<int, 4>{});
+    if constexpr (VEC > 2) by(std::integral_constant<int, 2>{});
+    if constexpr (VEC > 1) by(std::integral_constant<int, 1>{});
+}
 
 // Wave-wide DPP lane shifts (GFX9 family): wave_shr:1 gives lane i the value
 // of lane i-1, wave_shl:1 that of lane i+1; the lane without a source (0 or
@@ -359,10 +391,15 @@ __device__ __forceinline__ typename C::F xrow(const V& p, int v, int dx)
 // wait for loads issued in the same iteration.  The planes the ring and LDS
 // need are all < ns (the stencil reach ZHI <= the z-boundary width), so
 // slots whose load is skipped are never read.
+//
+// past (C::RAG): how many of the lane's values lie past the end of its row.
 template <class C, bool SYNC = true, class Load, class LoadAux, class Stage, class Compute>
-__device__ __forceinline__ void march(int k0, int k1, Load&& load, LoadAux&& load_aux,
+__device__ __forceinline__ void march(int k0, int k1, int past, Load&& load, LoadAux&& load_aux,
                                       Stage&& stage, Compute&& compute)
 {
+    auto enter = [&](typename C::F (&v)[C::VEC]) {
+        if constexpr (C::RAG) shift_down(v, past);
+    };
     using F = typename C::F;
     Slot<F, C::VEC, C::NH> ring[C::NP];
     ASlot<F, C::VEC, C::NA> aux[C::NP];
@@ -377,6 +414,8 @@ __device__ __forceinline__ void march(int k0, int k1, Load&& load, LoadAux&& loa
     for (int r = 0; r < C::RS; r++) load(k0 - C::ZLO + r, ring[r], true);
 #pragma unroll
     for (int d = 0; d < C::D; d++) load_aux(k0 + d, aux[d], true);
+#pragma unroll
+    for (int r = 0; r < C::ZLO + C::ZHI; r++) enter(ring[r].v);
     // LDS planes k0-LL .. k0+LR-1 (outside the ring when LL > ZL)
 #pragma unroll
     for (int dz = -C::LL; dz < C::LR; dz++) {
@@ -389,16 +428,20 @@ __device__ __forceinline__ void march(int k0, int k1, Load&& load, LoadAux&& loa
 #pragma unroll
             for (int v = 0; v < C::VEC; v++) t.v[v] = F(0);
             load(k0 + dz, t, true);
+            enter(t.v);
             stage(k0 + dz, t);
         }
     }
     auto plane = [&](auto phase, int k) {
         constexpr int P = decltype(phase)::value;
+        enter(ring[(P + C::ZLO + C::ZHI) % C::NP].v);
         stage(k + C::LR, ring[(P + C::ZLO + C::LR) % C::NP]);
         const int kp = k + C::ZHI + C::D;   // plane entering the ring
         load(kp, ring[(P + C::RS) % C::NP], kp <= k1 - 1 + C::ZHI);
         load_aux(k + C::D, aux[(P + C::D) % C::NP], k + C::D < k1);
         if constexpr (SYNC) __syncthreads();
+#pragma unroll
+        for (int a = 0; a < C::NAUX; a++) enter(aux[P % C::NP].a[a]);
         compute(phase, k, ring, aux);
     };
     int k = k0;
@@ -454,7 +497,9 @@ __device__ __forceinline__ void plane_tile(typename C::F* lds, int nx, int ny,
     // nothing to load).  Planes are addressed through one resource each:
     // base + k*sz, sz*sizeof(S) bytes (at most 2^31; the launchers check).
     const unsigned plane_bytes = (unsigned)(sz * (long long)sizeof(S));
-    const unsigned off_v = p_ok[0] ? (unsigned)(((long long)j * sy + x) * (long long)sizeof(S)) : KG_OOB;
+    const int past = C::RAG && x < nx ? max(x + C::VEC - nx, 0) : 0;
+    const unsigned off_v = p_ok[0] ? (unsigned)(((long long)j * sy + x - past) * (long long)sizeof(S))
+                                   : KG_OOB;
     unsigned off_h[C::NH];
 #pragma unroll
     for (int i = 0; i < C::NH; i++) {
@@ -470,9 +515,9 @@ __device__ __forceinline__ void plane_tile(typename C::F* lds, int nx, int ny,
 
     // One access per lane and slot (VEC values, then the halo value); values
     // a lane does not load (zeros) are never read for an interior point.  With
-    // VEC > 1 every lane with x < nx reads VEC values: callers guarantee that
-    // rows hold a multiple of VEC elements (nx % VEC == 0 in the dense
-    // layout, padded rows otherwise).
+    // VEC > 1 every lane with x < nx reads VEC values: unless C::RAG, callers
+    // guarantee that rows hold a multiple of VEC elements (nx % VEC == 0 in the
+    // dense layout, padded rows otherwise).
     auto load = [&](int k, Slot<F, C::VEC, C::NH>& s, bool want) {
         const __amdgpu_buffer_rsrc_t r = plane_rsrc(op.src, k, want);
         bload<T, C::VEC>(r, off_v, s.v);
@@ -514,7 +559,7 @@ __device__ __forceinline__ void plane_tile(typename C::F* lds, int nx, int ny,
     bool xmask[C::VEC];
 #pragma unroll
     for (int v = 0; v < C::VEC; v++) xmask[v] = x + v >= LO && x + v < nx - HI;
-    march<C>(k0, k1, load, load_aux, stage, [&](auto phase, int k, const auto& ring, const auto& aux) {
+    march<C>(k0, k1, past, load, load_aux, stage, [&](auto phase, int k, const auto& ring, const auto& aux) {
         constexpr int P = decltype(phase)::value;
         if (comp_row) {
             View<C, P> vw{lds, ring, aux, k, row, c, x < sy};
@@ -620,7 +665,7 @@ __device__ __forceinline__ void packed_tile(typename C::F* lds, int nx, int ny, 
     bool xmask[C::VEC];
 #pragma unroll
     for (int v = 0; v < C::VEC; v++) xmask[v] = x + v >= LO && x + v < nx - HI;
-    march<C>(k0, k1, load, load_aux, stage, [&](auto phase, int k, const auto& ring, const auto& aux) {
+    march<C>(k0, k1, 0, load, load_aux, stage, [&](auto phase, int k, const auto& ring, const auto& aux) {
         constexpr int P = decltype(phase)::value;
         if (comp_row) {
             PView<C, P> vw{L0, ring, aux, k, lane, cpr, true};
@@ -707,20 +752,6 @@ __device__ __forceinline__ void rows2_tile(int nx, int ny, long long sy, long lo
     });
 }
 
-// Single-grid launch of the direct row body over every plane of a dense
-// grid: tiles enumerated x fastest, then y, then plane, in tile order ORD
-// (kg_tile_order).
-template <class C, int LO, int HI, class Op, int PY, int ORD = 0>
-__global__ __launch_bounds__(64 * C::W)
-void rows2_kernel(int nx, int ny, int ntx, int nty, Op op)
-{
-    const unsigned b = kg_tile_order<ORD>(blockIdx.x, gridDim.x, (unsigned)ntx);
-    const int bx = (int)(b % (unsigned)ntx);
-    const int by = (int)((b / (unsigned)ntx) % (unsigned)nty);
-    const int k = (int)(b / ((unsigned)ntx * (unsigned)nty));
-    rows2_tile<C, LO, HI, Op, PY>(nx, ny, nx, (long long)nx * ny, bx, by, k, op);
-}
-
 // ------------------------------------------------------------ column march
 // For stencils that read only the xy-plane they write (gaussblur per plane,
 // the 2D kinds).  A wave owns one row piece of 64*VEC points of one plane
@@ -781,7 +812,8 @@ __device__ __forceinline__ void colmarch_tile(int nx, int ny, int ns, long long 
     if (k >= ns || y0 >= y1) return;
     const int x0 = bx * ColMarch<C>::TXW;
     const int x = x0 + lane * C::VEC;
-    const unsigned off_v = x < nx ? (unsigned)((long long)x * (long long)sizeof(S)) : KG_OOB;
+    const int past = C::RAG && x < nx ? max(x + C::VEC - nx, 0) : 0;
+    const unsigned off_v = x < nx ? (unsigned)((long long)(x - past) * (long long)sizeof(S)) : KG_OOB;
     // the H halo points of lane 0 (left of the piece) or lane 63 (right of
     // it) in one load: they lie in one row whenever the first does (nx and
     // x0 are multiples of VEC >= H), and start H*sizeof(S)-aligned
@@ -796,7 +828,16 @@ __device__ __forceinline__ void colmarch_tile(int nx, int ny, int ns, long long 
         const __amdgpu_buffer_rsrc_t r = make_rsrc(plane + (long long)(ok ? jr : 0) * sy,
                                                    ok ? row_bytes : 0u);
         bload<T, C::VEC>(r, off_v, s.v);
-        bload<T, C::NH>(r, off_h, s.h);
+        if constexpr (C::RAG) {   // the row may end between them
+#pragma unroll
+            for (int i = 0; i < C::NH; i++) {
+                F h[1];
+                bload<T, 1>(r, hx + i < nx ? off_h + i * (unsigned)sizeof(S) : KG_OOB, h);
+                s.h[i] = h[0];
+            }
+        } else {
+            bload<T, C::NH>(r, off_h, s.h);
+        }
     };
     auto no_aux = [&](int, ASlot<F, C::VEC, C::NA>&, bool) {};
     auto no_stage = [&](int, const Slot<F, C::VEC, C::NH>&) {};
@@ -814,7 +855,7 @@ __device__ __forceinline__ void colmarch_tile(int nx, int ny, int ns, long long 
             out[C::H + i] = dpp_shift<KG_DPP_WAVE_SHL1>(r.h[i], r.v[i]);
         }
     };
-    march<C, false>(y0, y1, load, no_aux, no_stage,
+    march<C, false>(y0, y1, past, load, no_aux, no_stage,
                     [&](auto phase, int j, const auto& ring, const auto&) {
         constexpr int P = decltype(phase)::value;
         if (j == y0) {   // the first row: the rows below and above it enter together

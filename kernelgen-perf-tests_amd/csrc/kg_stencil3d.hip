@@ -335,8 +335,8 @@ struct LapgsrbOp {
 #ifndef KG_WAVE_XS
 #define KG_WAVE_XS 0
 #endif
-template <int V> using LapCfg = kgp::Cfg<V, KG_LAP_W, 1, 0, 0, 1, 1, KG_LAP_D, 0, KG_LAP_KC,
-                                         kgp::F64, 64, false, V == 2 && KG_LAP_XS>;
+template <bool RAG> using LapCfg = kgp::Cfg<2, KG_LAP_W, 1, 0, 0, 1, 1, KG_LAP_D, 0, KG_LAP_KC,
+                                            kgp::F64, 64, false, KG_LAP_XS, RAG>;
 // gradient: W=12/D=2/KC=8 in chunks of 2 tile rows, one workgroup (12 waves)
 // per CU: 196 us (W=8 with 2 workgroups 201, 3 workgroups 208; W=12 with 2
 // 213; W=16 with 1 214; KC=16 224, D=3 209, XCD-contiguous 219).
@@ -346,10 +346,10 @@ template <int V> using LapCfg = kgp::Cfg<V, KG_LAP_W, 1, 0, 0, 1, 1, KG_LAP_D, 0
 #ifndef KG_GRAD_OCC
 #define KG_GRAD_OCC 1
 #endif
-template <int V> using GradCfg = kgp::Cfg<V, KG_GRAD_W, 1, 0, 0, 1, 1, 2, 0, 8, kgp::F64, 64, false,
-                                          V == 2 && KG_GRAD_XS>;
-template <int V> using WaveCfg = kgp::Cfg<V, 12, 2, 0, 0, 2, 2, 3, 1, 32, kgp::F64, 64, false,
-                                          V == 2 && KG_WAVE_XS>;
+template <bool RAG> using GradCfg = kgp::Cfg<2, KG_GRAD_W, 1, 0, 0, 1, 1, 2, 0, 8, kgp::F64, 64,
+                                             false, KG_GRAD_XS, RAG>;
+template <bool RAG> using WaveCfg = kgp::Cfg<2, 12, 2, 0, 0, 2, 2, 3, 1, 32, kgp::F64, 64, false,
+                                             KG_WAVE_XS, RAG>;
 // lapgsrb: 16-byte lanes (even nx, 16-byte aligned fields) take every
 // same-row x-neighbour, in planes k-1 .. k+1, from the neighbouring lanes'
 // registers by DPP shifts (x-shift mode), which leaves LDS only the 12
@@ -388,29 +388,28 @@ template <int V> using WaveCfg = kgp::Cfg<V, 12, 2, 0, 0, 2, 2, 3, 1, 32, kgp::F
 #ifndef KG_GSRB_WGPC
 #define KG_GSRB_WGPC 1
 #endif
-template <int V> using GsrbCfg = kgp::Cfg<V, (V == 2 ? KG_GSRB_W : 12), 2, 1, 1, 2, 2, KG_GSRB_D, 0,
-                                          KG_GSRB_KC, kgp::F64, 64, false, V == 2>;
+template <bool RAG> using GsrbCfg = kgp::Cfg<2, KG_GSRB_W, 2, 1, 1, 2, 2, KG_GSRB_D, 0, KG_GSRB_KC,
+                                             kgp::F64, 64, false, true, RAG>;
 #ifndef KG_WAVE_WGPC
 #define KG_WAVE_WGPC 0
 #endif
 
-// Launch Op on the plane engine; 16-byte lanes (VEC=2) need an even nx and
-// 16-byte aligned fields (al).
+// Launch Op on the plane engine, in the ragged form for an odd nx or fields that
+// are not 16-byte aligned (al).
 // ORD: tile order (kg_tile_order).  WGPC > 0: z-chunks longer than C::KC
 // planes when the launch would otherwise exceed about WGPC workgroups per
 // compute unit (each workgroup then marches further and fills its pipeline
 // fewer times); WGPC = 0 keeps C::KC.  OCC > 0: at most OCC resident
 // workgroups per compute unit, enforced by reserving unused dynamic LDS.
-template <template <int> class CfgT, template <class> class OpT, int LO, int HI, int ORD = 1,
+template <template <bool> class CfgT, template <class> class OpT, int LO, int HI, int ORD = 1,
           int WGPC = 0, int OCC = 0, class Fill>
 static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, Fill fill)
 {
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
     if (int rc = kg_check_plane_bytes((long long)nx * ny, 8)) return rc;
-    auto go = [&](auto vtag) -> int {
-        constexpr int V = decltype(vtag)::value;
-        using C = CfgT<V>;
+    auto go = [&](auto ragged) -> int {
+        using C = CfgT<decltype(ragged)::value>;
         using Op = OpT<C>;
         Op op{};
         fill(op);
@@ -437,8 +436,7 @@ static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
                       op);
         return kg_launch_end(ctx);
     };
-    if (nx % 2 == 0 && al) return go(std::integral_constant<int, 2>{});
-    return go(std::integral_constant<int, 1>{});
+    return nx % 2 == 0 && al ? go(std::false_type{}) : go(std::true_type{});
 }
 
 }  // namespace

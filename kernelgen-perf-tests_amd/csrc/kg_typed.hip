@@ -63,9 +63,6 @@
 #ifndef KG_GB3_YC32
 #define KG_GB3_YC32 16
 #endif
-#ifndef KG_ORD_ROWS2
-#define KG_ORD_ROWS2 0
-#endif
 
 namespace {
 
@@ -74,8 +71,29 @@ using namespace kgops;
 #define KG_REQUIRE(cond, msg) \
     do { if (!(cond)) return kg_set_error(KG_ERR_INVALID, "%s", msg); } while (0)
 
-// Single-grid launch of op Op in storage type T: 16-byte lanes (VEC = VMAX)
-// when nx is a multiple of VMAX, else one point per lane.
+// f(lanes per row as a constant) for rows of nx points, vec per lane.  BF16 rows of
+// 64 lanes are 512 points wide; narrower rows take 32 or 16 lanes (two or four
+// rows per wave) where fewer lanes then lie past the row's end, 32 counted 5 %
+// and 16 20 % dearer (what they cost on rows they fit: at 512 points 31, 31 and
+// 35 us).  Laplacian / wave13pt with 64, 32 and 16 lanes: 201x199x203 24 / 31, 12
+// / 19, 16 / 21 us; 301x203x151 21 / 25, 18 / 25, 17 / 23; 256^3 27 / 40, 25 /
+// 26, 26 / 26.  FP32 and FP64 tiles are half and a quarter as wide and gained
+// nothing (FP32 201x199x203 15, 18, 22).
+template <bool FOLD, class Fn>
+int with_lanes(int nx, int vec, Fn&& f)
+{
+    if constexpr (FOLD) {
+        auto lanes = [&](int lpr) { return (long long)((nx + lpr * vec - 1) / (lpr * vec)) * lpr; };
+        const long long t64 = lanes(64) * 100, t32 = lanes(32) * 105, t16 = lanes(16) * 120;
+        if (t16 < t32 && t16 < t64) return f(std::integral_constant<int, 16>{});
+        if (t32 < t64) return f(std::integral_constant<int, 32>{});
+    }
+    return f(std::integral_constant<int, 64>{});
+}
+
+// Single-grid launch of op Op in storage type T with 16-byte lanes (VEC = VMAX),
+// in the ragged form where nx is no multiple of VMAX or a field not aligned;
+// rows shorter than a lane take one point per lane.
 template <template <class> class OpT, class T, int VMAX, int W, int D, int KC, int ORD = KG_ORD_TYPED,
           class Fill>
 static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, Fill fill)
@@ -85,9 +103,10 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
     if (int rc = kg_check_plane_bytes((long long)nx * ny, (int)sizeof(typename T::S))) return rc;
     constexpr int LO = Bounds<OpT>::LO, HI = Bounds<OpT>::HI;
     constexpr int ZLO = Bounds<OpT>::ZLO, ZHI = Bounds<OpT>::ZHI;
-    auto go = [&](auto vtag) -> int {
+    auto go = [&](auto vtag, auto ragged, auto lanes) -> int {
         constexpr int V = decltype(vtag)::value;
-        using C = OpCfg<OpT, T, V, W, D, KC, 64, (V > 1) && KG_TYPED_XS>;
+        using C = OpCfg<OpT, T, V, W, D, KC, decltype(lanes)::value, (V > 1) && KG_TYPED_XS,
+                        decltype(ragged)::value>;
         using Op = OpT<C>;
         Op op{};
         fill(op);
@@ -102,43 +121,17 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
                       op);
         return kg_launch_end(ctx);
     };
-    if (nx % VMAX == 0 && al) return go(std::integral_constant<int, VMAX>{});
-    return go(std::integral_constant<int, 1>{});
-}
-
-// Per-plane stencils (gaussblur3) on the direct row body when nx % VEC == 0
-// and the fields are 16-byte aligned, else on the plane engine.  W waves
-// stacked in y per tile, PY output rows per lane.  Measured at 512^3 (cold):
-// FP64 W=8/PY=4 415 us (plane engine 492, PY=8 426, W=16 997); FP32
-// W=8/PY=8 232 us (plane engine 257, PY=4 267, PY=16 239).
-template <template <class> class OpT, class T, int VEC, int W, int PY, class Fill>
-static int launch_rows2(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, Fill fill)
-{
-    if (nx % VEC != 0 || !al) return launch_typed<OpT, T, VEC, 8, 2, 16>(ctx, name, nx, ny, ns, al, fill);
-    if (int rc = kg_check_ctx(ctx)) return rc;
-    if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
-    constexpr int LO = Bounds<OpT>::LO, HI = Bounds<OpT>::HI;
-    static_assert(Bounds<OpT>::ZLO == 0 && Bounds<OpT>::ZHI == 0, "every plane computed");
-    using C = OpCfg<OpT, T, VEC, W, 2, 16>;
-    using R2 = kgp::Rows2<C, PY>;
-    using Op = OpT<C>;
-    Op op{};
-    fill(op);
-    const int nxi = nx - LO - HI, nyi = ny - LO - HI;
-    const int ntx = (nx + R2::TXW - 1) / R2::TXW, nty = nyi > 0 ? (nyi + R2::TY - 1) / R2::TY : 0;
-    auto kern = kgp::rows2_kernel<C, LO, HI, Op, PY, KG_ORD_ROWS2>;
-    kg_register_kernel(name, (const void*)kern);
-    if (int rc = kg_launch_begin(ctx, name)) return rc;
-    if (nxi > 0 && nyi > 0 && ns > 0)
-        kg_launch(ctx, kern, dim3((unsigned)ntx * (unsigned)nty * (unsigned)ns), dim3(64 * C::W), 0,
-                  nx, ny, ntx, nty, op);
-    return kg_launch_end(ctx);
+    if (nx < VMAX)
+        return go(std::integral_constant<int, 1>{}, std::false_type{}, std::integral_constant<int, 64>{});
+    return with_lanes<sizeof(typename T::S) == 2>(nx, VMAX, [&](auto lanes) {
+        std::integral_constant<int, VMAX> v;
+        return nx % VMAX == 0 && al ? go(v, std::false_type{}, lanes) : go(v, std::true_type{}, lanes);
+    });
 }
 
 // Per-plane stencils on the column march (kgp::colmarch_tile): W waves per
-// workgroup, each marching YC rows of one plane with a D-row prefetch.  Same
-// requirements as the direct row body (nx % VEC == 0, 16-byte aligned
-// fields), else the plane engine.  gaussblur3 at 512^3, levels rotated,
+// workgroup, each marching YC rows of one plane with a D-row prefetch; rows of
+// any length and alignment (the ragged form).  gaussblur3 at 512^3, levels rotated,
 // first ten launches: FP32 W=4/D=4/YC=16 214 us against 255-264 on the
 // direct row body (YC=8 214, 12 225, 32 238, 64 256: fewer workgroups leave
 // a tail); FP64 W=4/D=2/YC=16 418 us against 451-472.  Keeping each row's
@@ -164,33 +157,33 @@ static int launch_rows2(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
 #ifndef KG_ORD_CM32
 #define KG_ORD_CM32 0
 #endif
-#ifndef KG_GB3_ENGINE
-#define KG_GB3_ENGINE 1
-#endif
 template <template <class> class OpT, class T, int VEC, int W, int D, int YC, int ORD, class Fill>
 static int launch_colmarch(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, Fill fill)
 {
-    if (nx % VEC != 0 || !al) return launch_typed<OpT, T, VEC, 8, 2, 16>(ctx, name, nx, ny, ns, al, fill);
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
     if (int rc = kg_check_plane_bytes((long long)nx * ny, (int)sizeof(typename T::S))) return rc;
     constexpr int LO = Bounds<OpT>::LO, HI = Bounds<OpT>::HI;
     static_assert(Bounds<OpT>::ZLO == 0 && Bounds<OpT>::ZHI == 0, "every plane computed");
     constexpr int H = Shape<OpT>::H;
-    using C = kgp::Cfg<VEC, W, H, 0, 0, H, H, D, 0, YC, T, 64, false, true>;
-    using Op = OpT<C>;
-    Op op{};
-    fill(op);
-    const int nxi = nx - LO - HI, nyi = ny - LO - HI;
-    const int ntx = (nx + kgp::ColMarch<C>::TXW - 1) / kgp::ColMarch<C>::TXW;
-    const int nty = nyi > 0 ? (nyi + W * YC - 1) / (W * YC) : 0;
-    auto kern = kgp::colmarch_kernel<C, LO, HI, Op, ORD>;
-    kg_register_kernel(name, (const void*)kern);
-    if (int rc = kg_launch_begin(ctx, name)) return rc;
-    if (nxi > 0 && nyi > 0 && ns > 0)
-        kg_launch(ctx, kern, dim3((unsigned)ntx * (unsigned)nty * (unsigned)ns), dim3(64 * W), 0,
-                  nx, ny, ns, ntx, nty, YC, op);
-    return kg_launch_end(ctx);
+    static_assert(VEC <= LO + HI + 1, "a row with an interior fills a lane");
+    auto go = [&](auto ragged) -> int {
+        using C = kgp::Cfg<VEC, W, H, 0, 0, H, H, D, 0, YC, T, 64, false, true, decltype(ragged)::value>;
+        using Op = OpT<C>;
+        Op op{};
+        fill(op);
+        const int nxi = nx - LO - HI, nyi = ny - LO - HI;
+        const int ntx = (nx + kgp::ColMarch<C>::TXW - 1) / kgp::ColMarch<C>::TXW;
+        const int nty = nyi > 0 ? (nyi + W * YC - 1) / (W * YC) : 0;
+        auto kern = kgp::colmarch_kernel<C, LO, HI, Op, ORD>;
+        kg_register_kernel(name, (const void*)kern);
+        if (int rc = kg_launch_begin(ctx, name)) return rc;
+        if (nxi > 0 && nyi > 0 && ns > 0)
+            kg_launch(ctx, kern, dim3((unsigned)ntx * (unsigned)nty * (unsigned)ns), dim3(64 * W), 0,
+                      nx, ny, ns, ntx, nty, YC, op);
+        return kg_launch_end(ctx);
+    };
+    return nx % VEC == 0 && al ? go(std::false_type{}) : go(std::true_type{});
 }
 
 // ------------------------------------------------------------ statistics
@@ -463,11 +456,7 @@ extern "C" int kg_gaussblur3_f64(kg_ctx* ctx, int nx, int ny, int ns, double s0,
     KG_REQUIRE(w0 && w1, "kg_gaussblur3_f64: null buffer");
     KG_REQUIRE(w0 != w1, "kg_gaussblur3_f64: w0 and w1 must be distinct");
     const double f = 1. / (s0 + 4 * (s1 + s2 + s4 + s8) + 8 * s5);   // gaussblur/gaussblur.c:65
-#if KG_GB3_ENGINE == 1
     return launch_colmarch<Gaussblur3Op, kgp::F64, 2, KG_GB3_W64, KG_GB3_D64, KG_GB3_YC64, KG_ORD_CM64>(ctx, "gaussblur3_f64", nx, ny, ns,
-#else
-    return launch_rows2<Gaussblur3Op, kgp::F64, 2, 8, 4>(ctx, "gaussblur3_f64", nx, ny, ns,
-#endif
                                                              kg_aligned16(w0, w1), [&](auto& op) {
         op.src = w0;
         op.dst = w1;
@@ -487,11 +476,7 @@ extern "C" int kg_gaussblur3_f32(kg_ctx* ctx, int nx, int ny, int ns, float s0, 
     KG_REQUIRE(w0 && w1, "kg_gaussblur3_f32: null buffer");
     KG_REQUIRE(w0 != w1, "kg_gaussblur3_f32: w0 and w1 must be distinct");
     const float f = 1.f / (s0 + 4 * (s1 + s2 + s4 + s8) + 8 * s5);
-#if KG_GB3_ENGINE == 1
     return launch_colmarch<Gaussblur3Op, kgp::F32, 4, KG_GB3_W32, KG_GB3_D32, KG_GB3_YC32, KG_ORD_CM32>(ctx, "gaussblur3_f32", nx, ny, ns,
-#else
-    return launch_rows2<Gaussblur3Op, kgp::F32, 4, 8, 8>(ctx, "gaussblur3_f32", nx, ny, ns,
-#endif
                                                              kg_aligned16(w0, w1), [&](auto& op) {
         op.src = w0;
         op.dst = w1;

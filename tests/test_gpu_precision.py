@@ -301,3 +301,19 @@ def test_typed_rejects_aliasing(gpu_ctx, kgmod):
         gpu_ctx.call("wave13pt_bf16", 4, 4, 4, 0.1, 0.2, 0.3, a, a, a)
     with pytest.raises(kgmod.KGError):
         gpu_ctx.field_stats(a, 7)
+
+
+@pytest.mark.parametrize("which,dtype", [("laplacian", "f32"), ("laplacian", "bf16"),
+                                         ("wave13pt", "f32"), ("wave13pt", "bf16"),
+                                         ("gaussblur3", "f32"), ("gaussblur3", "f64")])
+def test_typed_ragged_rows(gpu_ctx, oracle, which, dtype):
+    """Rows that are no multiple of a 16-byte lane, by every remainder: shorter
+    than a lane, around the 16-, 32- and 64-lane pieces, and past them."""
+    fn = f"{which}_{dtype}"
+    for si, nx in enumerate([5, 7, 9, 11, 63, 65, 127, 130, 131, 253, 255, 257, 258, 266, 511, 517, 1030]):
+        dims = (nx, 9 + si % 5, 6 + si % 3)
+        ins, out, coefs, rot = _case(which, dtype, dims, 400 + si)
+        got = _run_gpu(gpu_ctx, fn, dims, coefs, ins, out, 2, rot)
+        want = _run_oracle(oracle.lib, fn, dims, coefs, ins, out, 2, rot, f64 if dtype == "f64" else f32)
+        for g, w in zip(got, want):
+            assert g.tobytes() == w.tobytes(), f"{fn} {dims}"
