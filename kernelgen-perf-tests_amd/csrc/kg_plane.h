@@ -187,12 +187,10 @@ struct Cfg {
     // row that is no multiple of VEC reads the row's last VEC values and shifts
     // them down when they are first used (shift_down), so no load leaves its
     // row.  One value per lane, which such rows took before, against this: FP32
-    // at 333x257x131 laplacian 34 -> 22 us, wave13pt 58 -> 36, gaussblur3 39 -> 24;
-    // BF16 33 -> 21 and 47 -> 26; FP64 laplacian 42 -> 36, wave13pt 65 -> 55, lapgsrb
-    // (with LDS for every neighbour then) 72 -> 49, gaussblur3 57 -> 39.  FP64
-    // gradient, bound by its three stores, gains 3 % there and loses 14 % at
-    // 201x199x203, where its 128-point tiles make five rounds instead of nine of
-    // half the size.
+    // at 333x257x131 laplacian 35 -> 25 us, wave13pt 59 -> 38, gaussblur3 42 -> 29;
+    // BF16 34 -> 18 and 49 -> 27; FP64 laplacian 46 -> 40, gradient 91 -> 82, wave13pt
+    // 65 -> 56, lapgsrb (with LDS for every neighbour then) 72 -> 50, gaussblur3 58
+    // -> 44.
     static constexpr bool RAG = RAG_;
     static constexpr int NH = XS ? H : 1;             // halo values per ring slot
     static constexpr int RPW = 64 / LPR;             // rows per wave

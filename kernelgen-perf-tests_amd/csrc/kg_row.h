@@ -24,7 +24,7 @@ typedef double d2 __attribute__((ext_vector_type(2)));
 typedef d2 d2u __attribute__((aligned(8)));   // at any double
 
 template <int VEC_, int W_, int H_, int NF_, int LL_, int LR_, int ZL_, int ZR_, int D_, int NAUX_,
-          int YC_>
+          int YC_, bool RAG_ = false>
 struct Cfg {
     static constexpr int VEC = VEC_;   // points per lane along x (1 or 2)
     static constexpr int W = W_;       // waves side by side along x
@@ -37,6 +37,8 @@ struct Cfg {
     static constexpr int D = D_;       // prefetch distance (rows)
     static constexpr int NAUX = NAUX_; // side streams read at the point only
     static constexpr int YC = YC_;     // rows per workgroup
+    // rows of any length nx >= VEC and fields at any double (kgp::Cfg::RAG)
+    static constexpr bool RAG = RAG_;
     static constexpr int TXW = W * 64 * VEC;
     static constexpr int LW = TXW + 2 * H;
     static constexpr int NLS = LL + LR + 2;
@@ -120,8 +122,14 @@ void row_kernel(int nx, int ny, int ntx, Op op)
     const int hcol = hx < 0 ? -1 : hx - x0 + C::H;
     const bool h_ok = hx >= 0 && hx < nx;
     // Per-lane byte offsets within a row (kgp::KG_OOB: nothing to load).  With
-    // VEC = 2 callers guarantee an even nx, so a lane with x < nx may read two.
-    const unsigned off_v = x < nx ? (unsigned)x * 8u : kgp::KG_OOB;
+    // VEC = 2 a lane with x < nx reads two points: callers guarantee an even nx,
+    // or with C::RAG the last lane of an odd row reads the row's last two and
+    // shifts them when they are first used (enter).
+    const int past = C::RAG && x < nx ? max(x + C::VEC - nx, 0) : 0;
+    auto enter = [&](double (&v)[C::VEC]) {
+        if constexpr (C::RAG) kgp::shift_down(v, past);
+    };
+    const unsigned off_v = x < nx ? (unsigned)(x - past) * 8u : kgp::KG_OOB;
     const unsigned off_h = h_ok ? (unsigned)hx * 8u : kgp::KG_OOB;
     const unsigned row_bytes = (unsigned)nx * 8u;
     // Resource for row `row` of array base; empty unless want and 0 <= row < ny.
@@ -165,6 +173,10 @@ void row_kernel(int nx, int ny, int ntx, Op op)
 #pragma unroll
     for (int d = 0; d < C::D; d++) load_aux(j0 + d, aux[d]);
 #pragma unroll
+    for (int f = 0; f < C::NF; f++)
+#pragma unroll
+        for (int r = 0; r < C::ZL + C::ZHI; r++) enter(ring[f][r].v);
+#pragma unroll
     for (int dy = -C::LL; dy < C::LR; dy++)
 #pragma unroll
         for (int f = 0; f < C::NF; f++) {
@@ -173,6 +185,7 @@ void row_kernel(int nx, int ny, int ntx, Op op)
             } else {
                 Slot<C::VEC> t;
                 load(f, j0 + dy, t);
+                enter(t.v);
                 stage(f, j0 + dy, t);
             }
         }
@@ -184,12 +197,16 @@ void row_kernel(int nx, int ny, int ntx, Op op)
     auto row_step = [&](auto phase, int j) {
         constexpr int P = decltype(phase)::value;
 #pragma unroll
+        for (int f = 0; f < C::NF; f++) enter(ring[f][(P + C::ZL + C::ZHI) % C::NP].v);
+#pragma unroll
         for (int f = 0; f < C::NF; f++) stage(f, j + C::LR, ring[f][(P + C::ZL + C::LR) % C::NP]);
         const int jp = j + C::ZHI + C::D;
 #pragma unroll
         for (int f = 0; f < C::NF; f++) load(f, jp, ring[f][(P + C::RS) % C::NP], jp <= j1 - 1 + C::ZHI);
         load_aux(j + C::D, aux[(P + C::D) % C::NP], j + C::D < j1);
         __syncthreads();
+#pragma unroll
+        for (int a = 0; a < C::NAUX; a++) enter(aux[P % C::NP].a[a]);
         View<C, P> vw{lds, (const Slot<C::VEC>(*)[C::NP])ring, aux, j, col};
         op.run(vw, (long long)j * nx, x, xmask);
     };

@@ -138,42 +138,58 @@ struct WhisperingOp {
     }
 };
 
-// Row shapes from sweeps at 512x65536 (cold caches, 40-launch means) with
-// the prefetch rings kept in flight: jacobi/gameoflife D=2/YC=64 113 us (D=4
-// 141, W=8 118); gaussblur D=2/YC=32 116 us (D=3/YC=64 140); whispering with
-// 16-byte lanes, W=4/D=2/YC=8 589 us (8-byte lanes 610-643; later, first ten
-// launches of each: YC=4 584 us, 6 616, 12 644; D=1 633, D=3 584; hardware
-// and chunked tile orders 606 and 586, against 585-588 for this shape).
-// Whispering takes 258 registers, one wave per SIMD; held to 256 (two waves
-// per SIMD, 3 values spilled) it ran slower: 614-618 us against 572-573
-// (YC=6 615-628, 12 631-634, 16 660; D=1 605-622).
-//                     VEC W      H  NF LL LR ZL ZR D  NAUX YC
-template <int V> using WhCfg = kgr::Cfg<V, 8 / V, 1, 5, 0, 0, 1, 1, 2, 3, 8>;
+#ifndef KG_ORD_WH
+#define KG_ORD_WH 1
+#endif
+// Row shape of whispering from sweeps at 512x65536 (cold caches, 40-launch
+// means) with the prefetch rings kept in flight: 16-byte lanes, W=4/D=2/YC=8 589
+// us (8-byte lanes 610-643; later, first ten launches of each: YC=4 584 us, 6
+// 616, 12 644; D=1 633, D=3 584; hardware and chunked tile orders 606 and 586,
+// against 585-588 for this shape).  It takes 258 registers, one wave per SIMD;
+// held to 256 (two waves per SIMD, 3 values spilled) it ran slower: 614-618 us
+// against 572-573 (YC=6 615-628, 12 631-634, 16 660; D=1 605-622).
+// The tile is as many waves wide as fit the row (W: 1, 2 or 4 pieces of 128
+// points), so that narrow rows leave few lanes idle, and 2 rows high instead of
+// 8 (constants both: with the rows a launch argument the 512x65536 launch took
+// 627 us) where 8 would leave less than two waves per compute unit.  Cold
+// caches, against 512-point tiles of 8 rows (of 8-byte lanes where nx is odd):
+// 64x1024 13 -> 8 us, 100x4800 33 -> 14, 128x16384 87 -> 57, 200x40000 213 -> 162,
+// 301x30653 235 -> 198, 333x33667 269 -> 230, 511x60000 607 -> 569, 640x40000 528
+// -> 480; 512x65536 and 1000x10000 as before.
+//                                                    VEC W  H  NF LL LR ZL ZR D  NAUX YC
+template <int W, int YC, bool RAG> using WhCfg = kgr::Cfg<2, W, 1, 5, 0, 0, 1, 1, 2, 3, YC, RAG>;
 
-// Launch Op on the row engine; 16-byte lanes (VEC=2) need an even nx and
-// 16-byte aligned fields (al).
-template <template <int> class CfgT, template <class> class OpT, int LO, int HI, int VEC_EVEN,
-          int ORD = 1, class Fill>
-static int launch_row(kg_ctx* ctx, const char* name, int nx, int ny, bool al, Fill fill)
+// Launch whispering on the row engine, in the ragged form for an odd nx or
+// fields that are not 16-byte aligned (al).
+template <class Fill>
+static int launch_whispering(kg_ctx* ctx, int nx, int ny, bool al, Fill fill)
 {
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims2(nx, ny)) return rc;
-    auto go = [&](auto vtag) -> int {
-        constexpr int V = decltype(vtag)::value;
-        using C = CfgT<V>;
-        using Op = OpT<C>;
+    auto go = [&](auto w, auto yc, auto ragged) -> int {
+        using C = WhCfg<decltype(w)::value, decltype(yc)::value, decltype(ragged)::value>;
+        using Op = WhisperingOp<C>;
         Op op{};
         fill(op);
-        const kgr::Grid g = kgr::make_grid<C>(nx, ny, LO, HI);
-        auto kern = kgr::row_kernel<C, LO, HI, Op, ORD>;
-        kg_register_kernel(name, (const void*)kern);
-        if (int rc = kg_launch_begin(ctx, name)) return rc;
+        const kgr::Grid g = kgr::make_grid<C>(nx, ny, 1, 1);
+        auto kern = kgr::row_kernel<C, 1, 1, Op, KG_ORD_WH>;
+        kg_register_kernel("whispering", (const void*)kern);
+        if (int rc = kg_launch_begin(ctx, "whispering")) return rc;
         if (!g.empty)
             kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * C::W), 0, nx, ny, g.ntx, op);
         return kg_launch_end(ctx);
     };
-    if (VEC_EVEN == 2 && nx % 2 == 0 && al) return go(std::integral_constant<int, VEC_EVEN>{});
-    return go(std::integral_constant<int, 1>{});
+    auto high = [&](auto w, long long waves) {   // waves: side by side
+        const bool thin = waves * ((ny + 5) / 8) < 2 * ctx->cus;   // rows 1 .. ny-2 by 8
+        auto rag = [&](auto yc) {
+            return nx % 2 == 0 && al ? go(w, yc, std::false_type{}) : go(w, yc, std::true_type{});
+        };
+        return thin ? rag(std::integral_constant<int, 2>{}) : rag(std::integral_constant<int, 8>{});
+    };
+    const long long w1 = ((long long)nx + 127) / 128, w2 = (w1 + 1) / 2 * 2, w4 = (w1 + 3) / 4 * 4;
+    if (w4 <= w1) return high(std::integral_constant<int, 4>{}, w4);
+    if (w2 <= w1) return high(std::integral_constant<int, 2>{}, w2);
+    return high(std::integral_constant<int, 1>{}, w1);
 }
 
 // Direct march shapes (output rows per lane, waves per workgroup) from
@@ -208,9 +224,6 @@ static int launch_row(kg_ctx* ctx, const char* name, int nx, int ny, bool al, Fi
 #endif
 #ifndef KG_ORD_LIFE
 #define KG_ORD_LIFE 4
-#endif
-#ifndef KG_ORD_WH
-#define KG_ORD_WH 1
 #endif
 using J9D = kgr::DCfg<KG_J9_PY, KG_J9_ROWS, 1>;
 using JacD = kgr::DCfg<KG_JAC_PY, KG_J9_ROWS, 1>;
@@ -299,7 +312,7 @@ extern "C" int kg_whispering(kg_ctx* ctx, int nx, int ny, double mu, double epsi
     const long long n = (long long)nx * ny;
     const bool al = kg_aligned16(e_in, e_out, h0, h1, u_em0, u_em1, ca, cb, da, db) &&
                     kg_aligned16(e_in + n, e_out + n);
-    return launch_row<WhCfg, WhisperingOp, 1, 1, 2, KG_ORD_WH>(ctx, "whispering", nx, ny, al, [&](auto& op) {
+    return launch_whispering(ctx, nx, ny, al, [&](auto& op) {
         op.src[0] = h0;
         op.src[1] = ca;
         op.src[2] = cb;

@@ -189,6 +189,17 @@ def test_gpu_matches_oracle_thin_chunks(gpu_ctx, oracle, name):
             assert_bit_equal(got[role], want[role], f"{name} {dims} {role}")
 
 
+@pytest.mark.parametrize("dims", [(301, 1500), (255, 2100), (511, 1100), (256, 2100), (640, 900)])
+def test_gpu_whispering_tile_widths(gpu_ctx, oracle, dims):
+    """Tiles of 1, 2 and 4 row pieces with 8 rows each, odd and even rows."""
+    spec = K.SPECS["whispering"]
+    coefs, arrays = K.random_case(spec, dims, 1400)
+    want = oracle.run(spec, dims, coefs, arrays, 2)
+    got = K.GpuBackend(gpu_ctx).run(spec, dims, coefs, arrays, 2)
+    for role in want:
+        assert_bit_equal(got[role], want[role], f"whispering {dims} {role}")
+
+
 @pytest.mark.parametrize("name", ["laplacian", "wave13pt", "whispering", "gameoflife", "uxx1"])
 def test_gpu_matches_oracle_ten_steps(gpu_ctx, oracle, name):
     """Ten ping-pong steps (the suite's nt) at a mid size."""
