@@ -18,13 +18,10 @@
 // operators down to 3 x 3 vertices) and set u += e.  The FP32 inner solve
 // needs only a few digits per correction; FP64 residuals recover the rest.
 //
-// The FP32 levels are stored with rows padded to P = N rounded up to 4
-// floats, so that the sweeps and the prolongation work on 16-byte pieces:
-// a lane owns 4 points of PY rows, loads the rows it needs (pieces at x-4, x,
-// x+4) through the caches, and writes whole rows -- interior values, and 0 at
-// the boundary and padding points, which those arrays hold anyway -- so that
-// no cache line is written in part.
-#include "kg_internal.h"
+// The FP32 levels are stored with rows padded to P = N rounded up to 16
+// floats, so that their passes work on 16-byte pieces and write whole rows
+// (0 at the boundary and padding points): no cache line is written in part.
+#include "kg_plane.h"
 
 #include <chrono>
 #include <cmath>
@@ -32,215 +29,517 @@
 
 namespace {
 
-constexpr int PT = 16;   // 16 x 16 threads per workgroup (scalar kernels)
-// Tile order of the sweeps, the FP64 residual and the prolongation
-// (kg_tile_order): chunks of 2 tile rows per XCD, 8192^2 solve 17.7 ms
-// against 17.9-18.1 in hardware order (chunks of 4 or 8 rows 17.6-17.9),
+// Tile order of the V-cycle's passes and the FP64 residual (kg_tile_order):
+// chunks of 2 tile rows per XCD, 8192^2 solve 17.7 ms against 17.9-18.1 in
+// hardware order with the passes of that time (chunks of 4 or 8 rows 17.6-17.9),
 // bit-identical (the residual's partial sums stay indexed by tile).
 #ifndef KG_ORD_PJ
 #define KG_ORD_PJ 2
 #endif
-constexpr int VW = 4;    // waves per workgroup of the 4-point kernels, stacked in y
-constexpr int PY = 4;    // rows per lane of the 4-point kernels
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));   // at any element
 
-typedef __attribute__((address_space(1))) const f4 gf4;
+// ------------------------------------------------------------ a level's passes
+// A V-cycle visits a level twice: on the way down two damped Jacobi sweeps, the
+// residual and its full-weighting restriction, on the way up the bilinear
+// correction and two sweeps.  Each visit is one pass over the level (pj_down_k,
+// pj_up_k): a wave takes 256 columns, 4 per lane, and marches them along y; an
+// incoming row enters a window of three rows, which gives the first sweep of the
+// row before it, three of those give the second sweep of the row before that,
+// and so on, so that HBM sees u, f and the result once per visit.  The columns
+// beside a lane's 4 come from the neighbouring lanes by DPP.  Every stage makes
+// the wave's outermost column on either side invalid; the outer lanes hold only
+// such overlap (pieces start every 240 columns, 64-byte aligned).  Expressions and
+// orders are those of separate sweeps, residual and restriction, and so is the
+// result, bit for bit.
+//
+// Bound by HBM on the finest levels: u, f, u' and a quarter of it on the next
+// level are 871 MB at 8192^2, 203 us (4.3 TB/s; the best copy reaches 6.3) for
+// pj_up_k and 188 for pj_down_k.  Sweep pairs, residual and restriction,
+// prolongation and the addition to u as passes of their own took 14.2 of the 17.7 ms
+// of an 8192^2 solve (7.5, 3.3, 1.9, 1.5); it takes 10.4 so.  Rows of 64-byte
+// multiples and pieces of 240 columns, so that no wave writes part of a sector:
+// 5 % faster at 8192^2 than 248 columns of 4-float pitches.  The 4 waves of a
+// workgroup lie side by side; one above the other costs 2 % more.  Small levels
+// are bound by a wave's march: 6 us at 512 cells and below.
+constexpr int MW = 4;                  // waves per workgroup, side by side in x
+constexpr int PIECE = 240;             // columns a wave completes
 
-__device__ __forceinline__ f4 ldf4(const float* p) { return *(gf4*)p; }
-
-// The rows j0-1 .. j0+PY of a lane's 4-point column x (pieces at x-4, x, x+4
-// clamped into the padded row; clamped pieces feed only boundary points).
-struct Win4 {
-    float w[PY + 2][12];
+struct Coef {
+    float c0, c1, c2, cf;              // sweep: c0 u + c1 axis + c2 diag + cf f
+    float inv6h2;
 };
-__device__ __forceinline__ void load_win4(const float* __restrict__ u, int N, int P, int x, int j0,
-                                          Win4& W)
-{
-    const int xl = x >= 4 ? x - 4 : x, xr = x + 4 < P ? x + 4 : x;
-#pragma unroll
-    for (int q = 0; q < PY + 2; q++) {
-        const float* row = u + (long long)min(j0 - 1 + q, N - 1) * P;
-        const f4 a = ldf4(row + xl), b = ldf4(row + x), c = ldf4(row + xr);
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            W.w[q][v] = a[v];
-            W.w[q][4 + v] = b[v];
-            W.w[q][8 + v] = c[v];
-        }
+
+// Four columns of a row and the ones on either side of them.
+struct Row {
+    float v[4], l, r;
+    __device__ __forceinline__ float at(int i) const { return i < 0 ? l : i > 3 ? r : v[i]; }
+    __device__ __forceinline__ void sides()
+    {
+        l = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHR1>(0.f, v[3]);
+        r = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.f, v[0]);
     }
+};
+
+// damped Jacobi sweep of row b (a below, c above it): u' = c0 u + c1 (W + S + E +
+// N) + c2 (SW + NW + SE + NE) + cf f on the interior, 0 elsewhere
+__device__ __forceinline__ void pj_sweep(const Coef& k, const Row& a, const Row& b, const Row& c,
+                                         const float (&f)[4], bool row_in, const bool (&in)[4], Row& o)
+{
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const float val = k.c0 * b.v[v] + k.c1 * (b.at(v - 1) + a.v[v] + b.at(v + 1) + c.v[v]) +
+                          k.c2 * (a.at(v - 1) + c.at(v - 1) + a.at(v + 1) + c.at(v + 1)) + k.cf * f[v];
+        o.v[v] = row_in && in[v] ? val : 0.f;
+    }
+    o.sides();
 }
 
-// damped Jacobi sweep on 4-point pieces, u' = c0 u + c1 (W + S + E + N) +
-// c2 (SW + NW + SE + NE) + cf f; writes rows 1 .. N-2 whole (0 at the
-// boundary and padding)
-__global__ __launch_bounds__(64 * VW)
-void pj_smooth4_k(int N, int P, int ntx, float c0, float c1, float c2, float cf,
-                  const float* __restrict__ u, const float* __restrict__ f, float* __restrict__ uo)
+// r = f - (20 u - 4 (W + S + E + N) - (SW + NW + SE + NE)) / (6 h^2)
+__device__ __forceinline__ void pj_resid(const Coef& k, const Row& a, const Row& b, const Row& c,
+                                         const float (&f)[4], Row& o)
 {
-    const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
-    const unsigned tb = kg_tile_order<KG_ORD_PJ>(blockIdx.x, gridDim.x, (unsigned)ntx);
-    const int x = (int)(tb % (unsigned)ntx) * 256 + lane * 4;
-    const int j0 = 1 + ((int)(tb / (unsigned)ntx) * VW + w) * PY;
-    if (x >= P || j0 >= N - 1) return;
-    Win4 W;
-    load_win4(u, N, P, x, j0, W);
 #pragma unroll
-    for (int r = 0; r < PY; r++) {
-        const int j = j0 + r;
-        if (j >= N - 1) break;
-        const f4 fv = ldf4(f + (long long)j * P + x);
-        f4 o;
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-#define U(dx, dy) W.w[r + 1 + (dy)][4 + v + (dx)]
-            const float val = c0 * U(0, 0) + c1 * (U(-1, 0) + U(0, -1) + U(1, 0) + U(0, 1)) +
-                              c2 * (U(-1, -1) + U(-1, 1) + U(1, -1) + U(1, 1)) + cf * fv[v];
-#undef U
-            o[v] = (x + v >= 1 && x + v < N - 1) ? val : 0.f;
-        }
-        __builtin_nontemporal_store(o, (__attribute__((address_space(1))) f4*)(uo + (long long)j * P + x));
+    for (int v = 0; v < 4; v++) {
+        const float au = (20.f * b.v[v] - 4.f * (b.at(v - 1) + a.v[v] + b.at(v + 1) + c.v[v]) -
+                          (a.at(v - 1) + c.at(v - 1) + a.at(v + 1) + c.at(v + 1))) * k.inv6h2;
+        o.v[v] = f[v] - au;
     }
+    o.sides();
 }
 
-// Two damped Jacobi sweeps in one pass, bit-identical to two pj_smooth4_k
-// launches (same expression and order, no contraction): the lane forms the
-// first sweep's values on the block one point wider on every side than its
-// 4 points x PY rows (columns x-1 .. x+4, rows j0-1 .. j0+PY; 0 outside
-// rows/columns 1 .. N-2,
-// as the first launch would have written them), then the second sweep on
-// its own points.  u rows j0-2 .. j0+PY+1 and f rows j0-1 .. j0+PY come
-// through the caches; HBM sees each array once per two sweeps.
-#ifndef KG_SM2_PY
-// rows per lane: 8192^2 solve 19.0 ms (3 rows 19.1, 4 rows 19.4, 6 rows 19.0);
-// with the chunked tile order 17.0-17.2 ms (3 rows 17.2-17.3, 4 rows 17.5,
-// 6 rows 17.2-17.3)
-#define KG_SM2_PY 2
-#endif
-template <int PY>
-__global__ __launch_bounds__(64 * VW)
-void pj_smooth4x2_k(int N, int P, int ntx, float c0, float c1, float c2, float cf,
-                    const float* __restrict__ u, const float* __restrict__ f,
-                    float* __restrict__ uo)
-{
-    const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
-    const unsigned tb = kg_tile_order<KG_ORD_PJ>(blockIdx.x, gridDim.x, (unsigned)ntx);
-    const int x = (int)(tb % (unsigned)ntx) * 256 + lane * 4;
-    const int j0 = 1 + ((int)(tb / (unsigned)ntx) * VW + w) * PY;
-    if (x >= P || j0 >= N - 1) return;
-    const int xl = x >= 4 ? x - 4 : x, xr = x + 4 < P ? x + 4 : x;
-    // uu[q][c]: u at row j0-2+q, column x-2+c (c = 0 .. 7)
-    float uu[PY + 4][8];
+// What the marching passes share: the wave's columns and rows.  Rows 0 and N-1
+// and everything outside the grid count as 0 and are never read.
+struct March {
+    int N, P, x, yb, ye;               // lane's first column; rows [yb, ye) are completed
+    unsigned voff;                     // its byte offset in a row, or out of range
+    bool in[4], mine;                  // columns of the interior; the lane completes its columns
+    __device__ __forceinline__ bool setup(int N_, int P_, int ntx, int H)
+    {
+        N = N_;
+        P = P_;
+        const unsigned tb = kg_tile_order<KG_ORD_PJ>(blockIdx.x, gridDim.x, (unsigned)ntx);
+        const int lane = (int)(threadIdx.x & 63);
+        const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+        x = ((int)(tb % (unsigned)ntx) * MW + w) * PIECE - 4 + 4 * lane;
+        yb = (int)(tb / (unsigned)ntx) * H;
+        ye = min(yb + H, N - 1);
+        voff = x >= 0 && x < P ? (unsigned)x * 4u : kgp::KG_OOB;
 #pragma unroll
-    for (int q = 0; q < PY + 4; q++) {
-        const float* row = u + (long long)min(max(j0 - 2 + q, 0), N - 1) * P;
-        const f4 a = ldf4(row + xl), b = ldf4(row + x), c = ldf4(row + xr);
-        uu[q][0] = a[2];
-        uu[q][1] = a[3];
-#pragma unroll
-        for (int v = 0; v < 4; v++) uu[q][2 + v] = b[v];
-        uu[q][6] = c[0];
-        uu[q][7] = c[1];
+        for (int v = 0; v < 4; v++) in[v] = x + v >= 1 && x + v < N - 1;
+        mine = lane >= 1 && lane <= PIECE / 4 && x < P;
+        return x - 4 * lane < N - 4;   // the piece has a column
     }
-    // ff[q][c]: f at row j0-1+q, column x-1+c (c = 0 .. 5)
-    float ff[PY + 2][6];
-#pragma unroll
-    for (int q = 0; q < PY + 2; q++) {
-        const float* row = f + (long long)min(max(j0 - 1 + q, 0), N - 1) * P;
-        const f4 a = ldf4(row + xl), b = ldf4(row + x), c = ldf4(row + xr);
-        ff[q][0] = a[3];
-#pragma unroll
-        for (int v = 0; v < 4; v++) ff[q][1 + v] = b[v];
-        ff[q][5] = c[0];
+    __device__ __forceinline__ bool inside(int y) const { return y >= 1 && y < N - 1; }
+    __device__ __forceinline__ __amdgpu_buffer_rsrc_t row(const float* p, int y) const
+    {
+        const bool ok = inside(y);
+        return kgp::make_rsrc(p + (long long)(ok ? y : 0) * P, ok ? (unsigned)P * 4u : 0u);
     }
-    // first sweep: s1[q][c] at row j0-1+q, column x-1+c
-    float s1[PY + 2][6];
-#pragma unroll
-    for (int q = 0; q < PY + 2; q++) {
-        const int j = j0 - 1 + q;
-#pragma unroll
-        for (int c = 0; c < 6; c++) {
-            const int xc = x - 1 + c;
-#define U(dx, dy) uu[q + 1 + (dy)][c + 1 + (dx)]
-            const float val = c0 * U(0, 0) + c1 * (U(-1, 0) + U(0, -1) + U(1, 0) + U(0, 1)) +
-                              c2 * (U(-1, -1) + U(-1, 1) + U(1, -1) + U(1, 1)) + cf * ff[q][c];
-#undef U
-            s1[q][c] = (xc >= 1 && xc < N - 1 && j >= 1 && j < N - 1) ? val : 0.f;
+    __device__ __forceinline__ void load(const float* p, int y, float (&v)[4]) const
+    {
+        kgp::bload<kgp::F32, 4>(row(p, y), voff, v);
+    }
+    // whole rows: interior values, 0 on the boundary and the padding
+    __device__ __forceinline__ void store(float* p, int y, const Row& r) const
+    {
+        if (mine && y >= max(yb, 1) && y < ye) {
+            const f4 o = {r.v[0], r.v[1], r.v[2], r.v[3]};
+            __builtin_nontemporal_store(o, (__attribute__((address_space(1))) f4*)(p + (long long)y * P + x));
         }
     }
-    // second sweep on the lane's points
+};
+
+// Down: u' = two sweeps of u (ZERO: of the guess 0, which is not read) for the
+// right-hand side f, and the coarse right-hand side
+//   fc(I,J) = (4 r_C + 2 (r_W + r_E + r_S + r_N) + (r_SW + r_SE + r_NW + r_NE)) / 16
+// of the residual r of u' at the 3 x 3 fine points around (2I, 2J).  H: even.
+template <bool ZERO>
+__global__ __launch_bounds__(64 * MW)
+void pj_down_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* __restrict__ u,
+               const float* __restrict__ f, float* __restrict__ uo, float* __restrict__ fc)
+{
+    constexpr int D = 3;               // rows in flight
+    constexpr int LAG = ZERO ? 0 : 1;  // f enters one row after u
+    March m;
+    if (!m.setup(N, P, ntx, H)) return;
+    float pu[D][4], pf[D][4], fr[3][4];
+    Row ur[3], s1[3], s2[3], rr[3];
 #pragma unroll
-    for (int r = 0; r < PY; r++) {
-        const int j = j0 + r;
-        if (j >= N - 1) break;
-        f4 o;
+    for (int q = 0; q < 3; q++) {
+        ur[q] = s1[q] = s2[q] = rr[q] = Row{{0.f, 0.f, 0.f, 0.f}, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < 4; v++) fr[q][v] = 0.f;
+    }
+    const int first = m.yb - 3 - LAG, last = m.ye + 1 + LAG;   // incoming rows
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+        if constexpr (!ZERO) m.load(u, first + d, pu[d]);
+        m.load(f, first + d - LAG, pf[d]);
+    }
+    // At phase p row y enters slot p; slot p+2 (mod 3) holds the row before it.
+    // The first sweep's newest row is y - LAG, the second's y-1-LAG, the
+    // residual's y-2-LAG; each is kept in the slot of its phase.
+    auto step = [&](auto phase, int y) {
+        constexpr int p = decltype(phase)::value, p1 = (p + 2) % 3, p2 = (p + 1) % 3;
+#pragma unroll
+        for (int v = 0; v < 4; v++) fr[p][v] = pf[p][v];      // f row y - LAG
+        if constexpr (ZERO) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float val = 0.f + k.cf * fr[p][v];
+                s1[p].v[v] = m.inside(y) && m.in[v] ? val : 0.f;
+            }
+            s1[p].sides();
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++) ur[p].v[v] = pu[p][v];
+            ur[p].sides();
+            m.load(u, y + D, pu[p]);
+            pj_sweep(k, ur[p2], ur[p1], ur[p], fr[p], m.inside(y - 1), m.in, s1[p]);
+        }
+        m.load(f, y + D - LAG, pf[p]);
+        pj_sweep(k, s1[p2], s1[p1], s1[p], fr[p1], m.inside(y - 1 - LAG), m.in, s2[p]);
+        m.store(uo, y - 1 - LAG, s2[p]);
+        pj_resid(k, s2[p2], s2[p1], s2[p], fr[p2], rr[p]);
+        const int yr = y - 2 - LAG, J = (yr - 1) >> 1;        // residual row; its coarse row below
+        if ((yr & 1) && 2 * J >= m.yb && 2 * J < m.ye && J >= 1 && J < Nc - 1) {
+            const Row &a = rr[p2], &b = rr[p1], &c = rr[p];
+            f2 o;
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                const int v = 2 * q, I = (m.x >> 1) + q;
+                const float val = (4.f * b.v[v] + 2.f * (b.at(v - 1) + b.at(v + 1) + a.v[v] + c.v[v]) +
+                                   (a.at(v - 1) + a.at(v + 1) + c.at(v - 1) + c.at(v + 1))) * 0.0625f;
+                o[q] = I >= 1 && I < Nc - 1 ? val : 0.f;
+            }
+            if (m.mine) *(__attribute__((address_space(1))) f2*)(fc + (long long)J * Pc + (m.x >> 1)) = o;
+        }
+    };
+    for (int y = first; y <= last; y += 3)
+        kg_static_for<3>([&](auto p) {
+            if (y + decltype(p)::value <= last) step(p, y + decltype(p)::value);
+        });
+}
+
+// Up: u' = two sweeps of u plus the bilinear interpolation of the coarse e (e at
+// even/even points, the mean of the 2 or 4 coarse neighbours elsewhere).  ADD: u'
+// is not stored but added to the interior of the dense FP64 N x N field u64.
+template <bool ADD>
+__global__ __launch_bounds__(64 * MW)
+void pj_up_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* __restrict__ u,
+             const float* __restrict__ ec, const float* __restrict__ f, float* __restrict__ uo,
+             double* __restrict__ u64)
+{
+    constexpr int D = 3;
+    March m;
+    if (!m.setup(N, P, ntx, H)) return;
+    const unsigned coff = m.x >= 0 && m.x < P ? (unsigned)m.x * 2u : kgp::KG_OOB;   // column x/2
+    auto crow = [&](int J, float (&v)[2]) {
+        const bool ok = J >= 1 && J < Nc - 1;
+        kgp::bload<kgp::F32, 2>(kgp::make_rsrc(ec + (long long)(ok ? J : 0) * Pc, ok ? (unsigned)Pc * 4u : 0u),
+                                coff, v);
+    };
+    float pu[D][4], pf[D][4], pa[D][2], pb[D][2], fr[3][4];
+    Row vr[3], s1[3];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        vr[q] = s1[q] = Row{{0.f, 0.f, 0.f, 0.f}, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < 4; v++) fr[q][v] = 0.f;
+    }
+    const int first = m.yb - 2, last = m.ye + 1;
+    auto fetch = [&](int y, int d) {
+        m.load(u, y, pu[d]);
+        m.load(f, y - 1, pf[d]);
+        crow(y >> 1, pa[d]);
+        crow((y >> 1) + 1, pb[d]);
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) fetch(first + d, d);
+    // N is 4 q + 1: columns x .. x+3 of a lane left of column N-1 are in the row
+    const bool adds = m.mine && m.x < N - 1;
+    d2 w[2];
+    auto fetch64 = [&](int y) {
+        if (adds && y >= max(m.yb, 1) && y < m.ye) {
+            w[0] = *(const d2u*)(u64 + (long long)y * N + m.x);
+            w[1] = *(const d2u*)(u64 + (long long)y * N + m.x + 2);
+        }
+    };
+    auto step = [&](auto phase, int y) {
+        constexpr int p = decltype(phase)::value, p1 = (p + 2) % 3, p2 = (p + 1) % 3;
+        // coarse columns x/2, x/2+1, x/2+2 of rows y/2 and (odd y) y/2+1
+        const float a[3] = {pa[p][0], pa[p][1], kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.f, pa[p][0])};
+        const float b[3] = {pb[p][0], pb[p][1], kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.f, pb[p][0])};
+        const bool odd = y & 1;
 #pragma unroll
         for (int v = 0; v < 4; v++) {
-#define U(dx, dy) s1[r + 1 + (dy)][v + 1 + (dx)]
-            const float val = c0 * U(0, 0) + c1 * (U(-1, 0) + U(0, -1) + U(1, 0) + U(0, 1)) +
-                              c2 * (U(-1, -1) + U(-1, 1) + U(1, -1) + U(1, 1)) + cf * ff[r + 1][v + 1];
-#undef U
-            o[v] = (x + v >= 1 && x + v < N - 1) ? val : 0.f;
+            const int q = v >> 1;
+            const float e = !(v & 1) ? (odd ? 0.5f * (a[q] + b[q]) : a[q])
+                                     : (odd ? 0.25f * (a[q] + a[q + 1] + b[q] + b[q + 1])
+                                            : 0.5f * (a[q] + a[q + 1]));
+            vr[p].v[v] = m.inside(y) && m.in[v] ? pu[p][v] + e : 0.f;
+            fr[p][v] = pf[p][v];                               // f row y-1
         }
-        __builtin_nontemporal_store(o, (__attribute__((address_space(1))) f4*)(uo + (long long)j * P + x));
+        vr[p].sides();
+        if constexpr (ADD) fetch64(y - 2);
+        fetch(y + D, p);
+        pj_sweep(k, vr[p2], vr[p1], vr[p], fr[p], m.inside(y - 1), m.in, s1[p]);
+        Row o;
+        pj_sweep(k, s1[p2], s1[p1], s1[p], fr[p1], m.inside(y - 2), m.in, o);
+        if constexpr (!ADD) {
+            m.store(uo, y - 2, o);
+        } else if (adds && y - 2 >= max(m.yb, 1) && y - 2 < m.ye) {
+            double* q = u64 + (long long)(y - 2) * N + m.x;
+            *(d2u*)q = w[0] + d2{(double)o.v[0], (double)o.v[1]};
+            *(d2u*)(q + 2) = w[1] + d2{(double)o.v[2], (double)o.v[3]};
+        }
+    };
+    for (int y = first; y <= last; y += 3)
+        kg_static_for<3>([&](auto p) {
+            if (y + decltype(p)::value <= last) step(p, y + decltype(p)::value);
+        });
+}
+
+// ------------------------------------------------------------ the coarse levels
+// One workgroup runs the whole V-cycle from TOP cells per side (at most 128) down
+// to the 2-cell level (one unknown, solved exactly) and back up, with every
+// level's u in LDS and its right-hand side in the registers of the threads that
+// own the points.  A thread owns R = TOP^2/1024 rows of one column (one point on
+// the levels below 64 cells), so a wave reads consecutive LDS words.  As
+// launches these levels took 30 of the 40 of a 512 cell V-cycle, which bound its
+// solve (1.98 ms; 0.95 now).  The cycle from 128 cells takes 22 us, bound by one CU's
+// FP32 rate and LDS on the first level and by barriers below.
+constexpr int CTOP = 128;
+constexpr int CT = 1024;               // threads
+constexpr int CLV = 7;                 // levels of 128, 64, ..., 2 cells
+
+struct CCoef {
+    float c0, c1, c2, exact;           // exact: 6 h^2 / 20 of the 2-cell level
+    float cf[CLV], inv6h2[CLV];        // of the levels from TOP down
+};
+
+template <int n>
+struct CLevel {
+    static constexpr int N = n + 1, R = n * n > CT ? n * n / CT : 1;
+    static constexpr bool ONE = n <= 8;   // all points belong to the first wave, which works alone
+    // Thread t's column and first row.  Column n and row n are the boundary's:
+    // their threads compute along, on whatever LDS holds there, and put nothing.
+    static __device__ __forceinline__ int x(int t) { return 1 + t % n; }
+    static __device__ __forceinline__ int y(int t) { return 1 + t / n * R; }
+    static __device__ __forceinline__ bool works(int t) { return n * n >= CT || t < n * n; }
+    static __device__ __forceinline__ void sync()
+    {
+        if constexpr (ONE) {   // a wave's LDS operations stay in order
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __syncthreads();
+        }
     }
+    // v[r] = the thread's value of its row r / those values into a
+    template <class Val>
+    static __device__ __forceinline__ void each(int t, float (&v)[R], Val&& val)
+    {
+        const int q0 = y(t) * N + x(t);
+        if (!works(t)) return;
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = val(r, q0 + r * N);
+    }
+    static __device__ __forceinline__ void put(int t, const float (&v)[R], float* a)
+    {
+        const int q0 = y(t) * N + x(t);
+        if (!works(t) || x(t) == n) return;
+#pragma unroll
+        for (int r = 0; r < R - 1; r++) a[q0 + r * N] = v[r];
+        if (y(t) + R - 1 < n) a[q0 + (R - 1) * N] = v[R - 1];
+    }
+    static __device__ __forceinline__ float point(const CCoef& k, float cf, const float* u, int q, float f)
+    {
+        return k.c0 * u[q] + k.c1 * (u[q - 1] + u[q - N] + u[q + 1] + u[q + N]) +
+               k.c2 * (u[q - N - 1] + u[q + N - 1] + u[q - N + 1] + u[q + N + 1]) + cf * f;
+    }
+    // Two sweeps of the level in place; with zero from u = 0.
+    static __device__ __forceinline__ void smooth(const CCoef& k, float cf, float* u, const float (&f)[R],
+                                                  bool zero)
+    {
+        const int t = (int)threadIdx.x;
+        float o[R] = {};
+        if (zero) {
+            each(t, o, [&](int r, int) { return 0.f + cf * f[r]; });
+        } else {
+            each(t, o, [&](int r, int q) { return point(k, cf, u, q, f[r]); });
+            sync();
+        }
+        put(t, o, u);
+        sync();
+        each(t, o, [&](int r, int q) { return point(k, cf, u, q, f[r]); });
+        sync();
+        put(t, o, u);
+        sync();
+    }
+    // The boundary of the level's u.
+    static __device__ __forceinline__ void border(float* u)
+    {
+        for (int i = (int)threadIdx.x; i < N; i += CT) u[i] = u[n * N + i] = u[i * N] = u[i * N + n] = 0.f;
+    }
+    // One V-cycle on u (bordered; zero: u counts as 0 inside).  The memory past u
+    // is the coarser levels'; d is the level's place in k.
+    static __device__ __forceinline__ void cycle(const CCoef& k, int d, float* u, const float (&f)[R],
+                                                 bool zero)
+    {
+        const int t = (int)threadIdx.x;
+        if constexpr (n == 2) {
+            if (t == 0) u[N + 1] = k.exact * f[0];
+            sync();
+        } else {
+            using C = CLevel<n / 2>;
+            smooth(k, k.cf[d], u, f, zero);
+            float* uc = u + N * N;
+            const float inv = k.inv6h2[d];
+            // the residual, in the coarser levels' memory, then its restriction
+            float o[R] = {};
+            each(t, o, [&](int r, int q) {
+                const float au = (20.f * u[q] - 4.f * (u[q - 1] + u[q - N] + u[q + 1] + u[q + N]) -
+                                  (u[q - N - 1] + u[q + N - 1] + u[q - N + 1] + u[q + N + 1])) * inv;
+                return f[r] - au;
+            });
+            put(t, o, uc);
+            sync();
+            float fc[C::R] = {};
+            C::each(t, fc, [&](int r, int) {
+                const float* p = uc + 2 * (C::y(t) + r) * N + 2 * C::x(t);
+                return (4.f * p[0] + 2.f * (p[-1] + p[1] + p[-N] + p[N]) +
+                        (p[-N - 1] + p[-N + 1] + p[N - 1] + p[N + 1])) * 0.0625f;
+            });
+            sync();
+            C::border(uc);
+            if constexpr (C::ONE && !ONE) {   // the border and fc of an 8-cell level are the first wave's
+                if (t < 64) C::cycle(k, d + 1, uc, fc, true);
+                sync();
+            } else {
+                C::cycle(k, d + 1, uc, fc, true);
+            }
+            const int xo = x(t) & 1;
+            const float* e0 = uc + (x(t) >> 1);
+            each(t, o, [&](int r, int q) {
+                const int yy = y(t) + r;
+                const float *a = e0 + (yy >> 1) * C::N, *b = a + C::N;
+                const float even = xo ? 0.5f * (a[0] + a[1]) : a[0];
+                const float odd = xo ? 0.25f * (a[0] + a[1] + b[0] + b[1]) : 0.5f * (a[0] + b[0]);
+                return u[q] + (yy & 1 ? odd : even);
+            });
+            put(t, o, u);
+            sync();
+            smooth(k, k.cf[d], u, f, false);
+        }
+    }
+};
+
+template <int TOP>
+__global__ __launch_bounds__(CT)
+void pj_coarse_k(int P, CCoef k, const float* __restrict__ f, float* __restrict__ ug, int zero)
+{
+    using L = CLevel<TOP>;
+    // u of the level and behind it the coarser ones, or the residual of this one,
+    // and what the threads of the far boundary read past it
+    __shared__ float u[2 * L::N * L::N + 2 * L::N];
+    const int t = (int)threadIdx.x;
+    const int o0 = L::y(t) * P + L::x(t);
+    float fv[L::R] = {}, v[L::R] = {};
+    L::each(t, fv, [&](int r, int) { return f[o0 + r * P]; });
+    if (!zero) {
+        L::each(t, v, [&](int r, int) { return ug[o0 + r * P]; });
+        L::put(t, v, u);
+    }
+    L::border(u);
+    __syncthreads();
+    if (!L::ONE || t < 64) L::cycle(k, 0, u, fv, zero);
+    __syncthreads();
+    // interior rows, with 0 in columns 0 and N-1 (the other columns are not read)
+    for (int y = 1 + (t >> 6); y < TOP; y += CT / 64)
+        for (int x = t & 63; x < L::N; x += 64) ug[y * P + x] = u[y * L::N + x];
 }
 
 // The outer correction's FP64 residual, fused with its FP32 copy and its
 // squared norm: r = f - (20 u - 4 (u_W + u_S + u_E + u_N) - (u_SW + u_NW +
 // u_SE + u_NE)) / (6 h^2), summed in that order in FP64, written as
-// FP32 rows of pitch P, 0 on the boundary and the padding, and e = 0 (the
-// inner solve's initial guess) at the same points; the sum of r^2 over the
-// workgroup's points goes to part[blockIdx.x] (rows of a lane in order, then
-// lanes and waves by a fixed tree).  A workgroup of 4 waves takes 256
-// consecutive columns of RES_RY rows; a lane loads the RES_RY + 2 rows of
-// its column and both neighbours (side values from L1) and the RES_RY
-// values of f before the first use.
-constexpr int RES_RY = 8;
-
-__global__ __launch_bounds__(256)
-void pj_residual64_k(int N, int P, int ntx, double inv6h2, const double* __restrict__ u,
-                     const double* __restrict__ f, float* __restrict__ r, float* __restrict__ e,
-                     double* __restrict__ part)
+// FP32 rows of pitch P, 0 on the boundary columns; the sum of r^2 over the
+// workgroup's points goes to part[its tile] (rows of a lane in order, then lanes
+// and waves by a fixed tree).  A wave marches RES_H(n) rows of 128 columns, 2 per
+// lane (rows of u start at any multiple of 8 bytes); the columns beside a lane's 2
+// come by DPP, and the outer lanes only hold such columns.  Bound by HBM: 1.34 GB at
+// 8192^2 in 262 us (5.1 TB/s; tiles of 8 rows with side loads from L1 289 us; 16 or
+// 32 rows a wave 278 and 312).
+constexpr int RPIECE = 112;   // columns a wave completes
+constexpr int res_rows(int n) { return n >= 2048 ? 8 : n >= 1024 ? 4 : 2; }
+constexpr int res_ntx(int n) { return (n + 1 + MW * RPIECE - 1) / (MW * RPIECE); }
+constexpr int res_blocks_of(int n)
 {
-    __shared__ double wsum[4];
-    const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
+    return res_ntx(n) * ((n + res_rows(n) - 1) / res_rows(n));
+}
+
+__global__ __launch_bounds__(64 * MW)
+void pj_residual64_k(int N, int P, int ntx, int H, double inv6h2, const double* __restrict__ u,
+                     const double* __restrict__ f, float* __restrict__ r, double* __restrict__ part)
+{
+    constexpr int D = 3;                                       // rows in flight
+    __shared__ double wsum[MW];
+    const int lane = (int)(threadIdx.x & 63);
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const unsigned tb = kg_tile_order<KG_ORD_PJ>(blockIdx.x, gridDim.x, (unsigned)ntx);
-    const int x = (int)(tb % (unsigned)ntx) * 256 + w * 64 + lane;
-    const int j0 = (int)(tb / (unsigned)ntx) * RES_RY;
-    // clamped columns and rows: they only feed points that are not computed
-    const int xc = min(x, N - 1), xl = max(xc - 1, 0), xr = min(xc + 1, N - 1);
-    double v[RES_RY + 2][3], fv[RES_RY];
+    const int x = ((int)(tb % (unsigned)ntx) * MW + w) * RPIECE - 2 + 2 * lane;
+    const int yb = max((int)(tb / (unsigned)ntx) * H, 1);
+    const int ye = min((int)(tb / (unsigned)ntx + 1) * H, N - 1);
+    // 16 bytes inside the row; what lies past an end only feeds points that are
+    // not computed, except that column N-1 (even) is the second of its pair
+    const int xl = min(max(x, 0), N - 2);
+    const bool tail = x == N - 1;
+    const bool in0 = x >= 1 && x < N - 1, in1 = x + 1 >= 1 && x + 1 < N - 1;
+    const bool mine = lane >= 1 && lane <= RPIECE / 2;
+    struct Row2 { double l, a, b, r; };
+    Row2 ur[3];
+    d2 pu[D], pf[D];
+    auto row = [&](const double* p, int y) {
+        return *(const d2u*)(p + (long long)min(max(y, 0), N - 1) * N + xl);
+    };
+    const int first = yb - 1, last = ye;                       // incoming rows of u
 #pragma unroll
-    for (int q = 0; q < RES_RY + 2; q++) {
-        const long long o = (long long)min(max(j0 - 1 + q, 0), N - 1) * N;
-        v[q][0] = u[o + xl];
-        v[q][1] = u[o + xc];
-        v[q][2] = u[o + xr];
+    for (int d = 0; d < D; d++) {
+        pu[d] = row(u, first + d);
+        pf[d] = row(f, first + d - 1);
+        ur[d] = Row2{0.0, 0.0, 0.0, 0.0};
     }
-#pragma unroll
-    for (int q = 0; q < RES_RY; q++) fv[q] = f[(long long)min(j0 + q, N - 1) * N + xc];
     double acc = 0.0;
-#pragma unroll
-    for (int q = 0; q < RES_RY; q++) {
-        const int j = j0 + q;
-        if (j >= N) break;
-        float out = 0.f;
-        if (x >= 1 && x < N - 1 && j >= 1 && j < N - 1) {
-            const double(&a)[3] = v[q];
-            const double(&b)[3] = v[q + 1];
-            const double(&c)[3] = v[q + 2];
-            const double au = (20.0 * b[1] - 4.0 * (b[0] + a[1] + b[2] + c[1]) -
-                               (a[0] + c[0] + a[2] + c[2])) * inv6h2;
-            const double rv = fv[q] - au;
-            acc += rv * rv;
-            out = (float)rv;
+    auto step = [&](auto phase, int y) {
+        constexpr int p = decltype(phase)::value, p1 = (p + 2) % 3, p2 = (p + 1) % 3;
+        const d2 v = pu[p], fv = pf[p];
+        pu[p] = row(u, y + D);
+        pf[p] = row(f, y + D - 1);
+        Row2& c = ur[p];
+        c.a = tail ? v.y : v.x;
+        c.b = v.y;
+        c.l = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHR1>(0.0, c.b);
+        c.r = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.0, c.a);
+        if (y - 1 < yb) return;                                // row y-1 is the result's
+        const Row2 &a = ur[p2], &b = ur[p1];
+        const double au0 = (20.0 * b.a - 4.0 * (b.l + a.a + b.b + c.a) - (a.l + c.l + a.b + c.b)) * inv6h2;
+        const double au1 = (20.0 * b.b - 4.0 * (b.a + a.b + b.r + c.b) - (a.a + c.a + a.r + c.r)) * inv6h2;
+        const double r0 = in0 ? fv.x - au0 : 0.0, r1 = in1 ? fv.y - au1 : 0.0;
+        if (mine) {
+            acc += r0 * r0;
+            acc += r1 * r1;
+            const f2 o = {(float)r0, (float)r1};
+            if (x < P) __builtin_nontemporal_store(o, (__attribute__((address_space(1))) f2*)(r + (long long)(y - 1) * P + x));
         }
-        if (x < P) {
-            __builtin_nontemporal_store(out, r + (long long)j * P + x);
-            __builtin_nontemporal_store(0.f, e + (long long)j * P + x);
-        }
-    }
+    };
+    for (int y = first; y <= last; y += 3)
+        kg_static_for<3>([&](auto p) {
+            if (y + decltype(p)::value <= last) step(p, y + decltype(p)::value);
+        });
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) acc += __shfl_xor(acc, m);
     if (lane == 0) wsum[w] = acc;
@@ -255,7 +554,13 @@ void pj_sum_k(int n, double* __restrict__ part)
 {
     __shared__ double t[1024];
     double s = 0.0;
-    for (int i = (int)threadIdx.x; i < n; i += 1024) s += part[i];
+    for (int i = (int)threadIdx.x; i < n; i += 8 * 1024) {   // 8 loads in flight
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = i + q * 1024 < n ? part[i + q * 1024] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 8; q++) s += v[q];
+    }
     t[threadIdx.x] = s;
     __syncthreads();
     for (int m = 512; m >= 1; m >>= 1) {
@@ -265,190 +570,90 @@ void pj_sum_k(int n, double* __restrict__ part)
     if (threadIdx.x == 0) part[n] = t[0];
 }
 
-// Residual and full-weighting restriction in one pass (FP32): the coarse
-// right-hand side
-//   fc(I,J) = (4 r_C + 2 (r_W + r_E + r_S + r_N) + (r_SW + r_SE + r_NW + r_NE)) / 16
-// of the fine residual r = f - (20 u - 4 (u_W + u_S + u_E + u_N) - (u_SW +
-// u_NW + u_SE + u_NE)) / (6 h^2) at the 3 x 3 fine points around (2I, 2J),
-// summed in those orders; the fine residual is never stored.  Coarse
-// boundary 0; uc = 0 at the same points (the coarse solve's initial guess).
-template <int ORD>
-__global__ __launch_bounds__(PT * PT)
-void pj_resrestrict_k(int Nc, int Pc, int Pf, int ntx, float inv6h2, const float* __restrict__ u,
-                      const float* __restrict__ f, float* __restrict__ fc, float* __restrict__ uc)
-{
-    const unsigned tb = kg_tile_order<ORD>(blockIdx.x, gridDim.x, (unsigned)ntx);
-    const int I = (int)(tb % (unsigned)ntx) * PT + (int)threadIdx.x;
-    const int J = (int)(tb / (unsigned)ntx) * PT + (int)threadIdx.y;
-    if (I >= Nc || J >= Nc) return;
-    const long long oc = (long long)J * Pc + I;
-    uc[oc] = 0.f;
-    if (I == 0 || J == 0 || I == Nc - 1 || J == Nc - 1) {
-        fc[oc] = 0.f;
-        return;
-    }
-    // fine rows 2J-2 .. 2J+2 and columns 2I-2 .. 2I+2 lie in 0 .. Nf-1
-    const long long o = (long long)(2 * J) * Pf + 2 * I;
-    float uu[5][5];
-#pragma unroll
-    for (int dy = -2; dy <= 2; dy++)
-#pragma unroll
-        for (int dx = -2; dx <= 2; dx++) uu[dy + 2][dx + 2] = u[o + (long long)dy * Pf + dx];
-    float rr[3][3];
-#pragma unroll
-    for (int dy = -1; dy <= 1; dy++)
-#pragma unroll
-        for (int dx = -1; dx <= 1; dx++) {
-#define U(a, b) uu[dy + 2 + (b)][dx + 2 + (a)]
-            const float au = (20.f * U(0, 0) - 4.f * (U(-1, 0) + U(0, -1) + U(1, 0) + U(0, 1)) -
-                              (U(-1, -1) + U(-1, 1) + U(1, -1) + U(1, 1))) * inv6h2;
-#undef U
-            rr[dy + 1][dx + 1] = f[o + (long long)dy * Pf + dx] - au;
-        }
-#define R(a, b) rr[(b) + 1][(a) + 1]
-    fc[oc] = (4.f * R(0, 0) + 2.f * (R(-1, 0) + R(1, 0) + R(0, -1) + R(0, 1)) +
-              (R(-1, -1) + R(1, -1) + R(-1, 1) + R(1, 1))) * 0.0625f;
-#undef R
-}
-
-// u_f += bilinear interpolation of e_c on 4-point pieces of fine rows
-// (x multiple of 4, so fine points x, x+2 sit on coarse columns x/2, x/2+1);
-// e = e_c at even/even points, the mean of the 2 or 4 coarse neighbours
-// elsewhere; writes rows 1 .. Nf-2 whole (0 at the
-// boundary and padding).  One row per lane, 4 rows per workgroup.
-__global__ __launch_bounds__(256)
-void pj_prolong4_k(int Nf, int Pf, int Pc, int ntx, const float* __restrict__ ec,
-                   float* __restrict__ uf)
-{
-    const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
-    const unsigned tb = kg_tile_order<KG_ORD_PJ>(blockIdx.x, gridDim.x, (unsigned)ntx);
-    const int x = (int)(tb % (unsigned)ntx) * 256 + lane * 4;
-    const int j = 1 + (int)(tb / (unsigned)ntx) * 4 + w;
-    if (x >= Pf || j >= Nf - 1) return;
-    const int Nc = (Nf + 1) / 2;
-    const int I0 = x >> 1, J = j >> 1;
-    // coarse columns I0 .. I0+2 (clamped; clamped ones feed boundary or
-    // padding points only) of rows J and J+1 (odd j)
-    float a[3], b[3];
-#pragma unroll
-    for (int q = 0; q < 3; q++) {
-        const int I = min(I0 + q, Nc - 1);
-        a[q] = ec[(long long)J * Pc + I];
-        b[q] = (j & 1) ? ec[(long long)(J + 1) * Pc + I] : 0.f;
-    }
-    float* row = uf + (long long)j * Pf + x;
-    const f4 u = ldf4(row);
-    f4 o;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-        const int q = v >> 1;   // coarse column I0 + q of fine point x + v
-        float e;
-        if (!(v & 1) && !(j & 1)) e = a[q];
-        else if ((v & 1) && !(j & 1)) e = 0.5f * (a[q] + a[q + 1]);
-        else if (!(v & 1)) e = 0.5f * (a[q] + b[q]);
-        else e = 0.25f * (a[q] + a[q + 1] + b[q] + b[q + 1]);
-        o[v] = (x + v >= 1 && x + v < Nf - 1) ? u[v] + e : 0.f;
-    }
-    __builtin_nontemporal_store(o, (__attribute__((address_space(1))) f4*)row);
-}
-
-// exact solve on the coarsest level (3 x 3 vertices: one unknown)
-__global__ void pj_exact3_k(int P, float s, const float* __restrict__ f, float* __restrict__ u)
-{
-    if (threadIdx.x == 0) u[P + 1] = s * f[P + 1];
-}
-
-__global__ __launch_bounds__(256)
-void pj_zero_k(long long n, float* __restrict__ p)
-{
-    for (long long e = (long long)blockIdx.x * 256 + threadIdx.x; e < n; e += (long long)gridDim.x * 256)
-        p[e] = 0.f;
-}
-
-// dense N x N FP64 u += FP32 rows of pitch P
+// dense N x N FP64 u += FP32 rows of pitch P on the interior (a grid whose whole
+// V-cycle is the coarse kernel's)
 __global__ __launch_bounds__(256)
 void pj_add_k(int N, int P, const float* __restrict__ e, double* __restrict__ u)
 {
-    const long long n = (long long)N * N;
-    for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long long)gridDim.x * 256) {
-        const long long j = q / N, i = q - j * N;
-        u[q] += (double)e[j * P + i];
-    }
+    const int q = (int)(blockIdx.x * 256 + threadIdx.x), j = q / N, i = q - j * N;
+    if (i >= 1 && i < N - 1 && j >= 1 && j < N - 1) u[q] += (double)e[j * P + i];
 }
 
 struct Level {
-    int N, P;   // vertices per side, row pitch (N rounded up to 4)
+    int N, P;   // vertices per side, row pitch (N rounded up to 16)
     double h;
     float *u, *t, *f;
 };
 
-unsigned blocks1(long long n) { return (unsigned)std::min<long long>((n + 255) / 256, 256 * 64); }
-
-// workgroups of the 4-point kernels on level L
-struct Grid4 {
-    int ntx;
-    unsigned blocks;
-};
-Grid4 grid4(const Level& L)
+// Rows per wave of the marching passes (even): the most that leaves 8 waves per
+// CU, at least 2.  A wave also marches the 4 to 7 rows around its own, but on
+// small levels its latency is what counts: a 512 cell solve takes 1.20 ms at 8 rows,
+// 1.07 at 4, 1.03 at 2; at 8192 cells 16 to 24 rows are the best of 8 .. 128 by 2 %.
+int march_rows(const kg_ctx* ctx, int ntx, int N)
 {
-    Grid4 g;
-    g.ntx = (L.P + 255) / 256;
-    g.blocks = (unsigned)g.ntx * (unsigned)((L.N - 2 + VW * PY - 1) / (VW * PY));
-    return g;
+    for (int H : {16, 8, 4})
+        if ((long long)ntx * ((N - 2) / H + 1) >= 2LL * ctx->cus) return H;
+    return 2;
 }
 
-// n damped-Jacobi sweeps on level L (result in L.u)
-void smooth(hipStream_t st, Level& L, int n, double omega)
+constexpr double OMEGA = 0.8;   // damping; two sweeps before and two after the coarse levels
+
+float sweep_cf(double h) { return (float)(3 * OMEGA * h * h / 10); }
+float residual_scale(double h) { return (float)(1.0 / (6.0 * h * h)); }
+constexpr float C0 = (float)(1 - OMEGA), C1 = (float)(OMEGA / 5), C2 = (float)(OMEGA / 20);
+
+template <int TOP>
+void launch_coarse(hipStream_t st, const Level& L, bool zero)
 {
-    const float c0 = (float)(1 - omega), c1 = (float)(omega / 5), c2 = (float)(omega / 20);
-    const float cf = (float)(3 * omega * L.h * L.h / 10);
-    const Grid4 g = grid4(L);
-    for (int s = 0; s < n; s++) {
-        if (s + 1 < n) {   // two sweeps in one pass
-            constexpr int PY2 = KG_SM2_PY;
-            const unsigned b2 = (unsigned)g.ntx * (unsigned)((L.N - 2 + VW * PY2 - 1) / (VW * PY2));
-            hipLaunchKernelGGL(pj_smooth4x2_k<PY2>, dim3(b2), dim3(64 * VW), 0, st, L.N, L.P, g.ntx,
-                               c0, c1, c2, cf, L.u, L.f, L.t);
-            std::swap(L.u, L.t);
-            s++;
-            continue;
-        }
-        hipLaunchKernelGGL(pj_smooth4_k, dim3(g.blocks), dim3(64 * VW), 0, st, L.N, L.P, g.ntx, c0,
-                           c1, c2, cf, L.u, L.f, L.t);
-        // the boundary rows of t are 0 like u's (zeroed at allocation, never
-        // written), the boundary columns written as 0
-        std::swap(L.u, L.t);
+    CCoef k{};
+    k.c0 = C0;
+    k.c1 = C1;
+    k.c2 = C2;
+    k.exact = (float)(6.0 * 0.5 * 0.5 / 20.0);
+    int d = 0;
+    for (int n = TOP; n > 2; n /= 2, d++) {
+        k.cf[d] = sweep_cf(1.0 / n);
+        k.inv6h2[d] = residual_scale(1.0 / n);
     }
+    hipLaunchKernelGGL(pj_coarse_k<TOP>, dim3(1), dim3(CT), 0, st, L.P, k, (const float*)L.f, L.u,
+                       (int)zero);
 }
 
-void vcycle(hipStream_t st, Level* lv, int nl, int l, int pre, int post, double omega)
+// One V-cycle on level l from its u (zero: from 0), which ends in L.u, or, with
+// u64, is added to that field.  Rows 0 and N-1 of the levels' arrays are never
+// read or written.
+void vcycle(const kg_ctx* ctx, hipStream_t st, Level* lv, int l, bool zero, double* u64)
 {
     Level& L = lv[l];
-    if (l + 1 == nl) {
-        // 3 x 3 vertices: (A u)(1,1) = 20 u / (6 h^2) = f
-        hipLaunchKernelGGL(pj_exact3_k, dim3(1), dim3(64), 0, st, L.P,
-                           (float)(6.0 * L.h * L.h / 20.0), L.f, L.u);
+    if (L.N - 1 <= CTOP) {
+        switch (L.N - 1) {
+        case 2: launch_coarse<2>(st, L, zero); break;
+        case 4: launch_coarse<4>(st, L, zero); break;
+        case 8: launch_coarse<8>(st, L, zero); break;
+        case 16: launch_coarse<16>(st, L, zero); break;
+        case 32: launch_coarse<32>(st, L, zero); break;
+        case 64: launch_coarse<64>(st, L, zero); break;
+        default: launch_coarse<CTOP>(st, L, zero); break;
+        }
+        if (u64)
+            hipLaunchKernelGGL(pj_add_k, dim3((unsigned)((L.N * L.N + 255) / 256)), dim3(256), 0, st, L.N,
+                               L.P, (const float*)L.u, u64);
         return;
     }
-    smooth(st, L, pre, omega);
     Level& C = lv[l + 1];
-    // C.f = restricted residual, C.u = 0; C.t needs no clearing: every sweep
-    // rewrites its rows 1 .. N-2 whole and its boundary rows stay 0 from the
-    // workspace's set-up
-    // tiles in chunks of 2 tile rows per XCD on the large levels (8192^2
-    // solve 17.0 ms against 17.6 in hardware order, the same u bit for bit),
-    // hardware order on the others (1024^2: 2.2 ms against 2.3-2.4 chunked)
-    const int ntb = (C.N + PT - 1) / PT;   // tiles per side of the coarse level
-    auto rr = C.N > 1024 ? pj_resrestrict_k<2> : pj_resrestrict_k<0>;
-    hipLaunchKernelGGL(rr, dim3((unsigned)ntb * (unsigned)ntb), dim3(PT, PT), 0, st, C.N, C.P, L.P,
-                       ntb, (float)(1.0 / (6.0 * L.h * L.h)), L.u, L.f, C.f, C.u);
-    vcycle(st, lv, nl, l + 1, pre, post, omega);
-    {
-        const int ntx = (L.P + 255) / 256;
-        const unsigned blocks = (unsigned)ntx * (unsigned)((L.N - 2 + 3) / 4);
-        hipLaunchKernelGGL(pj_prolong4_k, dim3(blocks), dim3(256), 0, st, L.N, L.P, C.P, ntx, C.u, L.u);
-    }
-    smooth(st, L, post, omega);
+    const Coef k{C0, C1, C2, sweep_cf(L.h), residual_scale(L.h)};
+    const int ntx = (L.N + MW * PIECE - 1) / (MW * PIECE);
+    const int H = march_rows(ctx, ntx, L.N);
+    const unsigned blocks = (unsigned)ntx * (unsigned)((L.N - 1 + H - 1) / H);
+    auto down = zero ? pj_down_k<true> : pj_down_k<false>;
+    hipLaunchKernelGGL(down, dim3(blocks), dim3(64 * MW), 0, st, L.N, L.P, C.N, C.P, ntx, H, k,
+                       (const float*)L.u, (const float*)L.f, L.t, C.f);
+    std::swap(L.u, L.t);
+    vcycle(ctx, st, lv, l + 1, true, nullptr);
+    auto up = u64 ? pj_up_k<true> : pj_up_k<false>;
+    hipLaunchKernelGGL(up, dim3(blocks), dim3(64 * MW), 0, st, L.N, L.P, C.N, C.P, ntx, H, k,
+                       (const float*)L.u, (const float*)C.u, (const float*)L.f, L.t, u64);
+    std::swap(L.u, L.t);
 }
 
 // Levels n, n/2, ..., 2 cells per side: at most 14 for n <= 16384.
@@ -463,24 +668,19 @@ constexpr int MAX_N = 1 << 14;
 struct Workspace {
     int nl;
     Level lv[MAX_LEVELS];
-    int res_ntx, res_blocks;
+    int res_blocks;
     double* part;
     double* stats;
 };
 
 constexpr size_t align256(size_t b) { return (b + 255) / 256 * 256; }
-constexpr int pitch4(int N) { return (N + 3) / 4 * 4; }
-constexpr int res_blocks_of(int n)
-{
-    return (pitch4(n + 1) + 255) / 256 * ((n + 1 + RES_RY - 1) / RES_RY);
-}
-
+constexpr int pitch(int N) { return (N + 15) / 16 * 16; }
 // Bytes of the workspace of an n-cell solve (n a power of two >= 2).
 constexpr size_t workspace_bytes(int n, size_t stats_bytes)
 {
     size_t b = 0;
     for (int m = n; m >= 2; m /= 2) {
-        const size_t ne = (size_t)(m + 1) * (size_t)pitch4(m + 1);
+        const size_t ne = (size_t)(m + 1) * (size_t)pitch(m + 1);
         b += 3 * align256(ne * sizeof(float));
     }
     b += align256((size_t)(res_blocks_of(n) + 1) * sizeof(double));
@@ -493,8 +693,7 @@ void workspace_shape(Workspace& ws, int n)
 {
     ws.nl = 0;
     for (int m = n; m >= 2; m /= 2)
-        ws.lv[ws.nl++] = Level{m + 1, pitch4(m + 1), 1.0 / m, nullptr, nullptr, nullptr};
-    ws.res_ntx = (ws.lv[0].P + 255) / 256;
+        ws.lv[ws.nl++] = Level{m + 1, pitch(m + 1), 1.0 / m, nullptr, nullptr, nullptr};
     ws.res_blocks = res_blocks_of(n);
     ws.part = ws.stats = nullptr;
 }
@@ -517,18 +716,6 @@ void workspace_carve(Workspace& ws, char* base)
     ws.stats = (double*)(base + off);
 }
 
-// The levels' arrays start at 0: sweeps rely on boundary rows and padding
-// that they never write.
-void workspace_clear(hipStream_t st, Workspace& ws)
-{
-    for (int l = 0; l < ws.nl; l++) {
-        Level& L = ws.lv[l];
-        const long long ne = (long long)L.N * L.P;
-        for (float* p : {L.u, L.t, L.f})
-            hipLaunchKernelGGL(pj_zero_k, dim3(blocks1(ne)), dim3(256), 0, st, ne, p);
-    }
-}
-
 int check_args(kg_ctx* ctx, const char* who, int n, int nmax, const double* f, const double* u)
 {
     if (int rc = kg_check_ctx(ctx)) return rc;
@@ -540,7 +727,7 @@ int check_args(kg_ctx* ctx, const char* who, int n, int nmax, const double* f, c
     return KG_OK;
 }
 
-// The defect-correction loop on a carved and cleared workspace; the stream
+// The defect-correction loop on a carved workspace (of any contents); the stream
 // is synchronised on return.  Timing (events or the host clock) is the
 // caller's: t_start is called once the norm of f is known, right before the
 // first residual pass.
@@ -553,8 +740,6 @@ int solve(kg_ctx* ctx, int n, const double* f, double* u, double tol, int max_ou
     const int N = n + 1;
     const long long np = (long long)N * N;
     const double h = 1.0 / n;
-    const double omega = 0.8;
-    const int pre = 2, post = 2;
     if (max_outer < 1) max_outer = 1;
     if (vcycles < 1) vcycles = 1;
     double st_f[5];
@@ -570,8 +755,8 @@ int solve(kg_ctx* ctx, int n, const double* f, double* u, double tol, int max_ou
     for (;;) {
         // r = f - A u in FP64: its FP32 copy is the right-hand side of the
         // inner solve (F.f), its squared norm decides the stop
-        hipLaunchKernelGGL(pj_residual64_k, dim3(ws.res_blocks), dim3(256), 0, st, N, F.P, ws.res_ntx,
-                           1.0 / (6.0 * h * h), (const double*)u, f, F.f, F.u, ws.part);
+        hipLaunchKernelGGL(pj_residual64_k, dim3(ws.res_blocks), dim3(64 * MW), 0, st, N, F.P,
+                           res_ntx(n), res_rows(n), 1.0 / (6.0 * h * h), (const double*)u, f, F.f, ws.part);
         hipLaunchKernelGGL(pj_sum_k, dim3(1), dim3(1024), 0, st, ws.res_blocks, ws.part);
         double sumsq = 0.0;
         KG_HIP(hipMemcpyAsync(&sumsq, ws.part + ws.res_blocks, sizeof(double), hipMemcpyDeviceToHost, st));
@@ -579,10 +764,10 @@ int solve(kg_ctx* ctx, int n, const double* f, double* u, double tol, int max_ou
         rel = fnorm > 0 ? std::sqrt(sumsq) / fnorm : 0.0;
         if (rep && outer < KG_POISSON_HISTORY) rep->history[outer] = rel;
         if (rel < tol || outer >= max_outer) break;
-        // inner FP32 solve of A e = r from e = 0 (F.u, set by the residual pass)
-        for (int c = 0; c < vcycles; c++) vcycle(st, ws.lv, ws.nl, 0, pre, post, omega);
+        // inner FP32 solve of A e = r from e = 0, then u += e
+        for (int c = 0; c < vcycles; c++)
+            vcycle(ctx, st, ws.lv, 0, c == 0, c == vcycles - 1 ? u : nullptr);
         cycles += vcycles;
-        hipLaunchKernelGGL(pj_add_k, dim3(blocks1(np)), dim3(256), 0, st, F.N, F.P, (const float*)F.u, u);
         outer++;
     }
     KG_HIP(hipGetLastError());
@@ -670,8 +855,7 @@ extern "C" int kg_poisson_solve(kg_ctx* ctx, int n, const double* f, double* u, 
         return done(kg_set_error(KG_ERR_HIP, "kg_poisson_solve: hipEventCreate failed"));
     }
     workspace_carve(ws, base);
-    workspace_clear(st, ws);
-    kg_register_kernel("poisson_smooth", (const void*)pj_smooth4_k);
+    kg_register_kernel("poisson_smooth", (const void*)pj_up_k<false>);
     int outer = 0, cycles = 0;
     double rel = 0;
     if (int rc = solve(ctx, n, f, u, tol, max_outer, vcycles, ws, rep, &outer, &cycles, &rel,
@@ -702,9 +886,7 @@ extern "C" int kg_poisson_solve_noalloc(kg_ctx* ctx, int n, const double* f, dou
                             "workspace, more than the %zu reserved", n, workspace_bytes(n, STATS_BYTES),
                             NOALLOC_BYTES);
     workspace_carve(ws, g_scratch_ptr[ctx->device]);
-    // the previous call's contents are still there
-    workspace_clear(st, ws);
-    kg_register_kernel("poisson_smooth", (const void*)pj_smooth4_k);
+    kg_register_kernel("poisson_smooth", (const void*)pj_up_k<false>);
     int outer = 0, cycles = 0;
     double rel = 0;
     std::chrono::steady_clock::time_point t0;
@@ -716,4 +898,4 @@ extern "C" int kg_poisson_solve_noalloc(kg_ctx* ctx, int n, const double* f, dou
     return finish("kg_poisson_solve_noalloc", rep, ws, outer, cycles, rel, sec, tol);
 }
 
-int kg_preload_poisson() { return kg_preload_kernel((const void*)pj_smooth4_k); }
+int kg_preload_poisson() { return kg_preload_kernel((const void*)pj_up_k<false>); }

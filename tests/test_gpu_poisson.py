@@ -121,3 +121,72 @@ def test_poisson_rejects_bad_arguments(gpu_ctx, kgmod):
         kgmod.poisson_solve(gpu_ctx, 6, a, b)          # not a power of two
     with pytest.raises(kgmod.KGError):
         kgmod.poisson_solve(gpu_ctx, 8, a, a)          # f aliases u
+
+
+# ---- one correction against the same V-cycles in numpy, bit for bit ----
+F = np.float32
+
+
+def around(u):
+    """Centre, the axis neighbours' sum and the diagonal neighbours' sum of
+    the interior, in the order W + S + E + N and SW + NW + SE + NE."""
+    ax = u[1:-1, :-2] + u[:-2, 1:-1] + u[1:-1, 2:] + u[2:, 1:-1]
+    dg = u[:-2, :-2] + u[2:, :-2] + u[:-2, 2:] + u[2:, 2:]
+    return u[1:-1, 1:-1], ax, dg
+
+
+def sweeps(u, f, h):
+    for _ in range(2):
+        c, ax, dg = around(u)
+        u = np.pad(F(1 - 0.8) * c + F(0.8 / 5) * ax + F(0.8 / 20) * dg + F(3 * 0.8 * h * h / 10) * f[1:-1, 1:-1], 1)
+    return u
+
+
+def vcycle(u, f):
+    n = u.shape[0] - 1
+    h = 1.0 / n
+    if n == 2:
+        return np.pad(F(6 * h * h / 20) * f[1:-1, 1:-1], 1)
+    u = sweeps(u, f, h)
+    c, ax, dg = around(u)
+    r = np.pad(f[1:-1, 1:-1] - (F(20) * c - F(4) * ax - dg) * F(1 / (6 * h * h)), 1)
+    R = lambda dy, dx: r[2 + dy:n - 1 + dy:2, 2 + dx:n - 1 + dx:2]  # noqa: E731
+    fc = np.pad((F(4) * R(0, 0) + F(2) * (R(0, -1) + R(0, 1) + R(-1, 0) + R(1, 0)) +
+                 (R(-1, -1) + R(-1, 1) + R(1, -1) + R(1, 1))) * F(0.0625), 1)
+    a = vcycle(np.zeros_like(fc), fc)
+    e = np.zeros_like(u)
+    e[::2, ::2] = a
+    e[::2, 1::2] = F(0.5) * (a[:, :-1] + a[:, 1:])
+    e[1::2, ::2] = F(0.5) * (a[:-1] + a[1:])
+    e[1::2, 1::2] = F(0.25) * (a[:-1, :-1] + a[:-1, 1:] + a[1:, :-1] + a[1:, 1:])
+    u = u.copy()
+    u[1:-1, 1:-1] += e[1:-1, 1:-1]
+    return sweeps(u, f, h)
+
+
+@pytest.mark.parametrize("cycles", [1, 2])
+@pytest.mark.parametrize("n", [2, 4, 8, 16, 32, 64, 128, 256, 512, 1024, 2048])
+def test_poisson_one_correction(gpu_ctx, kgmod, n, cycles):
+    """u after one correction from a random guess: n up to 128 is the coarse
+    kernel's alone; 256 columns and up take 2 or more pieces of 240, 1 to 3
+    workgroups side by side and every count of rows per wave.  FP32
+    arithmetic is IEEE on both sides, so the two agree bit for bit."""
+    rng = np.random.default_rng(n)
+    f = rng.uniform(-1, 1, (n + 1, n + 1))
+    u0 = rng.uniform(-1, 1, (n + 1, n + 1))
+    u0[[0, -1]] = u0[:, [0, -1]] = 0
+    c, ax, dg = around(u0)
+    r = np.pad(f[1:-1, 1:-1] - (20 * c - 4 * ax - dg) * (1 / (6 * (1.0 / n) ** 2)), 1).astype(F)
+    e = np.zeros_like(r)
+    for _ in range(cycles):
+        e = vcycle(e, r)
+    want = u0 + e
+    for noalloc in (False, True) if n <= kgmod.POISSON_NOALLOC_MAX_N else (False,):
+        df, du = gpu_ctx.array(f), gpu_ctx.array(u0)
+        try:
+            kgmod.poisson_solve(gpu_ctx, n, df, du, tol=1e-30, max_outer=1, vcycles=cycles, noalloc=noalloc)
+        except kgmod.KGError as err:
+            assert "relative residual" in str(err)
+        np.testing.assert_array_equal(du.download().reshape(want.shape), want)
+        df.free()
+        du.free()
