@@ -4,8 +4,9 @@
 //
 // At the benchmark shape (512 x 256 x 256, 67 MFLOP) the step is latency
 // work, not throughput work: at the FP64 matrix peak it is under a
-// microsecond.  So the kernel is shaped for many short, independent waves
-// whose loads are all in flight before the first product:
+// microsecond.  So the kernel for such products (matmul_k) is shaped for many
+// short, independent waves whose loads are all in flight before the first product
+// (larger ones: matmul_tiles_k):
 //
 //   * a workgroup of KS = 4 waves owns one 16 x 16 tile of C (512 workgroups
 //     at 512 x 256: two per compute unit);
@@ -32,6 +33,7 @@ namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 typedef double v2d __attribute__((ext_vector_type(2)));
+typedef double v2u __attribute__((ext_vector_type(2), aligned(8)));   // at any element
 
 // Measured at 512 x 256 x 256 (40 back-to-back launches): 8.1 us (8.3
 // TFLOP/s) against 61 us for one wave per tile walking all of k with each
@@ -42,6 +44,9 @@ typedef double v2d __attribute__((ext_vector_type(2)));
 #endif
 #ifndef KG_MM_KC
 #define KG_MM_KC 64
+#endif
+#ifndef KG_ORD_MM
+#define KG_ORD_MM 8            // 2048^3: 278 us, 284 with 2 or 4
 #endif
 constexpr int KS = KG_MM_KS;   // waves per workgroup: the k range split KS ways
 constexpr int KC = KG_MM_KC;   // k values per chunk (KC/4 MFMA steps)
@@ -107,6 +112,171 @@ void matmul_k(int nx, int ny, int ns, int ntile_i, int kq, const double* __restr
     }
 }
 
+// Tiles of 16 T x 16 T (T = 2 or 4) for products large enough to fill the device
+// with them: every wave of the 4 holds the whole tile for its k range (the ranges,
+// their blocks of four products and the order in which they are added are
+// matmul_k's, and so is the result, bit for bit), so an operand read feeds T matrix
+// steps instead of one.  An MFMA step occupies its SIMD for 64 cycles: at T = 4 the
+// 16 of a k block take 1024 cycles for 4 KB of operands, which the caches deliver
+// straight into registers, 8 values of k ahead (a wave's next operands have 2048
+// cycles to arrive).  LDS only serves the final sum, in T T / 4 tiles at a time.
+//
+// Row m of tile 2p+q is row 32p + 2m + q: the operands of two tiles are one 16-byte
+// load of A, and a lane's results are pairs of rows.  Rows and columns past the
+// matrix read its last ones and are not stored.
+//
+// 2048^3 278 us (61.8 TFLOP/s), bound by the matrix cores, against 694 with 16 x 16
+// tiles, whose operand reads bound it; 1500^3 160 us (429), 1024^3 46 (104).  T = 2
+// reaches 44 TFLOP/s at 2048^3, bound by L1 (2 to 4 blocks in flight change nothing),
+// but gives a smaller product four times as many workgroups: 512 x 512 with k =
+// 2048 30 us (72 with T = 4, 48 with 16 x 16 tiles), 512^3 9.5 (24 and 15).
+template <int T>
+__global__ __launch_bounds__(64 * KS, T == 2 ? 6 : 2)
+void matmul_tiles_k(int nx, int ny, int ns, int ntile_i, int kq, const double* __restrict__ A,
+                    const double* __restrict__ B, double* __restrict__ C)
+{
+    constexpr int Q = T * T / KS;      // 16 x 16 tiles a wave sums and stores
+    __shared__ v4d part[KS][Q][64];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = (int)(threadIdx.x & 63);
+    const int lr = lane & 15, lg = lane >> 4;
+    const unsigned tb = kg_tile_order<KG_ORD_MM>(blockIdx.x, gridDim.x, (unsigned)ntile_i);
+    const int i0 = (int)(tb % (unsigned)ntile_i) * 16 * T, j0 = (int)(tb / (unsigned)ntile_i) * 16 * T;
+    const int kb = wave * kq, ke = min(kb + kq, ny);
+
+    v4d acc[T][T];
+#pragma unroll
+    for (int a = 0; a < T; a++)
+#pragma unroll
+        for (int b = 0; b < T; b++) {
+            const int j = j0 + 16 * b + lr;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int i = i0 + 32 * (a / 2) + 2 * (lg + 4 * r) + a % 2;
+                acc[a][b][r] = wave == 0 && i < nx && j < ns ? C[(long long)i + (long long)nx * j] : 0.0;
+            }
+        }
+
+    const double *pa[T / 2], *pb[T];   // operands of k = kb + 2 lg
+    bool tail[T / 2];                  // the lane's first row is the matrix's last
+#pragma unroll
+    for (int p = 0; p < T / 2; p++) {
+        const int i = i0 + 32 * p + 2 * lr;
+        tail[p] = i == nx - 1;
+        pa[p] = A + min(i, nx - 2) + (long long)nx * (kb + 2 * lg);
+    }
+#pragma unroll
+    for (int b = 0; b < T; b++) pb[b] = B + (long long)ny * min(j0 + 16 * b + lr, ns - 1) + kb + 2 * lg;
+
+    struct Ops { v2d a[T / 2][2], b[T]; };   // two MFMA steps: 8 values of k
+    Ops next;
+    auto load = [&](Ops& o) {
+#pragma unroll
+        for (int p = 0; p < T / 2; p++) {
+            o.a[p][0] = *(const v2u*)pa[p];
+            o.a[p][1] = *(const v2u*)(pa[p] + nx);
+            pa[p] += 8LL * nx;
+        }
+#pragma unroll
+        for (int b = 0; b < T; b++) {
+            o.b[b] = *(const v2u*)pb[b];
+            pb[b] += 8;
+        }
+    };
+    auto mult = [&](const Ops& o) {
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int p = 0; p < T / 2; p++) {
+                const double x = o.a[p][s].x, y = o.a[p][s].y;
+                const double a0 = tail[p] ? y : x;
+#pragma unroll
+                for (int b = 0; b < T; b++) {
+                    acc[2 * p][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, o.b[b][s], acc[2 * p][b], 0, 0, 0);
+                    acc[2 * p + 1][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(y, o.b[b][s], acc[2 * p + 1][b], 0, 0, 0);
+                }
+            }
+    };
+    const int nt = ke > kb ? (ke - kb) / 8 : 0;
+    if (nt > 0) load(next);
+    for (int t = 0; t < nt; t++) {
+        const Ops o = next;
+        if (t + 1 < nt) load(next);
+        mult(o);
+    }
+    if (kb + 8 * nt < ke) {            // the last 1 .. 7 values: 0 past them
+        const int k = kb + 8 * nt + 2 * lg;
+        const bool k0ok = k < ke, k1ok = k + 1 < ke;
+        Ops o;
+#pragma unroll
+        for (int p = 0; p < T / 2; p++) {
+            o.a[p][0] = o.a[p][1] = v2d{0.0, 0.0};
+            if (k0ok) o.a[p][0] = *(const v2u*)pa[p];
+            if (k1ok) o.a[p][1] = *(const v2u*)(pa[p] + nx);
+        }
+#pragma unroll
+        for (int b = 0; b < T; b++) {
+            o.b[b].x = k0ok ? pb[b][0] : 0.0;
+            o.b[b].y = k1ok ? pb[b][1] : 0.0;
+        }
+        mult(o);
+    }
+
+    // the four ranges' sums, in order; wave w adds and stores tiles w Q .. w Q + Q-1
+    kg_static_for<KS>([&](auto c) {
+        constexpr int w = decltype(c)::value;
+        if (w > 0) __syncthreads();
+        if (wave != w) {
+#pragma unroll
+            for (int q = 0; q < Q; q++) part[wave][q][lane] = acc[(w * Q + q) / T][(w * Q + q) % T];
+        }
+        __syncthreads();
+        if (wave == w) {
+#pragma unroll
+            for (int q = 0; q < Q; q++) {
+                const int a = (w * Q + q) / T, b = (w * Q + q) % T;
+                v4d sum = w == 0 ? acc[a][b] : part[0][q][lane];
+#pragma unroll
+                for (int v = 1; v < KS; v++) sum += v == w ? acc[a][b] : part[v][q][lane];
+                const int j = j0 + 16 * b + lr;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int i = i0 + 32 * (a / 2) + 2 * (lg + 4 * r) + a % 2;
+                    if (i < nx && j < ns) C[(long long)i + (long long)nx * j] = sum[r];
+                }
+            }
+        }
+    });
+}
+
+template <int T>
+void launch_tiles(kg_ctx* ctx, int nx, int ny, int ns, int kq, const double* A, const double* B, double* C)
+{
+    const int ti = (nx + 16 * T - 1) / (16 * T), tj = (ns + 16 * T - 1) / (16 * T);
+    kg_launch(ctx, matmul_tiles_k<T>, dim3((unsigned)((long long)ti * tj)), dim3(64 * KS), 0, nx, ny, ns, ti,
+              kq, A, B, C);
+}
+
+// The work of the busiest CU in 16 x 16 tiles when it is dealt out in tiles of T x T.
+long long busiest(const kg_ctx* ctx, int nx, int ns, int T)
+{
+    const long long t = (long long)((nx + 16 * T - 1) / (16 * T)) * ((ns + 16 * T - 1) / (16 * T));
+    return (t + ctx->cus - 1) / ctx->cus * T * T;
+}
+
+// Tile edge in units of 16.  A 16 x 16 tile of the result costs its CU 2.2, 3.0 and
+// 5.3 us per 1000 values of k at T = 4, 2 and 1, so a larger T is taken unless it leaves
+// the busiest CU too much: T = 4 up to 4/3 of T = 2 (equal times at 777 x 1333 x 901,
+// 16 against 12; at 301 x 2011 x 1203, 16 against 8, T = 2 is 1.4 times as fast),
+// T = 2 below twice T = 1 (3 against 4 at 333 x 257 x 421: 7.9 against 10.5 us; 2
+// against 4 at 512 x 256 x 256: 7.3 against 6.3).
+int tile_edge(const kg_ctx* ctx, int nx, int ns)
+{
+    const long long w1 = busiest(ctx, nx, ns, 1), w2 = busiest(ctx, nx, ns, 2), w4 = busiest(ctx, nx, ns, 4);
+    if (nx < 2 || w2 >= 2 * w1) return 1;   // (pairs of rows)
+    return 3 * w4 <= 4 * w2 ? 4 : 2;
+}
+
 }  // namespace
 
 extern "C" int kg_matmul(kg_ctx* ctx, int nx, int ny, int ns, const double* A, const double* B,
@@ -125,7 +295,10 @@ extern "C" int kg_matmul(kg_ctx* ctx, int nx, int ny, int ns, const double* A, c
     const int kq = ((ny + KS - 1) / KS + 3) / 4 * 4;
     kg_register_kernel("matmul_", (const void*)matmul_k);
     if (int rc = kg_launch_begin(ctx, "matmul_")) return rc;
-    if (tiles > 0)
+    const int edge = tile_edge(ctx, nx, ns);
+    if (edge == 4) launch_tiles<4>(ctx, nx, ny, ns, kq, A, B, C);
+    else if (edge == 2) launch_tiles<2>(ctx, nx, ny, ns, kq, A, B, C);
+    else if (tiles > 0)
         kg_launch(ctx, matmul_k, dim3((unsigned)tiles), dim3(64 * KS), 0, nx, ny, ns, ti, kq, A, B,
                   C);
     return kg_launch_end(ctx);

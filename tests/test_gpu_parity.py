@@ -283,3 +283,27 @@ def test_gpu_rejects_bad_arguments(gpu_ctx, kgmod):
         gpu_ctx.call("gameoflife", 8, 8, None, a)
     with pytest.raises(kgmod.KGError, match="invalid argument"):
         gpu_ctx.call("whispering", 8, 8, 0.5, 0.5, a, a, *[gpu_ctx.empty(64) for _ in range(8)])
+
+
+@pytest.mark.parametrize("dims", [(1024, 37, 1031), (1025, 1, 1023), (333, 257, 421), (515, 64, 513),
+                                  (2047, 35, 1025), (777, 130, 901), (1500, 100, 1501)])
+def test_gpu_matmul_tiles(gpu_ctx, kgmod, dims):
+    """Products tiled 32 x 32 and 64 x 64, at odd buffer addresses, against the
+    same product 16 columns at a time (16 x 16 tiles: few enough workgroups): an
+    element's arithmetic is the same, so the bits are.  Infinities and a NaN
+    in the last row and column stay there."""
+    nx, ny, ns = dims
+    rng = np.random.default_rng(nx)
+    A, B, C = (rng.uniform(-1, 1, s) for s in ((ny, nx), (ns, ny), (ns, nx)))   # column-major operands
+    A[0, -1], B[-1, 0], B[-1, -1] = np.inf, -np.inf, np.nan
+    a, b, c, d = (gpu_ctx.array(np.concatenate([[0.0], x.ravel()])) for x in (A, B, C, C))
+    def mm(n, pb, pc):
+        kgmod._check(gpu_ctx.lib, gpu_ctx.lib.kg_matmul(gpu_ctx.ptr, nx, ny, n, a.ptr + 8, pb, pc), "kg_matmul")
+    mm(ns, b.ptr + 8, c.ptr + 8)
+    for j in range(0, ns, 16):
+        mm(min(16, ns - j), b.ptr + 8 + 8 * ny * j, d.ptr + 8 + 8 * nx * j)
+    got, want = c.download()[1:], d.download()[1:]
+    np.testing.assert_array_equal(got.view(np.int64), want.view(np.int64))
+    assert np.isfinite(got.reshape(ns, nx)[:-1, :-1]).all()
+    for x in (a, b, c, d):
+        x.free()
