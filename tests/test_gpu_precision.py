@@ -317,3 +317,31 @@ def test_typed_ragged_rows(gpu_ctx, oracle, which, dtype):
         want = _run_oracle(oracle.lib, fn, dims, coefs, ins, out, 2, rot, f64 if dtype == "f64" else f32)
         for g, w in zip(got, want):
             assert g.tobytes() == w.tobytes(), f"{fn} {dims}"
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("src", [0, 1, 2])
+@pytest.mark.parametrize("dst", [0, 1, 2])
+def test_convert_lengths(gpu_ctx, kgmod, src, dst, off):
+    """Every pair of types, at and between the workgroups' pieces (512 lanes
+    of 2, 4 or 8 elements), on 16 byte boundaries and off them; nothing is
+    written around the result."""
+    npt = [np.float64, np.float32, np.uint16]
+    rng = np.random.default_rng(3 * src + dst)
+    for n in (1, 2, 1023, 1024, 1025, 2047, 2048, 4095, 4096, 4097, 9001):
+        v = rng.uniform(-2, 2, n) * 10.0 ** rng.integers(-45, 38, n)
+        v[::97] = np.inf
+        with np.errstate(over="ignore"):
+            x32 = v.astype(np.float32)
+        x = v if src == 0 else x32 if src == 1 else to_bf16(x32)
+        w32 = x32 if src < 2 else (x.astype(np.uint32) << 16).view(np.float32)
+        want = (x if src == 0 else w32.astype(np.float64)) if dst == 0 else w32 if dst == 1 else to_bf16(w32)
+        a = gpu_ctx.array(np.concatenate([np.zeros(off, npt[src]), x]))
+        fill = np.full(n + off + 8, 7, npt[dst])
+        b = gpu_ctx.array(fill)
+        kgmod._check(gpu_ctx.lib, gpu_ctx.lib.kg_convert(
+            gpu_ctx.ptr, dst, b.ptr + off * b.dtype.itemsize, src, a.ptr + off * a.dtype.itemsize, n), "kg_convert")
+        fill[off:off + n] = want
+        assert b.download().tobytes() == fill.tobytes(), n
+        a.free()
+        b.free()
