@@ -15,6 +15,7 @@
 // can wait for one row while the later ones stay in flight.  The cell at x-1
 // comes from the lane below (ds_bpermute), the cell at x+16 from the lane
 // above; the wave's end lanes load the 4 bytes beside their segment instead.
+// Rows may start at any byte.
 // The neighbour count is done four cells at a time in 32-bit words (SWAR):
 // counts are at most 8, so byte lanes never carry into each other.  Per row
 // the horizontal triple sum l+m+r is formed once and reused as the upper,
@@ -46,6 +47,10 @@ constexpr int LIFE_YC = LIFE_NP * LIFE_U;     // output rows per band
 constexpr int LIFE_SLOW_YC = 16;              // rows per workgroup, cell-wise kernel
 
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
+// at any byte
+typedef unsigned u2a __attribute__((ext_vector_type(2), aligned(1)));
+typedef unsigned u1a __attribute__((aligned(1)));
+typedef uint16_t u16a __attribute__((aligned(1)));
 
 // 0x01 in every byte lane whose byte is nonzero, 0x00 elsewhere.
 __device__ __forceinline__ unsigned nz_bytes(unsigned x)
@@ -58,10 +63,21 @@ struct LifeRow {
     unsigned h[4];   // per-cell sum of the cells at x-1, x, x+1 of this row
 };
 
+// Where a row ends in the middle of a lane's 16 cells (RAG), that lane takes the
+// row's last 16 cells, nx-16 .. nx-1, instead, and computes some of the lane's
+// below over again: no access crosses the row's end, whatever nx is.
+struct LifeLane {
+    int lane;
+    bool first, tail;   // takes x-1 from its side bytes; RAG: takes the row's end
+    int skip;           // RAG: place in the tail lane of the cell after the lane's below
+};
+
 // One row of a lane: raw = its 16 cells, side = the 4 bytes beside the wave's
-// segment (lane 0: cells x-4..x-1, lane 63: cells x+16..x+19, else unused).
-__device__ __forceinline__ LifeRow life_row(u4 raw, unsigned side, int lane)
+// segment (first: cells x-4..x-1, lane 63: cells x+13..x+16, else unused).
+template <bool RAG>
+__device__ __forceinline__ LifeRow life_row(u4 raw, unsigned side, const LifeLane& me)
 {
+    const int lane = me.lane;
     LifeRow row;
     row.m[0] = nz_bytes(raw.x);
     row.m[1] = nz_bytes(raw.y);
@@ -70,9 +86,15 @@ __device__ __forceinline__ LifeRow life_row(u4 raw, unsigned side, int lane)
     const unsigned s = nz_bytes(side);
     // cell x-1: top byte of the lane below; cell x+16: low byte of the lane above
     const unsigned below = (unsigned)__builtin_amdgcn_ds_bpermute((lane - 1) * 4, (int)row.m[3]);
-    const unsigned above = (unsigned)__builtin_amdgcn_ds_bpermute((lane + 1) * 4, (int)row.m[0]);
-    const unsigned l = (lane == 0 ? s : below) >> 24;
-    const unsigned r = (lane == 63 ? s : above) & 0xffu;
+    unsigned low = row.m[0];
+    if constexpr (RAG) {
+        const int q = me.skip >> 2;   // uniform
+        const unsigned a = q & 1 ? row.m[1] : row.m[0], b = q & 1 ? row.m[3] : row.m[2];
+        low = me.tail ? (q & 2 ? b : a) >> (8 * (me.skip & 3)) : low;
+    }
+    const unsigned above = (unsigned)__builtin_amdgcn_ds_bpermute((lane + 1) * 4, (int)low);
+    const unsigned l = (me.first ? s : below) >> 24;
+    const unsigned r = lane == 63 ? s >> 24 : above & 0xffu;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         // byte b of `left` is the cell at x-1 of byte b, of `right` at x+1
@@ -106,7 +128,7 @@ __device__ __forceinline__ uint8_t life_cell(const uint8_t* c0, long long o, int
     return (uint8_t)((n == 3) || (alive && n == 2));
 }
 
-// Rows with nx % 16 != 0 (the vector kernel below needs aligned rows): a
+// Rows shorter than 20 cells, or longer than the vector kernel's offsets: a
 // workgroup of 256 threads takes LIFE_SLOW_YC rows of 256 cells, cell by cell.
 __global__ __launch_bounds__(256)
 void life_u8_cells_k(int nx, int ny, int ntx, const uint8_t* __restrict__ c0,
@@ -123,14 +145,18 @@ void life_u8_cells_k(int nx, int ny, int ntx, const uint8_t* __restrict__ c0,
     }
 }
 
-// nx % 16 == 0 and 1 <= nx <= 2^24 (offsets within a band fit 31 bits).
-// Bands of 4 rows measured fastest at 4096^2 .. 16384^2 (16-row bands 15 %
-// slower).  Tile order KG_ORD_LIFE8: chunks of 8 bands per XCD, so a band's
-// neighbour rows and segments share its L2 (ping-pong steps, 50-launch means:
-// 8192^2 30.7 us, 16384^2 100 us; hardware order 31.4 / 107, XCD-contiguous
-// 37.9 / 108, chunks of 2, 4 or 16 bands within 2 %).  At 8192^2, 2 or 8
-// segments per workgroup ran 33.5 and 32.2 us against 31.0 for 4; 2 rows in
-// flight the same, 5 rows 32.4 us; two ring turns per band (D = 1) 31.1 us.
+// nx % 16 == 0, or with RAG any nx >= 20 (the tail lane reads its side bytes at
+// nx-20); nx <= 2^24 (offsets within a band fit 31 bits).
+// Bands of 4 rows measured fastest at 4096^2 .. 16384^2 (8 rows 3 % slower).  Tile
+// order KG_ORD_LIFE8: chunks of 8 bands per XCD, so a band's neighbour rows and
+// segments share its L2 (hardware order 2 % slower at 8192^2 and 7 % at 16384^2);
+// 8 segments per workgroup run alike at 8192^2 and 20 % slower at 4096^2.
+// A step of 8192^2 takes 22.5 us (6.0 TB/s, bound by memory): 31 us with the row's
+// end lanes storing 15 single cells and with stores that bypass the caches, which
+// the next step's loads then miss (25.9 with those alone; at 16384^2, where no level
+// stays cached, 102 against 97).  8000 x 8191 22.0 us (31.5 cell by cell), 5000 x
+// 4001 9.8 (42), 777 x 7000 8.2 (18.5).
+template <bool RAG>
 __global__ __launch_bounds__(64 * LIFE_WAVES)
 void life_u8_k(int nx, int ny, int nsx, const uint8_t* __restrict__ c0, uint8_t* __restrict__ c1)
 {
@@ -138,7 +164,7 @@ void life_u8_k(int nx, int ny, int nsx, const uint8_t* __restrict__ c0, uint8_t*
     const int sx = (int)(b % (unsigned)nsx);
     const int band = (int)(b / (unsigned)nsx);
     const int lane = (int)(threadIdx.x & 63);
-    const int x = (sx * LIFE_WAVES + (int)(threadIdx.x >> 6)) * LIFE_SEG + lane * LIFE_CW;
+    int x = (sx * LIFE_WAVES + (int)(threadIdx.x >> 6)) * LIFE_SEG + lane * LIFE_CW;
     const int j0 = 1 + band * LIFE_YC;            // first output row (< ny-1)
     const int j1 = min(j0 + LIFE_YC, ny - 1);     // output rows j0 .. j1-1
     // Resources cover exactly the band: input rows j0-1 .. j1, output rows
@@ -148,11 +174,18 @@ void life_u8_k(int nx, int ny, int nsx, const uint8_t* __restrict__ c0, uint8_t*
     const __amdgpu_buffer_rsrc_t rout =
         kgp::make_rsrc(c1 + (long long)j0 * nx, (unsigned)(j1 - j0) * (unsigned)nx);
     const bool xin = x < nx;
+    LifeLane me{lane, lane == 0, false, 0};
+    if constexpr (RAG) {
+        me.tail = xin && x + LIFE_CW > nx;
+        me.first |= me.tail;
+        me.skip = LIFE_CW - nx % LIFE_CW;
+        if (me.tail) x = nx - LIFE_CW;
+    }
     const unsigned vx = xin ? (unsigned)x : kgp::KG_OOB;
-    const unsigned sx_off = lane == 0 && xin && x >= 4 ? (unsigned)(x - 4)
-                          : lane == 63 && x + LIFE_CW < nx ? (unsigned)(x + LIFE_CW) : kgp::KG_OOB;
+    const unsigned sx_off = me.first && xin && x >= 4 ? (unsigned)(x - 4)
+                          : lane == 63 && x + LIFE_CW < nx ? (unsigned)(x + LIFE_CW - 3) : kgp::KG_OOB;
     // lanes whose 16 cells are all interior store a vector; the two lanes
-    // holding cell 0 or cell nx-1 store their other 15 cells one by one
+    // holding cell 0 or cell nx-1 store their other 15 cells in pieces
     const bool full = xin && x >= 1 && x + LIFE_CW <= nx - 1;
     const bool edge = xin && !full;
     const unsigned vst = full ? (unsigned)x : kgp::KG_OOB;
@@ -171,8 +204,8 @@ void life_u8_k(int nx, int ny, int nsx, const uint8_t* __restrict__ c0, uint8_t*
     load(1, raw1, s1);
 #pragma unroll
     for (int d = 0; d < LIFE_D; d++) load(2 + d, ring[d], side[d]);
-    LifeRow up = life_row(raw0, s0, lane);
-    LifeRow mid = life_row(raw1, s1, lane);
+    LifeRow up = life_row<RAG>(raw0, s0, me);
+    LifeRow mid = life_row<RAG>(raw1, s1, me);
     // Enter the loop with no load in flight (vmcnt(0)).  The ring's registers
     // before the loop need not be the ones the loop uses; a load still pending
     // there would make the compiler's wait at the loop head assume it was the
@@ -183,21 +216,30 @@ void life_u8_k(int nx, int ny, int nsx, const uint8_t* __restrict__ c0, uint8_t*
     auto step = [&](auto phase, int t) {
         constexpr int P = decltype(phase)::value;
         load(t + 2 + LIFE_D, ring[(P + LIFE_D) % LIFE_NP], side[(P + LIFE_D) % LIFE_NP]);
-        const LifeRow dn = life_row(ring[P], side[P], lane);
+        const LifeRow dn = life_row<RAG>(ring[P], side[P], me);
         unsigned res[4];
 #pragma unroll
         for (int q = 0; q < 4; q++)
             res[q] = life_rule(up.h[q] + (mid.h[q] - mid.m[q]) + dn.h[q], mid.m[q]);
         const unsigned ro = (unsigned)t * (unsigned)nx;
         const u4 out = {res[0], res[1], res[2], res[3]};
-        __builtin_amdgcn_raw_buffer_store_b128(out, rout, vst == kgp::KG_OOB ? vst : ro + vst, 0, 2);
+        __builtin_amdgcn_raw_buffer_store_b128(out, rout, vst == kgp::KG_OOB ? vst : ro + vst, 0, 0);
         if (edge && j0 + t < j1) {
-            uint8_t bytes[LIFE_CW];
-            __builtin_memcpy(bytes, res, sizeof bytes);
-            uint8_t* row = c1 + (long long)(j0 + t) * nx;
-#pragma unroll
-            for (int q = 0; q < LIFE_CW; q++)
-                if (x + q >= 1 && x + q < nx - 1) row[x + q] = bytes[q];
+            uint8_t* p = c1 + (long long)(j0 + t) * nx + x;
+            if (x == 0) {
+                p[1] = (uint8_t)(res[0] >> 8);
+                *(u16a*)(p + 2) = (uint16_t)(res[0] >> 16);
+                *(u1a*)(p + 4) = res[1];
+            } else {
+                *(u2a*)p = u2a{res[0], res[1]};
+            }
+            if (x + LIFE_CW == nx) {
+                *(u1a*)(p + 8) = res[2];
+                *(u16a*)(p + 12) = (uint16_t)res[3];
+                p[14] = (uint8_t)(res[3] >> 16);
+            } else {
+                *(u2a*)(p + 8) = u2a{res[2], res[3]};
+            }
         }
         up = mid;
         mid = dn;
@@ -217,14 +259,16 @@ extern "C" int kg_life_u8(kg_ctx* ctx, int nx, int ny, const uint8_t* c0, uint8_
     if (c0 == c1) return kg_set_error(KG_ERR_INVALID, "kg_life_u8: c0 and c1 must be distinct");
     if (((uintptr_t)c0 | (uintptr_t)c1) & (LIFE_CW - 1))
         return kg_set_error(KG_ERR_INVALID, "kg_life_u8: buffers must be 16-byte aligned");
-    const bool vec = nx % LIFE_CW == 0 && nx <= (1 << 24);
-    kg_register_kernel("life_u8", vec ? (const void*)life_u8_k : (const void*)life_u8_cells_k);
+    const bool rag = nx % LIFE_CW != 0;
+    const bool vec = (!rag || nx >= LIFE_CW + 4) && nx <= (1 << 24);
+    auto kern = rag ? life_u8_k<true> : life_u8_k<false>;
+    kg_register_kernel("life_u8", vec ? (const void*)kern : (const void*)life_u8_cells_k);
     if (int rc = kg_launch_begin(ctx, "life_u8")) return rc;
     if (nx > 2 && ny > 2) {
         if (vec) {
             const unsigned nsx = (unsigned)((nx + LIFE_TX - 1) / LIFE_TX);
             const unsigned nb = (unsigned)((ny - 2 + LIFE_YC - 1) / LIFE_YC);
-            kg_launch(ctx, life_u8_k, dim3(nsx * nb), dim3(64 * LIFE_WAVES), 0, nx, ny, (int)nsx,
+            kg_launch(ctx, kern, dim3(nsx * nb), dim3(64 * LIFE_WAVES), 0, nx, ny, (int)nsx,
                       c0, c1);
         } else {
             const unsigned ntx = (unsigned)((nx - 2 + 255) / 256);
@@ -237,6 +281,6 @@ extern "C" int kg_life_u8(kg_ctx* ctx, int nx, int ny, const uint8_t* c0, uint8_
 
 int kg_preload_life()
 {
-    if (int rc = kg_preload_kernel((const void*)life_u8_k)) return rc;
+    if (int rc = kg_preload_kernel((const void*)life_u8_k<false>)) return rc;
     return kg_preload_kernel((const void*)life_u8_cells_k);
 }

@@ -93,3 +93,15 @@ def test_life_u8_rejects_bad_arguments(gpu_ctx, kgmod):
     b = gpu_ctx.empty((80,), np.uint8)
     with pytest.raises(kgmod.KGError):
         gpu_ctx.call("life_u8", 8, 8, a.ptr + 1, b)
+
+
+@pytest.mark.parametrize("nx", [20, 21, 31, 33, 47, 1001, 1023, 1025, 1039, 1041, 2047, 4095, 4097, 4101, 5000])
+def test_life_u8_row_ends(gpu_ctx, oracle, nx):
+    """Rows that end in the middle of a lane's 16 cells: in a wave's first
+    lane, its last one and between, one to fifteen cells in, on whole and
+    partial bands, the last of which ends with the buffer."""
+    for ny in (3, 6, 9, 23):
+        cells = np.random.default_rng(nx * ny).integers(0, 2, (ny, nx)).astype(np.uint8)
+        for steps in (1, 3):
+            np.testing.assert_array_equal(_gpu_steps(gpu_ctx, cells, steps),
+                                          _oracle_steps(oracle, cells, steps), err_msg=f"{nx} x {ny}")
