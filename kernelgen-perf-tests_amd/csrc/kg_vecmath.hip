@@ -13,11 +13,12 @@
 // vecadd and sincos are one-read-per-input streams: each thread takes one
 // 16-byte piece of every array (two doubles or four floats), workgroups in
 // address order.  matvec keeps the reference's sequential sum per row
-// (bit-identical to an IEEE build), one lane per row: for 16-byte aligned
-// rows the lane streams its own row (matvec_rows_k: 512 x 65536 FP64 in
-// 63 us against 251 us for the LDS-staged form); otherwise a workgroup owns
-// 128 rows, stages column chunks of A in LDS with coalesced loads, and each
-// lane sums its own row from LDS in column order.
+// (bit-identical to an IEEE build), one lane per row: the lane streams its own
+// row (matvec_rows_k: 512 x 65536 FP64 in 60 us against 251 us for the LDS-staged
+// form, 511 x 60000 in 50 against 266, 509 x 300 in 16 against 184); only past the
+// 2 GiB that its offsets reach a workgroup owns 128 rows, stages column chunks of
+// A in LDS with coalesced loads, and each lane sums its own row from LDS in
+// column order.
 #include "kg_plane.h"
 
 #include <algorithm>
@@ -123,9 +124,8 @@ void matvec_k(int nx, int ny, const T* __restrict__ A, const T* __restrict__ x, 
     if (j < ny) y[j] = acc;
 }
 
-// Row-streaming form for rows of a multiple of per16 values on 16-byte
-// aligned A (every row starts on a 16-byte boundary): lane j sums row j
-// itself, reading it with 16-byte loads CH values at a time, the next chunk
+// Row-streaming form: lane j sums row j itself, reading it with 16-byte loads (at
+// any element address) CH values at a time, the next chunk
 // in flight while the current one is summed (two register buffers, named at
 // compile time so no copy waits for a load).  x[i] is the same for every
 // lane and comes through the scalar cache.  One lane per row leaves few
@@ -172,26 +172,32 @@ void matvec_rows_k(int nx, int ny, const T* __restrict__ A, const T* __restrict_
     constexpr int CH = mv_chunk<T>();
     const int j = (int)(blockIdx.x * 64 + threadIdx.x);
     const __amdgpu_buffer_rsrc_t r = kgp::make_rsrc(A, a_bytes);
+    // the sum over whole 16-byte pieces, then the values of a last part of one (a
+    // piece there could cross the end of A); loads past those feed nothing
+    const int whole = nx - nx % per16<T>();
     // lanes past the last row read nothing (offset beyond the resource)
     const unsigned row = j < ny ? (unsigned)((long long)j * nx * (long long)sizeof(T)) : kgp::KG_OOB;
     T b0[CH], b1[CH];
     T acc = 0;
     mv_load<T>(r, row, b0);
     int i0 = 0;
-    for (; i0 + 2 * CH <= nx; i0 += 2 * CH) {
+    for (; i0 + 2 * CH <= whole; i0 += 2 * CH) {
         mv_load<T>(r, row + (unsigned)((i0 + CH) * sizeof(T)), b1);
-        acc = mv_sum<T, true>(acc, b0, x, i0, nx);
-        if (i0 + 2 * CH < nx) mv_load<T>(r, row + (unsigned)((i0 + 2 * CH) * sizeof(T)), b0);
-        acc = mv_sum<T, true>(acc, b1, x, i0 + CH, nx);
+        acc = mv_sum<T, true>(acc, b0, x, i0, whole);
+        if (i0 + 2 * CH < whole) mv_load<T>(r, row + (unsigned)((i0 + 2 * CH) * sizeof(T)), b0);
+        acc = mv_sum<T, true>(acc, b1, x, i0 + CH, whole);
     }
-    if (i0 < nx) {   // a last chunk, in b0 (whole or in part)
-        acc = mv_sum<T, false>(acc, b0, x, i0, nx);
-        if (i0 + CH < nx) {
+    if (i0 < whole) {   // a last chunk, in b0 (whole or in part)
+        acc = mv_sum<T, false>(acc, b0, x, i0, whole);
+        if (i0 + CH < whole) {
             mv_load<T>(r, row + (unsigned)((i0 + CH) * sizeof(T)), b1);
-            acc = mv_sum<T, false>(acc, b1, x, i0 + CH, nx);
+            acc = mv_sum<T, false>(acc, b1, x, i0 + CH, whole);
         }
     }
-    if (j < ny) y[j] = acc;
+    if (j < ny) {
+        for (int i = whole; i < nx; i++) acc = acc + A[(long long)j * nx + i] * x[i];
+        y[j] = acc;
+    }
 }
 
 unsigned blocks_for(long long n) { return (unsigned)((n + 255) / 256); }
@@ -240,10 +246,10 @@ int matvec(kg_ctx* ctx, const char* who, const char* name, int nx, int ny, const
     if (!A || !x || !y) return kg_set_error(KG_ERR_INVALID, "%s: null buffer", who);
     if (y == A || y == x) return kg_set_error(KG_ERR_INVALID, "%s: y aliases an input", who);
     const long long a_bytes = (long long)nx * ny * (long long)sizeof(T);
-    const bool rows16 = nx % per16<T>() == 0 && !((uintptr_t)A & 15) && a_bytes < (1LL << 31);
-    kg_register_kernel(name, rows16 ? (const void*)matvec_rows_k<T> : (const void*)matvec_k<T>);
+    const bool rows = a_bytes < (1LL << 31);   // 32-bit offsets
+    kg_register_kernel(name, rows ? (const void*)matvec_rows_k<T> : (const void*)matvec_k<T>);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
-    if (ny > 0 && rows16 && nx > 0)
+    if (ny > 0 && rows && nx > 0)
         kg_launch(ctx, matvec_rows_k<T>, dim3((ny + 63) / 64), dim3(64), 0, nx, ny, A, x, y,
                   (unsigned)a_bytes);
     else if (ny > 0)

@@ -157,3 +157,19 @@ def test_sincos_f32(gpu_ctx, oracle, dims):
     oracle.lib.oracle_sincos_f32(C.c_size_t(n), vp(x), vp(y), vp(want))
     got = _gpu(gpu_ctx, "sincos_f32", dims, [x, y], np.zeros(n, np.float32))
     np.testing.assert_allclose(got, want, rtol=0, atol=SINCOS_TOL32)
+
+
+@pytest.mark.parametrize("ctype", [np.float64, np.float32])
+def test_matvec_row_ends(gpu_ctx, oracle, ctype):
+    """Rows of every remainder of a 16-byte piece, around one and two chunks,
+    on a buffer that starts at an odd element and ends with the last row."""
+    sfx = "" if ctype is np.float64 else "_f32"
+    for nx in (1, 2, 3, 5, 31, 32, 33, 34, 35, 63, 65, 66, 67, 96, 97, 127, 129, 130, 131, 193, 257):
+        for ny in (1, 63, 65, 130):
+            rng = np.random.default_rng(nx * 7 + ny)
+            A, x = rng.uniform(-1, 1, nx * ny).astype(ctype), rng.uniform(-1, 1, nx).astype(ctype)
+            want = np.zeros(ny, ctype)
+            getattr(oracle.lib, "oracle_matvec" + sfx)(nx, ny, vp(A), vp(x), vp(want))
+            for got in (_gpu(gpu_ctx, "matvec" + sfx, (nx, ny), [A, x], np.zeros(ny, ctype)),
+                        _gpu_shifted(gpu_ctx, "matvec" + sfx, (nx, ny), [A, x], np.zeros(ny, ctype), 1)):
+                np.testing.assert_array_equal(got, want, err_msg=f"{nx} x {ny}")
