@@ -1708,7 +1708,6 @@ extern "C" int kg_serve_run(kg_ctx* ctx, const kg_job* jobs, int njobs, size_t h
     double* check_res = nullptr;   // pinned: 5 statistics per job
     hipEvent_t checked = nullptr;
     bool checks_live = false;
-    const double* stats_res = ctx->stats + kg_stats_scratch_bytes() / sizeof(double) - 5;
     if (hipHostMalloc((void**)&check_res, sizeof(double) * 5 * (size_t)std::max(njobs, 1),
                       hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&checked, hipEventDisableTiming) != hipSuccess) {
@@ -1800,13 +1799,9 @@ extern "C" int kg_serve_run(kg_ctx* ctx, const kg_job* jobs, int njobs, size_t h
                 int lev = 0;
                 if ((rc = kg_batch_newest_level(b, x.id, &lev))) break;
                 if ((rc = kg_field_stats_launch(kg_stream(ctx), j.dtype, (size_t)g.sz * j.ns, g.lev[lev],
-                                                j.dtype, g.lev[lev ^ 1], ctx->stats)))
+                                                j.dtype, g.lev[lev ^ 1], ctx->stats,
+                                                check_res + 5 * x.job)))
                     break;
-                if (hipMemcpyAsync(check_res + 5 * x.job, stats_res, 5 * sizeof(double),
-                                   hipMemcpyDeviceToHost, kg_stream(ctx)) != hipSuccess) {
-                    rc = kg_set_error(KG_ERR_HIP, "kg_serve_run: convergence check copy failed");
-                    break;
-                }
                 x.check_at = x.done;
                 issued = true;
             }

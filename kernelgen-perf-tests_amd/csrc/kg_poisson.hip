@@ -311,7 +311,7 @@ void pj_up_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* 
 // own the points.  A thread owns R = TOP^2/1024 rows of one column (one point on
 // the levels below 64 cells), so a wave reads consecutive LDS words.  As
 // launches these levels took 30 of the 40 of a 512 cell V-cycle, which bound its
-// solve (1.98 ms; 0.95 now).  The cycle from 128 cells takes 22 us, bound by one CU's
+// solve (1.98 ms; 0.79 now).  The cycle from 128 cells takes 22 us, bound by one CU's
 // FP32 rate and LDS on the first level and by barriers below.
 constexpr int CTOP = 128;
 constexpr int CT = 1024;               // threads
@@ -547,10 +547,10 @@ void pj_residual64_k(int N, int P, int ntx, int H, double inv6h2, const double* 
     if (threadIdx.x == 0) part[tb] = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
 }
 
-// part[n] = sum of part[0 .. n) in a fixed order (one workgroup of 1024
+// out[0] = sum of part[0 .. n) in a fixed order (one workgroup of 1024
 // threads: strided per-thread sums, then a tree).
 __global__ __launch_bounds__(1024)
-void pj_sum_k(int n, double* __restrict__ part)
+void pj_sum_k(int n, const double* __restrict__ part, double* __restrict__ out)
 {
     __shared__ double t[1024];
     double s = 0.0;
@@ -567,7 +567,7 @@ void pj_sum_k(int n, double* __restrict__ part)
         if ((int)threadIdx.x < m) t[threadIdx.x] += t[threadIdx.x + m];
         __syncthreads();
     }
-    if (threadIdx.x == 0) part[n] = t[0];
+    if (threadIdx.x == 0) out[0] = t[0];
 }
 
 // dense N x N FP64 u += FP32 rows of pitch P on the interior (a grid whose whole
@@ -743,10 +743,11 @@ int solve(kg_ctx* ctx, int n, const double* f, double* u, double tol, int max_ou
     if (max_outer < 1) max_outer = 1;
     if (vcycles < 1) vcycles = 1;
     double st_f[5];
-    if (int rc = kg_field_stats_launch(st, KG_F64, (size_t)np, f, KG_F64, nullptr, ws.stats)) return rc;
-    KG_HIP(hipMemcpyAsync(st_f, ws.stats + kg_stats_scratch_bytes() / sizeof(double) - 5,
-                          sizeof st_f, hipMemcpyDeviceToHost, st));
-    KG_HIP(hipStreamSynchronize(st));
+    const bool host = ctx->host != nullptr;   // where the results come to
+    double* stats = host ? ctx->host : ws.stats + kg_stats_scratch_bytes() / sizeof(double) - 5;
+    double* sum = host ? ctx->host : ws.part + ws.res_blocks;
+    if (int rc = kg_field_stats_launch(st, KG_F64, (size_t)np, f, KG_F64, nullptr, ws.stats, stats)) return rc;
+    if (int rc = kg_bring_results(st, st_f, stats, 5, host)) return rc;
     const double fnorm = std::sqrt(st_f[1]);
     int outer = 0, cycles = 0;
     double rel = 0;
@@ -757,10 +758,10 @@ int solve(kg_ctx* ctx, int n, const double* f, double* u, double tol, int max_ou
         // inner solve (F.f), its squared norm decides the stop
         hipLaunchKernelGGL(pj_residual64_k, dim3(ws.res_blocks), dim3(64 * MW), 0, st, N, F.P,
                            res_ntx(n), res_rows(n), 1.0 / (6.0 * h * h), (const double*)u, f, F.f, ws.part);
-        hipLaunchKernelGGL(pj_sum_k, dim3(1), dim3(1024), 0, st, ws.res_blocks, ws.part);
+        hipLaunchKernelGGL(pj_sum_k, dim3(1), dim3(1024), 0, st, ws.res_blocks,
+                           (const double*)ws.part, sum);
         double sumsq = 0.0;
-        KG_HIP(hipMemcpyAsync(&sumsq, ws.part + ws.res_blocks, sizeof(double), hipMemcpyDeviceToHost, st));
-        KG_HIP(hipStreamSynchronize(st));
+        if (int rc = kg_bring_results(st, &sumsq, sum, 1, host)) return rc;
         rel = fnorm > 0 ? std::sqrt(sumsq) / fnorm : 0.0;
         if (rep && outer < KG_POISSON_HISTORY) rep->history[outer] = rel;
         if (rel < tol || outer >= max_outer) break;

@@ -156,6 +156,11 @@ extern "C" int kg_init(kg_ctx** out, int device)
         kg_destroy(c);
         return kg_set_error(KG_ERR_NOMEM, "kg_init: statistics scratch allocation failed");
     }
+    // without it results are copied from device memory
+    if (hipHostMalloc((void**)&c->host, KG_HOST_RESULTS * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        c->host = nullptr;
+    }
     int (*preload[])() = {kg_preload_stencil3d, kg_preload_tricubic, kg_preload_stencil2d,
                           kg_preload_matmul, kg_preload_util, kg_preload_life,
                           kg_preload_typed, kg_preload_batch, kg_preload_poisson,
@@ -171,6 +176,14 @@ extern "C" int kg_init(kg_ctx** out, int device)
         return rc;
     }
     *out = c;
+    return KG_OK;
+}
+
+int kg_bring_results(hipStream_t st, double* to, const double* from, int n, bool from_host)
+{
+    if (!from_host) KG_HIP(hipMemcpyAsync(to, from, n * sizeof(double), hipMemcpyDeviceToHost, st));
+    KG_HIP(hipStreamSynchronize(st));
+    if (from_host) memcpy(to, from, n * sizeof(double));
     return KG_OK;
 }
 
@@ -191,6 +204,7 @@ extern "C" int kg_destroy(kg_ctx* ctx)
         if (ctx->ev_stop[i]) (void)hipEventDestroy(ctx->ev_stop[i]);
     }
     if (ctx->stats) (void)hipFree(ctx->stats);
+    if (ctx->host) (void)hipHostFree(ctx->host);
     (void)hipStreamDestroy(ctx->queue);
     free(ctx->ev_start);
     free(ctx->ev_stop);

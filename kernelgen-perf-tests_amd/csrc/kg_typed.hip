@@ -284,26 +284,36 @@ void stats_final_k(int nblocks, const double* __restrict__ part, double* __restr
     if (t < 5) out[t] = red[t][0];
 }
 
-template <int DX, int DR>
-static void launch_stats(hipStream_t st, size_t n, const void* x, const void* r, double* part,
-                         double* out)
+// go(kernel, workgroups, args...) launches a kernel of KG_STATS_THREADS threads.
+template <int DX, int DR, class Go>
+static void launch_stats(Go&& go, size_t n, const void* x, const void* r, double* part, double* out)
 {
-    hipLaunchKernelGGL((stats_k<DX, DR>), dim3(KG_STATS_BLOCKS), dim3(KG_STATS_THREADS), 0, st, n,
-                       x, r, part);
-    hipLaunchKernelGGL(stats_final_k, dim3(1), dim3(KG_STATS_THREADS), 0, st, KG_STATS_BLOCKS,
-                       part, out);
+    go(stats_k<DX, DR>, KG_STATS_BLOCKS, n, x, r, part);
+    go(stats_final_k, 1, KG_STATS_BLOCKS, (const double*)part, out);
 }
 
-template <int DX>
-static int stats_dispatch_ref(hipStream_t st, int rdt, size_t n, const void* x, const void* r,
-                              double* part, double* out)
+template <int DX, class Go>
+static int stats_dispatch_ref(Go&& go, int rdt, size_t n, const void* x, const void* r, double* part,
+                              double* out)
 {
-    if (!r) launch_stats<DX, -1>(st, n, x, r, part, out);
-    else if (rdt == KG_F64) launch_stats<DX, KG_F64>(st, n, x, r, part, out);
-    else if (rdt == KG_F32) launch_stats<DX, KG_F32>(st, n, x, r, part, out);
-    else if (rdt == KG_BF16) launch_stats<DX, KG_BF16>(st, n, x, r, part, out);
+    if (!r) launch_stats<DX, -1>(go, n, x, r, part, out);
+    else if (rdt == KG_F64) launch_stats<DX, KG_F64>(go, n, x, r, part, out);
+    else if (rdt == KG_F32) launch_stats<DX, KG_F32>(go, n, x, r, part, out);
+    else if (rdt == KG_BF16) launch_stats<DX, KG_BF16>(go, n, x, r, part, out);
     else return kg_set_error(KG_ERR_INVALID, "kg_field_stats: unknown reference dtype %d", rdt);
     return KG_OK;
+}
+
+template <class Go>
+static int stats_dispatch(Go&& go, int dt, int rdt, size_t n, const void* x, const void* r, double* part,
+                          double* out)
+{
+    switch (dt) {
+    case KG_F64: return stats_dispatch_ref<KG_F64>(go, rdt, n, x, r, part, out);
+    case KG_F32: return stats_dispatch_ref<KG_F32>(go, rdt, n, x, r, part, out);
+    case KG_BF16: return stats_dispatch_ref<KG_BF16>(go, rdt, n, x, r, part, out);
+    default: return kg_set_error(KG_ERR_INVALID, "kg_field_stats: unknown dtype %d", dt);
+    }
 }
 
 // ------------------------------------------------------------ conversion
@@ -568,26 +578,24 @@ extern "C" int kg_field_stats(kg_ctx* ctx, int dtype, size_t n, const void* x, i
                "kg_field_stats: unknown reference dtype");
     int rc = KG_OK;
     double* dev = ctx->stats;   // KG_STATS_BLOCKS*5 partials followed by 5 results
+    double* res = ctx->host ? ctx->host : dev + KG_STATS_BLOCKS * 5;
     kg_register_kernel("field_stats", (const void*)stats_final_k);
     if ((rc = kg_launch_begin(ctx, "field_stats"))) return rc;
-    if ((rc = kg_field_stats_launch(kg_stream(ctx), dtype, n, x, ref_dtype, ref, dev))) return rc;
+    auto go = [&](auto kern, int blocks, auto... a) {
+        kg_launch(ctx, kern, dim3((unsigned)blocks), dim3(KG_STATS_THREADS), 0, a...);
+    };
+    if ((rc = stats_dispatch(go, dtype, ref_dtype, n, x, ref, dev, res))) return rc;
     if ((rc = kg_launch_end(ctx))) return rc;
-    KG_HIP(hipMemcpyAsync(out, dev + KG_STATS_BLOCKS * 5, 5 * sizeof(double), hipMemcpyDeviceToHost,
-                          kg_stream(ctx)));
-    KG_HIP(hipStreamSynchronize(kg_stream(ctx)));
-    return KG_OK;
+    return kg_bring_results(kg_stream(ctx), out, res, 5, ctx->host != nullptr);
 }
 
 int kg_field_stats_launch(hipStream_t st, int dtype, size_t n, const void* x, int ref_dtype,
-                          const void* ref, double* scratch)
+                          const void* ref, double* scratch, double* out)
 {
-    double* res = scratch + KG_STATS_BLOCKS * 5;
-    switch (dtype) {
-    case KG_F64: return stats_dispatch_ref<KG_F64>(st, ref_dtype, n, x, ref, scratch, res);
-    case KG_F32: return stats_dispatch_ref<KG_F32>(st, ref_dtype, n, x, ref, scratch, res);
-    case KG_BF16: return stats_dispatch_ref<KG_BF16>(st, ref_dtype, n, x, ref, scratch, res);
-    default: return kg_set_error(KG_ERR_INVALID, "kg_field_stats: unknown dtype %d", dtype);
-    }
+    auto go = [&](auto kern, int blocks, auto... a) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(KG_STATS_THREADS), 0, st, a...);
+    };
+    return stats_dispatch(go, dtype, ref_dtype, n, x, ref, scratch, out);
 }
 
 size_t kg_stats_scratch_bytes() { return (KG_STATS_BLOCKS * 5 + 5) * sizeof(double); }
