@@ -912,44 +912,67 @@ void shape_of(const kg_batch* b, const HostGrid& g, int& li, int& kc)
     }
 }
 
-// Most planes per tile for the untuned grids of a batch (shape_of's kc is cut
-// down to it).  A batch of few or small grids has fewer tiles than there are
-// workgroups, and a step then takes as long as its thickest tile.  A tile costs
-// about as much as KG_ITEM_PLANES planes to start, and the workgroups take the
-// tiles in rounds: the cap with the least of the longest tile and of the rounds
-// at the mean cost.  A step, against the default's 8 to 32 planes: 8 grids up to
-// 64^3 8.7 us (33.9), 40 FP32 grids up to 128^3 28.5 us (49.7), 40 FP64 ones
-// 45.8 us (53.8); 200 grids keep the default (306 us).  2 to 12 planes a tile's
-// start all choose alike; halving every tile until there are 1, 2 or 4 per
-// workgroup gave 35-43 us for the 40 FP32 grids and 47-59 for the FP64 ones.
-constexpr int KG_ITEM_PLANES = 5;
+// Most planes per tile for the untuned grids of a batch (capped_kc).  A batch of few
+// or small grids has fewer tiles than there are workgroups, and a step then takes
+// as long as its costliest tile.  A tile costs about as much as KG_ITEM_PLANES planes
+// to start, the planes beside its own and its planes, and the workgroups take the
+// tiles in rounds: the cap with the least of the costliest tile and of the rounds at
+// the mean cost.  A step, against the default's 8 to 32 planes: 8 grids up to 64^3
+// 8.3 us (33.9), 40 FP32 grids up to 128^3 23.7 (49.7), 40 FP64 ones 43.6 (53.8); 200
+// grids keep the default (306).  With gaussblur3's planes taken for as cheap as the
+// others' 28.3, 48.5 and, for 12 FP32 grids up to 128^3, 16.6 us (11.0 now).  6, 9 or
+// 12 planes a tile's start choose alike up to 40 grids; 6 cuts the 200 grids finer.
+constexpr int KG_ITEM_PLANES = 9;
+
+// What a plane of a tile costs against one of laplacian or wave13pt (0.54 us in a
+// tile of its own on an idle device): gaussblur3's 25 points 1.33 us in packed rows, 0.9
+// in the other shapes.
+double plane_cost(int kind, int li)
+{
+    return kind != KG_KIND_GAUSSBLUR3 || li == ROW2 || li == COL ? 1.0 : li == PACK ? 2.5 : 1.7;
+}
+
+// Planes per tile of grid g under the batch's cap.
+int capped_kc(const kg_batch* b, const HostGrid& g, int cap)
+{
+    if (b->tuned.count(size_class(g.spec))) return g.kc;
+    return std::max(2, std::min(g.kc, (int)(cap / plane_cost(g.spec.kind, g.li))));
+}
+
+// What a tile costs besides its planes: the start, and the planes it reads beside
+// its own.
+double tile_start(const HostGrid& g)
+{
+    const VarInfo& v = VARS[var_id(g.spec.kind, g.spec.dtype, g.li)];
+    return KG_ITEM_PLANES + v.zlo + v.zhi;
+}
 
 int planes_cap(const kg_batch* b, const std::vector<int>& order)
 {
     double best = 0;
-    int pick = KCS[NKC - 1];
-    for (int cap = KCS[NKC - 1]; cap >= 2; cap /= 2) {
-        long long items = 0, longest = 0;
-        double cost = 0;
+    int pick = 0;
+    for (int cap : {160, 112, 80, 56, 40, 32, 24, 20, 16, 12, 8, 6, 4, 2}) {
+        long long items = 0;
+        double cost = 0, longest = 0;
         for (int gi : order) {
             const HostGrid& g = b->grids[gi];
-            const int kc = b->tuned.count(size_class(g.spec)) ? g.kc : std::min(g.kc, cap);
+            const int kc = capped_kc(b, g, cap);
             const Cut c = cut_of(g, g.li, kc);
             if (!c.items()) continue;
-            const int thick = g.li == ROW2 ? 1 : kc;
             items += c.items();
-            cost += (double)c.items() * KG_ITEM_PLANES + (double)c.ntx * c.nty * c.planes;
-            longest = std::max<long long>(longest, KG_ITEM_PLANES + std::min(thick, c.planes));
+            const double start = tile_start(g), plane = plane_cost(g.spec.kind, g.li);
+            const int thick = g.li == ROW2 ? 1 : kc;
+            cost += c.items() * start + plane * c.ntx * c.nty * c.planes;
+            longest = std::max(longest, start + plane * std::min(thick, c.planes));
         }
         if (!items) break;
-        const double est = std::max((double)longest,
-                                    (double)((items + b->nwg - 1) / b->nwg) * cost / items);
+        const double est = std::max(longest, (double)((items + b->nwg - 1) / b->nwg) * cost / items);
         if (best == 0 || est < best) {
             best = est;
             pick = cap;
         }
     }
-    return pick;
+    return pick ? pick : 160;
 }
 
 // Upload descriptors and the work list (largest grids' tiles first).  With
@@ -990,7 +1013,7 @@ int build_work(kg_batch* b, int only_class = -1, int li_force = 0, int kc_force 
         const int cap = planes_cap(b, order);
         for (int gi : order) {
             HostGrid& g = b->grids[gi];
-            if (!b->tuned.count(size_class(g.spec))) g.kc = descs[gi].kc = std::min(g.kc, cap);
+            g.kc = descs[gi].kc = capped_kc(b, g, cap);
         }
     }
     std::vector<Item> items;
