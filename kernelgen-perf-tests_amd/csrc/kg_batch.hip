@@ -259,10 +259,17 @@ struct Item {
     int var;              // the grid's variant id (read with the item)
 };
 
+// Counters that all workgroups add to, each on a line of its own: with the eight of
+// the list on one line a step of 476 tiles (40 FP64 grids) took 43.6 us against
+// 36.2, a queue of 32 jobs 27.4 ms against 23.2.  (Workgroups that count their ends
+// per XCD first cost a step 0.3 us more.)
+struct alignas(128) BatchLine {
+    unsigned v;
+};
 struct BatchState {
     unsigned long long step;          // steps completed by the batch
-    unsigned counter[KG_NUM_XCD];     // next item of each XCD's part of the list
-    unsigned done;                    // workgroups finished this launch
+    BatchLine counter[KG_NUM_XCD];    // next item of each XCD's part of the list
+    BatchLine done;                   // workgroups finished this launch
 };
 
 // Not inlined: each variant then gets its own register allocation and the
@@ -511,7 +518,7 @@ void batch_k(const GridDesc* __restrict__ grids, const Item* __restrict__ items,
             while (left) {
                 const int p = (home + __builtin_ctz(left)) % KG_NUM_XCD;
                 int n = 0;
-                if (threadIdx.x == 0) n = (int)atomicAdd(&st->counter[p], 1u);
+                if (threadIdx.x == 0) n = (int)atomicAdd(&st->counter[p].v, 1u);
                 n = __builtin_amdgcn_readfirstlane(n);
                 if (n < queued(p)) {
                     got = part_lo(p + 1) - queued(p) + n;
@@ -521,7 +528,7 @@ void batch_k(const GridDesc* __restrict__ grids, const Item* __restrict__ items,
                 const int o = (home + (int)threadIdx.x) % KG_NUM_XCD;
                 bool some = false;
                 if (threadIdx.x < KG_NUM_XCD)
-                    some = (int)__hip_atomic_load(&st->counter[o], __ATOMIC_RELAXED,
+                    some = (int)__hip_atomic_load(&st->counter[o].v, __ATOMIC_RELAXED,
                                                   __HIP_MEMORY_SCOPE_AGENT) < queued(o);
                 left &= (unsigned)__ballot(some);
             }
@@ -535,10 +542,10 @@ void batch_k(const GridDesc* __restrict__ grids, const Item* __restrict__ items,
     // No fence: the state is only touched by atomics, each of them waited for,
     // and the levels are read by later launches.
     if (threadIdx.x == 0) {
-        if (atomicAdd(&st->done, 1u) == gridDim.x - 1) {
+        if (atomicAdd(&st->done.v, 1u) == gridDim.x - 1) {
             // every workgroup has taken its last item and read `step`
-            for (int x = 0; x < KG_NUM_XCD; x++) atomicExch(&st->counter[x], 0u);
-            atomicExch(&st->done, 0u);
+            for (int x = 0; x < KG_NUM_XCD; x++) atomicExch(&st->counter[x].v, 0u);
+            atomicExch(&st->done.v, 0u);
             atomicExch(&st->step, step + 1);
         }
     }
@@ -665,8 +672,8 @@ __global__ void state_set_k(BatchState* st, unsigned long long step)
 {
     if (threadIdx.x == 0) {
         atomicExch(&st->step, step);
-        for (int x = 0; x < KG_NUM_XCD; x++) atomicExch(&st->counter[x], 0u);
-        atomicExch(&st->done, 0u);
+        for (int x = 0; x < KG_NUM_XCD; x++) atomicExch(&st->counter[x].v, 0u);
+        atomicExch(&st->done.v, 0u);
     }
 }
 
@@ -918,7 +925,7 @@ void shape_of(const kg_batch* b, const HostGrid& g, int& li, int& kc)
 // to start, the planes beside its own and its planes, and the workgroups take the
 // tiles in rounds: the cap with the least of the costliest tile and of the rounds at
 // the mean cost.  A step, against the default's 8 to 32 planes: 8 grids up to 64^3
-// 8.3 us (33.9), 40 FP32 grids up to 128^3 23.7 (49.7), 40 FP64 ones 43.6 (53.8); 200
+// 8.3 us (33.9), 40 FP32 grids up to 128^3 23.7 (49.7), 40 FP64 ones 36.2 (53.8); 200
 // grids keep the default (306).  With gaussblur3's planes taken for as cheap as the
 // others' 28.3, 48.5 and, for 12 FP32 grids up to 128^3, 16.6 us (11.0 now).  6, 9 or
 // 12 planes a tile's start choose alike up to 40 grids; 6 cuts the 200 grids finer.
