@@ -37,7 +37,6 @@ namespace {
 #define KG_ORD_PJ 2
 #endif
 
-typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 typedef double d2 __attribute__((ext_vector_type(2)));
 typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));   // at any element
@@ -46,13 +45,13 @@ typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));   // at any 
 // A V-cycle visits a level twice: on the way down two damped Jacobi sweeps, the
 // residual and its full-weighting restriction, on the way up the bilinear
 // correction and two sweeps.  Each visit is one pass over the level (pj_down_k,
-// pj_up_k): a wave takes 256 columns, 4 per lane, and marches them along y; an
+// pj_up_k): a wave takes 64 V columns, V per lane, and marches them along y; an
 // incoming row enters a window of three rows, which gives the first sweep of the
 // row before it, three of those give the second sweep of the row before that,
 // and so on, so that HBM sees u, f and the result once per visit.  The columns
-// beside a lane's 4 come from the neighbouring lanes by DPP.  Every stage makes
+// beside a lane's V come from the neighbouring lanes by DPP.  Every stage makes
 // the wave's outermost column on either side invalid; the outer lanes hold only
-// such overlap (pieces start every 240 columns, 64-byte aligned).  Expressions and
+// such overlap (pieces start every 240 or 112 columns, 64-byte aligned).  Expressions and
 // orders are those of separate sweeps, residual and restriction, and so is the
 // result, bit for bit.
 //
@@ -60,37 +59,43 @@ typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));   // at any 
 // level are 871 MB at 8192^2, 203 us (4.3 TB/s; the best copy reaches 6.3) for
 // pj_up_k and 188 for pj_down_k.  Sweep pairs, residual and restriction,
 // prolongation and the addition to u as passes of their own took 14.2 of the 17.7 ms
-// of an 8192^2 solve (7.5, 3.3, 1.9, 1.5); it takes 10.4 so.  Rows of 64-byte
+// of an 8192^2 solve (7.5, 3.3, 1.9, 1.5); it takes 10.0 so.  Rows of 64-byte
 // multiples and pieces of 240 columns, so that no wave writes part of a sector:
 // 5 % faster at 8192^2 than 248 columns of 4-float pitches.  The 4 waves of a
 // workgroup lie side by side; one above the other costs 2 % more.  Small levels
-// are bound by a wave's march: 6 us at 512 cells and below.
+// are bound by a wave's march (6 us at 512 cells and below), whose steps V = 2 halves:
+// solves of 256 to 1024 cells 0.59, 0.80, 1.01 -> 0.56, 0.76, 0.96 ms.  It is taken where
+// 4 rows per wave leave a CU less than 8 waves; elsewhere V = 4 marches less overlap.
 constexpr int MW = 4;                  // waves per workgroup, side by side in x
-constexpr int PIECE = 240;             // columns a wave completes
+// columns a wave completes, V per lane: 1 or 2 lanes on either side are overlap
+template <int V> constexpr int edge_lanes() { return 4 / V; }
+template <int V> constexpr int piece() { return V == 4 ? 240 : 112; }
 
 struct Coef {
     float c0, c1, c2, cf;              // sweep: c0 u + c1 axis + c2 diag + cf f
     float inv6h2;
 };
 
-// Four columns of a row and the ones on either side of them.
+// A lane's columns of a row and the ones on either side of them.
+template <int V>
 struct Row {
-    float v[4], l, r;
-    __device__ __forceinline__ float at(int i) const { return i < 0 ? l : i > 3 ? r : v[i]; }
+    float v[V], l, r;
+    __device__ __forceinline__ float at(int i) const { return i < 0 ? l : i > V - 1 ? r : v[i]; }
     __device__ __forceinline__ void sides()
     {
-        l = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHR1>(0.f, v[3]);
+        l = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHR1>(0.f, v[V - 1]);
         r = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.f, v[0]);
     }
 };
 
 // damped Jacobi sweep of row b (a below, c above it): u' = c0 u + c1 (W + S + E +
 // N) + c2 (SW + NW + SE + NE) + cf f on the interior, 0 elsewhere
-__device__ __forceinline__ void pj_sweep(const Coef& k, const Row& a, const Row& b, const Row& c,
-                                         const float (&f)[4], bool row_in, const bool (&in)[4], Row& o)
+template <int V>
+__device__ __forceinline__ void pj_sweep(const Coef& k, const Row<V>& a, const Row<V>& b, const Row<V>& c,
+                                         const float (&f)[V], bool row_in, const bool (&in)[V], Row<V>& o)
 {
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
+    for (int v = 0; v < V; v++) {
         const float val = k.c0 * b.v[v] + k.c1 * (b.at(v - 1) + a.v[v] + b.at(v + 1) + c.v[v]) +
                           k.c2 * (a.at(v - 1) + c.at(v - 1) + a.at(v + 1) + c.at(v + 1)) + k.cf * f[v];
         o.v[v] = row_in && in[v] ? val : 0.f;
@@ -99,11 +104,12 @@ __device__ __forceinline__ void pj_sweep(const Coef& k, const Row& a, const Row&
 }
 
 // r = f - (20 u - 4 (W + S + E + N) - (SW + NW + SE + NE)) / (6 h^2)
-__device__ __forceinline__ void pj_resid(const Coef& k, const Row& a, const Row& b, const Row& c,
-                                         const float (&f)[4], Row& o)
+template <int V>
+__device__ __forceinline__ void pj_resid(const Coef& k, const Row<V>& a, const Row<V>& b, const Row<V>& c,
+                                         const float (&f)[V], Row<V>& o)
 {
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
+    for (int v = 0; v < V; v++) {
         const float au = (20.f * b.v[v] - 4.f * (b.at(v - 1) + a.v[v] + b.at(v + 1) + c.v[v]) -
                           (a.at(v - 1) + c.at(v - 1) + a.at(v + 1) + c.at(v + 1))) * k.inv6h2;
         o.v[v] = f[v] - au;
@@ -113,10 +119,11 @@ __device__ __forceinline__ void pj_resid(const Coef& k, const Row& a, const Row&
 
 // What the marching passes share: the wave's columns and rows.  Rows 0 and N-1
 // and everything outside the grid count as 0 and are never read.
+template <int V>
 struct March {
     int N, P, x, yb, ye;               // lane's first column; rows [yb, ye) are completed
     unsigned voff;                     // its byte offset in a row, or out of range
-    bool in[4], mine;                  // columns of the interior; the lane completes its columns
+    bool in[V], mine;                  // columns of the interior; the lane completes its columns
     __device__ __forceinline__ bool setup(int N_, int P_, int ntx, int H)
     {
         N = N_;
@@ -124,14 +131,14 @@ struct March {
         const unsigned tb = kg_tile_order<KG_ORD_PJ>(blockIdx.x, gridDim.x, (unsigned)ntx);
         const int lane = (int)(threadIdx.x & 63);
         const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-        x = ((int)(tb % (unsigned)ntx) * MW + w) * PIECE - 4 + 4 * lane;
+        x = ((int)(tb % (unsigned)ntx) * MW + w) * piece<V>() + V * (lane - edge_lanes<V>());
         yb = (int)(tb / (unsigned)ntx) * H;
         ye = min(yb + H, N - 1);
         voff = x >= 0 && x < P ? (unsigned)x * 4u : kgp::KG_OOB;
 #pragma unroll
-        for (int v = 0; v < 4; v++) in[v] = x + v >= 1 && x + v < N - 1;
-        mine = lane >= 1 && lane <= PIECE / 4 && x < P;
-        return x - 4 * lane < N - 4;   // the piece has a column
+        for (int v = 0; v < V; v++) in[v] = x + v >= 1 && x + v < N - 1;
+        mine = lane >= edge_lanes<V>() && lane < edge_lanes<V>() + piece<V>() / V && x < P;
+        return x - V * (lane - edge_lanes<V>()) < N;   // the piece has a column
     }
     __device__ __forceinline__ bool inside(int y) const { return y >= 1 && y < N - 1; }
     __device__ __forceinline__ __amdgpu_buffer_rsrc_t row(const float* p, int y) const
@@ -139,16 +146,19 @@ struct March {
         const bool ok = inside(y);
         return kgp::make_rsrc(p + (long long)(ok ? y : 0) * P, ok ? (unsigned)P * 4u : 0u);
     }
-    __device__ __forceinline__ void load(const float* p, int y, float (&v)[4]) const
+    __device__ __forceinline__ void load(const float* p, int y, float (&v)[V]) const
     {
-        kgp::bload<kgp::F32, 4>(row(p, y), voff, v);
+        kgp::bload<kgp::F32, V>(row(p, y), voff, v);
     }
     // whole rows: interior values, 0 on the boundary and the padding
-    __device__ __forceinline__ void store(float* p, int y, const Row& r) const
+    __device__ __forceinline__ void store(float* p, int y, const Row<V>& r) const
     {
         if (mine && y >= max(yb, 1) && y < ye) {
-            const f4 o = {r.v[0], r.v[1], r.v[2], r.v[3]};
-            __builtin_nontemporal_store(o, (__attribute__((address_space(1))) f4*)(p + (long long)y * P + x));
+            typedef float fv __attribute__((ext_vector_type(V)));
+            fv o;
+#pragma unroll
+            for (int v = 0; v < V; v++) o[v] = r.v[v];
+            __builtin_nontemporal_store(o, (__attribute__((address_space(1))) fv*)(p + (long long)y * P + x));
         }
     }
 };
@@ -157,22 +167,22 @@ struct March {
 // right-hand side f, and the coarse right-hand side
 //   fc(I,J) = (4 r_C + 2 (r_W + r_E + r_S + r_N) + (r_SW + r_SE + r_NW + r_NE)) / 16
 // of the residual r of u' at the 3 x 3 fine points around (2I, 2J).  H: even.
-template <bool ZERO>
+template <bool ZERO, int V>
 __global__ __launch_bounds__(64 * MW)
 void pj_down_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* __restrict__ u,
                const float* __restrict__ f, float* __restrict__ uo, float* __restrict__ fc)
 {
     constexpr int D = 3;               // rows in flight
     constexpr int LAG = ZERO ? 0 : 1;  // f enters one row after u
-    March m;
+    March<V> m;
     if (!m.setup(N, P, ntx, H)) return;
-    float pu[D][4], pf[D][4], fr[3][4];
-    Row ur[3], s1[3], s2[3], rr[3];
+    float pu[D][V], pf[D][V], fr[3][V];
+    Row<V> ur[3], s1[3], s2[3], rr[3];
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-        ur[q] = s1[q] = s2[q] = rr[q] = Row{{0.f, 0.f, 0.f, 0.f}, 0.f, 0.f};
+        ur[q] = s1[q] = s2[q] = rr[q] = Row<V>{};
 #pragma unroll
-        for (int v = 0; v < 4; v++) fr[q][v] = 0.f;
+        for (int v = 0; v < V; v++) fr[q][v] = 0.f;
     }
     const int first = m.yb - 3 - LAG, last = m.ye + 1 + LAG;   // incoming rows
 #pragma unroll
@@ -186,17 +196,17 @@ void pj_down_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float
     auto step = [&](auto phase, int y) {
         constexpr int p = decltype(phase)::value, p1 = (p + 2) % 3, p2 = (p + 1) % 3;
 #pragma unroll
-        for (int v = 0; v < 4; v++) fr[p][v] = pf[p][v];      // f row y - LAG
+        for (int v = 0; v < V; v++) fr[p][v] = pf[p][v];      // f row y - LAG
         if constexpr (ZERO) {
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
+            for (int v = 0; v < V; v++) {
                 const float val = 0.f + k.cf * fr[p][v];
                 s1[p].v[v] = m.inside(y) && m.in[v] ? val : 0.f;
             }
             s1[p].sides();
         } else {
 #pragma unroll
-            for (int v = 0; v < 4; v++) ur[p].v[v] = pu[p][v];
+            for (int v = 0; v < V; v++) ur[p].v[v] = pu[p][v];
             ur[p].sides();
             m.load(u, y + D, pu[p]);
             pj_sweep(k, ur[p2], ur[p1], ur[p], fr[p], m.inside(y - 1), m.in, s1[p]);
@@ -207,16 +217,18 @@ void pj_down_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float
         pj_resid(k, s2[p2], s2[p1], s2[p], fr[p2], rr[p]);
         const int yr = y - 2 - LAG, J = (yr - 1) >> 1;        // residual row; its coarse row below
         if ((yr & 1) && 2 * J >= m.yb && 2 * J < m.ye && J >= 1 && J < Nc - 1) {
-            const Row &a = rr[p2], &b = rr[p1], &c = rr[p];
-            f2 o;
+            const Row<V> &a = rr[p2], &b = rr[p1], &c = rr[p];
+            typedef float fc_t __attribute__((ext_vector_type(V / 2)));
+            float o[V / 2];
 #pragma unroll
-            for (int q = 0; q < 2; q++) {
+            for (int q = 0; q < V / 2; q++) {
                 const int v = 2 * q, I = (m.x >> 1) + q;
                 const float val = (4.f * b.v[v] + 2.f * (b.at(v - 1) + b.at(v + 1) + a.v[v] + c.v[v]) +
                                    (a.at(v - 1) + a.at(v + 1) + c.at(v - 1) + c.at(v + 1))) * 0.0625f;
                 o[q] = I >= 1 && I < Nc - 1 ? val : 0.f;
             }
-            if (m.mine) *(__attribute__((address_space(1))) f2*)(fc + (long long)J * Pc + (m.x >> 1)) = o;
+            if (m.mine)
+                *(__attribute__((address_space(1))) fc_t*)(fc + (long long)J * Pc + (m.x >> 1)) = __builtin_bit_cast(fc_t, o);
         }
     };
     for (int y = first; y <= last; y += 3)
@@ -228,28 +240,28 @@ void pj_down_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float
 // Up: u' = two sweeps of u plus the bilinear interpolation of the coarse e (e at
 // even/even points, the mean of the 2 or 4 coarse neighbours elsewhere).  ADD: u'
 // is not stored but added to the interior of the dense FP64 N x N field u64.
-template <bool ADD>
+template <bool ADD, int V>
 __global__ __launch_bounds__(64 * MW)
 void pj_up_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* __restrict__ u,
              const float* __restrict__ ec, const float* __restrict__ f, float* __restrict__ uo,
              double* __restrict__ u64)
 {
     constexpr int D = 3;
-    March m;
+    March<V> m;
     if (!m.setup(N, P, ntx, H)) return;
     const unsigned coff = m.x >= 0 && m.x < P ? (unsigned)m.x * 2u : kgp::KG_OOB;   // column x/2
-    auto crow = [&](int J, float (&v)[2]) {
+    auto crow = [&](int J, float (&v)[V / 2]) {
         const bool ok = J >= 1 && J < Nc - 1;
-        kgp::bload<kgp::F32, 2>(kgp::make_rsrc(ec + (long long)(ok ? J : 0) * Pc, ok ? (unsigned)Pc * 4u : 0u),
+        kgp::bload<kgp::F32, V / 2>(kgp::make_rsrc(ec + (long long)(ok ? J : 0) * Pc, ok ? (unsigned)Pc * 4u : 0u),
                                 coff, v);
     };
-    float pu[D][4], pf[D][4], pa[D][2], pb[D][2], fr[3][4];
-    Row vr[3], s1[3];
+    float pu[D][V], pf[D][V], pa[D][V / 2], pb[D][V / 2], fr[3][V];
+    Row<V> vr[3], s1[3];
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-        vr[q] = s1[q] = Row{{0.f, 0.f, 0.f, 0.f}, 0.f, 0.f};
+        vr[q] = s1[q] = Row<V>{};
 #pragma unroll
-        for (int v = 0; v < 4; v++) fr[q][v] = 0.f;
+        for (int v = 0; v < V; v++) fr[q][v] = 0.f;
     }
     const int first = m.yb - 2, last = m.ye + 1;
     auto fetch = [&](int y, int d) {
@@ -260,23 +272,29 @@ void pj_up_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* 
     };
 #pragma unroll
     for (int d = 0; d < D; d++) fetch(first + d, d);
-    // N is 4 q + 1: columns x .. x+3 of a lane left of column N-1 are in the row
+    // N is 4 q + 1: a lane's columns, left of column N-1, are in the row
     const bool adds = m.mine && m.x < N - 1;
-    d2 w[2];
+    d2 w[V / 2];
     auto fetch64 = [&](int y) {
         if (adds && y >= max(m.yb, 1) && y < m.ye) {
-            w[0] = *(const d2u*)(u64 + (long long)y * N + m.x);
-            w[1] = *(const d2u*)(u64 + (long long)y * N + m.x + 2);
+#pragma unroll
+            for (int q = 0; q < V / 2; q++) w[q] = *(const d2u*)(u64 + (long long)y * N + m.x + 2 * q);
         }
     };
     auto step = [&](auto phase, int y) {
         constexpr int p = decltype(phase)::value, p1 = (p + 2) % 3, p2 = (p + 1) % 3;
-        // coarse columns x/2, x/2+1, x/2+2 of rows y/2 and (odd y) y/2+1
-        const float a[3] = {pa[p][0], pa[p][1], kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.f, pa[p][0])};
-        const float b[3] = {pb[p][0], pb[p][1], kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.f, pb[p][0])};
+        // coarse columns x/2, x/2+1 (, x/2+2) of rows y/2 and (odd y) y/2+1
+        float a[V / 2 + 1], b[V / 2 + 1];
+#pragma unroll
+        for (int q = 0; q < V / 2; q++) {
+            a[q] = pa[p][q];
+            b[q] = pb[p][q];
+        }
+        a[V / 2] = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.f, a[0]);
+        b[V / 2] = kgp::dpp_shift<kgp::KG_DPP_WAVE_SHL1>(0.f, b[0]);
         const bool odd = y & 1;
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
+        for (int v = 0; v < V; v++) {
             const int q = v >> 1;
             const float e = !(v & 1) ? (odd ? 0.5f * (a[q] + b[q]) : a[q])
                                      : (odd ? 0.25f * (a[q] + a[q + 1] + b[q] + b[q + 1])
@@ -288,14 +306,15 @@ void pj_up_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* 
         if constexpr (ADD) fetch64(y - 2);
         fetch(y + D, p);
         pj_sweep(k, vr[p2], vr[p1], vr[p], fr[p], m.inside(y - 1), m.in, s1[p]);
-        Row o;
+        Row<V> o;
         pj_sweep(k, s1[p2], s1[p1], s1[p], fr[p1], m.inside(y - 2), m.in, o);
         if constexpr (!ADD) {
             m.store(uo, y - 2, o);
         } else if (adds && y - 2 >= max(m.yb, 1) && y - 2 < m.ye) {
             double* q = u64 + (long long)(y - 2) * N + m.x;
-            *(d2u*)q = w[0] + d2{(double)o.v[0], (double)o.v[1]};
-            *(d2u*)(q + 2) = w[1] + d2{(double)o.v[2], (double)o.v[3]};
+#pragma unroll
+            for (int h = 0; h < V / 2; h++)
+                *(d2u*)(q + 2 * h) = w[h] + d2{(double)o.v[2 * h], (double)o.v[2 * h + 1]};
         }
     };
     for (int y = first; y <= last; y += 3)
@@ -311,7 +330,7 @@ void pj_up_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* 
 // own the points.  A thread owns R = TOP^2/1024 rows of one column (one point on
 // the levels below 64 cells), so a wave reads consecutive LDS words.  As
 // launches these levels took 30 of the 40 of a 512 cell V-cycle, which bound its
-// solve (1.98 ms; 0.79 now).  The cycle from 128 cells takes 22 us, bound by one CU's
+// solve (1.98 ms; 0.77 now).  The cycle from 128 cells takes 22 us, bound by one CU's
 // FP32 rate and LDS on the first level and by barriers below.
 constexpr int CTOP = 128;
 constexpr int CT = 1024;               // threads
@@ -642,15 +661,18 @@ void vcycle(const kg_ctx* ctx, hipStream_t st, Level* lv, int l, bool zero, doub
     }
     Level& C = lv[l + 1];
     const Coef k{C0, C1, C2, sweep_cf(L.h), residual_scale(L.h)};
-    const int ntx = (L.N + MW * PIECE - 1) / (MW * PIECE);
-    const int H = march_rows(ctx, ntx, L.N);
+    const int ntx4 = (L.N + MW * piece<4>() - 1) / (MW * piece<4>());
+    const int H = march_rows(ctx, ntx4, L.N);
+    const bool narrow = H == 2;
+    const int ntx = narrow ? (L.N + MW * piece<2>() - 1) / (MW * piece<2>()) : ntx4;
     const unsigned blocks = (unsigned)ntx * (unsigned)((L.N - 1 + H - 1) / H);
-    auto down = zero ? pj_down_k<true> : pj_down_k<false>;
+    auto down = narrow ? (zero ? pj_down_k<true, 2> : pj_down_k<false, 2>)
+                       : (zero ? pj_down_k<true, 4> : pj_down_k<false, 4>);
     hipLaunchKernelGGL(down, dim3(blocks), dim3(64 * MW), 0, st, L.N, L.P, C.N, C.P, ntx, H, k,
                        (const float*)L.u, (const float*)L.f, L.t, C.f);
     std::swap(L.u, L.t);
     vcycle(ctx, st, lv, l + 1, true, nullptr);
-    auto up = u64 ? pj_up_k<true> : pj_up_k<false>;
+    auto up = narrow ? (u64 ? pj_up_k<true, 2> : pj_up_k<false, 2>) : (u64 ? pj_up_k<true, 4> : pj_up_k<false, 4>);
     hipLaunchKernelGGL(up, dim3(blocks), dim3(64 * MW), 0, st, L.N, L.P, C.N, C.P, ntx, H, k,
                        (const float*)L.u, (const float*)C.u, (const float*)L.f, L.t, u64);
     std::swap(L.u, L.t);
@@ -856,7 +878,7 @@ extern "C" int kg_poisson_solve(kg_ctx* ctx, int n, const double* f, double* u, 
         return done(kg_set_error(KG_ERR_HIP, "kg_poisson_solve: hipEventCreate failed"));
     }
     workspace_carve(ws, base);
-    kg_register_kernel("poisson_smooth", (const void*)pj_up_k<false>);
+    kg_register_kernel("poisson_smooth", (const void*)pj_up_k<false, 4>);
     int outer = 0, cycles = 0;
     double rel = 0;
     if (int rc = solve(ctx, n, f, u, tol, max_outer, vcycles, ws, rep, &outer, &cycles, &rel,
@@ -887,7 +909,7 @@ extern "C" int kg_poisson_solve_noalloc(kg_ctx* ctx, int n, const double* f, dou
                             "workspace, more than the %zu reserved", n, workspace_bytes(n, STATS_BYTES),
                             NOALLOC_BYTES);
     workspace_carve(ws, g_scratch_ptr[ctx->device]);
-    kg_register_kernel("poisson_smooth", (const void*)pj_up_k<false>);
+    kg_register_kernel("poisson_smooth", (const void*)pj_up_k<false, 4>);
     int outer = 0, cycles = 0;
     double rel = 0;
     std::chrono::steady_clock::time_point t0;
@@ -899,4 +921,4 @@ extern "C" int kg_poisson_solve_noalloc(kg_ctx* ctx, int n, const double* f, dou
     return finish("kg_poisson_solve_noalloc", rep, ws, outer, cycles, rel, sec, tol);
 }
 
-int kg_preload_poisson() { return kg_preload_kernel((const void*)pj_up_k<false>); }
+int kg_preload_poisson() { return kg_preload_kernel((const void*)pj_up_k<false, 4>); }
