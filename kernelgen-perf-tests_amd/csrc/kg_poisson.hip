@@ -29,12 +29,17 @@
 
 namespace {
 
-// Tile order of the V-cycle's passes and the FP64 residual (kg_tile_order):
-// chunks of 2 tile rows per XCD, 8192^2 solve 17.7 ms against 17.9-18.1 in
-// hardware order with the passes of that time (chunks of 4 or 8 rows 17.6-17.9),
-// bit-identical (the residual's partial sums stay indexed by tile).
+// Tile orders (kg_tile_order).  The marching passes deal single tile rows to the XCDs:
+// tile rows that share rows then run at the same time, which matters more than that
+// they share an L2, which their rows overflow (pj_up_k reads 1.4 times its input past
+// L2).  8192^2: pj_up_k 186 us, pj_down_k 182 and, from 0, 117; in chunks of 2 tile
+// rows 204, 187 and 131, in hardware order 204, 189 and 133.  The FP64 residual takes
+// chunks of 2 (259 us; single rows 272, chunks of 4 or 8 257-263).
 #ifndef KG_ORD_PJ
-#define KG_ORD_PJ 2
+#define KG_ORD_PJ 1
+#endif
+#ifndef KG_ORD_PJR
+#define KG_ORD_PJR 2
 #endif
 
 typedef float f2 __attribute__((ext_vector_type(2)));
@@ -56,10 +61,10 @@ typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));   // at any 
 // result, bit for bit.
 //
 // Bound by HBM on the finest levels: u, f, u' and a quarter of it on the next
-// level are 871 MB at 8192^2, 203 us (4.3 TB/s; the best copy reaches 6.3) for
-// pj_up_k and 188 for pj_down_k.  Sweep pairs, residual and restriction,
+// level are 871 MB at 8192^2, 186 us (4.7 TB/s; the best copy reaches 6.3) for
+// pj_up_k and 182 for pj_down_k.  Sweep pairs, residual and restriction,
 // prolongation and the addition to u as passes of their own took 14.2 of the 17.7 ms
-// of an 8192^2 solve (7.5, 3.3, 1.9, 1.5); it takes 10.0 so.  Rows of 64-byte
+// of an 8192^2 solve (7.5, 3.3, 1.9, 1.5); it takes 9.7 so.  Rows of 64-byte
 // multiples and pieces of 240 columns, so that no wave writes part of a sector:
 // 5 % faster at 8192^2 than 248 columns of 4-float pitches.  The 4 waves of a
 // workgroup lie side by side; one above the other costs 2 % more.  Small levels
@@ -509,7 +514,7 @@ void pj_residual64_k(int N, int P, int ntx, int H, double inv6h2, const double* 
     __shared__ double wsum[MW];
     const int lane = (int)(threadIdx.x & 63);
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const unsigned tb = kg_tile_order<KG_ORD_PJ>(blockIdx.x, gridDim.x, (unsigned)ntx);
+    const unsigned tb = kg_tile_order<KG_ORD_PJR>(blockIdx.x, gridDim.x, (unsigned)ntx);
     const int x = ((int)(tb % (unsigned)ntx) * MW + w) * RPIECE - 2 + 2 * lane;
     const int yb = max((int)(tb / (unsigned)ntx) * H, 1);
     const int ye = min((int)(tb / (unsigned)ntx + 1) * H, N - 1);
