@@ -320,8 +320,10 @@ int kg_launch_begin(kg_ctx* ctx, const char* name)
 
 int kg_launch_end(kg_ctx* ctx)
 {
+    // taken back first: what stayed would be the next launch's error
+    const hipError_t last = hipGetLastError();
     KG_HIP(ctx->launch_err);
-    KG_HIP(hipGetLastError());
+    KG_HIP(last);
     if (!ctx->timing) {
         ctx->last_is_stop = false;
         return KG_OK;
