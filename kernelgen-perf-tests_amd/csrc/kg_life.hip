@@ -128,7 +128,7 @@ __device__ __forceinline__ uint8_t life_cell(const uint8_t* c0, long long o, int
     return (uint8_t)((n == 3) || (alive && n == 2));
 }
 
-// Rows shorter than 20 cells, or longer than the vector kernel's offsets: a
+// Rows the vector kernel does not take, or not as fast (kg_life_u8): a
 // workgroup of 256 threads takes LIFE_SLOW_YC rows of 256 cells, cell by cell.
 __global__ __launch_bounds__(256)
 void life_u8_cells_k(int nx, int ny, int ntx, const uint8_t* __restrict__ c0,
@@ -259,21 +259,29 @@ extern "C" int kg_life_u8(kg_ctx* ctx, int nx, int ny, const uint8_t* c0, uint8_
     if (c0 == c1) return kg_set_error(KG_ERR_INVALID, "kg_life_u8: c0 and c1 must be distinct");
     if (((uintptr_t)c0 | (uintptr_t)c1) & (LIFE_CW - 1))
         return kg_set_error(KG_ERR_INVALID, "kg_life_u8: buffers must be 16-byte aligned");
+    // Ragged rows of a single cell-wise workgroup (258 cells) leave three of the vector
+    // kernel's four waves idle: cell by cell is faster once that kernel's bands no
+    // longer run all at once.  257 cells: 2000 rows 8.0 us cell by cell, 5.0 in lanes; 6000
+    // rows 8.8 and 7.7, 8000 rows 8.6 and 9.0, 200000 rows 89 and 132; 20 cells by 200000 rows
+    // 26 and 130; 259 cells by 200000 rows 166 and 132.
     const bool rag = nx % LIFE_CW != 0;
-    const bool vec = (!rag || nx >= LIFE_CW + 4) && nx <= (1 << 24);
+    const long long nsx = ((long long)nx + LIFE_TX - 1) / LIFE_TX, nb = ((long long)ny - 2 + LIFE_YC - 1) / LIFE_YC;
+    const bool narrow = rag && nx <= 258 && nb > 6LL * ctx->cus;
+    // a launch holds less than 2^32 work-items; the cell-wise kernel takes 2 to 4
+    // times as many rows of up to 770 cells
+    const bool many = rag && nsx * nb * 64 * LIFE_WAVES >= 1LL << 32;
+    const bool vec = (!rag || (nx >= LIFE_CW + 4 && !narrow && !many)) && nx <= (1 << 24);
     auto kern = rag ? life_u8_k<true> : life_u8_k<false>;
     kg_register_kernel("life_u8", vec ? (const void*)kern : (const void*)life_u8_cells_k);
     if (int rc = kg_launch_begin(ctx, "life_u8")) return rc;
     if (nx > 2 && ny > 2) {
         if (vec) {
-            const unsigned nsx = (unsigned)((nx + LIFE_TX - 1) / LIFE_TX);
-            const unsigned nb = (unsigned)((ny - 2 + LIFE_YC - 1) / LIFE_YC);
-            kg_launch(ctx, kern, dim3(nsx * nb), dim3(64 * LIFE_WAVES), 0, nx, ny, (int)nsx,
+            kg_launch(ctx, kern, dim3((unsigned)(nsx * nb)), dim3(64 * LIFE_WAVES), 0, nx, ny, (int)nsx,
                       c0, c1);
         } else {
-            const unsigned ntx = (unsigned)((nx - 2 + 255) / 256);
-            const unsigned nb = (unsigned)((ny - 2 + LIFE_SLOW_YC - 1) / LIFE_SLOW_YC);
-            kg_launch(ctx, life_u8_cells_k, dim3(ntx * nb), dim3(256), 0, nx, ny, (int)ntx, c0, c1);
+            const unsigned ntx = (unsigned)(((long long)nx - 2 + 255) / 256);
+            const unsigned nc = (unsigned)(((long long)ny - 2 + LIFE_SLOW_YC - 1) / LIFE_SLOW_YC);
+            kg_launch(ctx, life_u8_cells_k, dim3(ntx * nc), dim3(256), 0, nx, ny, (int)ntx, c0, c1);
         }
     }
     return kg_launch_end(ctx);

@@ -105,3 +105,36 @@ def test_life_u8_row_ends(gpu_ctx, oracle, nx):
         for steps in (1, 3):
             np.testing.assert_array_equal(_gpu_steps(gpu_ctx, cells, steps),
                                           _oracle_steps(oracle, cells, steps), err_msg=f"{nx} x {ny}")
+
+
+@pytest.mark.parametrize("nx,ny", [(20, 6147), (20, 6151), (100, 9001), (257, 7003), (258, 6300), (259, 7003), (20, 1538)])
+def test_life_u8_narrow_rows(gpu_ctx, oracle, nx, ny):
+    """Ragged rows on either side of the kernels' dividing line: 258 cells and
+    6 bands of 4 rows per compute unit (6144 rows on 256 of them)."""
+    cells = np.random.default_rng(nx + ny).integers(0, 2, (ny, nx)).astype(np.uint8)
+    for steps in (1, 2):
+        np.testing.assert_array_equal(_gpu_steps(gpu_ctx, cells, steps), _oracle_steps(oracle, cells, steps))
+
+
+@pytest.mark.parametrize("nx", [20, 259])
+def test_life_u8_rows_past_a_vector_launch(gpu_ctx, oracle, nx):
+    """More rows than the vector kernel's work-items in one launch can hold."""
+    period, ny = 1024, 2 ** 26 + 1029
+    cells = np.random.default_rng(nx).integers(0, 2, (period, nx)).astype(np.uint8)
+    a, b = gpu_ctx.empty((ny, nx), np.uint8), gpu_ctx.empty((ny, nx), np.uint8)
+    copy = lambda dst, src, n: gpu_ctx.lib.kg_d2d(gpu_ctx.ptr, dst, src, n)  # noqa: E731
+    first = gpu_ctx.array(cells)
+    assert copy(a.ptr, first.ptr, period * nx) == 0
+    rows = period
+    while rows < ny:                       # the board repeats every `period` rows
+        n = min(rows, ny - rows)
+        assert copy(a.ptr + rows * nx, a.ptr, n * nx) == 0
+        rows += n
+    gpu_ctx.call("life_u8", nx, ny, a, b)
+    for y in (1, 2 ** 25 + 7, 2 ** 26 - 40, ny - 81):
+        got = np.empty((80, nx), np.uint8)
+        assert gpu_ctx.lib.kg_d2h(gpu_ctx.ptr, got.ctypes.data, b.ptr + y * nx, got.nbytes) == 0
+        src = cells[np.arange(y - 1, y + 81) % period]
+        np.testing.assert_array_equal(got[:, 1:-1], _oracle_steps(oracle, src, 1)[1:-1, 1:-1], err_msg=f"row {y}")
+    for t in (a, b, first):
+        t.free()
