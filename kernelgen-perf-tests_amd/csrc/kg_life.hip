@@ -45,6 +45,7 @@ constexpr int LIFE_TX = LIFE_WAVES * LIFE_SEG;
 constexpr int LIFE_NP = LIFE_D + 1;           // ring slots
 constexpr int LIFE_YC = LIFE_NP * LIFE_U;     // output rows per band
 constexpr int LIFE_SLOW_YC = 16;              // rows per workgroup, cell-wise kernel
+constexpr long long LIFE_LLC = 256LL << 20;   // bytes of the device's last-level cache
 
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 // at any byte
@@ -153,10 +154,10 @@ void life_u8_cells_k(int nx, int ny, int ntx, const uint8_t* __restrict__ c0,
 // 8 segments per workgroup run alike at 8192^2 and 20 % slower at 4096^2.
 // A step of 8192^2 takes 22.5 us (6.0 TB/s, bound by memory): 31 us with the row's
 // end lanes storing 15 single cells and with stores that bypass the caches, which
-// the next step's loads then miss (25.9 with those alone; at 16384^2, where no level
-// stays cached, 102 against 97).  8000 x 8191 22.0 us (31.5 cell by cell), 5000 x
-// 4001 9.8 (42), 777 x 7000 8.2 (18.5).
-template <bool RAG>
+// the next step's loads then miss (26.6 with those alone).  8000 x 8191 22.0 us (31.5 cell
+// by cell), 5000 x 4001 9.8 (42), 777 x 7000 8.2 (18.5).
+// FAR: two levels that no cache holds; stores then bypass the caches (kg_life_u8).
+template <bool RAG, bool FAR>
 __global__ __launch_bounds__(64 * LIFE_WAVES)
 void life_u8_k(int nx, int ny, int nsx, const uint8_t* __restrict__ c0, uint8_t* __restrict__ c1)
 {
@@ -223,7 +224,8 @@ void life_u8_k(int nx, int ny, int nsx, const uint8_t* __restrict__ c0, uint8_t*
             res[q] = life_rule(up.h[q] + (mid.h[q] - mid.m[q]) + dn.h[q], mid.m[q]);
         const unsigned ro = (unsigned)t * (unsigned)nx;
         const u4 out = {res[0], res[1], res[2], res[3]};
-        __builtin_amdgcn_raw_buffer_store_b128(out, rout, vst == kgp::KG_OOB ? vst : ro + vst, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(out, rout, vst == kgp::KG_OOB ? vst : ro + vst, 0,
+                                               FAR ? 2 : 0);
         if (edge && j0 + t < j1) {
             uint8_t* p = c1 + (long long)(j0 + t) * nx + x;
             if (x == 0) {
@@ -271,7 +273,13 @@ extern "C" int kg_life_u8(kg_ctx* ctx, int nx, int ny, const uint8_t* c0, uint8_
     // times as many rows of up to 770 cells
     const bool many = rag && nsx * nb * 64 * LIFE_WAVES >= 1LL << 32;
     const bool vec = (!rag || (nx >= LIFE_CW + 4 && !narrow && !many)) && nx <= (1 << 24);
-    auto kern = rag ? life_u8_k<true> : life_u8_k<false>;
+    // Two levels beyond the last-level cache: cached stores only push out what the
+    // step still reads.  8192^2 23.0 us cached, 26.6 past the caches; 11520^2 (253 MiB) 44.2
+    // and 48.7; 12288^2 (288 MiB) 57.5 and 55.7; 16384^2 102.5 and 96.4; 24576^2 220 and 209;
+    // ragged 16385^2 123.9 and 120.8.
+    const bool far = 2LL * nx * ny > LIFE_LLC;
+    auto kern = rag ? (far ? life_u8_k<true, true> : life_u8_k<true, false>)
+                    : (far ? life_u8_k<false, true> : life_u8_k<false, false>);
     kg_register_kernel("life_u8", vec ? (const void*)kern : (const void*)life_u8_cells_k);
     if (int rc = kg_launch_begin(ctx, "life_u8")) return rc;
     if (nx > 2 && ny > 2) {
@@ -289,6 +297,6 @@ extern "C" int kg_life_u8(kg_ctx* ctx, int nx, int ny, const uint8_t* c0, uint8_
 
 int kg_preload_life()
 {
-    if (int rc = kg_preload_kernel((const void*)life_u8_k<false>)) return rc;
+    if (int rc = kg_preload_kernel((const void*)life_u8_k<false, false>)) return rc;
     return kg_preload_kernel((const void*)life_u8_cells_k);
 }

@@ -138,3 +138,10 @@ def test_life_u8_rows_past_a_vector_launch(gpu_ctx, oracle, nx):
         np.testing.assert_array_equal(got[:, 1:-1], _oracle_steps(oracle, src, 1)[1:-1, 1:-1], err_msg=f"row {y}")
     for t in (a, b, first):
         t.free()
+
+
+@pytest.mark.parametrize("nx,ny", [(16384, 8200), (11585, 11586)])
+def test_life_u8_levels_past_the_caches(gpu_ctx, oracle, nx, ny):
+    """Two levels of more than 256 MiB, whole and ragged rows."""
+    cells = np.random.default_rng(nx).integers(0, 2, (ny, nx)).astype(np.uint8)
+    np.testing.assert_array_equal(_gpu_steps(gpu_ctx, cells, 1), _oracle_steps(oracle, cells, 1))
