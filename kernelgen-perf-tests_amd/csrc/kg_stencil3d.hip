@@ -335,8 +335,8 @@ struct LapgsrbOp {
 #ifndef KG_WAVE_XS
 #define KG_WAVE_XS 0
 #endif
-template <bool RAG> using LapCfg = kgp::Cfg<2, KG_LAP_W, 1, 0, 0, 1, 1, KG_LAP_D, 0, KG_LAP_KC,
-                                            kgp::F64, 64, false, KG_LAP_XS, RAG>;
+template <int V, bool RAG> using LapCfg = kgp::Cfg<V, KG_LAP_W, 1, 0, 0, 1, 1, KG_LAP_D, 0, KG_LAP_KC,
+                                                   kgp::F64, 64, false, V == 2 && KG_LAP_XS, RAG>;
 // gradient: W=12/D=2/KC=8 in chunks of 2 tile rows, one workgroup (12 waves)
 // per CU: 196 us (W=8 with 2 workgroups 201, 3 workgroups 208; W=12 with 2
 // 213; W=16 with 1 214; KC=16 224, D=3 209, XCD-contiguous 219).
@@ -346,10 +346,10 @@ template <bool RAG> using LapCfg = kgp::Cfg<2, KG_LAP_W, 1, 0, 0, 1, 1, KG_LAP_D
 #ifndef KG_GRAD_OCC
 #define KG_GRAD_OCC 1
 #endif
-template <bool RAG> using GradCfg = kgp::Cfg<2, KG_GRAD_W, 1, 0, 0, 1, 1, 2, 0, 8, kgp::F64, 64,
-                                             false, KG_GRAD_XS, RAG>;
-template <bool RAG> using WaveCfg = kgp::Cfg<2, 12, 2, 0, 0, 2, 2, 3, 1, 32, kgp::F64, 64, false,
-                                             KG_WAVE_XS, RAG>;
+template <int V, bool RAG> using GradCfg = kgp::Cfg<V, KG_GRAD_W, 1, 0, 0, 1, 1, 2, 0, 8, kgp::F64, 64,
+                                                    false, V == 2 && KG_GRAD_XS, RAG>;
+template <int V, bool RAG> using WaveCfg = kgp::Cfg<V, 12, 2, 0, 0, 2, 2, 3, 1, 32, kgp::F64, 64, false,
+                                                    V == 2 && KG_WAVE_XS, RAG>;
 // lapgsrb: 16-byte lanes (even nx, 16-byte aligned fields) take every
 // same-row x-neighbour, in planes k-1 .. k+1, from the neighbouring lanes'
 // registers by DPP shifts (x-shift mode), which leaves LDS only the 12
@@ -388,28 +388,51 @@ template <bool RAG> using WaveCfg = kgp::Cfg<2, 12, 2, 0, 0, 2, 2, 3, 1, 32, kgp
 #ifndef KG_GSRB_WGPC
 #define KG_GSRB_WGPC 1
 #endif
-template <bool RAG> using GsrbCfg = kgp::Cfg<2, KG_GSRB_W, 2, 1, 1, 2, 2, KG_GSRB_D, 0, KG_GSRB_KC,
-                                             kgp::F64, 64, false, true, RAG>;
+template <int V, bool RAG> using GsrbCfg = kgp::Cfg<V, (V == 2 ? KG_GSRB_W : 12), 2, 1, 1, 2, 2,
+                                                    KG_GSRB_D, 0, KG_GSRB_KC, kgp::F64, 64, false,
+                                                    V == 2, RAG>;
 #ifndef KG_WAVE_WGPC
 #define KG_WAVE_WGPC 0
 #endif
 
-// Launch Op on the plane engine, in the ragged form for an odd nx or fields that
-// are not 16-byte aligned (al).
+// Where one point per lane takes the place of the ragged form's two, for an odd nx and
+// fields that are not 16-byte aligned.  Two make a tile 128 points wide instead of 64: a
+// row of up to 64 points leaves more than half of its lanes idle and pays for the wider
+// loads and the shifts all the same, and one of 129 to 192 fills 2 tiles no better than 3.
+// Time of one point per lane over that of two, for 33, 63 and 65 points a row and 32 M
+// points: laplacian 0.82, 0.86, 1.40; wave13pt 0.78, 0.90, 1.45; lapgsrb 0.78, 1.01, 1.96
+// (8 M: 0.77, 0.85, 1.81); gradient 0.76, 0.87, 1.30.  Below some thousand rows both
+// last a launch's 6 us: wave13pt 0.91 at 6300 rows of 63 points, 1.04 at 6200 of 13;
+// gradient 0.90 at 12100 of 33, 1.06 at 7300 of 55.
+// laplacian with 129 to 191 points a row 0.94-0.98 (32 M points), 0.93-1.02 (8 M), 1.0-1.09 (2
+// M), 193 1.15, 1.10, 1.11; wave13pt up to 160 points 1.0-1.06 (32 M), 0.93-1.07 (2 M),
+// 161 to 191 0.94-1.01 and 0.89-0.97.
+struct OneTake {
+    int nx;
+    long long rows, n;   // of the grid, and its points
+    OneTake(int nx_, int ny, int ns) : nx(nx_), rows((long long)ny * ns), n(nx_ * rows) {}
+    bool laplacian() const { return nx <= 64 || (nx > 128 && nx <= 192 && n >= 4000000); }
+    bool wave13pt() const { return (nx <= 64 && rows >= 6200) || (nx > 160 && nx <= 192); }
+    bool lapgsrb() const { return nx <= 64; }
+    bool gradient() const { return nx <= 64 && rows >= 9000; }
+};
+
+// Launch Op on the plane engine, for an odd nx or fields that are not 16-byte aligned
+// (al) in the ragged form or, with `one`, with one point per lane.
 // ORD: tile order (kg_tile_order).  WGPC > 0: z-chunks longer than C::KC
 // planes when the launch would otherwise exceed about WGPC workgroups per
 // compute unit (each workgroup then marches further and fills its pipeline
 // fewer times); WGPC = 0 keeps C::KC.  OCC > 0: at most OCC resident
 // workgroups per compute unit, enforced by reserving unused dynamic LDS.
-template <template <bool> class CfgT, template <class> class OpT, int LO, int HI, int ORD = 1,
+template <template <int, bool> class CfgT, template <class> class OpT, int LO, int HI, int ORD = 1,
           int WGPC = 0, int OCC = 0, class Fill>
-static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, Fill fill)
+static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, bool one, Fill fill)
 {
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
     if (int rc = kg_check_plane_bytes((long long)nx * ny, 8)) return rc;
-    auto go = [&](auto ragged) -> int {
-        using C = CfgT<decltype(ragged)::value>;
+    auto go = [&](auto vtag, auto ragged) -> int {
+        using C = CfgT<decltype(vtag)::value, decltype(ragged)::value>;
         using Op = OpT<C>;
         Op op{};
         fill(op);
@@ -436,7 +459,10 @@ static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
                       op);
         return kg_launch_end(ctx);
     };
-    return nx % 2 == 0 && al ? go(std::false_type{}) : go(std::true_type{});
+    std::integral_constant<int, 2> two;
+    if (nx % 2 == 0 && al) return go(two, std::false_type{});
+    if (one) return go(std::integral_constant<int, 1>{}, std::false_type{});
+    return go(two, std::true_type{});
 }
 
 }  // namespace
@@ -449,7 +475,8 @@ extern "C" int kg_laplacian(kg_ctx* ctx, int nx, int ny, int ns, double alpha, d
     KG_REQUIRE(w0 && w1, "kg_laplacian: null buffer");
     KG_REQUIRE(w0 != w1, "kg_laplacian: w0 and w1 must be distinct (out-of-place update)");
     return launch_plane<LapCfg, LaplacianOp, 1, 1, KG_ORD_LAP>(ctx, "laplacian", nx, ny, ns,
-                                                   kg_aligned16(w0, w1), [&](auto& op) {
+                                                   kg_aligned16(w0, w1), OneTake(nx, ny, ns).laplacian(),
+                                                   [&](auto& op) {
         op.src = w0;
         op.dst = w1;
         op.alpha = alpha;
@@ -483,7 +510,8 @@ extern "C" int kg_gradient(kg_ctx* ctx, int nx, int ny, int ns, double alpha, do
     KG_REQUIRE(u != ux && u != uy && u != uz && ux != uy && ux != uz && uy != uz,
                "kg_gradient: buffers must be distinct");
     return launch_plane<GradCfg, GradientOp, 1, 1, KG_ORD_GRAD, 0, KG_GRAD_OCC>(ctx, "gradient", nx, ny, ns,
-                                                         kg_aligned16(u, ux, uy, uz), [&](auto& op) {
+                                                         kg_aligned16(u, ux, uy, uz), OneTake(nx, ny, ns).gradient(),
+                                                         [&](auto& op) {
         op.src = u;
         op.ux = ux;
         op.uy = uy;
@@ -500,7 +528,8 @@ extern "C" int kg_wave13pt(kg_ctx* ctx, int nx, int ny, int ns, double m0, doubl
     KG_REQUIRE(w0 && w1 && w2, "kg_wave13pt: null buffer");
     KG_REQUIRE(w2 != w0 && w2 != w1, "kg_wave13pt: w2 aliases an input");
     return launch_plane<WaveCfg, Wave13ptOp, 2, 2, KG_ORD_WAVE, KG_WAVE_WGPC>(ctx, "wave13pt", nx, ny, ns,
-                                                   kg_aligned16(w0, w1, w2), [&](auto& op) {
+                                                   kg_aligned16(w0, w1, w2), OneTake(nx, ny, ns).wave13pt(),
+                                                   [&](auto& op) {
         op.src = w1;
         op.side[0] = w0;
         op.dst = w2;
@@ -538,7 +567,8 @@ extern "C" int kg_lapgsrb(kg_ctx* ctx, int nx, int ny, int ns, double c0, double
     KG_REQUIRE(w0 && w1, "kg_lapgsrb: null buffer");
     KG_REQUIRE(w0 != w1, "kg_lapgsrb: w0 and w1 must be distinct");
     return launch_plane<GsrbCfg, LapgsrbOp, 2, 2, KG_ORD_GSRB, KG_GSRB_WGPC>(ctx, "lapgsrb", nx, ny, ns,
-                                                         kg_aligned16(w0, w1), [&](auto& op) {
+                                                         kg_aligned16(w0, w1), OneTake(nx, ny, ns).lapgsrb(),
+                                                         [&](auto& op) {
         op.src = w0;
         op.dst = w1;
         op.c0 = c0;

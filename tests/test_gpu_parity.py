@@ -85,6 +85,26 @@ FULL3 = (512, 256, 256)
 FULL2 = (512, 65536)
 
 
+# either side of the lines between one and two points per lane: points a row, planes
+# and points of the grid
+ONE_POINT = [(21, 101, 97), (63, 60, 60), (64, 60, 60), (65, 30, 30), (129, 180, 181), (161, 11, 12),
+             (191, 30, 40), (192, 13, 9), (193, 13, 9), (301, 21, 3), (301, 21, 4), (301, 21, 5)]
+
+
+@pytest.mark.parametrize("name,dims", [(n, d) for n in ("laplacian", "divergence", "gradient", "wave13pt", "uxx1", "lapgsrb")
+                                       for d in ONE_POINT]
+                         + [("uxx1", (17, 600, 600)), ("uxx1", (55, 470, 470)), ("uxx1", (131, 9, 11)),
+                            ("divergence", (57, 20, 30)), ("gradient", (107, 90, 90))])
+def test_gpu_odd_rows_points_per_lane(gpu_ctx, oracle, name, dims):
+    spec = K.SPECS[name]
+    coefs, arrays = K.random_case(spec, dims, 40 + dims[0])
+    want = oracle.run(spec, dims, coefs, arrays, 1)
+    for offset in (0, 1):
+        got = K.GpuBackend(gpu_ctx).run(spec, dims, coefs, arrays, 1, offset=offset)
+        for role in want:
+            assert_bit_equal(got[role], want[role], f"{name} {dims} +{offset} {role}")
+
+
 @pytest.mark.parametrize("name", K.STENCILS)
 def test_gpu_matches_oracle_full_size_one_step(gpu_ctx, oracle, name):
     """The benchmark configuration (512x256x256 / 512x65536), one step, every
