@@ -407,6 +407,11 @@ template <int V, bool RAG> using GsrbCfg = kgp::Cfg<V, (V == 2 ? KG_GSRB_W : 12)
 // laplacian with 129 to 191 points a row 0.94-0.98 (32 M points), 0.93-1.02 (8 M), 1.0-1.09 (2
 // M), 193 1.15, 1.10, 1.11; wave13pt up to 160 points 1.0-1.06 (32 M), 0.93-1.07 (2 M),
 // 161 to 191 0.94-1.01 and 0.89-0.97.
+// gradient, whose three results of 8-byte alignment are stored in 16-byte pieces, gains
+// the least from two: 105 points a row 1.05 (32 M points), 1.02 (8 M), 0.93 (2 M), 113 to 191
+// 0.88-1.01, 0.90-0.98, 0.88-1.01; from 193 points on 0.98-1.21 (32 M), 0.95-1.09 (8 M),
+// 0.98-1.08 (4 M), but 0.86-0.98 (2 M and 1 M, where the fields stay cached; 1001 points a
+// row 1.1) and at 0.4 M points 1.0-1.15.
 struct OneTake {
     int nx;
     long long rows, n;   // of the grid, and its points
@@ -414,7 +419,11 @@ struct OneTake {
     bool laplacian() const { return nx <= 64 || (nx > 128 && nx <= 192 && n >= 4000000); }
     bool wave13pt() const { return (nx <= 64 && rows >= 6200) || (nx > 160 && nx <= 192); }
     bool lapgsrb() const { return nx <= 64; }
-    bool gradient() const { return nx <= 64 && rows >= 9000; }
+    bool gradient() const
+    {
+        return (nx <= 64 && rows >= 9000) || (nx >= 110 && nx <= 192 && n >= 600000) ||
+               (nx >= 100 && nx < 800 && n >= 600000 && n < 3000000);
+    }
 };
 
 // Launch Op on the plane engine, for an odd nx or fields that are not 16-byte aligned
