@@ -6,7 +6,8 @@
 // every global load prefetched a few planes ahead.  divergence and uxx1 read
 // each of their inputs at only a few offsets along one axis and run the direct
 // form: two points and a few planes per lane, every operand a 16-byte load
-// through the caches, all issued up front.
+// through the caches, all issued up front; narrow odd rows take a z-march with one
+// point per lane (OneTake).
 // Arithmetic is written in the reference's source order and the library is
 // built with -ffp-contract=off: results are bit-identical to an IEEE build of
 // the reference kernels.
@@ -46,12 +47,41 @@ namespace {
 using kgops::LaplacianOp;
 using kgops::Wave13ptOp;
 
+constexpr int TX = 64;   // column tiles of the z-march: one wave64 per x-row segment
+constexpr int TY = 4;    // 4 rows -> 256 threads per workgroup
+constexpr int KC = 16;   // z-planes per workgroup, at most
+
 #define KG_REQUIRE(cond, msg) \
     do { if (!(cond)) return kg_set_error(KG_ERR_INVALID, "%s", msg); } while (0)
 
 // --------------------------------------------------------------- divergence
 // divergence/divergence.c:93-96
 //
+// One point per lane: a 64 x 4 column tile marched along z (kg_zmarch.h).
+__global__ __launch_bounds__(TX * TY)
+void divergence_k(int nx, int ny, int ns, int ntx, int nty, int kc, double alpha, double beta, double gamma,
+                  double* __restrict__ u, const double* __restrict__ ux,
+                  const double* __restrict__ uy, const double* __restrict__ uz)
+{
+    kg_ztile t;
+    if (!kg_ztile_get<TX, TY, 1, 1, false>(nx, ny, ns, ntx, nty, kc, t)) return;
+    const long long sz = (long long)nx * ny;
+    const int sy = nx;
+    long long o = kg_off3(t.i, t.j, t.k0, nx, sz);
+    double zm = uz[o - sz];
+    double zc = uz[o];
+#pragma unroll 4
+    for (int k = t.k0; k < t.k1; k++) {
+        const double zp = uz[o + sz];
+        kg_st(&u[o], alpha * (ux[o + 1] - ux[o - 1]) +
+                     beta * (uy[o + sy] - uy[o - sy]) +
+                     gamma * (zp - zm));
+        zm = zc;
+        zc = zp;
+        o += sz;
+    }
+}
+
 // A lane owns points x, x+1 (x even) of row j and PZ consecutive planes; every
 // operand is a 16-byte load through the caches (ux as the aligned pairs at x-2, x, x+2; uy at rows
 // j-1, j+1; uz at planes k0-1 .. k0+PZ), all issued before the first use.
@@ -148,6 +178,43 @@ void divergence2_k(int nx, int ny, int ns, int ntx, int nty, double alpha, doubl
 // --------------------------------------------------------------------- uxx1
 // uxx1/uxx1.c:95-105, interior [2,n-1)^3, dth = 1/nx (:70)
 //
+// One point per lane, as for divergence.
+__global__ __launch_bounds__(TX * TY)
+void uxx1_k(int nx, int ny, int ns, int ntx, int nty, int kc, double c1, double c2, double dth,
+            const double* __restrict__ u0, double* __restrict__ u1,
+            const double* __restrict__ d1, const double* __restrict__ xx,
+            const double* __restrict__ xy, const double* __restrict__ xz)
+{
+    kg_ztile t;
+    if (!kg_ztile_get<TX, TY, 2, 1>(nx, ny, ns, ntx, nty, kc, t)) return;
+    const long long sz = (long long)nx * ny;
+    const int sy = nx;
+    long long o = kg_off3(t.i, t.j, t.k0, nx, sz);
+    // z-columns kept in registers: d1 at (i,j) and (i,j-1), planes k-1..k;
+    // xz at (i,j), planes k-2..k+1.
+    double d_c_m = d1[o - sz], d_y_m = d1[o - sy - sz];
+    double xz_m2 = xz[o - 2 * sz], xz_m1 = xz[o - sz], xz_c = xz[o];
+#pragma unroll 2
+    for (int k = t.k0; k < t.k1; k++) {
+        const double d_c = d1[o], d_y = d1[o - sy];
+        const double xz_p1 = xz[o + sz];
+        const double d = 0.25 * (d_c + d_y + d_c_m + d_y_m);
+        kg_st(&u1[o], u0[o] + (dth / d) * (
+            c1 * (xx[o] - xx[o - 1]) +
+            c2 * (xx[o + 1] - xx[o - 2]) +
+            c1 * (xy[o] - xy[o - sy]) +
+            c2 * (xy[o + sy] - xy[o - 2 * sy]) +
+            c1 * (xz_c - xz_m1) +
+            c2 * (xz_p1 - xz_m2)));
+        d_c_m = d_c;
+        d_y_m = d_y;
+        xz_m2 = xz_m1;
+        xz_m1 = xz_c;
+        xz_c = xz_p1;
+        o += sz;
+    }
+}
+
 // A lane owns points x, x+1 of row j and PZ planes; xx as the aligned pairs at x-2, x, x+2; xy at rows
 // j-2 .. j+1; d1 at rows j-1, j of planes k0-1 .. k0+PZ-1; xz at planes
 // k0-2 .. k0+PZ; u0 at the point.  ODD as for divergence: 95 us at 301x203x151
@@ -412,10 +479,28 @@ template <int V, bool RAG> using GsrbCfg = kgp::Cfg<V, (V == 2 ? KG_GSRB_W : 12)
 // 0.88-1.01, 0.90-0.98, 0.88-1.01; from 193 points on 0.98-1.21 (32 M), 0.95-1.09 (8 M),
 // 0.98-1.08 (4 M), but 0.86-0.98 (2 M and 1 M, where the fields stay cached; 1001 points a
 // row 1.1) and at 0.4 M points 1.0-1.15.
+// divergence and uxx1 (z-march against the direct form): divergence 0.71-0.77 at 5 to 9 points a
+// row, 0.85-0.98 at 33 to 41, at 47 to 55 0.94-0.99 from 10 M points on and 1.05-1.1 below, 1.0-1.05
+// at 63; 0.79-0.98 at 129 to 151, up to 191 0.88-0.97 from 10 M points on, 0.95-1.18 below.
+// uxx1 0.75-0.85 at 7 to 15 points a row; 0.82-0.93 at 21 from 4 M points on and at 27 to 41 from
+// 8 M on, 0.93-1.25 below; 0.89-0.97 at 51 to 61 from 12 M on, 1.05-1.22 below; 129 0.79-0.94, from
+// 131 on 1.0-1.35.
+// The direct form's lanes hold 4 planes: with 1 or 2 of them inside divergence 0.77-0.98 (3:
+// 0.97-1.07), uxx1 with 1 0.73-0.9 (2: 1.07-1.10).
 struct OneTake {
-    int nx;
+    int nx, ns;
     long long rows, n;   // of the grid, and its points
-    OneTake(int nx_, int ny, int ns) : nx(nx_), rows((long long)ny * ns), n(nx_ * rows) {}
+    OneTake(int nx_, int ny, int ns_) : nx(nx_), ns(ns_), rows((long long)ny * ns_), n(nx_ * rows) {}
+    bool divergence() const
+    {
+        const bool big = n >= 10000000;
+        return nx <= 44 || (big && nx <= 56) || (nx > 128 && nx <= (big ? 192 : 160)) || ns <= 4;
+    }
+    bool uxx1() const
+    {
+        return nx <= 16 || (nx <= 22 && n >= 3500000) || (nx <= 44 && n >= 7000000) ||
+               (nx <= 64 && n >= 10000000) || (nx > 128 && nx <= 130) || ns <= 4;
+    }
     bool laplacian() const { return nx <= 64 || (nx > 128 && nx <= 192 && n >= 4000000); }
     bool wave13pt() const { return (nx <= 64 && rows >= 6200) || (nx > 160 && nx <= 192); }
     bool lapgsrb() const { return nx <= 64; }
@@ -474,6 +559,24 @@ static int launch_plane(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
     return go(two, std::true_type{});
 }
 
+// A z-march kernel (one point per lane) over its grid.
+template <int LO, int HI, class... P, class... A>
+static int launch_zmarch(kg_ctx* ctx, const char* name, void (*kern)(int, int, int, int, int, int, P...),
+                         int nx, int ny, int ns, A... a)
+{
+    const kg_zgrid g0 = kg_zgrid_make(nx, ny, ns, LO, HI, TX, TY, KC);
+    // thinner chunks where 16 planes leave less than 4 workgroups per CU: divergence at
+    // 129x88x88 18.0 -> 12.4 us, uxx1 at 13x175x175 31 -> 21; above, uxx1 at 13x277x277 (1260
+    // workgroups) would go from 48 to 55, divergence at 47x291x292 from 33 to 36
+    const int kc = g0.blocks >= 4u * (unsigned)ctx->cus
+        ? KC : kg_fit_chunk(ctx, (long long)g0.ntx * g0.nty, ns - LO - HI, KC, 8, LO);
+    const kg_zgrid g = kg_zgrid_make(nx, ny, ns, LO, HI, TX, TY, kc);
+    kg_register_kernel(name, (const void*)kern);
+    if (int rc = kg_launch_begin(ctx, name)) return rc;
+    if (!g.empty) kg_launch(ctx, kern, dim3(g.blocks), dim3(TX, TY), 0, nx, ny, ns, g.ntx, g.nty, kc, a...);
+    return kg_launch_end(ctx);
+}
+
 }  // namespace
 
 // ============================================================ entry points
@@ -501,8 +604,11 @@ extern "C" int kg_divergence(kg_ctx* ctx, int nx, int ny, int ns, double alpha, 
     KG_REQUIRE(u != ux && u != uy && u != uz, "kg_divergence: output aliases an input");
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
-    const kg_zgrid g = kg_zgrid_make(nx, ny, ns, 1, 1, 128, DIV_ROWS, DIV_PZ);
     const bool even = nx % 2 == 0 && kg_aligned16(u, ux, uy, uz);
+    if (!even && OneTake(nx, ny, ns).divergence())
+        return launch_zmarch<1, 1>(ctx, "divergence", divergence_k, nx, ny, ns, alpha, beta, gamma, u, ux,
+                                   uy, uz);
+    const kg_zgrid g = kg_zgrid_make(nx, ny, ns, 1, 1, 128, DIV_ROWS, DIV_PZ);
     auto kern = even ? divergence2_k<false> : divergence2_k<true>;
     kg_register_kernel("divergence", (const void*)kern);
     if (int rc = kg_launch_begin(ctx, "divergence")) return rc;
@@ -558,9 +664,11 @@ extern "C" int kg_uxx1(kg_ctx* ctx, int nx, int ny, int ns, double c1, double c2
     const double dth = 1. / nx;   // uxx1/uxx1.c:70
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
+    const bool even = nx % 2 == 0 && kg_aligned16(u0, u1, d1, xx, xy, xz);
+    if (!even && OneTake(nx, ny, ns).uxx1())
+        return launch_zmarch<2, 1>(ctx, "uxx1", uxx1_k, nx, ny, ns, c1, c2, dth, u0, u1, d1, xx, xy, xz);
     // rows/planes from 2: the grid helper counts tiles from 0, one spare
     const kg_zgrid g = kg_zgrid_make(nx, ny, ns, 2, 1, 128, UXX_ROWS, UXX_PZ);
-    const bool even = nx % 2 == 0 && kg_aligned16(u0, u1, d1, xx, xy, xz);
     auto kern = even ? uxx1_2_k<false> : uxx1_2_k<true>;
     kg_register_kernel("uxx1", (const void*)kern);
     if (int rc = kg_launch_begin(ctx, "uxx1")) return rc;
