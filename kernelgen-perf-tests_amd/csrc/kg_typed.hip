@@ -91,12 +91,41 @@ int with_lanes(int nx, int vec, Fn&& f)
     return f(std::integral_constant<int, 64>{});
 }
 
+// Where one point per lane takes the place of 16-byte lanes for rows that are no multiple
+// of a lane or not aligned: rows of up to 64 points, which leave most of the lanes of a
+// 128 or 256 point tile idle, and what else the figures say.  Time of one point per lane
+// over that of 16-byte lanes, 33, 63 and 65 points a row, 32 M points: laplacian_f32 0.74,
+// 0.73, 1.39; wave13pt_f32 0.47, 0.54, 0.84 (8 M: 0.50, 0.58, 0.93; below some 6000 rows 1.04-1.12);
+// gaussblur3_f32 0.77, 0.76, 1.39; gaussblur3_f64 0.89, 0.86, 1.54 (4 M: 0.90, 0.93, 1.4; 2 M and up
+// to 20 points a row 1.0-1.2).
+// wave13pt_f32 with 65 to 125 and 257 to 320 points a row, which half fill their tiles: 0.84-0.96
+// and 0.88-0.94 at 32 M points, 0.92-1.0 and 1.14 at 16 M, 0.93-1.16 and 0.87-1.18 at 8 M.  gaussblur3 on small grids, where the column march's few
+// waves idle: FP32 0.4 M points 0.7-0.8, 1 M 0.8-1.07, 2 M 0.87-1.3; FP64 0.4 M 0.77-1.0, 1 M
+// 0.85-1.3; with 13 rows a plane and fewer 1.04-1.1.
+struct OneTake {
+    int nx, ny;
+    long long rows, n;   // of the grid, and its points
+    OneTake(int nx_, int ny_, int ns) : nx(nx_), ny(ny_), rows((long long)ny_ * ns), n(nx_ * rows) {}
+    bool laplacian_f32() const { return nx <= 64; }
+    bool wave13pt_f32() const
+    {
+        return (nx <= 64 && rows >= 6000) || (nx <= 125 && n >= 15000000) ||
+               (nx > 256 && nx <= 320 && n >= 24000000);
+    }
+    bool gaussblur3_f32() const { return nx <= 64 || (n < 1500000 && ny >= 16); }
+    bool gaussblur3_f64() const
+    {
+        return (nx > 20 && nx <= 64 && n >= 3000000) || (nx > 8 && n < 600000 && ny >= 16);
+    }
+};
+
 // Single-grid launch of op Op in storage type T with 16-byte lanes (VEC = VMAX),
 // in the ragged form where nx is no multiple of VMAX or a field not aligned;
-// rows shorter than a lane take one point per lane.
+// rows shorter than a lane, and with `one` those of the ragged form, take one point
+// per lane.
 template <template <class> class OpT, class T, int VMAX, int W, int D, int KC, int ORD = KG_ORD_TYPED,
           class Fill>
-static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, Fill fill)
+static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, bool one, Fill fill)
 {
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
@@ -121,7 +150,7 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
                       op);
         return kg_launch_end(ctx);
     };
-    if (nx < VMAX)
+    if (nx < VMAX || (one && !(nx % VMAX == 0 && al)))
         return go(std::integral_constant<int, 1>{}, std::false_type{}, std::integral_constant<int, 64>{});
     return with_lanes<sizeof(typename T::S) == 2>(nx, VMAX, [&](auto lanes) {
         std::integral_constant<int, VMAX> v;
@@ -131,7 +160,8 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
 
 // Per-plane stencils on the column march (kgp::colmarch_tile): W waves per
 // workgroup, each marching YC rows of one plane with a D-row prefetch; rows of
-// any length and alignment (the ragged form).  gaussblur3 at 512^3, levels rotated,
+// any length and alignment (the ragged form, or with `one` the plane engine with one
+// point per lane).  gaussblur3 at 512^3, levels rotated,
 // first ten launches: FP32 W=4/D=4/YC=16 214 us against 255-264 on the
 // direct row body (YC=8 214, 12 225, 32 238, 64 256: fewer workgroups leave
 // a tail); FP64 W=4/D=2/YC=16 418 us against 451-472.  Keeping each row's
@@ -158,8 +188,10 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
 #define KG_ORD_CM32 0
 #endif
 template <template <class> class OpT, class T, int VEC, int W, int D, int YC, int ORD, class Fill>
-static int launch_colmarch(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, Fill fill)
+static int launch_colmarch(kg_ctx* ctx, const char* name, int nx, int ny, int ns, bool al, bool one, Fill fill)
 {
+    if (one && !(nx % VEC == 0 && al))
+        return launch_typed<OpT, T, 1, 8, 2, 16>(ctx, name, nx, ny, ns, true, true, fill);
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims3(nx, ny, ns)) return rc;
     if (int rc = kg_check_plane_bytes((long long)nx * ny, (int)sizeof(typename T::S))) return rc;
@@ -465,7 +497,8 @@ extern "C" int kg_laplacian_f32(kg_ctx* ctx, int nx, int ny, int ns, float alpha
     KG_REQUIRE(w0 && w1, "kg_laplacian_f32: null buffer");
     KG_REQUIRE((const void*)w0 != (const void*)w1, "kg_laplacian_f32: w0 and w1 must be distinct");
     return launch_typed<LaplacianOp, kgp::F32, 4, KG_LF32_W, KG_LF32_D, KG_LF32_KC>(ctx, "laplacian_f32", nx, ny, ns,
-                                                            kg_aligned16(w0, w1), [&](auto& op) {
+                                                            kg_aligned16(w0, w1), OneTake(nx, ny, ns).laplacian_f32(),
+                                                            [&](auto& op) {
         op.src = w0;
         op.dst = w1;
         op.alpha = alpha;
@@ -479,7 +512,8 @@ extern "C" int kg_laplacian_bf16(kg_ctx* ctx, int nx, int ny, int ns, float alph
     KG_REQUIRE(w0 && w1, "kg_laplacian_bf16: null buffer");
     KG_REQUIRE((const void*)w0 != (const void*)w1, "kg_laplacian_bf16: w0 and w1 must be distinct");
     return launch_typed<LaplacianOp, kgp::BF16, KG_LBF_V, KG_LBF_W, KG_LBF_D, KG_LBF_KC>(ctx, "laplacian_bf16", nx, ny, ns,
-                                                             kg_aligned16(w0, w1), [&](auto& op) {
+                                                             kg_aligned16(w0, w1), false,
+                                                             [&](auto& op) {
         op.src = w0;
         op.dst = w1;
         op.alpha = alpha;
@@ -493,7 +527,8 @@ extern "C" int kg_wave13pt_f32(kg_ctx* ctx, int nx, int ny, int ns, float m0, fl
     KG_REQUIRE(w0 && w1 && w2, "kg_wave13pt_f32: null buffer");
     KG_REQUIRE(w2 != w0 && w2 != w1, "kg_wave13pt_f32: w2 aliases an input");
     return launch_typed<Wave13ptOp, kgp::F32, 4, KG_WF32_W, KG_WF32_D, KG_WF32_KC, KG_ORD_WF32>(ctx, "wave13pt_f32", nx, ny, ns,
-                                                            kg_aligned16(w0, w1, w2), [&](auto& op) {
+                                                            kg_aligned16(w0, w1, w2), OneTake(nx, ny, ns).wave13pt_f32(),
+                                                            [&](auto& op) {
         op.src = w1;
         op.side[0] = w0;
         op.dst = w2;
@@ -513,7 +548,8 @@ extern "C" int kg_wave13pt_bf16(kg_ctx* ctx, int nx, int ny, int ns, float m0, f
     // per workgroup, 2-plane prefetch; the measurements are listed with the
     // KG_WBF_* defaults above.
     return launch_typed<Wave13ptOp, kgp::BF16, KG_WBF_V, KG_WBF_W, KG_WBF_D, KG_WBF_KC, KG_ORD_WBF>(ctx, "wave13pt_bf16", nx, ny, ns,
-                                                             kg_aligned16(w0, w1, w2), [&](auto& op) {
+                                                             kg_aligned16(w0, w1, w2), false,
+                                                             [&](auto& op) {
         op.src = w1;
         op.side[0] = w0;
         op.dst = w2;
@@ -531,7 +567,8 @@ extern "C" int kg_gaussblur3_f64(kg_ctx* ctx, int nx, int ny, int ns, double s0,
     KG_REQUIRE(w0 != w1, "kg_gaussblur3_f64: w0 and w1 must be distinct");
     const double f = 1. / (s0 + 4 * (s1 + s2 + s4 + s8) + 8 * s5);   // gaussblur/gaussblur.c:65
     return launch_colmarch<Gaussblur3Op, kgp::F64, 2, KG_GB3_W64, KG_GB3_D64, KG_GB3_YC64, KG_ORD_CM64>(ctx, "gaussblur3_f64", nx, ny, ns,
-                                                             kg_aligned16(w0, w1), [&](auto& op) {
+                                                             kg_aligned16(w0, w1), OneTake(nx, ny, ns).gaussblur3_f64(),
+                                                             [&](auto& op) {
         op.src = w0;
         op.dst = w1;
         op.f = f;
@@ -551,7 +588,8 @@ extern "C" int kg_gaussblur3_f32(kg_ctx* ctx, int nx, int ny, int ns, float s0, 
     KG_REQUIRE(w0 != w1, "kg_gaussblur3_f32: w0 and w1 must be distinct");
     const float f = 1.f / (s0 + 4 * (s1 + s2 + s4 + s8) + 8 * s5);
     return launch_colmarch<Gaussblur3Op, kgp::F32, 4, KG_GB3_W32, KG_GB3_D32, KG_GB3_YC32, KG_ORD_CM32>(ctx, "gaussblur3_f32", nx, ny, ns,
-                                                             kg_aligned16(w0, w1), [&](auto& op) {
+                                                             kg_aligned16(w0, w1), OneTake(nx, ny, ns).gaussblur3_f32(),
+                                                             [&](auto& op) {
         op.src = w0;
         op.dst = w1;
         op.f = f;

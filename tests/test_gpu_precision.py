@@ -345,3 +345,20 @@ def test_convert_lengths(gpu_ctx, kgmod, src, dst, off):
         assert b.download().tobytes() == fill.tobytes(), n
         a.free()
         b.free()
+
+
+@pytest.mark.parametrize("which,dtype,dims", [
+    ("laplacian", "f32", (21, 9, 7)), ("laplacian", "f32", (63, 30, 20)), ("laplacian", "f32", (65, 30, 20)),
+    ("wave13pt", "f32", (33, 75, 81)), ("wave13pt", "f32", (63, 80, 74)), ("wave13pt", "f32", (101, 400, 400)),
+    ("wave13pt", "f32", (259, 312, 300)),
+    ("gaussblur3", "f32", (63, 40, 9)), ("gaussblur3", "f32", (301, 16, 9)), ("gaussblur3", "f32", (301, 71, 71)),
+    ("gaussblur3", "f64", (33, 350, 270)), ("gaussblur3", "f64", (301, 16, 9)), ("gaussblur3", "f64", (201, 71, 43))])
+def test_typed_points_per_lane(gpu_ctx, oracle, which, dtype, dims):
+    """Odd rows on either side of the lines between one point per lane and
+    16-byte lanes: points a row, rows and points of the grid."""
+    fn = f"{which}_{dtype}"
+    ins, out, coefs, rot = _case(which, dtype, dims, 900 + dims[0])
+    got = _run_gpu(gpu_ctx, fn, dims, coefs, ins, out, 1, rot)
+    want = _run_oracle(oracle.lib, fn, dims, coefs, ins, out, 1, rot, f64 if dtype == "f64" else f32)
+    for g, w in zip(got, want):
+        assert g.tobytes() == w.tobytes()
