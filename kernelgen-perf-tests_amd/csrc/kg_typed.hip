@@ -71,21 +71,29 @@ using namespace kgops;
 #define KG_REQUIRE(cond, msg) \
     do { if (!(cond)) return kg_set_error(KG_ERR_INVALID, "%s", msg); } while (0)
 
-// f(lanes per row as a constant) for rows of nx points, vec per lane.  BF16 rows of
-// 64 lanes are 512 points wide; narrower rows take 32 or 16 lanes (two or four
-// rows per wave) where fewer lanes then lie past the row's end, 32 counted 5 %
-// and 16 20 % dearer (what they cost on rows they fit: at 512 points 31, 31 and
-// 35 us).  Laplacian / wave13pt with 64, 32 and 16 lanes: 201x199x203 24 / 31, 12
-// / 19, 16 / 21 us; 301x203x151 21 / 25, 18 / 25, 17 / 23; 256^3 27 / 40, 25 /
-// 26, 26 / 26.  FP32 and FP64 tiles are half and a quarter as wide and gained
-// nothing (FP32 201x199x203 15, 18, 22).
-template <bool FOLD, class Fn>
-int with_lanes(int nx, int vec, Fn&& f)
+// f(lanes per row as a constant) for rows of nx points, vec per lane, of a grid of n points.
+// BF16 rows of 64 lanes are 512 points wide; narrower rows take 32 or 16 lanes (two or four
+// rows per wave) where fewer lanes then lie past the row's end.  What a lane costs more
+// than one of 64: 5 % with 32; with 16 20 %, 35 % for laplacian (H = 1) on grids beyond the
+// caches (12 M points), where it then takes 16 lanes for no more than 56 points a row; 64
+// lanes that a row fills by 60 % and more cost 11 % less, as memory bounds them (laplacian on
+// those grids only).
+// Laplacian / wave13pt with 64, 32 and 16 lanes: 201x199x203 24 / 31, 12 / 19, 16 / 21 us; 288^3
+// 39 / 53, 41 / 62, 47 / 53; 384^3 66 / 100, 72 / 114, 86 / 110; 576x576x100 47 / 80, 39 / 69, 44 /
+// 62; 248x512x512 101 / 151, 82 / 119, 118 / 135; 128x500x500, of the time with 64 lanes, 1 / 1, 0.79
+// / 0.61, 1.09 / 0.56; 264x174x174 laplacian 16 with 64 and 14 with 16, 384x144x144 13.7 and 11.9.
+// FP32 and FP64 tiles are half and a quarter as wide and gained nothing (FP32 201x199x203
+// 15, 18, 22).
+template <bool FOLD, int H, class Fn>
+int with_lanes(int nx, long long n, int vec, Fn&& f)
 {
     if constexpr (FOLD) {
         auto lanes = [&](int lpr) { return (long long)((nx + lpr * vec - 1) / (lpr * vec)) * lpr; };
-        const long long t64 = lanes(64) * 100, t32 = lanes(32) * 105, t16 = lanes(16) * 120;
-        if (t16 < t32 && t16 < t64) return f(std::integral_constant<int, 16>{});
+        const bool big = H != 1 || n >= 12000000;
+        const long long t64 = lanes(64) * (big && 10LL * nx >= 6LL * vec * lanes(64) ? 89 : 100);
+        const long long t32 = lanes(32) * 105, t16 = lanes(16) * (H == 1 && big ? 135 : 120);
+        const bool no16 = H == 1 && big && nx > 56;
+        if (!no16 && t16 < t32 && t16 < t64) return f(std::integral_constant<int, 16>{});
         if (t32 < t64) return f(std::integral_constant<int, 32>{});
     }
     return f(std::integral_constant<int, 64>{});
@@ -152,7 +160,7 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
     };
     if (nx < VMAX || (one && !(nx % VMAX == 0 && al)))
         return go(std::integral_constant<int, 1>{}, std::false_type{}, std::integral_constant<int, 64>{});
-    return with_lanes<sizeof(typename T::S) == 2>(nx, VMAX, [&](auto lanes) {
+    return with_lanes<sizeof(typename T::S) == 2, Shape<OpT>::H>(nx, (long long)nx * ny * ns, VMAX, [&](auto lanes) {
         std::integral_constant<int, VMAX> v;
         return nx % VMAX == 0 && al ? go(v, std::false_type{}, lanes) : go(v, std::true_type{}, lanes);
     });

@@ -362,3 +362,16 @@ def test_typed_points_per_lane(gpu_ctx, oracle, which, dtype, dims):
     want = _run_oracle(oracle.lib, fn, dims, coefs, ins, out, 1, rot, f64 if dtype == "f64" else f32)
     for g, w in zip(got, want):
         assert g.tobytes() == w.tobytes()
+
+
+@pytest.mark.parametrize("which,dims", [("laplacian", (72, 480, 470)), ("laplacian", (56, 540, 530)), ("laplacian", (288, 210, 200)),
+                                        ("laplacian", (288, 20, 9)), ("laplacian", (384, 20, 9)),
+                                        ("wave13pt", (288, 20, 9)), ("wave13pt", (312, 20, 9)), ("laplacian", (576, 20, 9)),
+                                        ("wave13pt", (573, 20, 9))])
+def test_bf16_lanes_per_row(gpu_ctx, oracle, which, dims):
+    """Rows on either side of the lines between 64, 32 and 16 lanes a row."""
+    ins, out, coefs, rot = _case(which, "bf16", dims, 950 + dims[0])
+    got = _run_gpu(gpu_ctx, which + "_bf16", dims, coefs, ins, out, 1, rot)
+    want = _run_oracle(oracle.lib, which + "_bf16", dims, coefs, ins, out, 1, rot, f32)
+    for g, w in zip(got, want):
+        assert g.tobytes() == w.tobytes()
