@@ -755,6 +755,7 @@ struct HostGrid {
     kg_grid_spec spec;
     bool alive;
     int li, kc;            // tile shape: LPRS[li], planes per tile
+    bool tuned;            // the shape is its size class's, tuned or set
     long long sy, sz;      // pitches (elements)
     size_t level_bytes;
     long long step0;
@@ -908,10 +909,11 @@ int ensure_device_arrays(kg_batch* b, int ndesc, int nitems)
 }
 
 // Shape of grid g: the tuned one of its size class, else the default.
-void shape_of(const kg_batch* b, const HostGrid& g, int& li, int& kc)
+void shape_of(const kg_batch* b, HostGrid& g, int& li, int& kc)
 {
     auto it = b->tuned.find(size_class(g.spec));
-    if (it != b->tuned.end()) {
+    g.tuned = it != b->tuned.end();
+    if (g.tuned) {
         li = it->second.first;
         kc = it->second.second;
     } else {
@@ -940,9 +942,9 @@ double plane_cost(int kind, int li)
 }
 
 // Planes per tile of grid g under the batch's cap.
-int capped_kc(const kg_batch* b, const HostGrid& g, int cap)
+int capped_kc(const HostGrid& g, int cap)
 {
-    if (b->tuned.count(size_class(g.spec))) return g.kc;
+    if (g.tuned) return g.kc;
     return std::max(2, std::min(g.kc, (int)(cap / plane_cost(g.spec.kind, g.li))));
 }
 
@@ -954,19 +956,31 @@ double tile_start(const HostGrid& g)
     return KG_ITEM_PLANES + v.zlo + v.zhi;
 }
 
+// Caps to choose from; the first leaves every default as it is.
+constexpr int KG_CAPS[] = {160, 112, 80, 56, 40, 32, 24, 20, 16, 12, 8, 6, 4, 2};
+// From this many rounds of tiles in the default cut on it is kept unseen, as it is where
+// no grid would take the cap: the choice costs the host 14 passes over the grids, at
+// every change of them (1000 grids: 580 us for one grid's joining and leaving with
+// a step after each, 330 without; 4096: 2490 and 1220).  With 2 rounds a step of 40 FP64
+// grids up to 128^3 takes 83 us, with 4 or more 70; 60 FP32 grids of 64 to 128 points a
+// side 133, 120; 80 149, with 4 154, with 6 137; 9 rounds and more gain no step anything.
+constexpr int KG_CAP_ROUNDS = 6;
+
 int planes_cap(const kg_batch* b, const std::vector<int>& order)
 {
+    if (std::all_of(order.begin(), order.end(), [&](int gi) { return b->grids[gi].tuned; })) return KG_CAPS[0];
     double best = 0;
     int pick = 0;
-    for (int cap : {160, 112, 80, 56, 40, 32, 24, 20, 16, 12, 8, 6, 4, 2}) {
+    for (int cap : KG_CAPS) {
         long long items = 0;
         double cost = 0, longest = 0;
         for (int gi : order) {
             const HostGrid& g = b->grids[gi];
-            const int kc = capped_kc(b, g, cap);
+            const int kc = capped_kc(g, cap);
             const Cut c = cut_of(g, g.li, kc);
             if (!c.items()) continue;
             items += c.items();
+            if (cap == KG_CAPS[0] && items >= (long long)KG_CAP_ROUNDS * b->nwg) return cap;
             const double start = tile_start(g), plane = plane_cost(g.spec.kind, g.li);
             const int thick = g.li == ROW2 ? 1 : kc;
             cost += c.items() * start + plane * c.ntx * c.nty * c.planes;
@@ -979,7 +993,7 @@ int planes_cap(const kg_batch* b, const std::vector<int>& order)
             pick = cap;
         }
     }
-    return pick ? pick : 160;
+    return pick ? pick : KG_CAPS[0];
 }
 
 // Upload descriptors and the work list (largest grids' tiles first).  With
@@ -1020,7 +1034,7 @@ int build_work(kg_batch* b, int only_class = -1, int li_force = 0, int kc_force 
         const int cap = planes_cap(b, order);
         for (int gi : order) {
             HostGrid& g = b->grids[gi];
-            g.kc = descs[gi].kc = capped_kc(b, g, cap);
+            g.kc = descs[gi].kc = capped_kc(g, cap);
         }
     }
     std::vector<Item> items;
