@@ -1235,14 +1235,23 @@ static int level_copy(kg_batch* b, int id, int level, void* host, bool up)
     const size_t h = (size_t)g.spec.ny * g.spec.ns;
     hipStream_t st = kg_stream(b->ctx);
     const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
-    if (w == dp) {   // rows without padding: the level is dense
+    // Row by row where that is as good: a row alone (8 KB 15 us, 26 as a block), two on their
+    // way to the host (19 us against 24 with the kernel that packs them; up 21 against 16, three
+    // down 26 and 25), and rows long enough to be worth a transfer's start each (3 of 800 KB down
+    // 126 us against 150, up 85 and 100, 8 323 and 377, 199 and 207; 100 of 400 KB down 3.4 ms
+    // and 3.7, up 1.6 and 1.25, 3 of them up 58 us and 73; 100 of 280 KB down 1.9 ms and 1.5).
+    const bool dense = w == dp;   // rows without padding
+    const bool long_rows = w >= ((size_t)(up && h > 4 ? 512 : 384) << 10);
+    const bool few = h == 1 || (h == 2 && !up) || (long_rows && (!dense || h <= 8));
+    if (dense && !few) {
         void* lev = g.lev[level];
         KG_HIP(hipMemcpyAsync(up ? lev : host, up ? host : lev, w * h, kind, st));
         KG_HIP(hipStreamSynchronize(st));
         return KG_OK;
     }
-    if (int rc = rows_reserve(b, w * h)) return rc;
-    if (b->rows_cap < w) {   // no memory for even one row: row by row
+    if (!few)
+        if (int rc = rows_reserve(b, w * h)) return rc;
+    if (few || b->rows_cap < w) {   // or without memory for even one row
         KG_HIP(up ? hipMemcpy2DAsync(g.lev[level], dp, host, w, w, h, kind, st)
                   : hipMemcpy2DAsync(host, w, g.lev[level], dp, w, h, kind, st));
         KG_HIP(hipStreamSynchronize(st));

@@ -313,3 +313,18 @@ def test_batch_work_queue_lengths(gpu_ctx, batch, ns, kc):
     batch.step(3, graph=False)
     batch.step(4, graph=True)
     _check_all(gpu_ctx, batch, specs, ids, init, 7, f"{ns} planes by {kc}")
+
+
+@pytest.mark.parametrize("dtype,dims", [(F64, (17, 1, 1)), (F32, (1001, 1, 1)), (F64, (17, 2, 1)), (F64, (17, 3, 1)),
+                                        (F32, (17, 1, 2)), (F64, (16, 1, 1)), (F64, (16, 2, 1)), (F64, (49151, 3, 1)), (F64, (49153, 3, 2)),
+                                        (F64, (65537, 3, 2)), (F32, (131073, 3, 1)), (F32, (131072, 3, 1))])
+def test_batch_levels_of_few_or_long_rows(batch, dtype, dims):
+    """Levels that move as one row, row by row and as packed blocks."""
+    t = np.float64 if dtype == F64 else np.float32
+    rng = np.random.default_rng(6)
+    gid = batch.add("laplacian", dtype, dims, COEFS["laplacian"])
+    lv = [rng.uniform(-1, 1, dims[::-1]).astype(t) for _ in range(2)]
+    for level, a in enumerate(lv):
+        batch.upload(gid, level, a)
+    for level in (1, 0):
+        assert np.array_equal(batch.download(gid, level), lv[level])
