@@ -338,7 +338,10 @@ int kg_batch_fill(kg_batch* b, unsigned long long seed);
 /* The comparison path: n steps as one plain launch per grid and step (same
  * tile bodies and results as kg_batch_step). */
 int kg_batch_step_sequential(kg_batch* b, int nsteps);
-/* HBM reserved by the batch's arena and bytes held by live grids. */
+/* HBM reserved by the batch -- its arena and, once a level whose rows are padded
+ * has moved to or from the host, the block such levels move through (a level's dense
+ * size, at most 64 MiB; without memory for it rows move one by one) -- and bytes
+ * held by live grids. */
 int kg_batch_memory(kg_batch* b, size_t* reserved, size_t* in_use);
 /* Fills the levels of one grid like kg_batch_fill (asynchronous); both levels
  * of a jacobi2 grid get the same values throughout. */
@@ -351,7 +354,9 @@ int kg_batch_fill_grid(kg_batch* b, int id, unsigned long long seed);
  * one step per tick together (continuous batching: one persistent launch per
  * tick over every active job).  KG_SERVE_SEQUENTIAL runs one job at a time
  * with one plain launch per step, for comparison.  Initial data come from the
- * job's seed (kg_batch_fill_grid).  A jacobi2 job with tol > 0 stops early
+ * job's seed (kg_batch_fill_grid).  hbm_budget counts the jobs' levels alone: the
+ * batch reserves them in chunks of 1 GiB and, for jobs with out, up to 64 MiB more
+ * (kg_batch_memory).  A jacobi2 job with tol > 0 stops early
  * once max |w_new - w_old| < tol (checked every 10 steps). */
 enum { KG_SERVE_CONTINUOUS = 0, KG_SERVE_SEQUENTIAL = 1 };
 

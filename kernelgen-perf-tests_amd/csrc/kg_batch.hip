@@ -1159,7 +1159,14 @@ extern "C" int kg_batch_add(kg_batch* b, const kg_grid_spec* spec, int* id)
     g.level_bytes = (size_t)g.sz * spec->ns * es;
     g.step0 = b->steps;
     for (int l = 0; l < nlev_of(spec->kind); l++) {
-        if (int rc = b->arena.alloc(g.level_bytes, &g.lev[l])) {
+        int rc = b->arena.alloc(g.level_bytes, &g.lev[l]);
+        if (rc == KG_ERR_NOMEM && b->rows) {   // a grid needs the memory more than level_copy
+            KG_HIP(hipFree(b->rows));
+            b->rows = nullptr;
+            b->rows_cap = 0;
+            rc = b->arena.alloc(g.level_bytes, &g.lev[l]);
+        }
+        if (rc) {
             for (int q = 0; q < l; q++) b->arena.release(g.lev[q], g.level_bytes);
             return rc;
         }
@@ -1458,7 +1465,7 @@ extern "C" int kg_batch_memory(kg_batch* b, size_t* reserved, size_t* in_use)
     size_t used = 0;
     for (const auto& g : b->grids)
         if (g.alive) used += Arena::up(g.level_bytes) * nlev_of(g.spec.kind);
-    if (reserved) *reserved = b->arena.reserved;
+    if (reserved) *reserved = b->arena.reserved + b->rows_cap;
     if (in_use) *in_use = used;
     return KG_OK;
 }

@@ -328,3 +328,13 @@ def test_batch_levels_of_few_or_long_rows(batch, dtype, dims):
         batch.upload(gid, level, a)
     for level in (1, 0):
         assert np.array_equal(batch.download(gid, level), lv[level])
+
+
+def test_batch_memory_counts_the_block_levels_move_through(batch):
+    dims = (17, 33, 9)
+    gid = batch.add("laplacian", F64, dims, COEFS["laplacian"])
+    reserved, used = batch.memory()
+    batch.upload(gid, 0, np.zeros(dims[::-1]))
+    assert batch.memory() == (reserved + 17 * 33 * 9 * 8, used)
+    batch.download(gid, 0)
+    assert batch.memory() == (reserved + 17 * 33 * 9 * 8, used)
