@@ -422,8 +422,14 @@ static int convert_to(hipStream_t st, int dd, size_t n, const void* src, void* d
     if (n == 0) return KG_OK;
     auto go = [&](auto dt) {
         constexpr int DD = decltype(dt)::value;
-        const size_t blocks = (n + Convert<DS, DD>::BLOCK - 1) / Convert<DS, DD>::BLOCK;
-        hipLaunchKernelGGL((convert_k<DS, DD>), dim3((unsigned)blocks), dim3(256), 0, st, n, src, dst);
+        typedef Convert<DS, DD> C;
+        // a launch holds less than 2^32 work-items (2^34 elements at 4 to a lane)
+        constexpr size_t most = ((size_t)1 << 24) - 1;
+        for (size_t i = 0; i < n; i += most * C::BLOCK) {
+            const size_t m = std::min(n - i, most * C::BLOCK);
+            hipLaunchKernelGGL((convert_k<DS, DD>), dim3((unsigned)((m + C::BLOCK - 1) / C::BLOCK)), dim3(256),
+                               0, st, m, (const typename C::S*)src + i, (typename C::D*)dst + i);
+        }
     };
     if (dd == KG_F64) go(std::integral_constant<int, KG_F64>{});
     else if (dd == KG_F32) go(std::integral_constant<int, KG_F32>{});

@@ -375,3 +375,35 @@ def test_bf16_lanes_per_row(gpu_ctx, oracle, which, dims):
     want = _run_oracle(oracle.lib, which + "_bf16", dims, coefs, ins, out, 1, rot, f32)
     for g, w in zip(got, want):
         assert g.tobytes() == w.tobytes()
+
+
+def test_convert_past_one_launch(gpu_ctx, kgmod):
+    """2^34 elements and more: beyond the work-items of one launch."""
+    n = 2 ** 34 + 4099
+    try:
+        src = kgmod.DeviceArray(gpu_ctx, (n,), np.float64)
+    except kgmod.KGError:
+        pytest.skip("no memory for the source")
+    try:
+        dst = kgmod.DeviceArray(gpu_ctx, (n,), np.uint16)
+    except kgmod.KGError:
+        src.free()
+        pytest.skip("no memory for the result")
+    lib, ctx = gpu_ctx.lib, gpu_ctx.ptr
+    rng = np.random.default_rng(4)
+    pieces = {at: rng.uniform(-1, 1, 6000).astype(np.float32).astype(np.float64)
+              for at in (0, 2 ** 34 - 1024 - 3000, 2 ** 34 - 3000, n - 6000) if at + 6000 <= n}
+    for at, v in pieces.items():
+        kgmod._check(lib, lib.kg_h2d(ctx, src.ptr + 8 * at, v.ctypes.data, v.nbytes), "kg_h2d")
+    rc = lib.kg_convert(ctx, kgmod.BF16, dst.ptr, kgmod.F64, src.ptr, n)
+    got = {at: np.empty(6000, np.uint16) for at in pieces}
+    for at, g in got.items():
+        lib.kg_d2h(ctx, g.ctypes.data, dst.ptr + 2 * at, g.nbytes)
+    back = {at: np.empty(6000) for at in pieces}       # the pieces may overlap
+    for at, v in back.items():
+        lib.kg_d2h(ctx, v.ctypes.data, src.ptr + 8 * at, v.nbytes)
+    src.free()
+    dst.free()
+    assert rc == 0
+    for at in pieces:
+        assert np.array_equal(got[at], to_bf16(back[at].astype(np.float32))), at
