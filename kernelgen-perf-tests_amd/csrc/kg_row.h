@@ -280,7 +280,7 @@ struct DView {
 template <class C>
 struct DGrid {
     int ntx;
-    unsigned blocks;
+    long long tile_rows;   // of ROWS * PY rows
     bool empty;
 };
 
@@ -290,9 +290,9 @@ static inline DGrid<C> make_dgrid(int nx, int ny, int lo, int hi)
     DGrid<C> g;
     const int nyi = ny - hi - lo, nxi = nx - hi - lo;
     g.empty = nxi <= 0 || nyi <= 0;
-    g.ntx = (nx + C::TXW - 1) / C::TXW;
+    g.ntx = (int)(((long long)nx + C::TXW - 1) / C::TXW);
     const int per = C::ROWS * C::PY;
-    g.blocks = g.empty ? 0u : (unsigned)g.ntx * (unsigned)((nyi + per - 1) / per);
+    g.tile_rows = g.empty ? 0 : ((long long)nyi + per - 1) / per;
     return g;
 }
 

@@ -246,8 +246,17 @@ static int launch_direct(kg_ctx* ctx, const char* name, int nx, int ny, const vo
                      : kgr::direct_kernel<DC, LO, HI, Op, ORD, true>;
     kg_register_kernel(name, (const void*)kern);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
-    if (!g.empty)
-        kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * DC::ROWS), 0, nx, ny, g.ntx, op);
+    // a launch holds less than 2^32 work-items: some 2^29 rows of up to 128 points, the tile
+    // rows past them go into further launches
+    const long long most = ((1LL << 32) - 1) / (64 * DC::ROWS) / g.ntx;
+    for (long long t = 0; t < g.tile_rows; t += most) {
+        const long long rows = std::min(g.tile_rows - t, most), y = t * DC::ROWS * DC::PY;
+        Op part = op;
+        part.src[0] += y * nx;
+        part.dst += y * nx;
+        kg_launch(ctx, kern, dim3((unsigned)(g.ntx * rows)), dim3(64 * DC::ROWS), 0, nx,
+                  (int)std::min<long long>(ny - y, rows * DC::ROWS * DC::PY + LO + HI), g.ntx, part);
+    }
     return kg_launch_end(ctx);
 }
 

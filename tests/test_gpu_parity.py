@@ -181,6 +181,43 @@ def test_gpu_fields_above_2GiB(gpu_ctx, oracle, name, dims):
         assert_bit_equal(got[role], want[role], f"{name} {dims} {role}")
 
 
+@pytest.mark.parametrize("name,nx", [("jacobi", 3), ("gaussblur", 5), ("gameoflife", 4)])
+def test_gpu_more_rows_than_a_launch_holds(gpu_ctx, oracle, kgmod, name, nx):
+    """Some 2^29 rows of one tile each; the field repeats every `period` rows."""
+    spec, period, ny = K.SPECS[name], 1024, 2 ** 29 + 1077
+    coefs, arrays = K.random_case(spec, (nx, period), 17)
+    src, dst = spec.arrays[:2]
+    try:
+        a = kgmod.DeviceArray(gpu_ctx, (ny, nx))
+    except kgmod.KGError:
+        pytest.skip("no memory for the first field")
+    try:
+        b = kgmod.DeviceArray(gpu_ctx, (ny, nx))
+    except kgmod.KGError:
+        a.free()
+        pytest.skip("no memory for the second field")
+    lib, ctx, row = gpu_ctx.lib, gpu_ctx.ptr, 8 * nx
+    block = np.asarray(arrays[src], np.float64).reshape(period, nx)
+    assert lib.kg_h2d(ctx, a.ptr, block.ctypes.data, block.nbytes) == 0
+    rows = period
+    while rows < ny:
+        n = min(rows, ny - rows)
+        assert lib.kg_d2d(ctx, a.ptr + rows * row, a.ptr, n * row) == 0
+        rows += n
+    gpu_ctx.call(name, nx, ny, *[coefs[c] for c in spec.coefs], a, b)
+    got = {y: np.empty((100, nx)) for y in (2, 2 ** 28, 2 ** 29 - 80, 2 ** 29 + 30, ny - 102)}
+    for y, g in got.items():
+        assert lib.kg_d2h(ctx, g.ctypes.data, b.ptr + y * row, g.nbytes) == 0
+    a.free()
+    b.free()
+    for y, g in got.items():
+        part = block[np.arange(y - 2, y + 102) % period]
+        state = {src: np.ascontiguousarray(part).ravel(), dst: np.zeros(104 * nx)}
+        oracle.step(spec, (nx, 104), coefs, state)
+        h = spec.lo
+        assert_bit_equal(g[:, h:nx - h], state[dst].reshape(104, nx)[2:-2, h:nx - h], f"row {y}")
+
+
 @pytest.mark.parametrize("dims", [(512, 520, 40), (512, 256, 200)])
 def test_gpu_lapgsrb_long_z_chunks(gpu_ctx, oracle, dims):
     """lapgsrb lengthens its z-chunks when the launch would exceed about two
