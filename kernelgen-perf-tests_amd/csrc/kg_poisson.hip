@@ -318,8 +318,11 @@ void pj_up_k(int N, int P, int Nc, int Pc, int ntx, int H, Coef k, const float* 
         } else if (adds && y - 2 >= max(m.yb, 1) && y - 2 < m.ye) {
             double* q = u64 + (long long)(y - 2) * N + m.x;
 #pragma unroll
-            for (int h = 0; h < V / 2; h++)
-                *(d2u*)(q + 2 * h) = w[h] + d2{(double)o.v[2 * h], (double)o.v[2 * h + 1]};
+            for (int h = 0; h < V / 2; h++) {
+                const d2 sum = w[h] + d2{(double)o.v[2 * h], (double)o.v[2 * h + 1]};
+                if (h == 0 && m.x == 0) q[1] = sum.y;          // column 0 is the caller's
+                else *(d2u*)(q + 2 * h) = sum;
+            }
         }
     };
     for (int y = first; y <= last; y += 3)

@@ -190,3 +190,23 @@ def test_poisson_one_correction(gpu_ctx, kgmod, n, cycles):
         np.testing.assert_array_equal(du.download().reshape(want.shape), want)
         df.free()
         du.free()
+
+
+@pytest.mark.parametrize("n", [2, 64, 128, 256, 1024])
+def test_poisson_leaves_the_boundary(gpu_ctx, kgmod, n):
+    """Not a bit of u's boundary changes: -0.0 stays, and values beside it."""
+    rng = np.random.default_rng(n)
+    u0 = np.zeros((n + 1, n + 1))
+    for edge in (np.s_[0], np.s_[-1], np.s_[:, 0], np.s_[:, -1]):
+        u0[edge] = np.where(rng.random(n + 1) < 0.5, -0.0, 5e-324)
+    df, du = gpu_ctx.array(rng.uniform(-1, 1, u0.shape)), gpu_ctx.array(u0)
+    try:
+        kgmod.poisson_solve(gpu_ctx, n, df, du, tol=1e-30, max_outer=2, vcycles=1)
+    except kgmod.KGError as err:
+        assert "relative residual" in str(err)
+    u = du.download().reshape(u0.shape)
+    df.free()
+    du.free()
+    for edge in (np.s_[0], np.s_[-1], np.s_[:, 0], np.s_[:, -1]):
+        assert np.array_equal(u[edge].view(np.uint64), u0[edge].view(np.uint64))
+    assert np.any(u[1:-1, 1:-1] != 0)
