@@ -29,12 +29,12 @@
 
 namespace {
 
-// Tile orders (kg_tile_order).  The marching passes deal single tile rows to the XCDs:
-// tile rows that share rows then run at the same time, which matters more than that
-// they share an L2, which their rows overflow (pj_up_k reads 1.4 times its input past
+// Tile orders (kg_tile_order).  In the marching passes each XCD takes a contiguous
+// eighth of the tile rows (1): tile rows that share rows then follow each other on
+// one XCD, although their rows overflow its L2 (pj_up_k reads 1.4 times its input past
 // L2).  8192^2: pj_up_k 186 us, pj_down_k 182 and, from 0, 117; in chunks of 2 tile
-// rows 204, 187 and 131, in hardware order 204, 189 and 133.  The FP64 residual takes
-// chunks of 2 (259 us; single rows 272, chunks of 4 or 8 257-263).
+// rows per XCD 204, 187 and 131, in hardware order 204, 189 and 133.  The FP64 residual
+// takes chunks of 2 (259 us; contiguous eighths 272, chunks of 4 or 8 257-263).
 #ifndef KG_ORD_PJ
 #define KG_ORD_PJ 1
 #endif

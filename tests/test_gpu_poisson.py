@@ -210,3 +210,10 @@ def test_poisson_leaves_the_boundary(gpu_ctx, kgmod, n):
     for edge in (np.s_[0], np.s_[-1], np.s_[:, 0], np.s_[:, -1]):
         assert np.array_equal(u[edge].view(np.uint64), u0[edge].view(np.uint64))
     assert np.any(u[1:-1, 1:-1] != 0)
+
+
+@pytest.mark.parametrize("cycles", [1, 2])
+def test_poisson_one_correction_16_rows_a_wave(gpu_ctx, kgmod, cycles):
+    """4096 cells: 16 rows per wave, the shape of the finest levels from here up
+    (256 to 2048 cells take 2, 4 and 8)."""
+    test_poisson_one_correction(gpu_ctx, kgmod, 4096, cycles)
