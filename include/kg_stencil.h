@@ -69,8 +69,9 @@ int kg_last_kernel_time(kg_ctx* ctx, double* seconds);
 int kg_timing_drain(kg_ctx* ctx, double* seconds, int cap, int* count);
 /* Name of the most recent launch's kernel and the registers it uses. */
 const char* kg_last_kernel_name(kg_ctx* ctx);
-/* Architected VGPRs per lane of the named entry point's main kernel (the
- * reference prints numRegs the same way: "<kernel> regcount = N"). */
+/* Architected VGPRs per lane of the named entry point's main kernel, in the form
+ * that its last launch in the process took (the reference prints numRegs the same
+ * way: "<kernel> regcount = N"). */
 int kg_kernel_regcount(kg_ctx* ctx, const char* kernel, int* vgprs);
 const char* kg_strerror(int status);
 const char* kg_last_error(void);

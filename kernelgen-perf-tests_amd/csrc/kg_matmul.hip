@@ -293,9 +293,10 @@ extern "C" int kg_matmul(kg_ctx* ctx, int nx, int ny, int ns, const double* A, c
         return kg_set_error(KG_ERR_INVALID, "kg_matmul: %lld tiles exceed one launch", tiles);
     // each wave's k range: a quarter of ny rounded up to whole MFMA steps
     const int kq = ((ny + KS - 1) / KS + 3) / 4 * 4;
-    kg_register_kernel("matmul_", (const void*)matmul_k);
-    if (int rc = kg_launch_begin(ctx, "matmul_")) return rc;
     const int edge = tile_edge(ctx, nx, ns);
+    kg_register_kernel("matmul_", edge == 4 ? (const void*)matmul_tiles_k<4>
+                                : edge == 2 ? (const void*)matmul_tiles_k<2> : (const void*)matmul_k);
+    if (int rc = kg_launch_begin(ctx, "matmul_")) return rc;
     if (edge == 4) launch_tiles<4>(ctx, nx, ny, ns, kq, A, B, C);
     else if (edge == 2) launch_tiles<2>(ctx, nx, ny, ns, kq, A, B, C);
     else if (tiles > 0)

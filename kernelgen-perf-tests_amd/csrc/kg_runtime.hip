@@ -45,7 +45,10 @@ void kg_register_kernel(const char* name, const void* func)
 {
     std::lock_guard<std::mutex> lk(g_reg_mu);
     for (int i = 0; i < g_nreg; i++)
-        if (strcmp(g_reg[i].name, name) == 0) return;
+        if (strcmp(g_reg[i].name, name) == 0) {
+            g_reg[i].func = func;   // the form launched last
+            return;
+        }
     if (g_nreg < 64) g_reg[g_nreg++] = {name, func};
 }
 

@@ -364,3 +364,18 @@ def test_gpu_matmul_tiles(gpu_ctx, kgmod, dims):
     assert np.isfinite(got.reshape(ns, nx)[:-1, :-1]).all()
     for x in (a, b, c, d):
         x.free()
+
+
+def test_gpu_regcount_is_the_launched_kernels(gpu_ctx):
+    """Each size's own kernel: a wave that holds a 64 x 64 tile of C takes more
+    registers than one with a 16 x 16 tile."""
+    def count(n):
+        bufs = [gpu_ctx.empty((n, n)) for _ in range(3)]
+        gpu_ctx.call("matmul", n, n, n, *bufs)
+        gpu_ctx.sync()
+        for b in bufs:
+            b.free()
+        return gpu_ctx.regcount("matmul_")
+    small, large = count(64), count(1536)
+    assert large > small > 0
+    assert count(64) == small
