@@ -937,6 +937,7 @@ void plane_kernel(int nx, int ny, int ns, int ntx, int nty, int kc, Op op)
 
 // Store the VEC results of a lane: one vector non-temporal store when all
 // points are interior, else per point.  Values are rounded to the storage type.
+// Rows start at any element (Cfg::RAG), so the vector is no more aligned than one.
 template <class T, int VEC>
 __device__ __forceinline__ void store(typename T::S* dst, long long ob, int x,
                                       const typename T::F (&r)[VEC], const bool (&xmask)[VEC])
@@ -953,7 +954,8 @@ __device__ __forceinline__ void store(typename T::S* dst, long long ob, int x,
         for (int v = 0; v < VEC; v++) s[v] = st_cvt<T>(r[v]);
         R raw;
         __builtin_memcpy(&raw, s, sizeof raw);
-        __builtin_nontemporal_store(raw, (gmem<R>*)(d + ob + x));
+        typedef R RU __attribute__((aligned(sizeof(S))));
+        __builtin_nontemporal_store(raw, (gmem<RU>*)(d + ob + x));
     } else {
 #pragma unroll
         for (int v = 0; v < VEC; v++)
