@@ -9,7 +9,8 @@
 //   * the work list is every (grid, tile) pair, tiles cut per grid with the
 //     tile shape of its size class (lanes per row 16/32/64 and planes per
 //     tile), largest grids first;
-//   * each resident workgroup pulls the next item from an atomic counter and
+//   * each resident workgroup takes the item of its own number first and further
+//     ones from atomic counters, one per XCD, and
 //     runs the plane engine's tile body for that grid's kind and type -- the
 //     same bodies as the single-grid kernels, so a grid's result is bit for
 //     bit what the single-grid entry point gives;
@@ -651,9 +652,9 @@ void launch_fill(hipStream_t st, void* p, int nx, int ny, int ns, long long sy, 
 
 // Rows of nx values between a padded level (row pitch sy) and a dense block,
 // one value per lane and turn; n = rows * nx values.  Moved by a strided host
-// copy instead, every row is a transfer of its own: 7 us a row (840 ms for the
+// copy instead, every row is a transfer of its own: 7 us a row (760 ms for the
 // 117,000 rows of 40 grids up to 128 points wide, 6 M values, that the packed
-// blocks bring to the host in 9 ms).  The rows are only touched once and the
+// blocks bring to the host in 3 ms).  The rows are only touched once and the
 // link to the host is a hundred times slower than HBM, so the simplest mapping
 // does.
 template <class S, bool PACK_ROWS>
@@ -935,7 +936,8 @@ constexpr int KG_ITEM_PLANES = 9;
 
 // What a plane of a tile costs against one of laplacian or wave13pt (0.54 us in a
 // tile of its own on an idle device): gaussblur3's 25 points 1.33 us in packed rows, 0.9
-// in the other shapes.
+// with 64 lanes a row.  ROW2 and COL, which gaussblur3 only has where a class is tuned or
+// its shape set, count as the others' planes: not measured, and never capped.
 double plane_cost(int kind, int li)
 {
     return kind != KG_KIND_GAUSSBLUR3 || li == ROW2 || li == COL ? 1.0 : li == PACK ? 2.5 : 1.7;

@@ -145,3 +145,10 @@ def test_life_u8_levels_past_the_caches(gpu_ctx, oracle, nx, ny):
     """Two levels of more than 256 MiB, whole and ragged rows."""
     cells = np.random.default_rng(nx).integers(0, 2, (ny, nx)).astype(np.uint8)
     np.testing.assert_array_equal(_gpu_steps(gpu_ctx, cells, 1), _oracle_steps(oracle, cells, 1))
+
+
+def test_life_u8_rows_past_the_vector_kernels_offsets(gpu_ctx, oracle):
+    """More than 2^24 cells a row: cell by cell, over many tiles side by side."""
+    nx, ny = 2 ** 24 + 37, 5
+    cells = np.random.default_rng(3).integers(0, 2, (ny, nx)).astype(np.uint8)
+    np.testing.assert_array_equal(_gpu_steps(gpu_ctx, cells, 1), _oracle_steps(oracle, cells, 1))

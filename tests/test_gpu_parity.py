@@ -379,3 +379,14 @@ def test_gpu_regcount_is_the_launched_kernels(gpu_ctx):
     small, large = count(64), count(1536)
     assert large > small > 0
     assert count(64) == small
+
+
+@pytest.mark.parametrize("nx,ns", [(16, 16), (512, 512), (1536, 1537)])
+def test_gpu_matmul_empty_sum(gpu_ctx, nx, ns):
+    """k = 0 in each tile size: C stays as it is."""
+    c = np.random.default_rng(nx).uniform(-1, 1, nx * ns)
+    a, b, dc = gpu_ctx.empty(1), gpu_ctx.empty(1), gpu_ctx.array(c)
+    gpu_ctx.call("matmul", nx, 0, ns, a, b, dc)
+    assert dc.download().tobytes() == c.tobytes()
+    for t in (a, b, dc):
+        t.free()

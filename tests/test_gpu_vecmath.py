@@ -173,3 +173,25 @@ def test_matvec_row_ends(gpu_ctx, oracle, ctype):
             for got in (_gpu(gpu_ctx, "matvec" + sfx, (nx, ny), [A, x], np.zeros(ny, ctype)),
                         _gpu_shifted(gpu_ctx, "matvec" + sfx, (nx, ny), [A, x], np.zeros(ny, ctype), 1)):
                 np.testing.assert_array_equal(got, want, err_msg=f"{nx} x {ny}")
+
+
+@pytest.mark.parametrize("name,code,np_t,nx,ny", [("matvec", 0, np.float64, 32768, 8200),
+                                                  ("matvec_f32", 1, np.float32, 65539, 8256)])
+def test_matvec_past_32_bit_offsets(gpu_ctx, kgmod, oracle, name, code, np_t, nx, ny):
+    """A of more than 2 GiB, which a lane cannot stream by 32-bit offsets: rows
+    in the first workgroup, across 2 GiB, and the last, against the oracle."""
+    a = kgmod.DeviceArray(gpu_ctx, (ny, nx), np_t)
+    gpu_ctx.call("fill_uniform", code, nx * ny, a, 11)
+    x = np.random.default_rng(9).uniform(-1, 1, nx).astype(np_t)
+    dx, dy = gpu_ctx.array(x), gpu_ctx.empty((ny,), np_t)
+    gpu_ctx.call(name, nx, ny, a, dx, dy)
+    y = dy.download()
+    for j in (0, 1, 127, 128, 8191, 8192, ny - 2):
+        rows = np.empty((2, nx), np_t)
+        assert gpu_ctx.lib.kg_d2h(gpu_ctx.ptr, rows.ctypes.data, a.ptr + j * nx * rows.itemsize, rows.nbytes) == 0
+        assert np.abs(rows).max() > 0.5
+        want = np.zeros(2, np_t)
+        getattr(oracle.lib, "oracle_" + name)(C.c_int(nx), C.c_int(2), vp(rows), vp(x), vp(want))
+        assert y[j:j + 2].tobytes() == want.tobytes(), j
+    for t in (a, dx, dy):
+        t.free()
