@@ -164,7 +164,7 @@ __device__ __forceinline__ T mv_sum(T acc, const T (&buf)[mv_chunk<T>()], const 
     return acc;
 }
 
-template <class T>
+template <class T, bool RAG>
 __global__ __launch_bounds__(64)
 void matvec_rows_k(int nx, int ny, const T* __restrict__ A, const T* __restrict__ x, T* __restrict__ y,
                    unsigned a_bytes)
@@ -172,9 +172,9 @@ void matvec_rows_k(int nx, int ny, const T* __restrict__ A, const T* __restrict_
     constexpr int CH = mv_chunk<T>();
     const int j = (int)(blockIdx.x * 64 + threadIdx.x);
     const __amdgpu_buffer_rsrc_t r = kgp::make_rsrc(A, a_bytes);
-    // the sum over whole 16-byte pieces, then the values of a last part of one (a
+    // RAG: the sum over whole 16-byte pieces, then the values of a last part of one (a
     // piece there could cross the end of A); loads past those feed nothing
-    const int whole = nx - nx % per16<T>();
+    const int whole = RAG ? nx - nx % per16<T>() : nx;
     // lanes past the last row read nothing (offset beyond the resource)
     const unsigned row = j < ny ? (unsigned)((long long)j * nx * (long long)sizeof(T)) : kgp::KG_OOB;
     T b0[CH], b1[CH];
@@ -195,7 +195,8 @@ void matvec_rows_k(int nx, int ny, const T* __restrict__ A, const T* __restrict_
         }
     }
     if (j < ny) {
-        for (int i = whole; i < nx; i++) acc = acc + A[(long long)j * nx + i] * x[i];
+        if constexpr (RAG)
+            for (int i = whole; i < nx; i++) acc = acc + A[(long long)j * nx + i] * x[i];
         y[j] = acc;
     }
 }
@@ -247,10 +248,13 @@ int matvec(kg_ctx* ctx, const char* who, const char* name, int nx, int ny, const
     if (y == A || y == x) return kg_set_error(KG_ERR_INVALID, "%s: y aliases an input", who);
     const long long a_bytes = (long long)nx * ny * (long long)sizeof(T);
     const bool rows = a_bytes < (1LL << 31);   // 32-bit offsets
-    kg_register_kernel(name, rows ? (const void*)matvec_rows_k<T> : (const void*)matvec_k<T>);
+    // rows of whole pieces without the code for a last part: 64 x 200000 FP32 12.1 us, 13.2
+    // with it
+    auto kern = nx % per16<T>() ? matvec_rows_k<T, true> : matvec_rows_k<T, false>;
+    kg_register_kernel(name, rows ? (const void*)kern : (const void*)matvec_k<T>);
     if (int rc = kg_launch_begin(ctx, name)) return rc;
     if (ny > 0 && rows && nx > 0)
-        kg_launch(ctx, matvec_rows_k<T>, dim3((ny + 63) / 64), dim3(64), 0, nx, ny, A, x, y,
+        kg_launch(ctx, kern, dim3((ny + 63) / 64), dim3(64), 0, nx, ny, A, x, y,
                   (unsigned)a_bytes);
     else if (ny > 0)
         kg_launch(ctx, matvec_k<T>, dim3((ny + MV_ROWS - 1) / MV_ROWS), dim3(MV_ROWS), 0, nx, ny, A,
