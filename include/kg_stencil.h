@@ -57,9 +57,13 @@ int kg_d2d(kg_ctx* ctx, void* dst, const void* src, size_t bytes);
 int kg_sync(kg_ctx* ctx);
 /* Per-launch device timing with HIP events (on by default): the newest
  * KG_TIMING_RING launches are kept.  A launch that queues behind the previous
- * one, still running, is timed from that one's end to its own (so it holds the
- * microsecond or so between them); a launch on an idle stream, or after work
- * that is not timed, from a start marker of its own. */
+ * one, still running, is timed from that one's end to its own, a launch on an idle
+ * stream, or after work that is not timed, from a start marker that is queued right
+ * before it.  Either way what passes on the stream before the kernel starts counts:
+ * about a microsecond while the stream is kept busy, but as long as the host takes to
+ * queue the kernel where the stream runs dry meanwhile.  A program that the system
+ * suspends there, or whose kernels end as fast as it launches them, finds that in single
+ * durations; medians over several launches do not. */
 #define KG_TIMING_RING 8192
 int kg_timing_enable(kg_ctx* ctx, int on);
 /* Duration in seconds of the most recent launch (waits for it). */

@@ -90,7 +90,9 @@ inline hipStream_t kg_stream(kg_ctx* ctx)
 // 32.8 us).  So a launch that queues behind the previous one, still running,
 // starts where that one stops (27.56 us reported for the 27.7 us kernel, 3.60
 // for the empty one's 3.5), and only a launch on an idle stream, where nothing
-// waits for it, records a start marker.
+// waits for it, records a start marker.  Should the previous launch end between
+// kg_launch_begin's look at it and the kernel's dispatch, that gap counts, as a gap
+// between a marker and its kernel does.
 int kg_launch_begin(kg_ctx* ctx, const char* name);
 int kg_launch_end(kg_ctx* ctx);
 
@@ -136,9 +138,9 @@ int kg_check_ctx(kg_ctx* ctx);
 int kg_check_dims3(int nx, int ny, int ns);
 int kg_check_dims2(int nx, int ny);
 int kg_check_plane_bytes(long long points, int elem_bytes);
-// True when every pointer is 16-byte aligned: the kernels' 16-byte lanes
-// (two doubles, four floats) are taken only then, 8-byte or narrower ones
-// otherwise.
+// True when every pointer is 16-byte aligned: together with rows of whole
+// 16-byte lanes (two doubles, four floats) kernels then take their aligned form,
+// otherwise the one for rows of any length and alignment or one point per lane.
 template <class... P>
 inline bool kg_aligned16(const P*... p)
 {
