@@ -1767,11 +1767,11 @@ extern "C" int kg_serve_run(kg_ctx* ctx, const kg_job* jobs, int njobs, size_t h
     // Convergence checks (jacobi2 jobs with tol > 0, every KG_SERVE_CHECK
     // steps) are issued after a tick and read after the next tick has been
     // queued: waiting for them then leaves the device busy with that tick.
-    double* check_res = nullptr;   // pinned: 5 statistics per job
+    double* check_res = nullptr;   // pinned, written by kernels: 5 statistics per job
     hipEvent_t checked = nullptr;
     bool checks_live = false;
     if (hipHostMalloc((void**)&check_res, sizeof(double) * 5 * (size_t)std::max(njobs, 1),
-                      hipHostMallocDefault) != hipSuccess ||
+                      hipHostMallocCoherent) != hipSuccess ||
         hipEventCreateWithFlags(&checked, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
         if (check_res) (void)hipHostFree(check_res);

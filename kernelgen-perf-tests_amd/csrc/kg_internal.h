@@ -40,7 +40,8 @@ struct kg_ctx {
 // A few doubles that a kernel writes straight to host memory arrive with the wait for
 // the stream; a copy of its own costs a launch, and one into unpinned memory a wait
 // more: kg_field_stats of 65536 points takes 33 us with the copy, 23
-// without, a Poisson solve of 512 cells 0.95 and 0.79 ms.
+// without, a Poisson solve of 512 cells 0.95 and 0.79 ms.  The memory is allocated as
+// coherent: what a kernel writes to it is there for any kind of wait, an event's included.
 constexpr int KG_HOST_RESULTS = 8;
 
 // Bytes of the context's kg_field_stats scratch.

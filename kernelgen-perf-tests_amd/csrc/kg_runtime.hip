@@ -160,7 +160,7 @@ extern "C" int kg_init(kg_ctx** out, int device)
         return kg_set_error(KG_ERR_NOMEM, "kg_init: statistics scratch allocation failed");
     }
     // without it results are copied from device memory
-    if (hipHostMalloc((void**)&c->host, KG_HOST_RESULTS * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+    if (hipHostMalloc((void**)&c->host, KG_HOST_RESULTS * sizeof(double), hipHostMallocCoherent) != hipSuccess) {
         (void)hipGetLastError();
         c->host = nullptr;
     }
