@@ -46,7 +46,7 @@ typedef double v2u __attribute__((ext_vector_type(2), aligned(8)));   // at any 
 #define KG_MM_KC 64
 #endif
 #ifndef KG_ORD_MM
-#define KG_ORD_MM 8            // 2048^3: 278 us, 284 with 2 or 4
+#define KG_ORD_MM 8            // 2048^3: 2 or 4 2 % slower
 #endif
 constexpr int KS = KG_MM_KS;   // waves per workgroup: the k range split KS ways
 constexpr int KC = KG_MM_KC;   // k values per chunk (KC/4 MFMA steps)
@@ -125,8 +125,9 @@ void matmul_k(int nx, int ny, int ns, int ntile_i, int kq, const double* __restr
 // load of A, and a lane's results are pairs of rows.  Rows and columns past the
 // matrix read its last ones and are not stored.
 //
-// 2048^3 278 us (61.8 TFLOP/s), bound by the matrix cores, against 694 with 16 x 16
-// tiles, whose operand reads bound it; 1500^3 160 us (429), 1024^3 46 (104).  T = 2
+// 2048^3 261 us (65.7 TFLOP/s), bound by the matrix cores, against 680 with 16 x 16
+// tiles, whose operand reads bound it; 1500^3 153 us (429), 1024^3 43 (91); launches queued
+// behind each other, 2048^3 waited for alone 280.  T = 2
 // reaches 44 TFLOP/s at 2048^3, bound by L1 (2 to 4 blocks in flight change nothing),
 // but gives a smaller product four times as many workgroups: 512 x 512 with k =
 // 2048 30 us (72 with T = 4, 48 with 16 x 16 tiles), 512^3 9.5 (24 and 15).

@@ -186,7 +186,7 @@ struct Cfg {
     // loads and stores VEC values from wherever they start; the last lane of a
     // row that is no multiple of VEC reads the row's last VEC values and shifts
     // them down when they are first used (shift_down), so no load leaves its
-    // row.  One value per lane, which such rows took before, against this: FP32
+    // row.  One value per lane, which narrow rows take (the launchers' OneTake), against this: FP32
     // at 333x257x131 laplacian 35 -> 25 us, wave13pt 59 -> 38, gaussblur3 42 -> 29;
     // BF16 34 -> 18 and 49 -> 27; FP64 laplacian 46 -> 40, gradient 91 -> 82, wave13pt
     // 65 -> 56, lapgsrb (with LDS for every neighbour then) 72 -> 50, gaussblur3 58

@@ -427,7 +427,7 @@ template <int V, bool RAG> using WaveCfg = kgp::Cfg<V, 12, 2, 0, 0, 2, 2, 3, 1, 
 // 129-137, 4 workgroups per CU 131-139); the same run timed the previous
 // shape (8-byte lanes, every neighbour from LDS, W=12/D=2) at 136 us and
 // 8-byte lanes in the x-shift mode at 149-178 us (twice the DPP moves per
-// point), so odd or unaligned grids keep the previous shape.  Back-to-back
+// point), so narrow odd or unaligned rows (OneTake) keep the previous shape.  Back-to-back
 // launches of this kernel slow down after about a dozen (101-107 us, then
 // 125-165 us, with the clock held down under the sustained load; laplacian
 // stays at 98-100 us), so shapes are compared on their first ten launches
