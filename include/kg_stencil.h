@@ -328,7 +328,8 @@ int kg_batch_info(kg_batch* b, double* points_per_step, double* bytes_per_step,
  * registers, planes_per_tile then counting the rows per wave), or
  * the flat body (lanes_per_row 0: points swept from cache, for small grids)
  * -- with 8/16/32/64 planes per tile, over reps launches on the batch's own
- * grids, and keeps the fastest.  Untuned classes take the direct row body
+ * grids, and keeps the one with which the whole batch's step should be fastest.
+ * Untuned classes take the direct row body
  * (jacobi2, life2), packed rows (rows up to 64 lanes) or 64 lanes per row, with
  * fewer planes per tile while the batch has too few tiles to fill the device.
  * Grid contents are preserved. */
