@@ -475,10 +475,12 @@ template <int V, bool RAG> using GsrbCfg = kgp::Cfg<V, (V == 2 ? KG_GSRB_W : 12)
 // M), 193 1.15, 1.10, 1.11; wave13pt up to 160 points 1.0-1.06 (32 M), 0.93-1.07 (2 M),
 // 161 to 191 0.94-1.01 and 0.89-0.97.
 // gradient, whose three results of 8-byte alignment are stored in 16-byte pieces, gains
-// the least from two: 105 points a row 1.05 (32 M points), 1.02 (8 M), 0.93 (2 M), 113 to 191
-// 0.88-1.01, 0.90-0.98, 0.88-1.01; from 193 points on 0.98-1.21 (32 M), 0.95-1.09 (8 M),
-// 0.98-1.08 (4 M), but 0.86-0.98 (2 M and 1 M, where the fields stay cached; 1001 points a
-// row 1.1, three planes 1.2) and at 0.4 M points 1.0-1.15.
+// the least from two, and loses where fields stay cached from call to call. Cold fields
+// of 32 M points: 105 points a row 1.05, 113 to 191 0.88-1.01, from 193 on 0.98-1.21; of 8 M
+// points 1.02, 0.90-0.98 and 0.95-1.06 up to 500 points a row, 1.0-1.1 above; of 2 M 0.93, 0.88-1.01,
+// 0.87-0.98. The same fields call after call: 97 to 105 points a row 0.88-0.91 (8 to 16 M points),
+// 193 to 351 0.80-0.93, 383 to 501 0.93-0.97, from 511 on 0.91-1.03. Three planes 1.2, 0.4 M points
+// 1.0-1.15.
 // divergence and uxx1 (z-march against the direct form): divergence 0.71-0.77 at 5 to 9 points a
 // row, 0.85-0.98 at 33 to 41, at 47 to 55 0.94-0.99 from 10 M points on and 1.05-1.1 below, 1.0-1.05
 // at 63; 0.79-0.98 at 129 to 151, up to 191 0.88-0.97 from 10 M points on, 0.95-1.18 below.
@@ -506,8 +508,8 @@ struct OneTake {
     bool lapgsrb() const { return nx <= 64; }
     bool gradient() const
     {
-        return (nx <= 64 && rows >= 9000) || (nx >= 110 && nx <= 192 && n >= 600000) ||
-               (nx >= 100 && nx < 800 && ns >= 16 && n >= 600000 && n < 3000000);
+        return (nx <= 64 && rows >= 9000) || (nx >= 110 && nx <= 192 && n >= 20000000) ||
+               (nx >= (n < 3000000 ? 100 : 106) && nx < 500 && ns >= 16 && n >= 600000 && n < 20000000);
     }
 };
 
