@@ -229,14 +229,44 @@ using J9D = kgr::DCfg<KG_J9_PY, KG_J9_ROWS, 1>;
 using JacD = kgr::DCfg<KG_JAC_PY, KG_J9_ROWS, 1>;
 using G25D = kgr::DCfg<KG_G25_PY, KG_G25_ROWS, 2>;
 
+// The row engine with one point per lane, 256 points by 64 rows (32 for H = 2) a tile.
+//                                 VEC W  H  NF LL LR ZL ZR D  NAUX YC
+using J9Row = kgr::Cfg<1, 4, 1, 1, 1, 1, 0, 0, 2, 0, 64>;
+using G25Row = kgr::Cfg<1, 4, 2, 1, 2, 2, 0, 0, 2, 0, 32>;
+
+// Rows of 129 to 192 points need two of the direct march's 128 point tiles and fill them
+// no better than the row engine's one of 256: on large grids, which memory and not the
+// latency of a march bounds, that engine is the faster (odd nx or fields off 16 bytes).
+// Its time over the direct march's: gameoflife 32 M points, 129 to 161 a row 0.87-0.89, 193
+// 0.95, 205 1.10; 64 M 0.81-0.85 and 0.91; 16 M 0.98-1.05. jacobi and gaussblur 64 M points,
+// 129 to 161 a row 0.90-0.97, 171 0.99, 191 1.0; 32 M 0.93-1.03.
+static bool row_engine(bool life, int nx, int ny)
+{
+    const long long n = (long long)nx * ny;
+    return nx > 128 && (life ? nx <= 200 && n >= 24000000 : nx <= 168 && n >= 40000000);
+}
+
 // Single-field stencils on the direct march: its aligned form when nx is even and
-// both fields are 16-byte aligned, else the form for any row length.
-template <class DC, template <class> class OpT, int LO, int HI, int ORD, class Fill>
+// both fields are 16-byte aligned, else the form for any row length or, with `row`, the
+// row engine.
+template <class DC, class RC, template <class> class OpT, int LO, int HI, int ORD, class Fill>
 static int launch_direct(kg_ctx* ctx, const char* name, int nx, int ny, const void* in,
-                         const void* out, Fill fill)
+                         const void* out, bool row, Fill fill)
 {
     if (int rc = kg_check_ctx(ctx)) return rc;
     if (int rc = kg_check_dims2(nx, ny)) return rc;
+    if (row && (nx % 2 != 0 || !kg_aligned16(in, out))) {
+        using Op = OpT<RC>;
+        Op op{};
+        fill(op);
+        const kgr::Grid g = kgr::make_grid<RC>(nx, ny, LO, HI);
+        auto kern = kgr::row_kernel<RC, LO, HI, Op, 1>;
+        kg_register_kernel(name, (const void*)kern);
+        if (int rc = kg_launch_begin(ctx, name)) return rc;
+        if (!g.empty)
+            kg_launch(ctx, kern, dim3(g.blocks), dim3(64 * RC::W), 0, nx, ny, g.ntx, op);
+        return kg_launch_end(ctx);
+    }
     using Op = OpT<DC>;
     Op op{};
     fill(op);
@@ -270,7 +300,8 @@ extern "C" int kg_jacobi(kg_ctx* ctx, int nx, int ny, double c0, double c1, doub
 {
     KG_REQUIRE(w0 && w1, "kg_jacobi: null buffer");
     KG_REQUIRE(w0 != w1, "kg_jacobi: w0 and w1 must be distinct");
-    return launch_direct<JacD, JacobiOp, 1, 1, KG_ORD_JAC>(ctx, "jacobi_", nx, ny, w0, w1, [&](auto& op) {
+    return launch_direct<JacD, J9Row, JacobiOp, 1, 1, KG_ORD_JAC>(ctx, "jacobi_", nx, ny, w0, w1,
+                                                                 row_engine(false, nx, ny), [&](auto& op) {
         op.src[0] = w0;
         op.dst = w1;
         op.c0 = c0;
@@ -285,7 +316,8 @@ extern "C" int kg_gaussblur(kg_ctx* ctx, int nx, int ny, double s0, double s1, d
     KG_REQUIRE(w0 && w1, "kg_gaussblur: null buffer");
     KG_REQUIRE(w0 != w1, "kg_gaussblur: w0 and w1 must be distinct");
     const double f = 1. / (s0 + 4 * (s1 + s2 + s4 + s8) + 8 * s5);   // gaussblur/gaussblur.c:65
-    return launch_direct<G25D, GaussblurOp, 2, 2, KG_ORD_GAUSS>(ctx, "gaussblur", nx, ny, w0, w1, [&](auto& op) {
+    return launch_direct<G25D, G25Row, GaussblurOp, 2, 2, KG_ORD_GAUSS>(ctx, "gaussblur", nx, ny, w0, w1,
+                                                                      row_engine(false, nx, ny), [&](auto& op) {
         op.src[0] = w0;
         op.dst = w1;
         op.f = f;
@@ -302,7 +334,8 @@ extern "C" int kg_gameoflife(kg_ctx* ctx, int nx, int ny, const double* u0, doub
 {
     KG_REQUIRE(u0 && u1, "kg_gameoflife: null buffer");
     KG_REQUIRE(u0 != u1, "kg_gameoflife: u0 and u1 must be distinct");
-    return launch_direct<J9D, GameoflifeOp, 1, 1, KG_ORD_LIFE>(ctx, "gameoflife", nx, ny, u0, u1, [&](auto& op) {
+    return launch_direct<J9D, J9Row, GameoflifeOp, 1, 1, KG_ORD_LIFE>(ctx, "gameoflife", nx, ny, u0, u1,
+                                                                   row_engine(true, nx, ny), [&](auto& op) {
         op.src[0] = u0;
         op.dst = u1;
     });

@@ -181,6 +181,20 @@ def test_gpu_fields_above_2GiB(gpu_ctx, oracle, name, dims):
         assert_bit_equal(got[role], want[role], f"{name} {dims} {role}")
 
 
+@pytest.mark.parametrize("name,dims", [("gameoflife", (129, 186100)), ("gameoflife", (199, 120700)),
+                                       ("jacobi", (129, 310100)), ("jacobi", (167, 239600)),
+                                       ("gaussblur", (130, 307800)), ("gaussblur", (167, 239600))])
+def test_gpu_large_grids_of_half_filled_rows(gpu_ctx, oracle, name, dims):
+    """Odd rows, and even ones off 16 bytes, of 129 to 200 points on grids large
+    enough for the row engine's tiles."""
+    spec = K.SPECS[name]
+    coefs, arrays = K.random_case(spec, dims, 60 + dims[0])
+    want = oracle.run(spec, dims, coefs, arrays, 1)
+    got = K.GpuBackend(gpu_ctx).run(spec, dims, coefs, arrays, 1, offset=1)
+    for role in want:
+        assert_bit_equal(got[role], want[role], f"{name} {dims} {role}")
+
+
 @pytest.mark.parametrize("name,nx", [("jacobi", 3), ("gaussblur", 5), ("gameoflife", 4)])
 def test_gpu_more_rows_than_a_launch_holds(gpu_ctx, oracle, kgmod, name, nx):
     """Some 2^29 rows of one tile each; the field repeats every `period` rows."""
