@@ -71,45 +71,48 @@ using namespace kgops;
 #define KG_REQUIRE(cond, msg) \
     do { if (!(cond)) return kg_set_error(KG_ERR_INVALID, "%s", msg); } while (0)
 
-// f(lanes per row as a constant) for rows of nx points, vec per lane, of a grid of n points.
-// BF16 rows of 64 lanes are 512 points wide; narrower rows take 32 or 16 lanes (two or four
-// rows per wave) where fewer lanes then lie past the row's end.  What a lane costs more
-// than one of 64: 5 % with 32; with 16 20 %, 35 % for laplacian (H = 1) on grids beyond the
-// caches (12 M points), where it then takes 16 lanes for no more than 56 points a row; 64
-// lanes that a row fills by 60 % and more cost 11 % less, as memory bounds them (laplacian on
-// those grids only).
+// f(lanes per row as a constant) for rows of nx points, vec per lane, of a grid of n points;
+// whole: not the ragged form.  BF16 rows of 64 lanes are 512 points wide; narrower rows
+// take 32 or 16 lanes (two or four rows per wave) where fewer lanes then lie past the row's
+// end.  A lane of 32 costs 5 % more than one of 64, one of 16 20 %.  Memory bounds
+// whole rows sooner: 64 lanes that a row fills by 60 % and more cost 11 % less, and for
+// laplacian (H = 1) on grids beyond the caches (12 M points) one of 16 35 % more, which it
+// then takes for no more than 56 points a row.
 // Laplacian / wave13pt with 64, 32 and 16 lanes: 201x199x203 24 / 31, 12 / 19, 16 / 21 us; 288^3
 // 39 / 53, 41 / 62, 47 / 53; 384^3 66 / 100, 72 / 114, 86 / 110; 576x576x100 47 / 80, 39 / 69, 44 /
 // 62; 248x512x512 101 / 151, 82 / 119, 118 / 135; 128x500x500, of the time with 64 lanes, 1 / 1, 0.79
-// / 0.61, 1.09 / 0.56; 264x174x174 laplacian 16 with 64 and 14 with 16, 384x144x144 13.7 and 11.9.
+// / 0.61, 1.09 / 0.56; 264x174x174 laplacian 16 with 64 and 14 with 16, 384x144x144 13.7 and 11.9;
+// ragged 65x701x702 100 with 32 and 73 with 16, 257x352x353 65 with 64 and 53 with 16.
 // FP32 and FP64 tiles are half and a quarter as wide and gained nothing (FP32 201x199x203
 // 15, 18, 22).
 template <bool FOLD, int H, class Fn>
-int with_lanes(int nx, long long n, int vec, Fn&& f)
+int with_lanes(int nx, long long n, int vec, bool whole, Fn&& f)
 {
     if constexpr (FOLD) {
         auto lanes = [&](int lpr) { return (long long)((nx + lpr * vec - 1) / (lpr * vec)) * lpr; };
-        const bool big = H != 1 || n >= 12000000;
-        const long long t64 = lanes(64) * (big && 10LL * nx >= 6LL * vec * lanes(64) ? 89 : 100);
-        const long long t32 = lanes(32) * 105, t16 = lanes(16) * (H == 1 && big ? 135 : 120);
-        const bool no16 = H == 1 && big && nx > 56;
+        const bool bound = whole && (H != 1 || n >= 12000000);
+        const long long t64 = lanes(64) * (bound && 10LL * nx >= 6LL * vec * lanes(64) ? 89 : 100);
+        const long long t32 = lanes(32) * 105, t16 = lanes(16) * (H == 1 && bound ? 135 : 120);
+        const bool no16 = H == 1 && bound && nx > 56;
         if (!no16 && t16 < t32 && t16 < t64) return f(std::integral_constant<int, 16>{});
         if (t32 < t64) return f(std::integral_constant<int, 32>{});
     }
     return f(std::integral_constant<int, 64>{});
 }
 
-// Where one point per lane takes the place of 16-byte lanes for rows that are no multiple
-// of a lane or not aligned: rows of up to 64 points, which leave most of the lanes of a
-// 128 or 256 point tile idle, and what else the figures say.  Time of one point per lane
-// over that of 16-byte lanes, 33, 63 and 65 points a row, 32 M points: laplacian_f32 0.74,
-// 0.73, 1.39; wave13pt_f32 0.47, 0.54, 0.84 (8 M: 0.50, 0.58, 0.93; below some 6000 rows 1.04-1.12);
-// gaussblur3_f32 0.77, 0.76, 1.39; gaussblur3_f64 0.89, 0.86, 1.54 (4 M: 0.90, 0.93, 1.4; 2 M and up
-// to 20 points a row 1.0-1.2).
+// Where one point per lane takes the place of 16-byte lanes for rows that are no multiple of a lane
+// or not aligned: rows of up to 64 points, which leave most of the lanes of a 128 or 256 point tile
+// idle, and what else the figures say.  Time of one point per lane over that of 16-byte lanes, 33,
+// 63 and 65 points a row, 32 M points: laplacian_f32 0.74, 0.73, 1.39; wave13pt_f32 0.47, 0.54,
+// 0.84 (8 M: 0.50, 0.58, 0.93; below some 6000 rows 1.04-1.12); gaussblur3_f32 0.77, 0.76, 1.39;
+// gaussblur3_f64 0.89, 0.86, 1.54 (4 M: 0.90, 0.93, 1.4; 2 M and up to 20 points a row 1.0-1.2).
 // wave13pt_f32 with 65 to 125 and 257 to 320 points a row, which half fill their tiles: 0.84-0.96
-// and 0.88-0.94 at 32 M points, 0.92-1.0 and 1.14 at 16 M, 0.93-1.16 and 0.87-1.18 at 8 M.  gaussblur3 on small grids, where the column march's few
-// waves idle: FP32 0.4 M points 0.7-0.8, 1 M 0.8-1.07, 2 M 0.87-1.3; FP64 0.4 M 0.77-1.0, 1 M
-// 0.85-1.3; with 13 rows a plane and fewer 1.04-1.1.
+// and 0.88-0.94 at 32 M points, 0.92-1.0 and 1.14 at 16 M, 0.93-1.16 and 0.87-1.18 at 8 M.
+// gaussblur3 on small grids, where the column march's few waves idle: FP32 0.4 M points 0.7-0.8, 1
+// M 0.8-1.07, 2 M 0.87-1.3; FP64 0.4 M 0.77-1.0, 1 M 0.85-1.3; with 13 rows a plane and fewer
+// 1.04-1.1.  laplacian_bf16, whose narrow rows fold (with_lanes), only with 53, 55, 59, 61 and 63
+// points a row: 0.83-0.94 (16 to 64 M points), 0.90-1.01 (8 M); 1.0 at 51, 1.06 with one point past
+// the lanes (57), 1.01-1.16 for 54, 58 and 60, 0.94-1.17 for 62, 1.01-1.84 elsewhere.
 struct OneTake {
     int nx, ny;
     long long rows, n;   // of the grid, and its points
@@ -120,6 +123,7 @@ struct OneTake {
         return (nx <= 64 && rows >= 6000) || (nx <= 125 && n >= 15000000) ||
                (nx > 256 && nx <= 320 && n >= 24000000);
     }
+    bool laplacian_bf16() const { return nx > 52 && nx < 64 && nx % 2 && nx % 8 != 1 && n >= 6000000; }
     bool gaussblur3_f32() const { return nx <= 64 || (n < 1500000 && ny >= 16); }
     bool gaussblur3_f64() const
     {
@@ -160,9 +164,11 @@ static int launch_typed(kg_ctx* ctx, const char* name, int nx, int ny, int ns, b
     };
     if (nx < VMAX || (one && !(nx % VMAX == 0 && al)))
         return go(std::integral_constant<int, 1>{}, std::false_type{}, std::integral_constant<int, 64>{});
-    return with_lanes<sizeof(typename T::S) == 2, Shape<OpT>::H>(nx, (long long)nx * ny * ns, VMAX, [&](auto lanes) {
+    const bool whole = nx % VMAX == 0 && al;
+    const long long n = (long long)nx * ny * ns;
+    return with_lanes<sizeof(typename T::S) == 2, Shape<OpT>::H>(nx, n, VMAX, whole, [&](auto lanes) {
         std::integral_constant<int, VMAX> v;
-        return nx % VMAX == 0 && al ? go(v, std::false_type{}, lanes) : go(v, std::true_type{}, lanes);
+        return whole ? go(v, std::false_type{}, lanes) : go(v, std::true_type{}, lanes);
     });
 }
 
@@ -526,7 +532,7 @@ extern "C" int kg_laplacian_bf16(kg_ctx* ctx, int nx, int ny, int ns, float alph
     KG_REQUIRE(w0 && w1, "kg_laplacian_bf16: null buffer");
     KG_REQUIRE((const void*)w0 != (const void*)w1, "kg_laplacian_bf16: w0 and w1 must be distinct");
     return launch_typed<LaplacianOp, kgp::BF16, KG_LBF_V, KG_LBF_W, KG_LBF_D, KG_LBF_KC>(ctx, "laplacian_bf16", nx, ny, ns,
-                                                             kg_aligned16(w0, w1), false,
+                                                             kg_aligned16(w0, w1), OneTake(nx, ny, ns).laplacian_bf16(),
                                                              [&](auto& op) {
         op.src = w0;
         op.dst = w1;

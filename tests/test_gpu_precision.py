@@ -364,7 +364,9 @@ def test_typed_points_per_lane(gpu_ctx, oracle, which, dtype, dims):
         assert g.tobytes() == w.tobytes()
 
 
-@pytest.mark.parametrize("which,dims", [("laplacian", (72, 480, 470)), ("laplacian", (56, 540, 530)), ("laplacian", (288, 210, 200)),
+@pytest.mark.parametrize("which,dims", [("laplacian", (72, 480, 470)), ("laplacian", (56, 540, 530)),
+                                        ("laplacian", (55, 335, 335)), ("laplacian", (57, 330, 330)),
+                                        ("laplacian", (288, 210, 200)), ("laplacian", (257, 220, 220)),
                                         ("laplacian", (288, 20, 9)), ("laplacian", (384, 20, 9)),
                                         ("wave13pt", (288, 20, 9)), ("wave13pt", (312, 20, 9)), ("laplacian", (576, 20, 9)),
                                         ("wave13pt", (573, 20, 9))])
