@@ -2,7 +2,8 @@
 // gameoflife, whispering (the reference runs them at nx x (ny*ns), e.g.
 // 512 x 65536).  The single-field stencils (jacobi, gaussblur, gameoflife)
 // run on the direct row march of kg_row.h (every neighbour loaded through
-// the caches, a few output rows per lane); whispering, with five fields and
+// the caches, a few output rows per lane; some large grids of ragged rows on the
+// row-staged engine, row_engine below); whispering, with five fields and
 // three side streams, on the row-staged engine: x-neighbours and diagonal
 // neighbours from LDS rows, the lane's own column from registers, every load
 // prefetched a few rows ahead.  Arithmetic is in the reference's source order
