@@ -1419,8 +1419,13 @@ extern "C" int kg_batch_tune(kg_batch* b, int reps, int* classes_tuned)
     std::map<int, std::vector<Shape>> shapes;
     float empty = 0, total = 0;
     const int listed = b->nitems;
+    // one slow launch here would take the work of every shape for nothing
     b->nitems = 0;
     int rc = trial(empty);
+    for (int i = 0; i < 7 && !rc; i++) {
+        float ms = 0;
+        if (!(rc = trial(ms))) empty = std::min(empty, ms);
+    }
     b->nitems = listed;
     for (const auto& cls : classes) {
         float least = 1e30f;
