@@ -317,7 +317,8 @@ def test_batch_work_queue_lengths(gpu_ctx, batch, ns, kc):
 
 @pytest.mark.parametrize("dtype,dims", [(F64, (17, 1, 1)), (F32, (1001, 1, 1)), (F64, (17, 2, 1)), (F64, (17, 3, 1)),
                                         (F32, (17, 1, 2)), (F64, (16, 1, 1)), (F64, (16, 2, 1)), (F64, (49151, 3, 1)), (F64, (49153, 3, 2)),
-                                        (F64, (65537, 3, 2)), (F32, (131073, 3, 1)), (F32, (131072, 3, 1))])
+                                        (F64, (65537, 3, 2)), (F32, (131073, 3, 1)), (F32, (131072, 3, 1)),
+                                        (F64, (4096, 1, 1)), (F64, (98304, 3, 1)), (F32, (98304, 3, 3))])
 def test_batch_levels_of_few_or_long_rows(batch, dtype, dims):
     """Levels that move as one row, row by row and as packed blocks."""
     t = np.float64 if dtype == F64 else np.float32
