@@ -342,7 +342,7 @@ int kg_batch_set_shape(kg_batch* b, int id, int lanes_per_row, int planes_per_ti
  * boundary cells of (seed, grid, element), shared by the levels. */
 int kg_batch_fill(kg_batch* b, unsigned long long seed);
 /* The comparison path: n steps as one plain launch per grid and step (same
- * tile bodies and results as kg_batch_step). */
+ * tile bodies, shapes and results as kg_batch_step, for which the shapes are tuned). */
 int kg_batch_step_sequential(kg_batch* b, int nsteps);
 /* HBM reserved by the batch -- its arena and, once a level whose rows are padded
  * has moved to or from the host, the block such levels move through (a level's dense

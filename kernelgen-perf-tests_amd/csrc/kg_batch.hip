@@ -1247,11 +1247,12 @@ static int level_copy(kg_batch* b, int id, int level, void* host, bool up)
     // Row by row where that is as good.  Padded rows: one (8 KB 15 us, 26 as a block), two on their
     // way to the host (19 us against 24 with the kernel that packs them; up 21 against 16, three
     // down 26 and 25), and rows long enough to be worth a transfer's start each (3 of 800 KB down
-    // 126 us against 150, up 85 and 100, 8 323 and 377, 199 and 207; 100 of 400 KB down 3.4 ms
-    // and 3.7, up 1.6 and 1.25, 3 of them up 58 us and 73; 100 of 280 KB down 1.9 ms and 1.5).
-    // Rows without padding are a block already, and one transfer: one row of up to 16 KB
-    // (down 14 us against 23; 32 KB 14 and 11), two of them down (20 and 22), three to eight down of 0.5 to 1 MB (of 768 KB 126 us
-    // and 137, 8 of them 324 and 348; of 512 KB 95 and 90, of 1 MB 181 and 176; up equal).
+    // 126 us against 150, up 85 and 100, 8 323 and 377, 199 and 207; 100 of 400 KB down 3.4 ms and
+    // 3.7, up 1.6 and 1.25, 3 of them up 58 us and 73; 100 of 280 KB down 1.9 ms and 1.5). Rows
+    // without padding are a block already, and one transfer: one row of up to 16 KB (down 14 us
+    // against 23; 32 KB 14 and 11), two of them down (20 and 22), three to eight down of 0.5 to 1
+    // MB (of 768 KB 126 us and 137, 8 of them 324 and 348; of 512 KB 95 and 90, of 1 MB 181 and
+    // 176; up equal).
     const bool dense = w == dp;
     const bool long_rows = w >= ((size_t)(up && h > 4 ? 512 : 384) << 10);
     const bool few = dense ? (w * h <= 16384 && (h == 1 || (h == 2 && !up))) ||
